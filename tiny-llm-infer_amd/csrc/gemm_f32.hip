@@ -1,0 +1,183 @@
+// Matrix product of the float32 path: y[M,N] = x[M,K] . W[N,K]^T, everything float32, on the matrix cores' float32
+// instruction (v_mfma_f32_16x16x4_f32: float32 products and sums, 157 TFLOP/s against the vector units' same
+// rate but with a sixteenth of the operand reads), W row-major as it is held.  K must be a multiple of 4.
+//
+// A row's result does not depend on the number of rows beside it: k goes to the eight waves of a workgroup in eight
+// ranges that depend on K alone, every range is summed in the same order whatever the tiles, and the ranges are
+// added in their order.
+//
+// What bounds it: for few rows the reading of W (4 bytes an element once, straight into the operand registers, no LDS:
+// every wave owns its range of k, so nothing is read twice in a workgroup but x); from about 48 rows on the matrix cores.
+// Lane l holds A[l%16][l/16], B[l/16][l%16], D[(l/16)*4 .. +4][l%16] of a 16 x 16 x 4 product.  The four k of a product may
+// be any as long as A and B agree: lane group c = l/16 takes four k in a row, [kb + 4c, kb + 4c + 4), one 16-byte load that
+// serves four products, so that a row of W is read in pieces of 64 bytes, the next piece by the next load.
+//
+// Measured with 1 to 5 rows at width 1,024 (the tiled kernel of the vector units in gemm_plain.hip, which walks k with one
+// load in flight, before): q/k/v (6.3 MB) 156 -> 5.8 us, output and down projection (4.2 and 16.8 MB) 378 -> 9.1 us on
+// average, gate/up with its activation (33.6 MB) 160 -> 11.5 us, the head (134 MB) 201 -> 29 us = 4.6 TB/s.  Error against
+// float64 of the logits of four layers 2.9e-6 -> 1.1e-6.
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+#define GF_RANGES 8
+
+// RT tiles of 16 rows of W and MT tiles of 16 rows of x a workgroup; U steps of 16 k are asked for together, the next U
+// while these are multiplied.  GATED: W holds N gate rows, then N up rows; tiles come in pairs of both and y is
+// act(gate) * up * scale.
+template <int RT, int MT, int U, bool GATED>
+__global__ void __launch_bounds__(GF_RANGES * 64)
+gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int M, int N, int K,
+                GateOut gate) {
+    constexpr int TOGETHER = GATED ? 2 : 1;                    // row tiles that are finished together
+    __shared__ float red[GF_RANGES][TOGETHER * MT][64][4];
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int r = lane % 16, c = lane / 16;
+    const int n_base = blockIdx.x * (16 * RT / TOGETHER), m_base = blockIdx.y * (16 * MT);
+
+    f32x4 acc[RT][MT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    // rows past the end read a valid one and are never stored
+    const float* w_row[RT];
+    const float* x_row[MT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        const int n = min(n_base + (t / TOGETHER) * 16 + r, N - 1);
+        w_row[t] = w + (size_t)(n + (GATED && (t & 1) ? N : 0)) * K + c * 4;
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) x_row[m] = x + (size_t)min(m_base + m * 16 + r, M - 1) * K + c * 4;
+
+    const int steps = (K + 15) / 16, each = (steps + GF_RANGES - 1) / GF_RANGES;
+    const int first = min(wave * each, steps), count = min(steps - first, each);
+    // the last step of k may be partial: it is left to the end, where loads are looked after one by one
+    const int whole = min(count, max(0, K / 16 - first));
+    const int batches = whole / U;
+
+    f32x4 a[2][U][RT], b[2][U][MT];
+    auto load = [&](int s, int batch) __attribute__((always_inline)) {
+        const int kb = (first + batch * U) * 16;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) b[s][u][m] = *reinterpret_cast<const f32x4*>(x_row[m] + kb + u * 16);
+#pragma unroll
+            for (int t = 0; t < RT; ++t) a[s][u][t] = *reinterpret_cast<const f32x4*>(w_row[t] + kb + u * 16);
+        }
+    };
+    auto multiply = [&](int s, int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+                    acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][u][t][j], b[s][u][m][j], acc[t][m], 0, 0, 0);
+    };
+    auto multiply_all = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) multiply(s, u);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (batches > 0) {
+        load(0, 0);
+        int i = 0;
+        for (; i + 2 < batches; i += 2) {
+            load(1, i + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply_all(0);
+            load(0, i + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply_all(1);
+        }
+        if (i + 1 < batches) {
+            load(1, i + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply_all(0);
+            multiply_all(1);
+        } else {
+            multiply_all(0);
+        }
+    }
+    for (int s = batches * U; s < count; ++s) {
+        const int k = (first + s) * 16;
+        const bool in = k + c * 4 < K;                         // (K is a multiple of 4)
+        const f32x4 zero = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < MT; ++m) b[0][0][m] = in ? *reinterpret_cast<const f32x4*>(x_row[m] + k) : zero;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) a[0][0][t] = in ? *reinterpret_cast<const f32x4*>(w_row[t] + k) : zero;
+        multiply(0, 0);
+    }
+
+#pragma unroll
+    for (int t0 = 0; t0 < RT; t0 += TOGETHER) {
+        if (t0 > 0) __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TOGETHER; ++t)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) *reinterpret_cast<f32x4*>(red[wave][t * MT + m][lane]) = acc[t0 + t][m];
+        __syncthreads();
+        if (wave < MT) {
+            const int row = m_base + wave * 16 + r, n0 = n_base + (t0 / TOGETHER) * 16 + c * 4;
+            float s[TOGETHER][4];
+#pragma unroll
+            for (int t = 0; t < TOGETHER; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    s[t][e] = 0.f;
+                    for (int range = 0; range < GF_RANGES; ++range) s[t][e] += red[range][t * MT + wave][lane][e];
+                }
+            if (row < M && n0 < N) {
+                if constexpr (GATED) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[0][e] = gate_unit(s[0][e], s[1][e], gate);
+                }
+                const int ld = GATED ? gate.ld : N;
+                store4(y + (size_t)row * ld + n0, s[0], N - n0, (ld & 3) == 0 && ((uintptr_t)y & 15) == 0);
+            }
+        }
+    }
+}
+
+template <int RT, int MT, int U>
+static int launch_f32(const float* x, const float* w, float* y, int M, int N, int K, const GateOut& gate, hipStream_t s) {
+    constexpr int COLS = 16 * RT;
+    const dim3 grid((N + (gate.on ? COLS / 2 : COLS) - 1) / (gate.on ? COLS / 2 : COLS), (M + 16 * MT - 1) / (16 * MT));
+    if (grid.y > 65535) return tli_fail("gemm_f32: %d rows exceed the grid limit", M);
+    if (gate.on) {
+        if constexpr (RT > 1) gemm_f32_kernel<RT, MT, U, true><<<grid, GF_RANGES * 64, 0, s>>>(x, w, y, M, N, K, gate);
+    } else {
+        gemm_f32_kernel<RT, MT, U, false><<<grid, GF_RANGES * 64, 0, s>>>(x, w, y, M, N, K, gate);
+    }
+    return tli_check_launch("gemm_f32");
+}
+
+// y[M,N] = x[M,K] . w[N,K]^T in float32; gated: w is [2 N, K], gate rows before up rows, and y[M, y_ld] takes
+// act(gate) * up * act_scale (y_ld 0: N).
+extern "C" int tli_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K, int gated, int act, float act_scale,
+                            int y_ld, void* stream) {
+    const GateOut gate = gate_out(gated, act, act_scale, y_ld, N);
+    if (const char* fault = gate_out_fault(gate, N)) return tli_fail("gemm_f32: %s", fault);
+    if (M <= 0 || N <= 0) return 0;
+    if (K <= 0 || K % 4) return tli_fail("gemm_f32: K = %d must be a positive multiple of 4", K);
+    if (((uintptr_t)x | (uintptr_t)w) & 15) return tli_fail("gemm_f32: operands must be 16-byte aligned");
+    const float *xp = (const float*)x, *wp = (const float*)w;
+    float* yp = (float*)y;
+    hipStream_t s = (hipStream_t)stream;
+    // Few rows: one tile of W a workgroup while that gives less than two workgroups a compute unit, two beyond (x is then
+    // read half as often).  Many rows: 64 x 64 outputs a workgroup where that fills the chip, else 32 x 64 or 16 x 64.
+    const long tiles = ((long)(gated ? 2 : 1) * N + 15) / 16, units = tli_compute_units();
+    if (M <= 16) return tiles < 2 * units && !gated ? launch_f32<1, 1, 8>(xp, wp, yp, M, N, K, gate, s)
+                                                    : launch_f32<2, 1, 4>(xp, wp, yp, M, N, K, gate, s);
+    if (M <= 32) return tiles < 2 * units && !gated ? launch_f32<1, 2, 4>(xp, wp, yp, M, N, K, gate, s)
+                                                    : launch_f32<2, 2, 4>(xp, wp, yp, M, N, K, gate, s);
+    const long blocks = tiles * ((M + 63) / 64);
+    if (blocks >= 4 * units) return launch_f32<4, 4, 1>(xp, wp, yp, M, N, K, gate, s);
+    if (blocks >= 2 * units || gated) return launch_f32<2, 4, 2>(xp, wp, yp, M, N, K, gate, s);
+    return launch_f32<1, 4, 2>(xp, wp, yp, M, N, K, gate, s);
+}

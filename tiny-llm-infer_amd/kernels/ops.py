@@ -84,6 +84,7 @@ def load_library():
         "tli_keys_values_to_cache": [P, P, P, P, P, I, I, P, I, I, I, I, I, I, P, F, P, P, I, P],
         "tli_attention_plain": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, I, P],
         "tli_gemm_plain": [P, P, P, I, I, I, I, I, I, P],
+        "tli_gemm_f32": [P, P, P, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_fused_bf16": [P, P, P, I, I, I, I, P, I, F, P, P, P, P, I, I, F, I, P],
         "tli_gemm_mid_bf16": [P, P, P, P, I, I, I, I, I, I, I, I, F, I, P],
@@ -494,9 +495,19 @@ class HipOps:
             return y
         w = getattr(matrix, "w", matrix)
         self._want(w, "linear matrix")
+        if out_dtype == torch.float32 and self._f32_product_takes(x, w):
+            self._call(self.lib.tli_gemm_f32, x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, 0, *_NO_GATE,
+                       self._stream())
+            return y
         self._call(self.lib.tli_gemm_plain, x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K,
                    _dtype_code(x.dtype), _dtype_code(w.dtype), _dtype_code(out_dtype), self._stream())
         return y
+
+    @staticmethod
+    def _f32_product_takes(x, w) -> bool:
+        """Whether the float32 product on the matrix cores takes these operands: rows of whole 16-byte pieces."""
+        return (x.dtype == torch.float32 and w.dtype == torch.float32 and x.shape[1] % 4 == 0
+                and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
     def _product_into_residual(self, p: PendingProduct, resid, weight, eps) -> NormedRows:
         """resid += x W^T, and the rows of the norm that follows, its factor still owed."""
@@ -664,6 +675,15 @@ class HipOps:
             self._want(x, "linear input", torch.bfloat16, (M, _shape_of(m)[1]))
             y, y_at, ld = self._rows_into(into, M, m.inter, x.dtype)
             return self._linear_rows(x, gated, y, M, 2 * m.inter, K, 1, gate=(y_at, act, float(scale), ld))
+        if not self.plain_products and x.dtype == torch.float32 and getattr(m, "dtype", None) == torch.float32 and M > 0:
+            w = m.w
+            self._want(x, "linear input", torch.float32, (M, w.shape[1]))
+            self._want(w, "linear matrix", torch.float32, (2 * m.inter, K))
+            if self._f32_product_takes(x, w):
+                y, y_at, ld = self._rows_into(into, M, m.inter, x.dtype)
+                self._call(self.lib.tli_gemm_f32, x.data_ptr(), w.data_ptr(), y_at, M, m.inter, K, 1, act, float(scale), ld,
+                           self._stream())
+                return y
         return self.swiglu(self.linear(x, m), activation=activation, scale=scale, into=into)
 
     def swiglu(self, gu: torch.Tensor, limit: float = 0.0, slope: float = 1.0, activation: str = "silu", scale: float = 1.0,
