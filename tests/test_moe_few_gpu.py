@@ -1,0 +1,115 @@
+"""The routed experts of few rows in two launches, the shared expert among them, beside float64: tiles of 16 rows and their
+edges, more experts than pairs and fewer, k of less than a step of 128 and of more steps than waves, experts that hand
+their input on; and a row's independence of the rows beside it."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+BF = torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from tiny_llm_infer_amd.kernels.ops import HipOps
+    return HipOps(DEV)
+
+
+# (rows, experts, of which identity, top, width, hidden units, hidden units of the shared expert or 0)
+SIZES = [(1, 4, 0, 2, 72, 40, 48), (5, 6, 2, 3, 128, 64, 0), (8, 16, 0, 2, 2048, 512, 1024), (16, 40, 0, 2, 264, 200, 96),
+         (17, 8, 1, 4, 136, 272, 32), (32, 3, 0, 1, 1000, 2304, 16), (33, 64, 0, 1, 96, 48, 112), (64, 16, 0, 8, 512, 136, 256)]
+
+
+def make(ops, size, kind):
+    from tiny_llm_infer_amd.parts.base import BuildEnv
+    from tiny_llm_infer_amd.parts.linear import GatedMatrix, as_matrix, fuse_rows
+    T, E, identity, top, D, ff, sff = size
+    g = torch.Generator(device=DEV).manual_seed(T + ff)
+    env = BuildEnv(dtype=BF, device=torch.device(DEV), ops=ops, max_model_len=64)
+
+    def rnd(*shape, std=1.0):
+        return (torch.randn(shape, generator=g, device=DEV) * std).to(BF)
+    gated = kind in ("silu", "limited")
+    w = {"x": rnd(T, D), "gate": rnd(E, ff, D, std=D ** -0.5), "up": rnd(E, ff, D, std=D ** -0.5), "down": rnd(E, D, ff, std=ff ** -0.5)}
+    packed = ops.pack_experts(torch.cat([w["gate"], w["up"]], 1) if gated else w["up"], w["down"], gated=gated)
+    scores = torch.rand(T, E + identity, generator=g, device=DEV)
+    weights, ids = torch.topk(scores, top, dim=1)
+    shared = (None, None, None)
+    if sff:
+        w["sg"], w["su"], w["sd"] = rnd(sff, D, std=D ** -0.5), rnd(sff, D, std=D ** -0.5), rnd(D, sff, std=sff ** -0.5)
+        up = GatedMatrix(w["sg"], w["su"], env) if kind == "silu" else fuse_rows([w["sg"], w["su"]], env) if gated else as_matrix(w["su"], env)
+        shared = (up, as_matrix(w["sd"], env), torch.rand(T, generator=g, device=DEV))
+    return w, packed, ids.to(torch.int32).contiguous(), weights.contiguous(), shared
+
+
+def plain(w, ids, weights, gate, E, kind):
+    x = w["x"].double()
+
+    def expert(h, wg, wu, wd):
+        u = h @ wu.double().T
+        if kind == "silu":
+            a = torch.nn.functional.silu(h @ wg.double().T) * u
+        elif kind == "limited":
+            z = torch.clamp(h @ wg.double().T, max=1.5)
+            a = z * torch.sigmoid(1.702 * z) * (torch.clamp(u, -1.5, 1.5) + 1)
+        else:
+            a = torch.relu(u) ** 2
+        return a @ wd.double().T
+    out = torch.zeros_like(x)
+    for t in range(x.shape[0]):
+        for j in range(ids.shape[1]):
+            e, by = int(ids[t, j]), float(weights[t, j])
+            if e >= E:
+                out[t] += by * x[t]
+            elif kind == "relu2":
+                out[t] += expert(by * x[t], None, w["up"][e], w["down"][e])
+            else:
+                out[t] += by * expert(x[t], w["gate"][e], w["up"][e], w["down"][e])
+    if gate is not None:
+        out += gate.double()[:, None] * expert(x, w["sg"], w["su"], w["sd"])
+    return out
+
+
+@pytest.mark.parametrize("kind", ["silu", "limited", "relu2"])
+@pytest.mark.parametrize("size", SIZES)
+def test_experts_of_few_rows(ops, size, kind):
+    T, E, identity = size[:3]
+    if kind == "relu2" and identity:
+        pytest.skip("experts whose weight goes on their input all have matrices")
+    w, packed, ids, weights, (up, down, gate) = make(ops, size, kind)
+    how = {"silu": {}, "limited": dict(limit=1.5, slope=1.702, shared_limit=1.5), "relu2": dict(activation="relu2", weight_on_input=True)}[kind]
+
+    def few(at):
+        return ops.resolve(ops.experts_of_few_rows(w["x"][at].clone(), ids[at].clone(), weights[at].clone(), packed, up, down,
+                                                   None if gate is None else gate[at].clone(), handed_on=identity > 0, **how))
+    got = few(slice(0, T))
+    want = plain(w, ids, weights, gate, E, kind)
+    # hidden units and results are rounded to bfloat16 (2^-9 of their size each): the sum over ff rounded units is off by
+    # 2^-9 of the root of the sum of their squares, which is the size of the result itself; five times that for the largest
+    scale = float(want.square().mean().sqrt())
+    assert float((got.double() - want).abs().max()) <= 5 * 2.0 ** -9 * scale + 2.0 ** -8 * float(want.abs().max())
+    for at in (slice(0, 1), slice(T - 1, T), slice(T // 2, T)):
+        assert torch.equal(few(at), got[at]), "a row's result depends on the rows beside it"
+
+
+def test_layer_norm_of_unfinished_sums(ops):
+    """The layer norm adds up the parts, and rounds their sum, as the reduction of its own does."""
+    from tiny_llm_infer_amd.kernels.ops import DeferredSum
+    g = torch.Generator(device=DEV).manual_seed(1)
+    for rows, n in ((1, 64), (5, 100), (3, 5120), (2, 17000)):
+        parts = [DeferredSum(torch.randn((p, rows, n), generator=g, device=DEV), BF) for p in (3, 2)]
+        weight = torch.rand(n, generator=g, device=DEV)
+        resid = torch.randn((rows, n), generator=g, device=DEV)
+        for deltas in (parts[:1], parts, [ops.resolve(parts[0]), parts[1]]):
+            mine, want = resid.clone(), resid.clone()
+            y = ops.add_layernorm(mine, deltas, (weight,), 1e-5, BF)[0]
+            z = ops.add_layernorm(want, [ops.resolve(d) for d in deltas], (weight,), 1e-5, BF)[0]
+            assert torch.equal(y, z) and torch.equal(mine, want)
+
+
+def test_sizes_that_other_kernels_take(ops):
+    w, packed, ids, weights, (up, down, gate) = make(ops, (65, 8, 0, 2, 64, 32, 0), "silu")
+    assert ops.experts_of_few_rows(w["x"], ids, weights, packed, None, None, None) is None
+    w, packed, ids, weights, _ = make(ops, (2, 300, 0, 2, 64, 32, 0), "silu")
+    assert ops.experts_of_few_rows(w["x"], ids, weights, packed, None, None, None) is None

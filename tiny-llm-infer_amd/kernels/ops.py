@@ -107,7 +107,7 @@ def load_library():
         "tli_conv_heads": [P, P, P, P, P, P, P, P, P, P, I, I, P, I, I, I, I, I, I, I, I, I, P],
         "tli_attention_biased_plain": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P, P, P, I, I, I, P],
         "tli_attention_biased_mfma_bf16": [P, P, P, P, P, P, I, I, I, P, I, I, I, I, I, I, F, P, P, P, I, I, I, P],
-        "tli_add_layernorm": [P, P, P, P, P, P, P, P, I, I, I, F, I, P],
+        "tli_add_layernorm": [P, P, I, P, I, P, P, P, P, P, I, I, I, F, I, P],
         "tli_delta_prepare": [P, I, P, P, P, ctypes.c_longlong, ctypes.c_longlong, P, P, P, P, P, P, P, P, P, P, P, P, P,
                               I, I, I, I, I, I, I, I, P],
         "tli_delta_recurrence": [P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, P],
@@ -116,6 +116,8 @@ def load_library():
         "tli_moe_route": [P, ctypes.c_longlong, ctypes.c_longlong, P, P, P, I, I, I, I, I, F, I, I, I, I, P, P],
         "tli_moe_router_bf16": [P, P, I, P, P, P, I, I, I, I, I, F, I, I, I, I, P, P],
         "tli_moe_experts": [P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, F, I, I, P],
+        "tli_moe_few_takes": [I, I, I, I, I],
+        "tli_moe_few_bf16": [P, P, P, P, P, P, P, P, P, P, ctypes.c_longlong, P, P, P, I, I, I, I, I, I, I, F, F, F, I, I, P],
         "tli_norm_add": [P, P, P, P, I, I, F, I, P],
         "tli_residual_rows": [P, P, ctypes.c_longlong, P],
         "tli_attention_sized_plain": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, F, I, I, I, I, P, P],
@@ -1208,16 +1210,21 @@ class HipOps:
     # ---- layer norm ------------------------------------------------------------------------------
     def add_layernorm(self, resid, deltas, weights, eps, out_dtype, rows=None, num_rows=None):
         """``resid`` (float32 [T, n]) takes the sum of ``deltas`` (none, one or two tensors [T, n] of
-        ``out_dtype``: what the parts before still owe it); returns the layer norm (no bias) of its rows
+        ``out_dtype``, or unfinished products: what the parts before still owe it); returns the layer norm (no bias) of its rows
         once for every weight vector of ``weights`` (one or two: norms of the same rows share their mean
         and variance).  With ``rows`` only those rows are computed and ``resid`` stays as it is."""
         total, n = resid.shape
         self._want(resid, "residual", torch.float32)
-        deltas = tuple(deltas)
+        deltas, parts = list(deltas), [0, 0]
         if len(deltas) > 2 or not 1 <= len(weights) <= 2:
             raise KernelError("add_layernorm takes at most two deltas and one or two weight vectors")
-        for d in deltas:
-            self._want(d, "residual delta", out_dtype, (total, n))
+        for i, d in enumerate(deltas):
+            if isinstance(d, DeferredSum) and d.dtype == out_dtype == torch.bfloat16:
+                deltas[i], parts[i] = d.parts, d.parts.shape[0]
+                self._want(d.parts, "partial sums of the residual delta", torch.float32, (parts[i], total, n))
+                continue
+            deltas[i] = self.resolve(d)
+            self._want(deltas[i], "residual delta", out_dtype, (total, n))
         for w in weights:
             self._want(w, "norm weight", torch.float32, (n,))
         out_rows = total
@@ -1229,7 +1236,7 @@ class HipOps:
         outs = [torch.empty((out_rows, n), dtype=out_dtype, device=self.device) for _ in weights]
         d1 = deltas[0] if deltas else None
         d2 = deltas[1] if len(deltas) > 1 else None
-        self._call(self.lib.tli_add_layernorm, resid.data_ptr(), _ptr(d1), _ptr(d2), weights[0].data_ptr(),
+        self._call(self.lib.tli_add_layernorm, resid.data_ptr(), _ptr(d1), parts[0], _ptr(d2), parts[1], weights[0].data_ptr(),
                    _ptr(weights[1]) if len(weights) > 1 else None, outs[0].data_ptr(),
                    outs[1].data_ptr() if len(weights) > 1 else None, _ptr(rows), out_rows, total, n, float(eps),
                    _dtype_code(out_dtype), self._stream())
@@ -1476,6 +1483,59 @@ class HipOps:
                        out[t0:t1].data_ptr(), t1 - t0, top, n, ff, E, _dtype_code(x.dtype), float(limit), float(slope), act,
                        on_input, self._stream())
         return out
+
+    FEW_EXPERT_ROWS = 64         # up to so many rows the experts, the shared one with them, are two launches without a sort
+
+    def experts_of_few_rows(self, x, ids, weights, packed, shared_up, shared_down, shared_gate, limit=0.0, slope=1.0,
+                            shared_limit=0.0, activation=None, weight_on_input=False, handed_on=False):
+        """``apply_experts`` with the shared expert's products taken in, for few rows: ``shared_up`` its gate and up matrices (a
+        ``GatedMatrix``, or a ``Matrix`` of gate rows before up rows; without a gate the up matrix), ``shared_down`` (both None:
+        no shared expert); ``handed_on``: ids from E on may occur.  ``ids`` names no expert twice in a row.  The result is a
+        ``DeferredSum``, a part for every place of the choice and one for the shared expert; None where these kernels do not
+        apply."""
+        T, n = x.shape
+        if (packed is None or x.dtype != torch.bfloat16 or self.plain_products or self.moe_tile or not 0 < T <= self.FEW_EXPERT_ROWS):
+            return None
+        E, ff, top = packed["experts"], packed["inter"], ids.shape[1]
+        if packed["hidden"] != n or not self.lib.tli_moe_few_takes(T, top, E, n, ff):
+            return None
+        act = -1
+        if activation is not None:
+            self.check_activation(activation)
+            act = self.ACTIVATIONS[activation]
+        s_ff, s_gate, s_up, s_down, s_step = 0, None, None, None, 0
+        if shared_up is not None:
+            tiled, gated = getattr(shared_up, "tiled", None), getattr(shared_up, "gated", None)
+            s_down = getattr(shared_down, "tiled", None)
+            s_ff = _shape_of(shared_down)[1]
+            block = (n + 127) // 128 * 2048                       # elements of a block of 16 rows
+            if s_down is None or s_ff % 8 or (act < 0 and s_ff % 16):
+                return None
+            if act >= 0:
+                if tiled is None:
+                    return None
+                s_up, s_step = tiled.data_ptr(), block
+            elif gated is not None:                               # blocks of gate and up rows in turn
+                s_gate, s_up, s_step = gated.data_ptr(), gated.data_ptr() + 2 * block, 2 * block
+            elif tiled is not None:
+                s_gate, s_up, s_step = tiled.data_ptr(), tiled.data_ptr() + 2 * block * (s_ff // 16), block
+            else:
+                return None
+            if _shape_of(shared_up) != ((s_ff if act >= 0 else 2 * s_ff), n) or _shape_of(shared_down)[0] != n:
+                raise KernelError("the shared expert's matrices do not fit the rows")
+        self._want(x, "expert input")
+        self._want(ids, "chosen experts", torch.int32, (T, top))
+        self._want(weights, "experts' weights", torch.float32, (T, top))
+        if shared_gate is not None:
+            self._want(shared_gate, "shared expert's gate", torch.float32, (T,))
+        parts = torch.empty((top + (1 if s_ff else 0), T, n), dtype=torch.float32, device=self.device)
+        hid = torch.empty((T * top, ff), dtype=torch.bfloat16, device=self.device)
+        s_hid = torch.empty((T, s_ff), dtype=torch.bfloat16, device=self.device) if s_ff else None
+        self._call(self.lib.tli_moe_few_bf16, x.data_ptr(), ids.data_ptr(), weights.data_ptr(), None if act >= 0 else packed["gate"].data_ptr(),
+                   packed["up"].data_ptr(), packed["down"].data_ptr(), hid.data_ptr(), s_gate, s_up, None if s_down is None else s_down.data_ptr(), s_step,
+                   _ptr(shared_gate), _ptr(s_hid), parts.data_ptr(), 1 if handed_on else 0, T, top, E, n, ff, s_ff, float(limit), float(slope), float(shared_limit), act,
+                   1 if weight_on_input else 0, self._stream())
+        return DeferredSum(parts, torch.bfloat16)
 
     # ---- blocks that norm what a sublayer gives ------------------------------------------------------------
     def residual_rows(self, resid: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:

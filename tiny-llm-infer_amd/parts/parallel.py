@@ -41,12 +41,12 @@ class ParallelBlock(Block):
             if a is not None and b is not None and a[1] == b[1]:
                 self.pair = ((a[0], b[0]), a[1])
 
-    def _owed(self, pending) -> Tuple[torch.Tensor, ...]:
-        ops = self.env.ops
-        return tuple(ops.resolve(y) for y in (pending or ()) if y is not None)
+    def _owed(self, pending) -> tuple:
+        return tuple(y for y in (pending or ()) if y is not None)
 
-    def _one(self, owed: Tuple[torch.Tensor, ...]) -> Optional[torch.Tensor]:
+    def _one(self, owed: tuple) -> Optional[torch.Tensor]:
         """What is owed as one tensor, for a norm of another kind, which takes one."""
+        owed = tuple(self.env.ops.resolve(y) for y in owed)
         if not owed:
             return None
         return owed[0] if len(owed) == 1 else (owed[0].to(torch.float32) + owed[1].to(torch.float32)).to(owed[0].dtype)
