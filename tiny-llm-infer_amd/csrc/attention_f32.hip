@@ -1,0 +1,154 @@
+// Attention of the float32 path over the paged cache, a workgroup a (row, head): as attention_plain.hip, which walks 256 keys
+// at a time with a key a thread and stays for what this kernel does not take (heads that are no multiple of 64, pages of fewer
+// than four slots) and as its reference.
+//
+// The keys go to the four waves in blocks of 16, in turn; a wave keeps a running maximum, sum and output of its own, and the
+// four are joined at the end.  In a block four lanes share a key (lane 16 c + j: quarter c of key j, 16 bytes a load), then a
+// lane takes every 64th output element and the block's 16 values of it, four to a load.  What bounds a decode step's few short
+// rows is the chain of loads of one block after the other, which is a quarter as long here and has all its loads in flight:
+// 5 rows of up to 52 keys, 16 heads of 64: 15.9 -> 4.8 us, most of it the launch.
+// The order of additions depends on the row's first and last key alone.
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+#define AF_WAVES 4
+
+template <int DH>            // head_dim / 64
+__global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
+    const float* __restrict__ q, float* __restrict__ out, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
+    const int* __restrict__ positions, const int* __restrict__ seq_of_row, const int* __restrict__ tables, int table_width,
+    int page_size, int num_pages, int heads, int kv_heads, float scale, int window) {
+    constexpr int D = DH * 64;
+    __shared__ __attribute__((aligned(16))) float p_s[AF_WAVES][16];
+    __shared__ float m_s[AF_WAVES], l_s[AF_WAVES], o_s[AF_WAVES][D];
+    const int row = blockIdx.x, head = blockIdx.y;
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int j = lane % 16, c = lane / 16;
+    const int g = head / (heads / kv_heads);
+    const int pos = positions[row];
+    const int* table = tables + (size_t)seq_of_row[row] * table_width;
+    const int lo = window > 0 ? max(0, pos - window + 1) : 0;
+    const size_t page_stride = (size_t)kv_heads * page_size * D;
+    const float* k_head = k_cache + (size_t)g * page_size * D;
+    const float* v_head = v_cache + (size_t)g * page_size * D;
+
+    // this lane's quarter of the query: elements 16 i + 4 c .. + 4
+    f32x4 qv[DH * 4];
+    {
+        const float* q_row = q + ((size_t)row * heads + head) * D + c * 4;
+#pragma unroll
+        for (int i = 0; i < DH * 4; ++i) qv[i] = *reinterpret_cast<const f32x4*>(q_row + i * 16);
+    }
+    float m = -INFINITY, l = 0.f, o[DH];
+#pragma unroll
+    for (int i = 0; i < DH; ++i) o[i] = 0.f;
+    auto page_of = [&](int t) { return t <= pos ? table[t / page_size] : -1; };
+
+    for (int base = (lo / 16 + wave) * 16; base <= pos; base += 16 * AF_WAVES) {
+        const int t = base + j;
+        const int page = page_of(t);
+        const bool seen = t >= lo && page >= 0 && page < num_pages;
+        const float* kp = k_head + (size_t)(seen ? page : 0) * page_stride + (size_t)(t % page_size) * D + c * 4;
+        f32x4 kv[DH * 4];
+#pragma unroll
+        for (int i = 0; i < DH * 4; ++i) kv[i] = *reinterpret_cast<const f32x4*>(kp + i * 16);
+        // the values of the block: groups of four slots never straddle a page
+        int v_page[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v_page[u] = page_of(base + 4 * u);
+        f32x4 vv[DH][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const bool held = v_page[u] >= 0 && v_page[u] < num_pages;
+            const float* vp = v_head + (size_t)(held ? v_page[u] : 0) * page_stride + (size_t)lane * page_size + (base + 4 * u) % page_size;
+#pragma unroll
+            for (int i = 0; i < DH; ++i) vv[i][u] = *reinterpret_cast<const f32x4*>(vp + (size_t)i * 64 * page_size);
+        }
+        f32x4 dot = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < DH * 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dot[e] = fmaf(qv[i][e], kv[i][e], dot[e]);
+        const float s = quad_rows_sum((dot[0] + dot[1]) + (dot[2] + dot[3])) * scale;
+        const float score = seen ? s : -INFINITY;
+        float top = score;
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 16));
+        const float m_new = fmaxf(m, top);
+        if (m_new == -INFINITY) continue;                       // (nothing of this block is seen: the same for the whole wave)
+        const float p = seen ? expf(score - m_new) : 0.f;
+        const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
+        float sum = p;
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 16);
+        l = l * corr + sum;
+        m = m_new;
+        if (c == 0) p_s[wave][j] = p;
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < DH; ++i) o[i] *= corr;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const f32x4 w = *reinterpret_cast<const f32x4*>(&p_s[wave][4 * u]);
+#pragma unroll
+            for (int i = 0; i < DH; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[i] = fmaf(w[e], vv[i][u][e], o[i]);
+        }
+        wave_lds_sync();
+    }
+    if (lane == 0) {
+        m_s[wave] = m;
+        l_s[wave] = l;
+    }
+#pragma unroll
+    for (int i = 0; i < DH; ++i) o_s[wave][i * 64 + lane] = o[i];
+    __syncthreads();
+    float best = m_s[0];
+#pragma unroll
+    for (int w = 1; w < AF_WAVES; ++w) best = fmaxf(best, m_s[w]);
+    float total = 0.f, share[AF_WAVES];
+#pragma unroll
+    for (int w = 0; w < AF_WAVES; ++w) {
+        share[w] = m_s[w] == -INFINITY ? 0.f : expf(m_s[w] - best);
+        total += l_s[w] * share[w];
+    }
+    const float inv = total > 0.f ? 1.0f / total : 0.f;
+    for (int d = threadIdx.x; d < D; d += AF_WAVES * 64) {
+        float y = 0.f;
+#pragma unroll
+        for (int w = 0; w < AF_WAVES; ++w) y = fmaf(share[w], o_s[w][d], y);
+        out[((size_t)row * heads + head) * D + d] = y * inv;
+    }
+}
+
+extern "C" int tli_attention_f32_takes(int head_dim, int page_size) {
+    return head_dim > 0 && head_dim % 64 == 0 && head_dim <= 256 && page_size >= 4 && page_size % 4 == 0;
+}
+
+// As tli_attention_plain, float32.
+extern "C" int tli_attention_f32(const void* q, void* out, const void* k_cache, const void* v_cache, const int* positions,
+                                 const int* seq_of_row, const int* tables, int table_width, int page_size, int num_pages, int rows,
+                                 int heads, int kv_heads, int head_dim, float scale, int window, void* stream) {
+    if (rows <= 0) return 0;
+    if (!tli_attention_f32_takes(head_dim, page_size))
+        return tli_fail("attention_f32: heads of %d (64, 128, 192, 256) or pages of %d slots are not taken", head_dim, page_size);
+    if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || heads > 65535)
+        return tli_fail("attention_f32: %d heads cannot be grouped over %d kv heads", heads, kv_heads);
+    if (table_width <= 0 || num_pages <= 0) return tli_fail("attention_f32: bad cache geometry");
+    if (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) return tli_fail("attention_f32: operands must be 16-byte aligned");
+    const dim3 grid(rows, heads);
+#define TLI_AF(DH)                                                                                                                 \
+    attention_f32_kernel<DH><<<grid, AF_WAVES * 64, 0, (hipStream_t)stream>>>((const float*)q, (float*)out, (const float*)k_cache, \
+                                                                               (const float*)v_cache, positions, seq_of_row, tables, \
+                                                                               table_width, page_size, num_pages, heads, kv_heads, scale, window)
+    switch (head_dim / 64) {
+        case 1: TLI_AF(1); break;
+        case 2: TLI_AF(2); break;
+        case 3: TLI_AF(3); break;
+        default: TLI_AF(4); break;
+    }
+#undef TLI_AF
+    return tli_check_launch("attention_f32");
+}

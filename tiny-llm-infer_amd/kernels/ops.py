@@ -83,6 +83,8 @@ def load_library():
         "tli_values_to_cache": [P, P, P, P, I, I, P, I, I, I, I, I, I, P],
         "tli_keys_values_to_cache": [P, P, P, P, P, I, I, P, I, I, I, I, I, I, P, F, P, P, I, P],
         "tli_attention_plain": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, I, P],
+        "tli_attention_f32_takes": [I, I],
+        "tli_attention_f32": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, P],
         "tli_gemm_plain": [P, P, P, I, I, I, I, I, I, P],
         "tli_gemm_f32": [P, P, P, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, I, I, F, I, P],
@@ -791,6 +793,12 @@ class HipOps:
                        T, g.tables.data_ptr(), g.table_width, g.page_size, kc.shape[0], heads, kv_heads,
                        head_dim, float(scale), int(window or 0), self._prefill_mode(step, T), _ptr(sinks),
                        self._stream())
+            return out
+        if (q.dtype == torch.float32 and not self.force_plain and self.lib.tli_attention_f32_takes(head_dim, g.page_size)
+                and (q.data_ptr() | kc.data_ptr() | vc.data_ptr()) % 16 == 0):
+            self._call(self.lib.tli_attention_f32, q.data_ptr(), out.data_ptr(), kc.data_ptr(), vc.data_ptr(), step.positions.data_ptr(),
+                       step.seq_of_row.data_ptr(), g.tables.data_ptr(), g.table_width, g.page_size, kc.shape[0], T, heads, kv_heads,
+                       head_dim, float(scale), int(window or 0), self._stream())
             return out
         self._call(self.lib.tli_attention_plain, q.data_ptr(), out.data_ptr(), kc.data_ptr(),
                    vc.data_ptr(), step.positions.data_ptr(), step.seq_of_row.data_ptr(),
