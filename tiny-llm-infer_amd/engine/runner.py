@@ -140,10 +140,11 @@ class ModelRunner:
         self.steps_run = 0
         # Decode steps (one token for every request, every logit wanted) launch the same
         # kernels with the same arguments whenever (requests, table width, reach, skew) agree:
-        # their launch sequence is recorded once as a HIP graph and replayed.
+        # their launch sequence is recorded once as a HIP graph and replayed.  (float32 steps too: launched one by
+        # one, the 40 kernels of a small model's step take the host longer than the device: 6.1 -> 4.5 ms for 16 steps of
+        # four layers of 1,024.)
         parts = [model.embedding, model.final_norm, model.head] + list(model.blocks)
-        self.use_graphs = (env.device.type == "cuda" and env.dtype == torch.bfloat16
-                           and all(p.replayable for p in parts))
+        self.use_graphs = env.device.type == "cuda" and all(p.replayable for p in parts)
         self.graphs = {}
         self.graph_pool = None
         self.graph_replays = 0
