@@ -25,7 +25,9 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 // RT tiles of 16 rows of W and MT tiles of 16 rows of x a workgroup; U steps of 16 k are asked for together, the next U
 // while these are multiplied.  GATED: W holds N gate rows, then N up rows; tiles come in pairs of both and y is
 // act(gate) * up * scale.
-template <int RT, int MT, int U, bool GATED>
+// CT < 16 (one tile of W): a workgroup takes CT of a tile's 16 columns, its lanes of the others repeating them, so that a matrix
+// of few rows is read by more compute units.
+template <int RT, int MT, int U, bool GATED, int CT = 16>
 __global__ void __launch_bounds__(GF_RANGES * 64)
 gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int M, int N, int K,
                 GateOut gate) {
@@ -33,7 +35,8 @@ gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float*
     __shared__ float red[GF_RANGES][TOGETHER * MT][64][4];
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     const int r = lane % 16, c = lane / 16;
-    const int n_base = blockIdx.x * (16 * RT / TOGETHER), m_base = blockIdx.y * (16 * MT);
+    static_assert(CT == 16 || RT == 1, "part of one tile");
+    const int n_base = blockIdx.x * (CT == 16 ? 16 * RT / TOGETHER : CT), m_base = blockIdx.y * (16 * MT);
 
     f32x4 acc[RT][MT];
 #pragma unroll
@@ -46,7 +49,7 @@ gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float*
     const float* x_row[MT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
-        const int n = min(n_base + (t / TOGETHER) * 16 + r, N - 1);
+        const int n = min(n_base + (t / TOGETHER) * 16 + r % CT, N - 1);
         w_row[t] = w + (size_t)(n + (GATED && (t & 1) ? N : 0)) * K + c * 4;
     }
 #pragma unroll
@@ -132,7 +135,7 @@ gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float*
                     s[t][e] = 0.f;
                     for (int range = 0; range < GF_RANGES; ++range) s[t][e] += red[range][t * MT + wave][lane][e];
                 }
-            if (row < M && n0 < N) {
+            if (row < M && n0 < N && c * 4 < CT) {
                 if constexpr (GATED) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) s[0][e] = gate_unit(s[0][e], s[1][e], gate);
@@ -142,6 +145,12 @@ gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float*
             }
         }
     }
+}
+
+template <int MT, int U, int CT>
+static int launch_f32_part(const float* x, const float* w, float* y, int M, int N, int K, const GateOut& gate, hipStream_t s) {
+    gemm_f32_kernel<1, MT, U, false, CT><<<dim3((N + CT - 1) / CT, (M + 16 * MT - 1) / (16 * MT)), GF_RANGES * 64, 0, s>>>(x, w, y, M, N, K, gate);
+    return tli_check_launch("gemm_f32");
 }
 
 template <int RT, int MT, int U>
@@ -172,6 +181,13 @@ extern "C" int tli_gemm_f32(const void* x, const void* w, void* y, int M, int N,
     // Few rows: one tile of W a workgroup while that gives less than two workgroups a compute unit, two beyond (x is then
     // read half as often).  Many rows: 64 x 64 outputs a workgroup where that fills the chip, else 32 x 64 or 16 x 64.
     const long tiles = ((long)(gated ? 2 : 1) * N + 15) / 16, units = tli_compute_units();
+    // parts of a tile while that gives no more than a workgroup a compute unit (1,024 columns of k 4,096: 64 workgroups of
+    // whole tiles, 256 of quarters: 16 decode steps of four layers of width 1,024 4.47 -> 4.19 ms)
+    if (M <= 32 && !gated && tiles * 2 <= units) {
+        const bool four = tiles * 4 <= units;
+        if (M <= 16) return four ? launch_f32_part<1, 8, 4>(xp, wp, yp, M, N, K, gate, s) : launch_f32_part<1, 8, 8>(xp, wp, yp, M, N, K, gate, s);
+        return four ? launch_f32_part<2, 4, 4>(xp, wp, yp, M, N, K, gate, s) : launch_f32_part<2, 4, 8>(xp, wp, yp, M, N, K, gate, s);
+    }
     if (M <= 16) return tiles < 2 * units && !gated ? launch_f32<1, 1, 8>(xp, wp, yp, M, N, K, gate, s)
                                                     : launch_f32<2, 1, 4>(xp, wp, yp, M, N, K, gate, s);
     if (M <= 32) return tiles < 2 * units && !gated ? launch_f32<1, 2, 4>(xp, wp, yp, M, N, K, gate, s)
