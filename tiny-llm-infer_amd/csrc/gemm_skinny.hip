@@ -15,6 +15,12 @@
 // any 32 values of k as long as A and B agree: lane group c = l/16 takes the 32
 // consecutive k  [kb + 32c, kb + 32c + 32)  of a 128-wide step, 8 per MFMA.
 //
+// The rows of x of a step go through LDS (up to 16 rows; see XR below), and where whole tiles of 16 columns leave half the
+// compute units without one a workgroup takes half a tile.  Measured with 8 rows, cold weights, launches of a chain (straight
+// into the operand registers, whole tiles, before): 2,048 columns into the residual of k 8,192 13.2 -> 9.8 us, of k 12,288 15.3 ->
+// 12.6; 4,096 columns of k 4,096 9.0 -> 8.0, of k 12,288 19.9 -> 18.9; 24,576 of k 4,096 (gated) 33.3 -> 32.9.  A chain of launches
+// costs 2.5 us each before the first byte; what is left goes by at 6.4 TB/s.
+//
 // A workgroup owns 16*RT output columns; its waves take the 128-wide k steps in
 // turn and their partial sums are added through LDS in wave order, so the
 // result does not depend on the launch.
@@ -39,6 +45,7 @@
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_any;     // four floats at any multiple of four bytes
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 union Pack16 {
     uint4 u;
@@ -78,14 +85,20 @@ struct SkinnyFuse {
 };
 
 template <int RT, int MT, int WAVES, typename TO, bool TILED = false, bool GATED = false, int DEPTH = 2,
-          int FUSE = FUSE_NONE>
+          int FUSE = FUSE_NONE, int XR = 0, bool WHOLE = false, bool HALF = false>
 __global__ void __launch_bounds__(WAVES * 64)
 gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, TO* __restrict__ y,
                    int M, int N, int K, SkinnyFuse fuse) {
+    static_assert(XR == 0 || MT == 1, "one tile of rows goes through LDS");
+    // HALF: a workgroup takes half a tile, 8 columns (lanes of the other half repeat them), so that twice as many compute
+    // units read a matrix of few rows
+    static_assert(!HALF || (RT == 1 && MT == 1 && TILED && !GATED), "half a tile of a tiled matrix");
+    constexpr int COLS = HALF ? 8 : 16 * RT;
     __shared__ float red[WAVES][RT * MT][64][4];
+    __shared__ u32x4_t x_lds[XR ? WAVES : 1][16][16];            // a wave's rows of one step, chunk q of row r at q ^ r
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     const int r = lane % 16, c = lane / 16;
-    const int n_base = blockIdx.x * (16 * RT);
+    const int n_base = blockIdx.x * COLS;
     if constexpr (FUSE == FUSE_NONE && TILED && !GATED) x += fuse.inputs.at(n_base);
 
     f32x4 acc[RT][MT];
@@ -105,7 +118,8 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
         w_row[t] = w + (size_t)(w_ok[t] ? n : 0) * K;
         if (TILED)   // blocks of 16 rows x 128 k = 4 KiB, stored [j][lane][8]: one load instruction
                      // of a wave reads 1 KiB in a row
-            w_row[t] = w + ((size_t)(blockIdx.x * RT + t) * ((K + 127) / 128)) * 2048 + lane * 8;
+            w_row[t] = HALF ? w + ((size_t)(blockIdx.x / 2) * ((K + 127) / 128)) * 2048 + (16 * c + 8 * (blockIdx.x % 2) + r % 8) * 8
+                            : w + ((size_t)(blockIdx.x * RT + t) * ((K + 127) / 128)) * 2048 + lane * 8;
     }
     const bf16_t* x_row[MT];
 #pragma unroll
@@ -116,16 +130,28 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
     // 4*(RT+MT)*(DEPTH-1) 16-byte loads in flight.  The main loop takes whole steps only
     // and none of its loads is under a branch: after a branch that may have issued loads
     // the compiler waits for all loads in flight, which would undo the prefetching.
-    Pack16 a[DEPTH][RT][4], b[DEPTH][MT][4];
+    Pack16 a[DEPTH][RT][4], b[XR ? 1 : DEPTH][MT][4];
+    // XR > 0: x goes through LDS.  A lane asks for 16 bytes of a row that its 15 neighbours go on with (a load instruction
+    // takes four rows of 256 bytes), and the operands are read from LDS; straight into the operand registers every load
+    // instruction takes 16 bytes from each of 64 places, which keeps the vector cache busy for longer than the weights do.
+    u32x4_t x_step[XR ? DEPTH : 1][XR ? XR : 1];
+    const bf16_t* x_piece[XR ? XR : 1];
+#pragma unroll
+    for (int i = 0; i < XR; ++i) x_piece[i] = x + (size_t)min(i * 4 + c, M - 1) * K + r * 8;
     auto load_step = [&](auto STAGE, int kb) {
         constexpr int S = decltype(STAGE)::value;
         const int k = kb + c * 32;
         // x first: it comes from L2 and loads complete in the order of issue
+        if constexpr (XR > 0) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
+            for (int i = 0; i < XR; ++i) x_step[S][i] = *reinterpret_cast<const u32x4_t*>(x_piece[i] + kb);
+        } else {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                b[S][m][j].u = *reinterpret_cast<const uint4*>(x_row[m] + k + j * 8);
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    b[S][m][j].u = *reinterpret_cast<const uint4*>(x_row[m] + k + j * 8);
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -135,15 +161,26 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
                 else
                     a[S][t][j].u = *reinterpret_cast<const uint4*>(w_row[t] + k + j * 8);
     };
-    auto mma_step = [&](auto STAGE) {
+    auto mma_step = [&](auto STAGE, auto DIRECT) {
         constexpr int S = decltype(STAGE)::value;
+        constexpr int B = XR ? 0 : S;
+        if constexpr (XR > 0 && !decltype(DIRECT)::value) {
+            // (a wave's LDS instructions run in their order: no step overtakes the one before.  Rows from 4 XR on are
+            // whatever lies there: they meet no other row's sums and are never stored)
+#pragma unroll
+            for (int i = 0; i < XR; ++i) x_lds[wave][i * 4 + c][r ^ (i * 4 + c)] = x_step[S][i];
+            wave_lds_sync();
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[0][0][j].w = x_lds[wave][r][(4 * c + j) ^ r];
+            wave_lds_sync();
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int t = 0; t < RT; ++t)
 #pragma unroll
                 for (int m = 0; m < MT; ++m)
-                    acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[S][t][j].v, b[S][m][j].v,
+                    acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[S][t][j].v, b[B][m][j].v,
                                                                         acc[t][m], 0, 0, 0);
         // keeps the scheduler from moving the loads of the next step (issued after this
         // in program order) ahead of these products, where they would have to be waited
@@ -170,7 +207,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
                 if (FULL || i + I + DEPTH - 1 < mine)
                     load_step(std::integral_constant<int, (I + DEPTH - 1) % DEPTH>{}, k_of(i + I + DEPTH - 1));
                 __builtin_amdgcn_sched_barrier(0);
-                mma_step(std::integral_constant<int, I>{});
+                mma_step(std::integral_constant<int, I>{}, std::false_type{});
                 self(self, i, std::integral_constant<int, I + 1>{}, FULL_T);
             }
         }
@@ -206,7 +243,14 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
         {   // wave t < RT finishes tile t: its residual values and norm weights (the other
             // waves ask for the same as wave 0, which costs nothing and keeps the loads
             // free of branches; rows and columns past the end repeat the last)
-            const int n0 = n_base + (wave < RT ? wave : 0) * 16 + c * 4;
+            const int n0 = n_base + (wave < RT ? wave : 0) * 16 + (HALF ? c % 2 : c) * 4;
+            if constexpr (WHOLE) {                     // rows of whole pieces of four columns: a load each
+                const int col = min(n0, N - 4);
+                const f32x4 h = *reinterpret_cast<const f32x4*>(fuse.resid + (size_t)min(r, M - 1) * N + col);
+                const f32x4_any v = *reinterpret_cast<const f32x4_any*>(fuse.norm_w + col);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) h_old[e] = h[e], nw[e] = v[e];
+            } else
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int col = min(n0 + e, N - 1);
@@ -234,7 +278,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
 #pragma unroll
             for (int m = 0; m < MT; ++m) b[0][m][j].u = load16_or_zero(x_row[m] + k + j * 8, in);
         }
-        mma_step(std::integral_constant<int, 0>{});
+        mma_step(std::integral_constant<int, 0>{}, std::true_type{});
     }
 
 #pragma unroll
@@ -296,7 +340,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
         for (int wv = 0; wv < WAVES; ++wv)
 #pragma unroll
             for (int i = 0; i < 4; ++i) s[i] += red[wv][tile][lane][i];
-        const int row = m * 16 + r;
+        const int row = HALF && c >= 2 ? M : m * 16 + r;       // (nothing is stored of what a half tile repeats)
         const int n0 = n_base + t * 16 + c * 4;
         if (FUSE == FUSE_RESIDUAL) {
             // (MT == 1 and tile == wave: the values asked for at the start are this tile's)
@@ -326,34 +370,56 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
     }
 }
 
-#ifndef PIPE_DEPTH
-#define PIPE_DEPTH 2
-#endif
+// Up to 16 rows go through LDS, four, eight or sixteen of them.
+#define SKINNY_ROWS(M, LAUNCH)          \
+    if ((M) <= 4) { LAUNCH(1); }        \
+    else if ((M) <= 8) { LAUNCH(2); }   \
+    else { LAUNCH(4); }
 
 template <int RT, int MT, int WAVES>
 static int launch_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N, int K, int y_dtype,
-                         int tiled, const GateOut& gate, const InputGroups& inputs, const OutUnit& unit, hipStream_t s) {
+                         int tiled, const GateOut& gate, const InputGroups& inputs, const OutUnit& unit, hipStream_t s, bool half = false) {
     SkinnyFuse plain{};
     plain.unit = unit;
     plain.gate = gate;
     plain.inputs = inputs;
     const int blocks = (N + 16 * RT - 1) / (16 * RT);
-    constexpr int D = (MT == 1 && RT <= 2) ? PIPE_DEPTH : 2;    // deep prefetch where the registers allow
-    if (tiled == 2) {       // gated: pairs of row tiles, silu(gate)*up written as bfloat16
-        gemm_skinny_kernel<RT, MT, WAVES, bf16_t, true, true, D><<<blocks, WAVES * 64, 0, s>>>(x, w, (bf16_t*)y, M, N, K, plain);
-    } else if (tiled) {
-        if (y_dtype == TLI_BF16)
-            gemm_skinny_kernel<RT, MT, WAVES, bf16_t, true, false, D><<<blocks, WAVES * 64, 0, s>>>(x, w, (bf16_t*)y, M, N, K, plain);
-        else
-            gemm_skinny_kernel<RT, MT, WAVES, float, true, false, D><<<blocks, WAVES * 64, 0, s>>>(x, w, (float*)y, M, N, K, plain);
+    constexpr bool CAN_HALF = RT == 1 && MT == 1;
+    if constexpr (CAN_HALF) {
+        if (half && tiled == 1) {
+#define SKINNY_HALF(TO, XR) \
+    gemm_skinny_kernel<1, 1, WAVES, TO, true, false, 2, FUSE_NONE, XR, false, true><<<(N + 7) / 8, WAVES * 64, 0, s>>>(x, w, (TO*)y, M, N, K, plain)
+#define SKINNY_HALF_BF16(XR) SKINNY_HALF(bf16_t, XR)
+#define SKINNY_HALF_F32(XR) SKINNY_HALF(float, XR)
+            if (y_dtype == TLI_BF16) SKINNY_ROWS(M, SKINNY_HALF_BF16)
+            else SKINNY_ROWS(M, SKINNY_HALF_F32)
+            return tli_check_launch("gemm_skinny");
+        }
+    }
+#define SKINNY_LAUNCH(TO, TILED, GATED, XR) \
+    gemm_skinny_kernel<RT, MT, WAVES, TO, TILED, GATED, 2, FUSE_NONE, XR><<<blocks, WAVES * 64, 0, s>>>(x, w, (TO*)y, M, N, K, plain)
+#define SKINNY_GATED(XR) SKINNY_LAUNCH(bf16_t, true, true, XR)
+#define SKINNY_BF16(XR) SKINNY_LAUNCH(bf16_t, true, false, XR)
+#define SKINNY_F32(XR) SKINNY_LAUNCH(float, true, false, XR)
+    if constexpr (MT == 1) {
+        if (tiled == 2) SKINNY_ROWS(M, SKINNY_GATED)       // pairs of row tiles, silu(gate)*up written as bfloat16
+        else if (tiled && y_dtype == TLI_BF16) SKINNY_ROWS(M, SKINNY_BF16)
+        else if (tiled) SKINNY_ROWS(M, SKINNY_F32)
+        else if (y_dtype == TLI_BF16) SKINNY_LAUNCH(bf16_t, false, false, 0);
+        else SKINNY_LAUNCH(float, false, false, 0);
     } else {
-        if (y_dtype == TLI_BF16)
-            gemm_skinny_kernel<RT, MT, WAVES, bf16_t, false><<<blocks, WAVES * 64, 0, s>>>(x, w, (bf16_t*)y, M, N, K, SkinnyFuse{});
-        else
-            gemm_skinny_kernel<RT, MT, WAVES, float, false><<<blocks, WAVES * 64, 0, s>>>(x, w, (float*)y, M, N, K, SkinnyFuse{});
+        if (tiled == 2) SKINNY_GATED(0);
+        else if (tiled && y_dtype == TLI_BF16) SKINNY_BF16(0);
+        else if (tiled) SKINNY_F32(0);
+        else if (y_dtype == TLI_BF16) SKINNY_LAUNCH(bf16_t, false, false, 0);
+        else SKINNY_LAUNCH(float, false, false, 0);
     }
     return tli_check_launch("gemm_skinny");
 }
+
+// Half tiles where whole ones leave half of the chip or more without a workgroup, and the matrix is not so small that its
+// product is all launch and latency.
+static bool half_tiles(int M, int N, int tiled) { return M <= 16 && tiled == 1 && N >= 1024 && (N + 15) / 16 <= tli_compute_units() / 2; }
 
 template <int MT>
 static int pick_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N, int K, int y_dtype,
@@ -361,11 +427,12 @@ static int pick_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N, 
     // cfg 0: by shape.  Narrow outputs get one 16-column tile per workgroup so that
     // even N = 4096 gives 256 workgroups; wide outputs share x over two tiles.
     const long tiles = (N + 15) / 16;
-    if (cfg == 0) cfg = tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
+    if (cfg == 0) cfg = half_tiles(M, N, tiled) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
     if (tiled == 2 && cfg < 20) cfg = 24;          // gated needs pairs of row tiles
     switch (cfg) {
         case 14: return launch_skinny<1, MT, 4>(x, w, y, M, N, K, y_dtype, tiled, gate, inputs, unit, s);
         case 18: return launch_skinny<1, MT, 8>(x, w, y, M, N, K, y_dtype, tiled, gate, inputs, unit, s);
+        case 8: return launch_skinny<1, MT, 8>(x, w, y, M, N, K, y_dtype, tiled, gate, inputs, unit, s, true);
         case 24: return launch_skinny<2, MT, 4>(x, w, y, M, N, K, y_dtype, tiled, gate, inputs, unit, s);
         case 28: return launch_skinny<2, MT, 8>(x, w, y, M, N, K, y_dtype, tiled, gate, inputs, unit, s);
         default: return tli_fail("gemm_skinny: unknown configuration %d", cfg);
@@ -426,20 +493,38 @@ extern "C" int tli_gemm_skinny_unit_bf16(const void* x, const void* w, void* y, 
 
 template <int RT, int WAVES>
 static int launch_skinny_fused(const bf16_t* x, const bf16_t* w, bf16_t* y, int M, int N, int K, int gated,
-                               const SkinnyFuse& f, hipStream_t s) {
+                               const SkinnyFuse& f, hipStream_t s, bool half = false) {
     const int blocks = (N + 16 * RT - 1) / (16 * RT);
-    if (f.resid)
-        gemm_skinny_kernel<RT, 1, WAVES, bf16_t, true, false, PIPE_DEPTH, FUSE_RESIDUAL><<<blocks, WAVES * 64, 0, s>>>(x, w, y, M, N, K, f);
-    else if (gated)
-        gemm_skinny_kernel<RT, 1, WAVES, bf16_t, true, true, PIPE_DEPTH, FUSE_RSTD><<<blocks, WAVES * 64, 0, s>>>(x, w, y, M, N, K, f);
-    else
-        gemm_skinny_kernel<RT, 1, WAVES, bf16_t, true, false, PIPE_DEPTH, FUSE_RSTD><<<blocks, WAVES * 64, 0, s>>>(x, w, y, M, N, K, f);
+#define SKINNY_FUSED(GATED, FUSE, XR, ...) \
+    gemm_skinny_kernel<RT, 1, WAVES, bf16_t, true, GATED, 2, FUSE, XR, ##__VA_ARGS__><<<blocks, WAVES * 64, 0, s>>>(x, w, y, M, N, K, f)
+#define SKINNY_RESIDUAL(XR) SKINNY_FUSED(false, FUSE_RESIDUAL, XR)
+#define SKINNY_RESIDUAL_WHOLE(XR) SKINNY_FUSED(false, FUSE_RESIDUAL, XR, true)
+#define SKINNY_RSTD_GATED(XR) SKINNY_FUSED(true, FUSE_RSTD, XR)
+#define SKINNY_RSTD(XR) SKINNY_FUSED(false, FUSE_RSTD, XR)
+#define SKINNY_RESIDUAL_HALF(XR) \
+    gemm_skinny_kernel<1, 1, WAVES, bf16_t, true, false, 2, FUSE_RESIDUAL, XR, true, true><<<(N + 7) / 8, WAVES * 64, 0, s>>>(x, w, y, M, N, K, f)
+#define SKINNY_RSTD_HALF(XR) \
+    gemm_skinny_kernel<1, 1, WAVES, bf16_t, true, false, 2, FUSE_RSTD, XR, false, true><<<(N + 7) / 8, WAVES * 64, 0, s>>>(x, w, y, M, N, K, f)
+    if constexpr (RT == 1) {
+        if (half) {
+            if (f.resid) SKINNY_ROWS(M, SKINNY_RESIDUAL_HALF)
+            else SKINNY_ROWS(M, SKINNY_RSTD_HALF)
+            return tli_check_launch("gemm_skinny (norm taken in)");
+        }
+    }
+    if (f.resid && N % 4 == 0) SKINNY_ROWS(M, SKINNY_RESIDUAL_WHOLE)
+    else if (f.resid) SKINNY_ROWS(M, SKINNY_RESIDUAL)
+    else if (gated) SKINNY_ROWS(M, SKINNY_RSTD_GATED)
+    else SKINNY_ROWS(M, SKINNY_RSTD)
     return tli_check_launch("gemm_skinny (norm taken in)");
 }
 
+// How many partial sums of squares a row has after a product into the residual: one for every 8 or 16 columns.
+extern "C" int tli_gemm_skinny_parts(int M, int N) { return half_tiles(M, N, 1) && N % 4 == 0 ? (N + 7) / 8 : (N + 15) / 16; }
+
 // The product with a norm taken in (see the top of this file), for up to 16 rows and W in the
 // decode layout.  Either  resid != null:  resid[M,N] += x . W^T (float32), xw[M,N] =
-// bfloat16(norm_w * resid), ssq_out[ceil(N/16)][M] = partial sums of resid^2 (y is not used);
+// bfloat16(norm_w * resid), ssq_out[tli_gemm_skinny_parts(M, N)][M] = partial sums of resid^2 (y is not used);
 // or  ssq_in != null:  y = (x . W^T) / sqrt(sum(ssq_in[parts_in][M]) / K + eps), through the
 // SwiGLU of a gated matrix if `gated` (y then [M, N/2]).
 extern "C" int tli_gemm_skinny_fused_bf16(const void* x, const void* w, void* y, int M, int N, int K, int gated,
@@ -463,11 +548,13 @@ extern "C" int tli_gemm_skinny_fused_bf16(const void* x, const void* w, void* y,
     const bf16_t* xp = (const bf16_t*)x;
     const bf16_t* wp = (const bf16_t*)w;
     const long tiles = (N + 15) / 16;
-    if (cfg == 0) cfg = tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
+    const bool half = !gated && half_tiles(M, N, 1) && (!resid || N % 4 == 0);     // (as tli_gemm_skinny_parts says)
+    if (cfg == 0) cfg = half ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
     if (gated && cfg < 20) cfg = 24;
     switch (cfg) {
         case 14: return launch_skinny_fused<1, 4>(xp, wp, (bf16_t*)y, M, N, K, gated, f, s);
         case 18: return launch_skinny_fused<1, 8>(xp, wp, (bf16_t*)y, M, N, K, gated, f, s);
+        case 8: return launch_skinny_fused<1, 8>(xp, wp, (bf16_t*)y, M, N, K, gated, f, s, true);
         case 24: return launch_skinny_fused<2, 4>(xp, wp, (bf16_t*)y, M, N, K, gated, f, s);
         case 28: return launch_skinny_fused<2, 8>(xp, wp, (bf16_t*)y, M, N, K, gated, f, s);
         default: return tli_fail("gemm_skinny: unknown configuration %d", cfg);
