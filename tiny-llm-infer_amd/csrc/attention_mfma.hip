@@ -982,22 +982,34 @@ attention_decode_solo_kernel(bf16_t* __restrict__ out, bf16_t* __restrict__ k_ca
 // grid (heads, rows); one thread per output element
 __global__ void attention_merge_splits_kernel(const float* __restrict__ partial, bf16_t* __restrict__ out,
                                               int heads, int head_dim, int splits) {
-    const int head = blockIdx.x, row = blockIdx.y;
-    const float* src = partial + ((size_t)row * heads + head) * splits * (head_dim + 2);
+    // A lane holds the maximum and sum of one split (64 at a time), so that a head waits for memory twice and not once a
+    // split: eight splits of 128 elements 8.7 -> 4.7 us.
+    const int head = blockIdx.x, row = blockIdx.y, lane = threadIdx.x;
+    const size_t step = head_dim + 2;
+    const float* src = partial + ((size_t)row * heads + head) * splits * step;
     float m = -INFINITY;
-    for (int s = 0; s < splits; ++s) m = fmaxf(m, src[(size_t)s * (head_dim + 2) + head_dim]);
+    for (int s0 = 0; s0 < splits; s0 += 64)
+        if (s0 + lane < splits) m = fmaxf(m, src[(s0 + lane) * step + head_dim]);
+    m = wave_max(m);
     const float base = (m == -INFINITY) ? 0.f : m;
     float l = 0.f;
-    for (int s = 0; s < splits; ++s) {
-        const float* p = src + (size_t)s * (head_dim + 2);
-        l += p[head_dim + 1] * __builtin_amdgcn_exp2f(p[head_dim] - base);
-    }
+    for (int s0 = 0; s0 < splits; s0 += 64)
+        if (s0 + lane < splits) l += src[(s0 + lane) * step + head_dim + 1] * __builtin_amdgcn_exp2f(src[(s0 + lane) * step + head_dim] - base);
+    l = wave_sum(l);
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    for (int d = threadIdx.x; d < head_dim; d += blockDim.x) {
+    for (int d = lane; d < head_dim; d += 64) {
         float a = 0.f;
-        for (int s = 0; s < splits; ++s) {
-            const float* p = src + (size_t)s * (head_dim + 2);
-            a += p[d] * __builtin_amdgcn_exp2f(p[head_dim] - base);
+        for (int s0 = 0; s0 < splits; s0 += 8) {
+            float v[8], w[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float* p = src + min(s0 + e, splits - 1) * step;
+                v[e] = p[d];
+                w[e] = p[head_dim];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (s0 + e < splits) a = fmaf(v[e], __builtin_amdgcn_exp2f(w[e] - base), a);
         }
         out[((size_t)row * heads + head) * head_dim + d] = f32_to_bf16(a * inv);
     }
