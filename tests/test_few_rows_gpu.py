@@ -1,0 +1,88 @@
+"""Decode products whose columns are taken in half tiles of eight (1,024 to 2,048 outputs, up to 16 rows), beside float64 at
+the edges of their tiles; and decode attention where a row's keys are cut into many short splits."""
+import math
+
+import pytest
+import torch
+
+from test_long_context_gpu import close, fill, make_step, ref_attention_dev, rnd_dev
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+BF = torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from tiny_llm_infer_amd.kernels.ops import HipOps
+    return HipOps(DEV)
+
+
+def allowed(x, w, extra=0.0):
+    """K float32 additions of exact products, and the rounding of the result to bfloat16."""
+    terms = x.double().abs() @ w.double().abs().T + extra
+    return (x.shape[1] * 2.0 ** -24) * terms
+
+
+# (rows, outputs, k): either end of the range and one past it on both sides, outputs that end inside a half tile, between the
+# halves of one and not in whole float4s; k of one step and of a ragged last one; 1, 4, 5, 8, 9 and 16 rows (the rows' loads)
+HALF_SIZES = [(1, 1024, 128), (4, 1500, 264), (5, 2048, 1032), (8, 1030, 72), (9, 1031, 640), (16, 1992, 2056), (3, 1016, 256),
+              (2, 2064, 256), (17, 1024, 256)]
+
+
+@pytest.mark.parametrize("mnk", HALF_SIZES)
+def test_half_tiles(ops, mnk):
+    from tiny_llm_infer_amd.parts.base import BuildEnv
+    from tiny_llm_infer_amd.parts.linear import Matrix
+    M, N, K = mnk
+    env = BuildEnv(dtype=BF, device=torch.device(DEV), ops=ops, max_model_len=64)
+    x, w = rnd_dev((M, K), 1), rnd_dev((N, K), 2, 0.05)
+    m = Matrix(w, env)
+    want, tol = x.double() @ w.double().T, allowed(x, w)
+    y32 = ops.linear(x, m, out_dtype=torch.float32)
+    assert bool(((y32.double() - want).abs() <= tol).all())
+    y = ops.linear(x, m)
+    assert bool(((y.double() - want).abs() <= tol + 2.0 ** -8 * want.abs()).all())
+    unit = ops.linear_act(x, m, "relu2")
+    relu = want.clamp(min=0)
+    assert bool(((unit.double() - relu * relu).abs() <= 2 * relu * tol + tol * tol + 2.0 ** -7 * relu * relu).all())
+    if M > 16:
+        return
+    # into the residual: the sum, the next norm's rows and their sums of squares
+    resid, nw = rnd_dev((M, N), 3).float(), 1 + rnd_dev((N,), 4, 0.2).float()
+    r = resid.clone()
+    normed = ops.add_rmsnorm(r, ops.linear(x, m, deferred=True), nw, 1e-5, BF, lazy=True)
+    h = resid.double() + want
+    slack = allowed(x, w, resid.double().abs()) + 2.0 ** -23 * h.abs()
+    assert bool(((r.double() - h).abs() <= slack).all())
+    assert torch.allclose(normed.ssq.sum(0).double(), (h * h).sum(-1), rtol=1e-4)
+    # and from normed rows, back to a product of half tiles
+    back = rnd_dev((1536, N), 5, 0.05)
+    if N % 8 == 0:
+        z = ops.linear(normed, Matrix(back, env))
+        n = nw.double() * h / torch.sqrt((h * h).mean(-1, keepdim=True) + 1e-5)
+        # the normed rows are rounded to bfloat16 once, the result once
+        limit = 2.0 ** -8 * (n.abs() @ back.double().abs().T) + 2.0 ** -8 * (n @ back.double().T).abs() + 1e-3
+        assert bool(((z.double() - n @ back.double().T).abs() <= limit).all())
+
+
+# heads, kv heads, head_dim, page, lengths, splits: eight splits of 128 keys at the first length that is split; sixteen and
+# more of 256; counts that are no multiple of eight; two workgroups a compute unit; rows far too short for most splits
+SPLITS = [(32, 8, 128, 16, [513], 8), (32, 8, 128, 16, [1024, 1, 129, 640], 8), (16, 2, 64, 8, [4096], 16),
+          (8, 4, 256, 16, [4097], 32), (32, 8, 128, 16, [2100, 2049, 700], 11), (32, 8, 128, 16, [1500] * 9, 4),
+          (32, 8, 128, 32, [3000, 5, 2900, 2500, 3100, 4000, 2049, 128, 3000, 3500, 127, 3300], 6)]
+
+
+@pytest.mark.parametrize("case", SPLITS, ids=lambda c: f"{len(c[4])}x{c[4][0]}-{c[1]}x{c[2]}")
+def test_short_splits(ops, case):
+    heads, kv_heads, hd, page, lens, splits = case
+    num_pages = sum((n + page - 1) // page for n in lens) + 5
+    step, tables, pos, seq = make_step(lens, [1] * len(lens), page, num_pages, 5, kv_heads, hd, BF, None)
+    if ops.DECODE_WORKGROUPS == 256:
+        assert ops._decode_splits(len(lens), step.reach, step.cache.group, heads, kv_heads, hd, None)[0] == splits
+    ks, vs = fill(step, tables, lens, kv_heads, hd, 100)
+    q = rnd_dev((len(pos), heads * hd), 50)
+    scale = 1 / math.sqrt(hd)
+    out = ops.paged_attention(q, step, step.cache, heads, kv_heads, hd, scale, None)
+    close(out, ref_attention_dev(q, ks, vs, pos, seq, heads, kv_heads, scale, None), "short splits")

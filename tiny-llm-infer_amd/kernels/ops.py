@@ -221,7 +221,7 @@ class HipOps:
     MID_ROWS_TO_PLAIN = 256      # a product without a gate: up to this many (two blocks of 128 rows side by side)
     DECODE_WORKGROUPS = 256      # the device's compute units (set to what the device reports when the library is loaded):
                                  # the decode attention splits a row's keys to come near one workgroup for each
-    DECODE_SPLIT_KEYS = 1024     # a split walks at least this many keys
+    DECODE_SPLIT_KEYS = 256      # a split of a few rows walks this many keys
     # A step of prompt portions whose first sequences decode: the prefill kernel takes a row that decodes
     # as a sequence of one row, beside its other workgroups; the decode kernel is a second launch (8 to 10
     # us) that runs before it, but splits a long row's keys and puts four waves on a row.  Those rows go
@@ -939,27 +939,45 @@ class HipOps:
         keys of the average one."""
         reach = reach if not window else min(reach, (window + 31) // 32 * 32 + 32)
         groups = T * kv_heads * ((heads // kv_heads + 15) // 16)
-        # A split costs a pass that merges the parts (4 to 5 us) and a workgroup that walks no more than
-        # 1,500 keys is done in the time of the shortest split run (13 to 17 us against 17.5), so: no split
-        # up to a reach of 2,048 keys; beyond, towards one workgroup a compute unit, half of that for 16
-        # (row, kv head) pairs and fewer (more parts than that cost more in the merge than they save in the
-        # walk), and splits of at least 1,024 keys, of 4,096 from a quarter of the compute units on (there
-        # the workgroups already share the memory's rate between them).  Measured at heads of 128, 1 to 64
-        # rows of 600 to 32,768 keys, every power of two of splits: this rule is within 8% of the best
-        # everywhere; the one before (256 workgroups, 512 keys) was up to 45% over it at 1,024 keys and 20%
-        # over it at 1 and 2 rows of 16,384 keys and more.
+        # A workgroup fetches its keys at about 45 bytes a ns whatever the rest of the chip does, so a few
+        # long rows are done the sooner the more workgroups walk them, until there is one a compute unit.
+        # Against that stand the pass that merges the parts (3 to 5 us; it sums eight of them at once) and
+        # the fixed part of a workgroup.  Measured at 32 query and 8 kv heads of 128 (2 and 32 kv heads and
+        # heads of 256 agree), from raw projections, us, unsplit / this rule:
+        #   1 row of 520 keys 10.2 / 9.2, of 1,500 19.4 / 12.0; 8 rows of 520 11.4 / 11.9, of 1,000 20.2 /
+        #   16.0; up to a reach of 512 keys no split is better (1 row of 300 keys 8.5 / 9.3).
+        #   1 row of 3,000 keys 32.0 / 12.8, of 8,000 97 / 18.1, of 32,000 (32 splits) 34.7, with 16 40.3.
+        #   16 rows of 2,000 keys 40.0 / 33.4, of 6,000 103 / 86; of 600 16.9 and in two splits 18.9.
+        #   24 rows of 2,100 keys 46.0, in two splits 50.5, of 5,000 98 and 107: from more pairs than half
+        #   the compute units on the memory's rate is what bounds them.
+        # Hence: towards a workgroup a compute unit of splits of 256 keys (eight splits of 128 at a reach of
+        # 1,024; more than 32 only of 1,024 keys each); from a quarter of the units to half of them two
+        # workgroups a unit of 512 keys; fewer than four splits never pay.  Splits of at least 1,024 keys,
+        # the rule when the merge took twice as long: 18.5 at 1 row of 3,000 keys, 24 at 2 rows of 6,000.
         # Sequences of unequal lengths: the workgroups of the short ones are done early, so the step's
-        # rows count as that many fewer of the longest one's length (32 rows, one of 4,000 keys and 31 of
-        # 300: 40 us unsplit, 30 us in four splits; 16 rows of 64 to 2,304 keys: 24.3 and 22.5 us).  With a
-        # window every row walks about as many keys.
+        # rows count as that many fewer of the longest one's length; but each of the short rows' workgroups
+        # costs 5 ns all the same, so beyond eight splits there are two workgroups a unit over all rows, and
+        # never more than eight a unit unless splits would grow beyond 2,048 keys (31 rows of 200 keys and
+        # one of 4,000: 54.5 unsplit, 35.1 in eight, 48.1 in sixteen), and no split of more rows than a
+        # quarter of the units below a reach of 4,096 (one of 900 keys beside 15 of 200: 15.0 and in eight
+        # 17.2).  With a window every row walks about as many keys.
+        every = groups
+        units = self.DECODE_WORKGROUPS
+        least = 4 * self.DECODE_SPLIT_KEYS
         if skew > 1 and not window:
             groups = max(1, groups // skew)
-        units = self.DECODE_WORKGROUPS
+            least = least if every <= units // 4 else 16 * self.DECODE_SPLIT_KEYS
         splits = 1
-        if reach > 2 * self.DECODE_SPLIT_KEYS and groups < units:
-            aim = units // 2 if groups <= units // 16 else units
-            least = self.DECODE_SPLIT_KEYS if groups <= units // 4 else 4 * self.DECODE_SPLIT_KEYS
-            splits = max(1, min((aim + groups - 1) // groups, reach // least, 64))
+        if reach >= least and groups <= units // 2:
+            if groups <= units // 4:
+                splits = min(-(-units // groups), max(8, min(reach // self.DECODE_SPLIT_KEYS, 32), reach // 1024), 64)
+            else:
+                splits = min(-(-2 * units // groups), reach // 512, 64)
+            if skew > 1 and not window:
+                cap = min(8 * units // every, max(8, 2 * units // every))
+                splits = min(splits, max(cap, reach // 2048))
+            if splits < 4:
+                splits = 1
         # (a split's block table entries are kept in LDS: at most 2046 pages a split)
         splits = max(splits, -(-reach // (2046 * g.page_size // 128 * 128)))
         per_split = ((reach + splits - 1) // splits + 127) // 128 * 128
