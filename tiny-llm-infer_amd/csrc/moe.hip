@@ -17,9 +17,9 @@
 // down:    y_c = sum_j weight_j (a_j . Wd_e(j)[c])  (+ shared gate * shared_c), summed in the order of
 //          the choice, so that a row's result does not depend on what else is in the step.
 //
-// These kernels walk the pairs one by one, each reading its expert's matrices: what a decode step
-// needs anyway, and the float32 path.  Steps of many rows in bfloat16 sort the pairs by expert and
-// multiply tile by tile (moe_grouped.hip).
+// These kernels walk the pairs one by one, each reading its expert's matrices: the float32 path, and
+// what the others do not take.  Steps of up to 64 rows in bfloat16 go expert by expert (moe_few.hip),
+// steps of more rows sort the pairs by expert and multiply tile by tile (moe_grouped.hip).
 #include "common.h"
 
 #define MOE_MAX_TOP 32
@@ -102,7 +102,14 @@ __device__ __forceinline__ void wave_best(float& v, int& index) {
     }
 }
 
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
+
+// A workgroup a row: what bounds it is the time of a fetch from memory and the chain of lane exchanges of the choice, so a
+// wave makes COLS of the logits at once (17 of them, 16 experts and a shared gate, took two rounds of fetches before) and the
+// correction comes in beside them.  8 rows of 2,048, 16 experts and a shared gate: 7.1 us before, 6.4 now.
 #define ROUTER_THREADS 1024
+#define ROUTER_WAVES (ROUTER_THREADS / TLI_WAVE)
+template <int COLS>
 __global__ __launch_bounds__(ROUTER_THREADS) void moe_router_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int D,
                                                                     int* __restrict__ ids, float* __restrict__ weights,
                                                                     float* __restrict__ shared_gate, int E, int top, int groups,
@@ -114,21 +121,33 @@ __global__ __launch_bounds__(ROUTER_THREADS) void moe_router_kernel(const bf16_t
     const size_t t = blockIdx.x;
     const int lane = threadIdx.x % TLI_WAVE, wave = threadIdx.x / TLI_WAVE;
     const bf16_t* xr = x + t * D;
-    for (int e = wave; e < E + (has_shared ? 1 : 0); e += ROUTER_THREADS / TLI_WAVE) {
-        const bf16_t* we = w + (size_t)e * D;
-        float a = 0.f;
-#pragma unroll 4
-        for (int i = lane * 8; i < D; i += TLI_WAVE * 8) {
-            const uint4 p = *reinterpret_cast<const uint4*>(xr + i), q = *reinterpret_cast<const uint4*>(we + i);
-            const uint32_t u[4] = {p.x, p.y, p.z, p.w}, v[4] = {q.x, q.y, q.z, q.w};
+    const int cols = E + (has_shared ? 1 : 0);
+    for (int e = threadIdx.x; e < E; e += ROUTER_THREADS) c[e] = correction ? correction[e] : 0.f;     // (fetched beside the rows)
+    for (int e0 = wave; e0 < cols; e0 += COLS * ROUTER_WAVES) {
+        constexpr int UNROLL = COLS > 2 ? 2 : 4;
+        const bf16_t* we[COLS];                    // (past the last row: the last one again, its sum not kept)
+        float a[COLS];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                a = fmaf(__uint_as_float(u[k] << 16), __uint_as_float(v[k] << 16), a);
-                a = fmaf(__uint_as_float(u[k] & 0xFFFF0000u), __uint_as_float(v[k] & 0xFFFF0000u), a);
-            }
+        for (int j = 0; j < COLS; ++j) we[j] = w + (size_t)min(e0 + j * ROUTER_WAVES, cols - 1) * D, a[j] = 0.f;
+#pragma unroll UNROLL
+        for (int i = lane * 8; i < D; i += TLI_WAVE * 8) {
+            const u32x4_t u = *reinterpret_cast<const u32x4_t*>(xr + i);
+            u32x4_t v[COLS];
+#pragma unroll
+            for (int j = 0; j < COLS; ++j) v[j] = *reinterpret_cast<const u32x4_t*>(we[j] + i);
+#pragma unroll
+            for (int j = 0; j < COLS; ++j)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    a[j] = fmaf(__uint_as_float(u[k] << 16), __uint_as_float(v[j][k] << 16), a[j]);
+                    a[j] = fmaf(__uint_as_float(u[k] & 0xFFFF0000u), __uint_as_float(v[j][k] & 0xFFFF0000u), a[j]);
+                }
         }
-        a = wave_sum(a);
-        if (lane == 0) s[e] = a;
+#pragma unroll
+        for (int j = 0; j < COLS; ++j) {
+            const float sum = wave_sum(a[j]);
+            if (lane == 0 && e0 + j * ROUTER_WAVES < cols) s[e0 + j * ROUTER_WAVES] = sum;
+        }
     }
     __syncthreads();
     if (wave > 0) return;
@@ -146,7 +165,7 @@ __global__ __launch_bounds__(ROUTER_THREADS) void moe_router_kernel(const bf16_t
     } else {
         for (int e = lane; e < E; e += TLI_WAVE) s[e] = 1.0f / (1.0f + expf(-s[e]));
     }
-    for (int e = lane; e < E; e += TLI_WAVE) c[e] = correction ? s[e] + correction[e] : s[e];
+    for (int e = lane; e < E; e += TLI_WAVE) c[e] = correction ? s[e] + c[e] : s[e];
     wave_lds_sync();
     const int per = E / groups;
     unsigned long long open = ~0ull;               // the `keep` best groups, a bit each (groups <= 64: one a lane)
@@ -283,9 +302,14 @@ extern "C" int tli_moe_router_bf16(const void* x, const void* w, int D, int* ids
         return tli_fail("moe_router: bad sizes (experts %d, top %d (at most %d), groups %d (at most 64), keep %d, width %d)", E, top,
                         MOE_MAX_TOP, groups, keep, D);
     if (((uintptr_t)x | (uintptr_t)w) & 15) return tli_fail("moe_router: operands must be 16-byte aligned");
-    moe_router_kernel<<<T, ROUTER_THREADS, (size_t)(2 * E + 1) * sizeof(float), (hipStream_t)stream>>>(
-        (const bf16_t*)x, (const bf16_t*)w, D, ids, weights, shared_gate, E, top, groups, keep, scale, has_shared, softmax_scores,
-        group_by_max, normalize, correction);
+    const int rounds = (E + (has_shared ? 1 : 0) + ROUTER_WAVES - 1) / ROUTER_WAVES;
+#define ROUTER_LAUNCH(COLS)                                                                                              \
+    moe_router_kernel<COLS><<<T, ROUTER_THREADS, (size_t)(2 * E + 1) * sizeof(float), (hipStream_t)stream>>>(            \
+        (const bf16_t*)x, (const bf16_t*)w, D, ids, weights, shared_gate, E, top, groups, keep, scale, has_shared,       \
+        softmax_scores, group_by_max, normalize, correction)
+    if (rounds == 1) ROUTER_LAUNCH(1);
+    else if (rounds == 2) ROUTER_LAUNCH(2);
+    else ROUTER_LAUNCH(4);
     return tli_check_launch("moe_router");
 }
 
