@@ -1,6 +1,7 @@
 // Plain attention over the paged cache: one workgroup per (head, row), any
-// sizes, float32 or bfloat16 storage, float32 arithmetic.  This is the
-// attention of the float32 path and the reference beside the tuned kernels.
+// sizes, float32 or bfloat16 storage, float32 arithmetic.  It takes what
+// attention_f32.hip leaves of the float32 path (heads of other sizes, pages that
+// are no multiple of four) and is the reference beside the tuned kernels.
 //
 // Row at position p, head h, kv head g = h / (heads / kv_heads):
 //   s_t = (q_h . K_t,g) * scale   for t = lo..p,  lo = 0 or p - window + 1

@@ -1,9 +1,9 @@
 // Plain tiled matrix product y[M,N] = x[M,K] . W[N,K]^T for any sizes and for
 // float32 or bfloat16 inputs, float32 accumulation in a fixed order (k
 // ascending, no split over k), so a row's result does not depend on how many
-// other rows are in the batch.  This is the matrix product of the float32 path
-// (plain FMA, no reduced-precision matrix mode) and the reference beside the
-// MFMA kernels.  Weights are [out, in] row-major as the reference stores them
+// other rows are in the batch.  It takes what gemm_f32.hip leaves of the float32
+// path (rows that are not whole 16-byte pieces, mixed types) and is the reference
+// beside the MFMA kernels (plain FMA, no reduced-precision matrix mode).  Weights are [out, in] row-major as the reference stores them
 // (kernels/src/matmul_kernel_cpu.cpp:27-35).
 #include "common.h"
 

@@ -282,8 +282,8 @@ class HipOps:
         return self.many_rows != "own"
 
     def use_plain_kernels(self) -> None:
-        """Every product, attention and norm through the plain kernels, bfloat16 too
-        (what the float32 path runs): to tell a fault of a tuned kernel from one elsewhere."""
+        """Every product, attention and norm through the plain kernels, bfloat16 and float32:
+        to tell a fault of a tuned kernel from one elsewhere."""
         self.force_plain = self.plain_products = self.separate_norms = self.unfused_decode = True
 
     # ---- helpers ----------------------------------------------------------
