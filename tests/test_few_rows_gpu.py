@@ -1,4 +1,4 @@
-"""Decode products whose columns are taken in half tiles of eight (1,024 to 2,048 outputs, up to 16 rows), beside float64 at
+"""Decode products whose columns are taken in half tiles of eight (up to 2,048 outputs and 16 rows), beside float64 at
 the edges of their tiles; and decode attention where a row's keys are cut into many short splits."""
 import math
 
@@ -25,10 +25,10 @@ def allowed(x, w, extra=0.0):
     return (x.shape[1] * 2.0 ** -24) * terms
 
 
-# (rows, outputs, k): either end of the range and one past it on both sides, outputs that end inside a half tile, between the
+# (rows, outputs, k): either end of the range into the residual and one past it on both sides, and few outputs; outputs that end inside a half tile, between the
 # halves of one and not in whole float4s; k of one step and of a ragged last one; 1, 4, 5, 8, 9 and 16 rows (the rows' loads)
 HALF_SIZES = [(1, 1024, 128), (4, 1500, 264), (5, 2048, 1032), (8, 1030, 72), (9, 1031, 640), (16, 1992, 2056), (3, 1016, 256),
-              (2, 2064, 256), (17, 1024, 256)]
+              (2, 2064, 256), (17, 1024, 256), (2, 8, 128), (16, 17, 264), (6, 250, 2048), (11, 72, 4096)]
 
 
 @pytest.mark.parametrize("mnk", HALF_SIZES)

@@ -417,9 +417,12 @@ static int launch_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N
     return tli_check_launch("gemm_skinny");
 }
 
-// Half tiles where whole ones leave half of the chip or more without a workgroup, and the matrix is not so small that its
-// product is all launch and latency.
-static bool half_tiles(int M, int N, int tiled) { return M <= 16 && tiled == 1 && N >= 1024 && (N + 15) / 16 <= tli_compute_units() / 2; }
+// Half tiles where whole ones leave half of the chip or more without a workgroup.  Cold weights, 8 rows, whole and half: 64
+// columns of k 2,048 3.68 and 3.46 us, 256 of 4,096 5.16 and 4.64, 768 of 6,144 7.51 and 6.64; 1 and 16 rows gain as much.
+// Into the residual only from 1,024 columns on: each half tile leaves sums of squares that the next product adds up.
+static bool half_tiles(int M, int N, int tiled, bool into_residual) {
+    return M <= 16 && tiled == 1 && (N + 15) / 16 <= tli_compute_units() / 2 && (!into_residual || (N >= 1024 && N % 4 == 0));
+}
 
 template <int MT>
 static int pick_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N, int K, int y_dtype,
@@ -427,7 +430,7 @@ static int pick_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N, 
     // cfg 0: by shape.  Narrow outputs get one 16-column tile per workgroup so that
     // even N = 4096 gives 256 workgroups; wide outputs share x over two tiles.
     const long tiles = (N + 15) / 16;
-    if (cfg == 0) cfg = half_tiles(M, N, tiled) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
+    if (cfg == 0) cfg = half_tiles(M, N, tiled, false) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
     if (tiled == 2 && cfg < 20) cfg = 24;          // gated needs pairs of row tiles
     switch (cfg) {
         case 14: return launch_skinny<1, MT, 4>(x, w, y, M, N, K, y_dtype, tiled, gate, inputs, unit, s);
@@ -520,7 +523,7 @@ static int launch_skinny_fused(const bf16_t* x, const bf16_t* w, bf16_t* y, int 
 }
 
 // How many partial sums of squares a row has after a product into the residual: one for every 8 or 16 columns.
-extern "C" int tli_gemm_skinny_parts(int M, int N) { return half_tiles(M, N, 1) && N % 4 == 0 ? (N + 7) / 8 : (N + 15) / 16; }
+extern "C" int tli_gemm_skinny_parts(int M, int N) { return half_tiles(M, N, 1, true) ? (N + 7) / 8 : (N + 15) / 16; }
 
 // The product with a norm taken in (see the top of this file), for up to 16 rows and W in the
 // decode layout.  Either  resid != null:  resid[M,N] += x . W^T (float32), xw[M,N] =
@@ -548,7 +551,7 @@ extern "C" int tli_gemm_skinny_fused_bf16(const void* x, const void* w, void* y,
     const bf16_t* xp = (const bf16_t*)x;
     const bf16_t* wp = (const bf16_t*)w;
     const long tiles = (N + 15) / 16;
-    const bool half = !gated && half_tiles(M, N, 1) && (!resid || N % 4 == 0);     // (as tli_gemm_skinny_parts says)
+    const bool half = !gated && half_tiles(M, N, 1, resid != nullptr);     // (as tli_gemm_skinny_parts says)
     if (cfg == 0) cfg = half ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
     if (gated && cfg < 20) cfg = 24;
     switch (cfg) {
