@@ -1,6 +1,8 @@
 """The routed experts of few rows in two launches, the shared expert among them, beside float64: tiles of 16 rows and their
 edges, more experts than pairs and fewer, k of less than a step of 128 and of more steps than waves, experts that hand
 their input on; and a row's independence of the rows beside it."""
+import math
+
 import pytest
 import torch
 
@@ -113,3 +115,58 @@ def test_sizes_that_other_kernels_take(ops):
     assert ops.experts_of_few_rows(w["x"], ids, weights, packed, None, None, None) is None
     w, packed, ids, weights, _ = make(ops, (2, 300, 0, 2, 64, 32, 0), "silu")
     assert ops.experts_of_few_rows(w["x"], ids, weights, packed, None, None, None) is None
+
+
+# (experts, top, groups, kept groups): more places than lanes share experts; several experts a lane; groups of which some are out
+CHOICES = [(16, 2, 1, 1), (64, 8, 1, 1), (40, 3, 4, 2), (130, 32, 1, 1)]
+
+
+def _diverged(x):
+    """Rows that hold no numbers, among others that do: all NaN, one NaN, an infinity of either sign, one past another."""
+    x = x.clone()
+    x[0], x[1, 3], x[5, 2], x[6, 7], x[11, :2] = math.nan, math.nan, math.inf, -math.inf, math.inf
+    x[8], x[9] = math.nan, math.nan
+    return x, [2, 3, 4, 7, 10, 12, 13, 14, 15]
+
+
+@pytest.mark.parametrize("score", ["sigmoid", "softmax"])
+@pytest.mark.parametrize("choice", CHOICES)
+def test_choice_for_rows_that_hold_no_numbers(ops, choice, score):
+    """Whatever a row holds, its choice is of different experts, and the other rows' is what it is without it."""
+    E, top, groups, keep = choice
+    g = torch.Generator(device=DEV).manual_seed(E)
+    x = torch.randn((16, 72), generator=g, device=DEV).to(BF)
+    rows = (torch.randn((E + 1, 72), generator=g, device=DEV) * 0.3).to(BF)
+    bad, healthy = _diverged(x)
+    want = ops.router(x, rows, E, top, groups, keep, 1.0, True, score=score)
+    got = ops.router(bad, rows, E, top, groups, keep, 1.0, True, score=score)
+    for a, b in zip(got, want):
+        assert torch.equal(a[healthy], b[healthy])
+    z = torch.randn((3, E + 1), generator=g, device=DEV)
+    z[1], z[2, E // 2] = math.nan, math.nan
+    from_logits = ops.route_experts(z, E, top, groups, keep, 1.0, True, score=score)[0]
+    for ids in (got[0], from_logits):
+        assert int(ids.min()) >= 0 and int(ids.max()) < E
+        assert bool((ids.sort(dim=1).values.diff(dim=1) > 0).all()), "an expert was chosen twice"
+    assert torch.equal(got[0][0], from_logits[1]), "the two kernels choose differently for a row of NaNs"
+
+
+@pytest.mark.parametrize("sizes", [(16, 4), (64, 8)])
+def test_diverged_rows_leave_the_others_alone(ops, sizes):
+    """Router and experts of 16 rows, eight of them diverged, some before healthy ones in the step: the healthy rows are bit for
+    bit what they are without them.  (The memory that the parts come from holds NaNs beforehand.)"""
+    E, top = sizes
+    w, packed, _, _, _ = make(ops, (16, E, 0, top, 128, 64, 0), "silu")
+    rows = (torch.randn((E, 128), generator=torch.Generator(device=DEV).manual_seed(3), device=DEV) * 0.3).to(BF)
+    bad, healthy = _diverged(w["x"])
+    bad[12] = math.nan
+    healthy.remove(12)
+
+    def run(x):
+        ids, weights, _ = ops.router(x, rows, E, top, 1, 1, 1.0, False)
+        stale = torch.full((top, 16, 128), math.nan, device=DEV)
+        del stale
+        return ops.resolve(ops.experts_of_few_rows(x, ids, weights, packed, None, None, None))
+    want, got = run(w["x"]), run(bad)
+    assert torch.equal(got[healthy], want[healthy])
+    assert bool(got[[0, 8, 9, 12]].isnan().all())

@@ -24,6 +24,11 @@
 
 #define MOE_MAX_TOP 32
 
+// What the choice goes by.  A score that is no number (a row with a NaN or an infinity in it) counts as the lowest: a NaN
+// compares as neither larger nor smaller, the lanes of a choice would not agree on the largest, and an expert could be chosen
+// twice.
+__device__ __forceinline__ float choice_score(float v) { return v != v ? -INFINITY : v; }
+
 __global__ void moe_route_kernel(const float* __restrict__ z, long long z_row, long long z_col, int* __restrict__ ids,
                                  float* __restrict__ weights, float* __restrict__ shared_gate, int T, int E,
                                  int top, int groups, int keep, float scale, int has_shared, int softmax_scores,
@@ -45,7 +50,7 @@ __global__ void moe_route_kernel(const float* __restrict__ z, long long z_row, l
     } else {
         for (int e = 0; e < E; ++e) s[e] = 1.0f / (1.0f + expf(-zr[(size_t)e * z_col]));
     }
-    for (int e = 0; e < E; ++e) c[e] = correction ? s[e] + correction[e] : s[e];
+    for (int e = 0; e < E; ++e) c[e] = choice_score(correction ? s[e] + correction[e] : s[e]);
     if (has_shared) shared_gate[t] = 1.0f / (1.0f + expf(-zr[(size_t)E * z_col]));
     const int per = E / groups;
     // the `keep` best groups, as a bit a group (groups <= 64)
@@ -165,7 +170,7 @@ __global__ __launch_bounds__(ROUTER_THREADS) void moe_router_kernel(const bf16_t
     } else {
         for (int e = lane; e < E; e += TLI_WAVE) s[e] = 1.0f / (1.0f + expf(-s[e]));
     }
-    for (int e = lane; e < E; e += TLI_WAVE) c[e] = correction ? s[e] + c[e] : s[e];
+    for (int e = lane; e < E; e += TLI_WAVE) c[e] = choice_score(correction ? s[e] + c[e] : s[e]);
     wave_lds_sync();
     const int per = E / groups;
     unsigned long long open = ~0ull;               // the `keep` best groups, a bit each (groups <= 64: one a lane)
