@@ -170,3 +170,26 @@ def test_diverged_rows_leave_the_others_alone(ops, sizes):
     want, got = run(w["x"]), run(bad)
     assert torch.equal(got[healthy], want[healthy])
     assert bool(got[[0, 8, 9, 12]].isnan().all())
+
+
+@pytest.mark.parametrize("size", [(3, 4, 0, 2, 72, 40, 48), (16, 16, 0, 3, 136, 72, 0), (17, 8, 1, 4, 136, 272, 32), (20, 200, 0, 4, 96, 48, 0),
+                                  (64, 5, 0, 8, 128, 64, 16)])
+@pytest.mark.parametrize("kind", ["silu", "relu2"])
+def test_rows_that_name_an_expert_twice(ops, size, kind):
+    """More pairs of an expert than rows: the slots are filled several times, and no part is left as the memory was."""
+    T, E, identity, top, D = size[:5]
+    if kind == "relu2" and identity:
+        pytest.skip("experts whose weight goes on their input all have matrices")
+    w, packed, ids, weights, (up, down, gate) = make(ops, (T, max(E, top), identity, top, *size[4:]), kind)
+    E = max(E, top)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    ids = torch.randint(0, 2, (T, top), generator=g, device=DEV, dtype=torch.int32) + E - 2 + identity
+    weights = torch.rand((T, top), generator=g, device=DEV)
+    how = {"silu": {}, "relu2": dict(activation="relu2", weight_on_input=True)}[kind]
+    stale = torch.full((top + 1, T, D), math.nan, device=DEV)
+    del stale
+    got = ops.resolve(ops.experts_of_few_rows(w["x"], ids, weights, packed, up, down, gate, handed_on=identity > 0, **how))
+    want = plain(w, ids, weights, gate, E, kind)
+    # as for test_experts_of_few_rows; terms of the same expert add up, by at most the root of their number (8 places: 3 times)
+    scale = float(want.square().mean().sqrt())
+    assert float((got.double() - want).abs().max()) <= 15 * 2.0 ** -9 * scale + 2.0 ** -8 * float(want.abs().max())

@@ -5,7 +5,8 @@
 //            shared expert for every row
 //   down:    part[j, row] = weight[row, j] (hid[row, j] . Wd_e) for the j-th expert of a row's choice, and behind them
 //            part[top, row] = shared gate * (hid . Wd) of the shared expert; experts that hand their input on give weight * x.
-//            The sum of the parts, in their order, is the block's output: whoever reads it adds them up.
+//            The sum of the parts, in their order, is the block's output: whoever reads it adds them up.  Every part is written,
+//            whichever experts a row names.
 //
 // Both are one kernel: a workgroup takes 32 rows of one expert's matrix (16 gate and 16 up rows of a gated one) and finds
 // that expert's pairs of (row, place in the choice) itself, by looking through the choice: there is no sort.
@@ -95,6 +96,35 @@ __device__ __forceinline__ void in_steps(int count, L load, M multiply) {
 #define FEW_UP 1                 // hidden units of up rows alone
 #define FEW_DOWN 2
 
+// The pairs of an expert that found no slot, without the matrix cores: there are slots for as many pairs as rows, so these are
+// only of choices that name an expert more than once in a row.  A wave a pair, a lane an output of the workgroup's two tiles
+// `a` and `b` of W and one half of every 128 of k.
+template <int KIND>
+__device__ __forceinline__ void pairs_without_slot(const FewExperts& f, int e, int slots, const bf16_t* a, const bf16_t* b, int block, int K) {
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, waves = blockDim.x / 64;
+    const bf16_t* w = lane % 32 < 16 ? a : b;
+    for (int p = 0, n = 0; p < f.T * f.top; ++p) {
+        if (f.ids[p] != e) continue;
+        const int rank = n++;
+        if (rank < slots || rank % waves != wave) continue;
+        const bf16_t* x = KIND == FEW_DOWN ? f.hid + (size_t)p * K : f.x + (size_t)(p / f.top) * K;
+        float s = 0.f;
+        for (int i = 0; i < (K + 127) / 128 * 64; ++i) {             // (64 of 128 a step: c of two, j of four, eight in a row)
+            const int kb = i / 64, c = lane / 32 * 2 + i / 32 % 2, j = i / 8 % 4, k = kb * 128 + c * 32 + i % 32;
+            if (k < K) s = fmaf(bf16_to_f32(w[(size_t)kb * 2048 + j * 512 + (16 * c + lane % 16) * 8 + i % 8]), bf16_to_f32(x[k]), s);
+        }
+        s += __shfl_xor(s, 32, 64);
+        const float other = __shfl_xor(s, 16, 64);
+        const int unit = KIND == FEW_GATED ? block * 16 + lane % 16 : block * 32 + lane % 32;
+        if (KIND == FEW_DOWN) {
+            if (lane < 32 && unit < f.D)
+                f.part[((size_t)(p % f.top) * f.T + p / f.top) * f.D + unit] = (f.weights ? f.weights[p] : 1.0f) * s;
+        } else if (lane < (KIND == FEW_GATED ? 16 : 32) && unit < f.ff) {
+            from_f32(f.hid + (size_t)p * f.ff + unit, KIND == FEW_GATED ? gated_unit(s, other, f.unit.limit, f.unit.slope) : act_of(f.unit.of_pair(p) * s, f.unit.kind));
+        }
+    }
+}
+
 // Blocks 0 .. s_blocks-1 are the shared expert's (FEW_DOWN: also of the experts that hand their input on); then `blocks` for each candidate expert: expert y where there are no more
 // experts than pairs, else the expert of pair y, if no pair before it has the same.
 template <int RB, int KIND>
@@ -109,7 +139,7 @@ __global__ void __launch_bounds__(256) moe_few_kernel(FewExperts f, int s_blocks
     const int block = shared ? blockIdx.x : (blockIdx.x - s_blocks) % blocks;
     const int P = f.T * f.top;
     int* mine = slots[wave];
-    int e = 0, n = 0;                                        // the expert, and its number of pairs
+    int e = 0, n = 0;                                        // the expert, and its number of pairs with a slot
     if (DOWN && shared && f.handed_on) {
         for (int i = threadIdx.x; i < P * 32; i += WAVES * 64) {
             const int p = i / 32, t = p / f.top, col = block * 32 + i % 32;
@@ -135,7 +165,14 @@ __global__ void __launch_bounds__(256) moe_few_kernel(FewExperts f, int s_blocks
             n += __popcll(mask);
         }
         if (n == 0) return;
-        n = min(n, 16 * RB);
+        if (n > 16 * RB) {
+            const int K = DOWN ? f.ff : f.D, kb = (K + 127) / 128, tiles = ((DOWN ? f.D : f.ff) + 15) / 16;
+            const size_t expert = (size_t)e * tiles * kb * 2048, step = (size_t)kb * 2048;
+            const bf16_t* u = (DOWN ? f.down : f.up) + expert;
+            if (GATED) pairs_without_slot<KIND>(f, e, 16 * RB, f.gate + expert + block * step, u + block * step, block, K);
+            else pairs_without_slot<KIND>(f, e, 16 * RB, u + 2 * block * step, u + min(2 * block + 1, tiles - 1) * step, block, K);
+            n = 16 * RB;
+        }
         wave_lds_sync();
         for (int s = lane; s < 16 * RB; s += 64)
             if (s >= n) mine[s] = mine[0];
@@ -256,7 +293,7 @@ extern "C" int tli_moe_few_takes(int T, int top, int E, int D, int ff) {
 
 // gate_t, up_t, down_t as for tli_moe_grouped_bf16; hid [T * top, ff], s_hid [T, s_ff]: scratch; the shared expert (s_ff > 0): s_gate
 // (act < 0) and s_up at the first block of 16 rows, blocks s_step elements apart, s_down tiled [D, s_ff].  part [top, T, D], one
-// more with a shared expert: see the top of this file.  No row of ids names an expert twice.
+// more with a shared expert: see the top of this file.
 extern "C" int tli_moe_few_bf16(const void* x, const int* ids, const float* weights, const void* gate_t, const void* up_t,
                                 const void* down_t, void* hid, const void* s_gate, const void* s_up, const void* s_down, long long s_step,
                                 const float* s_weight, void* s_hid, float* part, int handed_on, int T, int top, int E, int D, int ff, int s_ff, float limit,
