@@ -193,3 +193,22 @@ def test_rows_that_name_an_expert_twice(ops, size, kind):
     # as for test_experts_of_few_rows; terms of the same expert add up, by at most the root of their number (8 places: 3 times)
     scale = float(want.square().mean().sqrt())
     assert float((got.double() - want).abs().max()) <= 15 * 2.0 ** -9 * scale + 2.0 ** -8 * float(want.abs().max())
+
+
+def test_an_infinity_at_the_end_of_k(ops):
+    """Rows whose last values are infinite, with k no multiple of 128: the sums are infinite and not NaN, in the hidden units
+    and (these being infinite) in the outputs; the other rows are what they are without them."""
+    T, E, top, D, ff = 5, 4, 2, 72, 200
+    w, packed, ids, weights, _ = make(ops, (T, E, 0, top, D, ff, 0), "relu2")
+    down = w["down"].abs().clamp(min=0.01)
+    up = w["up"].clone()
+    up[:, :, D - 1] = 0.5
+    packed = ops.pack_experts(up, down, gated=False)
+
+    def run(x):
+        return ops.resolve(ops.experts_of_few_rows(x, ids, weights + 0.1, packed, None, None, None, activation="relu2"))
+    x = w["x"].clone()
+    x[3, D - 1] = math.inf
+    got, without = run(x), run(w["x"])
+    assert bool((got[3] == math.inf).all())
+    assert torch.equal(got[[0, 1, 2, 4]], without[[0, 1, 2, 4]])

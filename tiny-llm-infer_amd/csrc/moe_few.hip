@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(256) moe_few_kernel(FewExperts f, int s_blocks
     constexpr bool GATED = KIND == FEW_GATED, DOWN = KIND == FEW_DOWN;
     __shared__ float red[WAVES][2 * RB][64][4];
     __shared__ int slots[WAVES][16 * RB];                   // the pair (of the shared expert: the row) of every slot
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);       // (in a scalar register)
     const int r = lane % 16, c = lane / 16;
     const bool shared = (int)blockIdx.x < s_blocks;
     const int block = shared ? blockIdx.x : (blockIdx.x - s_blocks) % blocks;
@@ -197,11 +197,16 @@ __global__ void __launch_bounds__(256) moe_few_kernel(FewExperts f, int s_blocks
             a_row[1] = u + expert + (size_t)min(2 * block + 1, all - 1) * step + lane * 8;
         }
     }
-    const bf16_t* x_row[RB];
+    // Rows are read through a buffer descriptor, of which an offset past the end gives zeros: that is what lanes past the end
+    // of k ask for.  (The tiles of W are zeros there, but a zero times whatever lies behind the row, or times an infinity that
+    // stands in for it, need not be one.)
+    const bf16_t* inputs = DOWN ? (shared ? f.s_hid : f.hid) : f.x;
+    const auto buffer = __builtin_amdgcn_make_buffer_rsrc((void*)inputs, 0, (DOWN && !shared ? P : f.T) * K * 2, 0x00020000);
+    int x_row[RB];                                            // in bytes
 #pragma unroll
     for (int m = 0; m < RB; ++m) {
         const int slot = mine[m * 16 + r];
-        x_row[m] = DOWN ? (shared ? f.s_hid : f.hid) + (size_t)slot * K : f.x + (size_t)(shared ? slot : slot / f.top) * K;
+        x_row[m] = (DOWN || shared ? slot : slot / f.top) * K * 2;
     }
 
     f32x4 acc[2][RB];
@@ -213,12 +218,13 @@ __global__ void __launch_bounds__(256) moe_few_kernel(FewExperts f, int s_blocks
     auto load = [&](auto STAGE, int i) __attribute__((always_inline)) {
         constexpr int S = decltype(STAGE)::value;
         const int kb = wave + i * WAVES;
-        // (past the end of k the tiles of W are zeros: there a row's last values stand in)
 #pragma unroll
         for (int m = 0; m < RB; ++m)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                b[S][m][j].u = *reinterpret_cast<const uint4*>(x_row[m] + min(kb * 128 + c * 32 + j * 8, K - 8));
+            for (int j = 0; j < 4; ++j) {
+                const int k = kb * 128 + c * 32 + j * 8;
+                b[S][m][j].w = __builtin_amdgcn_raw_buffer_load_b128(buffer, k < K ? x_row[m] + 2 * k : -16, 0, 0);
+            }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -288,7 +294,8 @@ __global__ void __launch_bounds__(256) moe_few_kernel(FewExperts f, int s_blocks
 
 // Whether the kernels above take these sizes.
 extern "C" int tli_moe_few_takes(int T, int top, int E, int D, int ff) {
-    return T > 0 && T <= FEW_MAX_ROWS && E > 0 && E <= FEW_MAX_EXPERTS && top > 0 && D > 0 && ff > 0 && D % 8 == 0 && ff % 8 == 0;
+    return T > 0 && T <= FEW_MAX_ROWS && E > 0 && E <= FEW_MAX_EXPERTS && top > 0 && D > 0 && ff > 0 && D % 8 == 0 && ff % 8 == 0 &&
+           (long long)T * D < 1 << 30 && (long long)T * top * ff < 1 << 30;       // (offsets into rows are 32 bits of bytes)
 }
 
 // gate_t, up_t, down_t as for tli_moe_grouped_bf16; hid [T * top, ff], s_hid [T, s_ff]: scratch; the shared expert (s_ff > 0): s_gate
@@ -299,7 +306,7 @@ extern "C" int tli_moe_few_bf16(const void* x, const int* ids, const float* weig
                                 const float* s_weight, void* s_hid, float* part, int handed_on, int T, int top, int E, int D, int ff, int s_ff, float limit,
                                 float slope, float s_limit, int act, int weight_on_input, void* stream) {
     if (T <= 0) return 0;
-    if (!tli_moe_few_takes(T, top, E, D, ff) || s_ff < 0 || s_ff % 8)
+    if (!tli_moe_few_takes(T, top, E, D, ff) || s_ff < 0 || s_ff % 8 || (long long)T * s_ff >= 1 << 30)
         return tli_fail("moe_few: bad sizes (%d rows, %d of %d experts, width %d, %d and %d hidden units)", T, top, E, D, ff, s_ff);
     if (act >= TLI_ACT_KINDS || (act < 0 && (weight_on_input || !gate_t))) return tli_fail("moe_few: bad activation");
     if (s_ff && (!s_up || !s_down || !s_hid || s_step <= 0 || (act < 0 && (!s_gate || s_ff % 16)))) return tli_fail("moe_few: bad shared expert");
