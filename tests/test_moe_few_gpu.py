@@ -212,3 +212,23 @@ def test_an_infinity_at_the_end_of_k(ops):
     got, without = run(x), run(w["x"])
     assert bool((got[3] == math.inf).all())
     assert torch.equal(got[[0, 1, 2, 4]], without[[0, 1, 2, 4]])
+
+
+def test_rows_and_experts_of_the_faster_way(ops):
+    """Beyond 32 rows only up to 32 experts go to the kernels of few rows; what the part gives is the same either way."""
+    from tiny_llm_infer_amd.kernels.ops import DeferredSum
+    from tiny_llm_infer_amd.config import PartSpec
+    from tiny_llm_infer_amd.parts.base import BuildEnv, build_part
+    env = BuildEnv(dtype=BF, device=torch.device(DEV), ops=ops, max_model_len=64)
+    g = torch.Generator(device=DEV).manual_seed(4)
+    for E, rows, few in ((32, 64, True), (33, 32, True), (33, 33, False), (200, 64, False), (33, 1, True)):
+        part = build_part("ffn", PartSpec("routed_experts", {"hidden_size": 64, "experts": E, "top": 2, "intermediate_size": 32},
+                                          {"router": "router", "experts": "e{}."}))
+        part.load({d.name: (torch.randn(d.shape, generator=g, device=DEV) * d.shape[1] ** -0.5).to(BF) for d in part.tensors()}, env)
+        x = torch.randn((rows, 64), generator=g, device=DEV).to(BF)
+        y = part.forward(x, None)
+        assert isinstance(y, DeferredSum) == few, (E, rows)
+        ids, weights, _ = ops.router(x, part.w_router, E, 2, 1, 1, 1.0, False)
+        other = ops.apply_experts(x, ids, weights, None, None, part.packed, None, None)
+        # hidden units, parts and results are rounded to bfloat16 on the way: a few of its steps at the size of the largest
+        assert float((ops.resolve(y).double() - other.double()).abs().max()) <= 2.0 ** -6 * float(other.double().abs().max())

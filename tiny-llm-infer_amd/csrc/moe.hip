@@ -18,7 +18,7 @@
 //          the choice, so that a row's result does not depend on what else is in the step.
 //
 // These kernels walk the pairs one by one, each reading its expert's matrices: the float32 path, and
-// what the others do not take.  Steps of up to 64 rows in bfloat16 go expert by expert (moe_few.hip),
+// what the others do not take.  Steps of few rows in bfloat16 (up to 64, or 32 of many experts) go expert by expert (moe_few.hip),
 // steps of more rows sort the pairs by expert and multiply tile by tile (moe_grouped.hip).
 #include "common.h"
 

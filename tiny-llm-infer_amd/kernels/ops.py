@@ -1513,6 +1513,16 @@ class HipOps:
 
     FEW_EXPERT_ROWS = 64         # up to so many rows the experts, the shared one with them, are two launches without a sort
 
+    def few_expert_rows(self, experts: int) -> int:
+        """Up to how many rows ``experts_of_few_rows`` is the faster way for so many experts.  From 33 rows on its workgroups
+        multiply slots for 64 pairs of an expert, most of them empty where the experts are many.  Measured against the sorted
+        products, the sum of the parts left out and (in brackets) counted in, width 2,048 unless named: up to 32 rows 1.2 to
+        4.3 times as fast at 4 to 256 experts; 64 rows, 16 experts of which 2 are chosen 1.25 (1.19) times, 24 of which 4 1.08
+        (1.01), 32 of which 2 (width 4,096) 1.20 (1.18), 32 of which 4 with a shared one 1.23 (1.16), 32 of which 4 (width 1,024)
+        1.05 (0.96), 64 of which 8 0.99 (0.96), 128 of which 8 0.85 (0.83), 256 of which 8 0.87 (0.85); 33 rows, 128 and 256
+        0.91 (0.88)."""
+        return self.FEW_EXPERT_ROWS if experts <= 32 else 32
+
     def experts_of_few_rows(self, x, ids, weights, packed, shared_up, shared_down, shared_gate, limit=0.0, slope=1.0,
                             shared_limit=0.0, activation=None, weight_on_input=False, handed_on=False):
         """``apply_experts`` with the shared expert's products taken in, for few rows: ``shared_up`` its gate and up matrices (a

@@ -138,7 +138,7 @@ class RoutedExperts(FeedForward):
         ids, weights, shared_gate = ops.router(x, self.w_router, self.outputs, self.top, self.groups, self.keep, self.scale,
                                                self.has_gate, **how)
         few = getattr(ops, "experts_of_few_rows", None)
-        if few is not None:
+        if few is not None and x.shape[0] <= ops.few_expert_rows(self.experts):
             y = few(x, ids, weights, self.packed, self.shared_gate_up, self.shared_down, shared_gate, limit=self.limit, slope=self.slope,
                     shared_limit=self.shared_limit, activation=None if self.gated else self.activation, weight_on_input=self.weight_on == "input",
                     handed_on=self.identity > 0)
