@@ -75,9 +75,10 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
         float top = score;
 #pragma unroll
         for (int off = 8; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 16));
+        if (!__any(score != -INFINITY)) continue;               // (nothing of this block counts: the same for the whole wave)
+        // (a maximum passes NaNs over, the weights and their sum do not: a row with a NaN in it comes out as NaNs)
         const float m_new = fmaxf(m, top);
-        if (m_new == -INFINITY) continue;                       // (nothing of this block is seen: the same for the whole wave)
-        const float p = seen ? expf(score - m_new) : 0.f;
+        const float p = score == -INFINITY ? 0.f : expf(score - m_new);
         const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
         float sum = p;
 #pragma unroll
