@@ -60,3 +60,20 @@ def test_rows_that_hold_no_numbers(ops, case):
     got, plain = run(ops, case, step, bad), run(ops, case, step, bad, plain=True)
     assert torch.equal(got.isnan(), plain.isnan()) and bool(got[0, :hd].isnan().all()) and bool(got[1, hd:2 * hd].isnan().all())
     assert torch.equal(got[3:], want[3:])
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}-{c[1]}x{c[2]}-page{c[3]}-window{c[6]}")
+def test_slots_that_no_row_sees_may_hold_anything(ops, case):
+    """NaNs and infinities in pages that nobody holds, in slots behind a sequence's end and before its window."""
+    step, pos, seq, ks, vs, q = setup(case)
+    want = run(ops, case, step, q)
+    page, window = case[3], case[6]
+    tables = step.cache.group.tables.cpu().numpy()
+    unseen = torch.ones((step.cache.k.shape[0], page), dtype=torch.bool)
+    for p, s in zip(pos, seq):
+        for t in range(0 if window is None else max(0, p - window + 1), p + 1):
+            unseen[int(tables[s, t // page]), t % page] = False
+    for fill in (math.nan, math.inf):
+        step.cache.k.masked_fill_(unseen.to(DEV)[:, None, :, None], fill)
+        step.cache.v.masked_fill_(unseen.to(DEV)[:, None, None, :], fill)
+        assert torch.equal(run(ops, case, step, q), want), fill

@@ -9,6 +9,7 @@
 // 5 rows of up to 52 keys, 16 heads of 64: 15.9 -> 4.8 us, most of it the launch.
 // The order of additions depends on the row's first and last key alone.
 #include "common.h"
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
@@ -78,7 +79,7 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
         if (!__any(score != -INFINITY)) continue;               // (nothing of this block counts: the same for the whole wave)
         // (a maximum passes NaNs over, the weights and their sum do not: a row with a NaN in it comes out as NaNs)
         const float m_new = fmaxf(m, top);
-        const float p = score == -INFINITY ? 0.f : expf(score - m_new);
+        const float p = !seen ? -0.f : score == -INFINITY ? 0.f : expf(score - m_new);
         const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
         float sum = p;
 #pragma unroll
@@ -89,14 +90,22 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
         wave_lds_sync();
 #pragma unroll
         for (int i = 0; i < DH; ++i) o[i] *= corr;
+        auto add = [&](auto WHOLE) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const f32x4 w = *reinterpret_cast<const f32x4*>(&p_s[wave][4 * u]);
+            for (int u = 0; u < 4; ++u) {
+                const f32x4 w = *reinterpret_cast<const f32x4*>(&p_s[wave][4 * u]);
 #pragma unroll
-            for (int i = 0; i < DH; ++i)
+                for (int i = 0; i < DH; ++i)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[i] = fmaf(w[e], vv[i][u][e], o[i]);
-        }
+                    for (int e = 0; e < 4; ++e) {
+                        const float next = fmaf(w[e], vv[i][u][e], o[i]);
+                        o[i] = decltype(WHOLE)::value || __float_as_int(w[e]) >= 0 ? next : o[i];
+                    }
+            }
+        };
+        // what lies in a slot that is not this row's (its weight is -0) need not be a number, and 0 times it need not be 0
+        if (__all(seen)) add(std::true_type{});
+        else add(std::false_type{});
         wave_lds_sync();
     }
     if (lane == 0) {
