@@ -86,3 +86,20 @@ def test_short_splits(ops, case):
     scale = 1 / math.sqrt(hd)
     out = ops.paged_attention(q, step, step.cache, heads, kv_heads, hd, scale, None)
     close(out, ref_attention_dev(q, ks, vs, pos, seq, heads, kv_heads, scale, None), "short splits")
+
+
+@pytest.mark.parametrize("n", [4112, 4128, 16400])
+def test_an_odd_number_of_tiles_two_a_workgroup(ops, n):
+    """Workgroups of two tiles of 16 columns, the last of them with one: right sums, and no sums of squares beyond a row's own
+    (the NaNs behind them stay)."""
+    M, K, parts = 5, 136, (n + 15) // 16
+    x, w = rnd_dev((M, K), 1), rnd_dev((n, K), 2, 0.05)
+    tiled = ops.tile_matrix(w)
+    resid, nw = rnd_dev((M, n), 3).float(), 1 + rnd_dev((n,), 4, 0.2).float()
+    r, ssq, xw = resid.clone(), torch.full((parts + 2, M), math.nan, device=DEV), torch.empty((M, n), dtype=BF, device=DEV)
+    ops._call(ops.lib.tli_gemm_skinny_fused_bf16, x.data_ptr(), tiled.data_ptr(), None, M, n, K, 0, None, 0, 0.0, r.data_ptr(), nw.data_ptr(),
+              xw.data_ptr(), ssq.data_ptr(), 0, 0, 1.0, 0, ops._stream())
+    h = resid.double() + x.double() @ w.double().T
+    assert bool(((r.double() - h).abs() <= allowed(x, w, resid.double().abs()) + 2.0 ** -23 * h.abs()).all())
+    assert torch.allclose(ssq[:parts].sum(0).double(), (h * h).sum(-1), rtol=1e-4)
+    assert bool(ssq[parts:].isnan().all())

@@ -117,9 +117,9 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
         w_ok[t] = n < N;
         w_row[t] = w + (size_t)(w_ok[t] ? n : 0) * K;
         if (TILED)   // blocks of 16 rows x 128 k = 4 KiB, stored [j][lane][8]: one load instruction
-                     // of a wave reads 1 KiB in a row
+                     // of a wave reads 1 KiB in a row (past an odd number of tiles: the last one again)
             w_row[t] = HALF ? w + ((size_t)(blockIdx.x / 2) * ((K + 127) / 128)) * 2048 + (16 * c + 8 * (blockIdx.x % 2) + r % 8) * 8
-                            : w + ((size_t)(blockIdx.x * RT + t) * ((K + 127) / 128)) * 2048 + lane * 8;
+                            : w + ((size_t)min((int)blockIdx.x * RT + t, (N - 1) / 16) * ((K + 127) / 128)) * 2048 + lane * 8;
     }
     const bf16_t* x_row[MT];
 #pragma unroll
@@ -356,7 +356,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
                 store4(fuse.xw + (size_t)row * N + n0, hw, N - n0, (N & 3) == 0);
             }
             ssq = quad_rows_sum(ssq);                  // over the tile's 16 columns
-            if (c == 0 && row < M) fuse.ssq_out[(size_t)(blockIdx.x * RT + t) * M + row] = ssq;
+            if (c == 0 && row < M && (HALF || RT == 1 || n_base + t * 16 < N)) fuse.ssq_out[(size_t)(blockIdx.x * RT + t) * M + row] = ssq;
             continue;
         }
         if (FUSE == FUSE_RSTD) {
