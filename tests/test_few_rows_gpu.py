@@ -103,3 +103,33 @@ def test_an_odd_number_of_tiles_two_a_workgroup(ops, n):
     assert bool(((r.double() - h).abs() <= allowed(x, w, resid.double().abs()) + 2.0 ** -23 * h.abs()).all())
     assert torch.allclose(ssq[:parts].sum(0).double(), (h * h).sum(-1), rtol=1e-4)
     assert bool(ssq[parts:].isnan().all())
+
+
+@pytest.mark.parametrize("cfg", [0, 8, 14, 18, 24, 28])
+@pytest.mark.parametrize("n", [1024, 1500, 2048, 2064, 4112])
+def test_partial_sums_of_every_launch_shape(ops, n, cfg):
+    """Into the residual through each launch shape: as many sums of squares a row as tli_gemm_skinny_parts says, all of them
+    written (there are NaNs before), and no more."""
+    M, K = 5, 256
+    x, w = rnd_dev((M, K), 1), rnd_dev((n, K), 2, 0.05)
+    tiled = ops.tile_matrix(w)
+    resid, nw = rnd_dev((M, n), 3).float(), 1 + rnd_dev((n,), 4, 0.2).float()
+    parts = ops.lib.tli_gemm_skinny_parts(M, n, cfg)
+    ssq = torch.full((parts + 2, M), math.nan, device=DEV)
+    xw = torch.empty((M, n), dtype=BF, device=DEV)
+    r = resid.clone()
+    ops._call(ops.lib.tli_gemm_skinny_fused_bf16, x.data_ptr(), tiled.data_ptr(), None, M, n, K, 0, None, 0, 0.0, r.data_ptr(), nw.data_ptr(),
+              xw.data_ptr(), ssq.data_ptr(), cfg, 0, 1.0, 0, ops._stream())
+    h = resid.double() + x.double() @ w.double().T
+    assert torch.allclose(ssq[:parts].sum(0).double(), (h * h).sum(-1), rtol=1e-4)
+    assert bool(ssq[parts:].isnan().all())
+
+
+def test_half_tiles_want_whole_pieces_of_a_residual(ops):
+    from tiny_llm_infer_amd.kernels.ops import KernelError
+    x, tiled = rnd_dev((2, 128), 1), ops.tile_matrix(rnd_dev((1030, 128), 2))
+    r, nw = torch.zeros((2, 1030), device=DEV), torch.ones(1030, device=DEV)
+    xw, ssq = torch.empty((2, 1030), dtype=BF, device=DEV), torch.empty((200, 2), device=DEV)
+    with pytest.raises(KernelError):
+        ops._call(ops.lib.tli_gemm_skinny_fused_bf16, x.data_ptr(), tiled.data_ptr(), None, 2, 1030, 128, 0, None, 0, 0.0, r.data_ptr(),
+                  nw.data_ptr(), xw.data_ptr(), ssq.data_ptr(), 8, 0, 1.0, 0, ops._stream())

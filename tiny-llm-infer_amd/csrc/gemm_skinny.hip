@@ -522,12 +522,19 @@ static int launch_skinny_fused(const bf16_t* x, const bf16_t* w, bf16_t* y, int 
     return tli_check_launch("gemm_skinny (norm taken in)");
 }
 
+// The launch shape `cfg` of the product with a norm taken in (0: by the sizes), and whether it takes half tiles.
+static int fused_shape(int M, int N, int gated, bool into_residual, int cfg) {
+    const long tiles = (N + 15) / 16;
+    if (cfg == 0) cfg = !gated && half_tiles(M, N, 1, into_residual) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
+    return gated && cfg < 20 ? 24 : cfg;
+}
+
 // How many partial sums of squares a row has after a product into the residual: one for every 8 or 16 columns.
-extern "C" int tli_gemm_skinny_parts(int M, int N) { return half_tiles(M, N, 1, true) ? (N + 7) / 8 : (N + 15) / 16; }
+extern "C" int tli_gemm_skinny_parts(int M, int N, int cfg) { return fused_shape(M, N, 0, true, cfg) == 8 ? (N + 7) / 8 : (N + 15) / 16; }
 
 // The product with a norm taken in (see the top of this file), for up to 16 rows and W in the
 // decode layout.  Either  resid != null:  resid[M,N] += x . W^T (float32), xw[M,N] =
-// bfloat16(norm_w * resid), ssq_out[tli_gemm_skinny_parts(M, N)][M] = partial sums of resid^2 (y is not used);
+// bfloat16(norm_w * resid), ssq_out[tli_gemm_skinny_parts(M, N, cfg)][M] = partial sums of resid^2 (y is not used);
 // or  ssq_in != null:  y = (x . W^T) / sqrt(sum(ssq_in[parts_in][M]) / K + eps), through the
 // SwiGLU of a gated matrix if `gated` (y then [M, N/2]).
 extern "C" int tli_gemm_skinny_fused_bf16(const void* x, const void* w, void* y, int M, int N, int K, int gated,
@@ -550,10 +557,8 @@ extern "C" int tli_gemm_skinny_fused_bf16(const void* x, const void* w, void* y,
     hipStream_t s = (hipStream_t)stream;
     const bf16_t* xp = (const bf16_t*)x;
     const bf16_t* wp = (const bf16_t*)w;
-    const long tiles = (N + 15) / 16;
-    const bool half = !gated && half_tiles(M, N, 1, resid != nullptr);     // (as tli_gemm_skinny_parts says)
-    if (cfg == 0) cfg = half ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
-    if (gated && cfg < 20) cfg = 24;
+    cfg = fused_shape(M, N, gated, resid != nullptr, cfg);
+    if (cfg == 8 && resid && N % 4) return tli_fail("gemm_skinny: half tiles into a residual of %d columns (a multiple of 4)", N);
     switch (cfg) {
         case 14: return launch_skinny_fused<1, 4>(xp, wp, (bf16_t*)y, M, N, K, gated, f, s);
         case 18: return launch_skinny_fused<1, 8>(xp, wp, (bf16_t*)y, M, N, K, gated, f, s);

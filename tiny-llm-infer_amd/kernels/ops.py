@@ -90,7 +90,7 @@ def load_library():
         "tli_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_fused_bf16": [P, P, P, I, I, I, I, P, I, F, P, P, P, P, I, I, F, I, P],
         "tli_gemm_mid_bf16": [P, P, P, P, I, I, I, I, I, I, I, I, F, I, P],
-        "tli_gemm_skinny_parts": [I, I],
+        "tli_gemm_skinny_parts": [I, I, I],
         "tli_gemm_mid_splits": [I, I, I],
         "tli_gemm_mid_splits_rows": [I, I, I, I],
         "tli_gemm_mid_reduce": [P, P, I, I, I, I, P],
@@ -523,7 +523,7 @@ class HipOps:
         if tuple(resid.shape) != (M, N):
             raise KernelError(f"the product gives {(M, N)}, the residual is {tuple(resid.shape)}")
         xw = torch.empty((M, N), dtype=torch.bfloat16, device=self.device)
-        ssq = torch.empty((self.lib.tli_gemm_skinny_parts(M, N), M), dtype=torch.float32, device=self.device)
+        ssq = torch.empty((self.lib.tli_gemm_skinny_parts(M, N, 0), M), dtype=torch.float32, device=self.device)
         self._call(self.lib.tli_gemm_skinny_fused_bf16, x.data_ptr(), m.tiled.data_ptr(), None, M, N, K, 0,
                    None, 0, 0.0, resid.data_ptr(), weight.data_ptr(), xw.data_ptr(), ssq.data_ptr(), 0, *_NO_GATE,
                    self._stream())
