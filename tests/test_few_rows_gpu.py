@@ -133,3 +133,35 @@ def test_half_tiles_want_whole_pieces_of_a_residual(ops):
     with pytest.raises(KernelError):
         ops._call(ops.lib.tli_gemm_skinny_fused_bf16, x.data_ptr(), tiled.data_ptr(), None, 2, 1030, 128, 0, None, 0, 0.0, r.data_ptr(),
                   nw.data_ptr(), xw.data_ptr(), ssq.data_ptr(), 8, 0, 1.0, 0, ops._stream())
+
+
+# (outputs, k): half tiles on either side of their lines (k as long as the outputs are many, 256) and of the rows' way through
+# LDS (1,024); a tile a workgroup; two, of eight and of four waves, on either side of k 4,096, ragged ends of k
+WAYS = [(256, 256), (264, 256), (1016, 1016), (1024, 1032), (72, 128), (3000, 1024), (3000, 1000), (4096, 2056), (8192, 4096), (8200, 4088),
+        (16640, 4104), (16640, 520)]
+
+
+@pytest.mark.parametrize("nk", WAYS)
+def test_a_row_is_the_same_by_either_way_of_its_operands(ops, nk):
+    """16 rows, 8, 5 and 1 of them: whether they go through LDS or straight into the operand registers, and by whole tiles or
+    half ones, a row's sums are those of one order."""
+    from tiny_llm_infer_amd.kernels.ops import NormedRows
+    from tiny_llm_infer_amd.parts.base import BuildEnv
+    from tiny_llm_infer_amd.parts.linear import GatedMatrix, Matrix
+    N, K = nk
+    env = BuildEnv(dtype=BF, device=torch.device(DEV), ops=ops, max_model_len=64)
+    x, w = rnd_dev((16, K), 1), rnd_dev((N, K), 2, 0.05)
+    ssq = torch.rand((4, 16), device=DEV) * K / 4
+    m = Matrix(w, env)
+    gated = GatedMatrix(w[:N // 32 * 16], w[-(N // 32 * 16):], env)
+
+    def forms(rows):
+        normed = NormedRows(x[rows].contiguous(), ssq[:, rows].contiguous(), 1e-5)
+        return [ops.linear(x[rows].contiguous(), m), ops.linear(x[rows].contiguous(), m, out_dtype=torch.float32), ops.linear(normed, m),
+                ops.linear_swiglu(normed, gated), ops.linear_swiglu(x[rows].contiguous(), gated)]
+    want = x.double() @ w.double().T
+    all_rows = forms(slice(0, 16))
+    assert bool(((all_rows[1].double() - want).abs() <= allowed(x, w)).all())
+    for rows in (slice(0, 1), slice(3, 8), slice(8, 16)):
+        for a, b in zip(forms(rows), all_rows):
+            assert torch.equal(a, b[rows])

@@ -15,10 +15,10 @@
 // any 32 values of k as long as A and B agree: lane group c = l/16 takes the 32
 // consecutive k  [kb + 32c, kb + 32c + 32)  of a 128-wide step, 8 per MFMA.
 //
-// The rows of x of a step go through LDS (up to 16 rows; see XR below), and where whole tiles of 16 columns leave half the
-// compute units without one a workgroup takes half a tile.  Measured with 8 rows, cold weights, launches of a chain (straight
+// The rows of x of a step go through LDS where that pays (through_lds below), and where whole tiles of 16 columns leave half the
+// compute units without one a workgroup takes half a tile (half_tiles).  Measured with 8 rows, cold weights, launches of a chain (straight
 // into the operand registers, whole tiles, before): 2,048 columns into the residual of k 8,192 13.2 -> 9.8 us, of k 12,288 15.3 ->
-// 12.6; 4,096 columns of k 4,096 9.0 -> 8.0, of k 12,288 19.9 -> 18.9; 24,576 of k 4,096 (gated) 33.3 -> 32.9.  A chain of launches
+// 12.6; 4,096 columns of k 4,096 9.0 -> 8.0, of k 12,288 19.9 -> 18.9; 24,576 of k 4,096 (gated) 31.6 -> 31.3.  A chain of launches
 // costs 2.5 us each before the first byte; what is left goes by at 6.4 TB/s.
 //
 // A workgroup owns 16*RT output columns; its waves take the 128-wide k steps in
@@ -116,10 +116,12 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
         const int n = n_base + t * 16 + r;
         w_ok[t] = n < N;
         w_row[t] = w + (size_t)(w_ok[t] ? n : 0) * K;
+        // (past an odd number of tiles: the last one again; a gated matrix has pairs of them)
+        const int tile = GATED || t == 0 ? blockIdx.x * RT + t : min((int)blockIdx.x * RT + t, (N - 1) / 16);
         if (TILED)   // blocks of 16 rows x 128 k = 4 KiB, stored [j][lane][8]: one load instruction
-                     // of a wave reads 1 KiB in a row (past an odd number of tiles: the last one again)
+                     // of a wave reads 1 KiB in a row
             w_row[t] = HALF ? w + ((size_t)(blockIdx.x / 2) * ((K + 127) / 128)) * 2048 + (16 * c + 8 * (blockIdx.x % 2) + r % 8) * 8
-                            : w + ((size_t)min((int)blockIdx.x * RT + t, (N - 1) / 16) * ((K + 127) / 128)) * 2048 + lane * 8;
+                            : w + ((size_t)tile * ((K + 127) / 128)) * 2048 + lane * 8;
     }
     const bf16_t* x_row[MT];
 #pragma unroll
@@ -370,10 +372,28 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
     }
 }
 
-// Up to 16 rows go through LDS, four, eight or sixteen of them.
-#define SKINNY_ROWS(M, LAUNCH)          \
-    if ((M) <= 4) { LAUNCH(1); }        \
+// Where the rows of x (up to 16) go through LDS.  It takes a fetch less of 64 places a load instruction and costs a trip through
+// LDS in every step, which shows where a wave has few steps and where the matrix alone keeps the memory busy.  Cold weights,
+// through LDS and straight into the operand registers, us:
+//   into the residual: always.  4,096 columns of k 4,096, 16 rows 9.05 and 9.56; 2,048 of 2,048, 1 row 4.22 and 4.78.
+//   half tiles: from k 1,024 on.  256 columns of k 4,096, 8 rows 4.94 and 5.77, of 1,024 2.94 and 3.22, of 512 2.62 and 2.67.
+//   a tile a workgroup: 9 to 16 rows of k 1,024 and more.  4,096 columns normed, 16 rows of k 3,072 7.19 and 7.91, of 512 3.71 and
+//   3.58; 8 rows of k 2,048 5.65 and 5.51, of 4,096 8.16 and 8.17.
+//   two tiles: from k 4,096 on, and float outputs (the logits) from 9 rows on.  24,576 gated columns of k 4,096, 8 rows 31.4 and
+//   31.7; 12,288 of 4,096 19.1 and 19.7, 16 rows of 2,048 13.0 and 12.5, of 512 6.77 and 5.65; 32,768 float columns, 8 rows of k
+//   2,048 21.9 and 21.6, of 5,120 49.4 and 49.2, 16 rows 50.8 and 51.6.
+static bool through_lds(int M, int K, bool two_tiles, bool half, bool float_out) {
+    if (half) return K >= 1024;
+    return two_tiles ? K >= 4096 && (M > 8 || !float_out) : M > 8 && K >= 1024;
+}
+// (four, eight or sixteen rows)
+#define SKINNY_ROWS(M, LDS, LAUNCH)     \
+    if (!(LDS)) { LAUNCH(0); }          \
+    else if ((M) <= 4) { LAUNCH(1); }   \
     else if ((M) <= 8) { LAUNCH(2); }   \
+    else { LAUNCH(4); }
+#define SKINNY_ROWS_16(LDS, LAUNCH)     \
+    if (!(LDS)) { LAUNCH(0); }          \
     else { LAUNCH(4); }
 
 template <int RT, int MT, int WAVES>
@@ -391,8 +411,9 @@ static int launch_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N
     gemm_skinny_kernel<1, 1, WAVES, TO, true, false, 2, FUSE_NONE, XR, false, true><<<(N + 7) / 8, WAVES * 64, 0, s>>>(x, w, (TO*)y, M, N, K, plain)
 #define SKINNY_HALF_BF16(XR) SKINNY_HALF(bf16_t, XR)
 #define SKINNY_HALF_F32(XR) SKINNY_HALF(float, XR)
-            if (y_dtype == TLI_BF16) SKINNY_ROWS(M, SKINNY_HALF_BF16)
-            else SKINNY_ROWS(M, SKINNY_HALF_F32)
+            const bool lds = through_lds(M, K, false, true, false);
+            if (y_dtype == TLI_BF16) SKINNY_ROWS(M, lds, SKINNY_HALF_BF16)
+            else SKINNY_ROWS(M, lds, SKINNY_HALF_F32)
             return tli_check_launch("gemm_skinny");
         }
     }
@@ -402,9 +423,12 @@ static int launch_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N
 #define SKINNY_BF16(XR) SKINNY_LAUNCH(bf16_t, true, false, XR)
 #define SKINNY_F32(XR) SKINNY_LAUNCH(float, true, false, XR)
     if constexpr (MT == 1) {
-        if (tiled == 2) SKINNY_ROWS(M, SKINNY_GATED)       // pairs of row tiles, silu(gate)*up written as bfloat16
-        else if (tiled && y_dtype == TLI_BF16) SKINNY_ROWS(M, SKINNY_BF16)
-        else if (tiled) SKINNY_ROWS(M, SKINNY_F32)
+        const bool lds = through_lds(M, K, RT == 2, false, y_dtype != TLI_BF16);
+        if (tiled == 2) SKINNY_ROWS(M, lds, SKINNY_GATED)       // pairs of row tiles, silu(gate)*up written as bfloat16
+        else if (tiled && y_dtype == TLI_BF16) {
+            if constexpr (RT == 2) SKINNY_ROWS(M, lds, SKINNY_BF16)
+            else SKINNY_ROWS_16(lds, SKINNY_BF16)
+        } else if (tiled) SKINNY_ROWS_16(lds, SKINNY_F32)
         else if (y_dtype == TLI_BF16) SKINNY_LAUNCH(bf16_t, false, false, 0);
         else SKINNY_LAUNCH(float, false, false, 0);
     } else {
@@ -419,9 +443,12 @@ static int launch_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N
 
 // Half tiles where whole ones leave half of the chip or more without a workgroup.  Cold weights, 8 rows, whole and half: 64
 // columns of k 2,048 3.68 and 3.46 us, 256 of 4,096 5.16 and 4.64, 768 of 6,144 7.51 and 6.64; 1 and 16 rows gain as much.
-// Into the residual only from 1,024 columns on: each half tile leaves sums of squares that the next product adds up.
-static bool half_tiles(int M, int N, int tiled, bool into_residual) {
-    return M <= 16 && tiled == 1 && (N + 15) / 16 <= tli_compute_units() / 2 && (!into_residual || (N >= 1024 && N % 4 == 0));
+// Not where k is shorter than the columns are many, or than two steps: 2,048 columns of k 512 2.97 and 3.06, normed 3.31 and
+// 3.55, 256 of 128 2.14 and 2.26.  Into the residual only from 1,024 columns on (each half tile leaves sums of squares that the
+// next product adds up), there of every k: 2,048 columns of k 256 3.41 and 3.21.
+static bool half_tiles(int M, int N, int K, int tiled, bool into_residual) {
+    if (M > 16 || tiled != 1 || (N + 15) / 16 > tli_compute_units() / 2) return false;
+    return into_residual ? N >= 1024 && N % 4 == 0 : K >= N && K >= 256;
 }
 
 template <int MT>
@@ -430,7 +457,7 @@ static int pick_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N, 
     // cfg 0: by shape.  Narrow outputs get one 16-column tile per workgroup so that
     // even N = 4096 gives 256 workgroups; wide outputs share x over two tiles.
     const long tiles = (N + 15) / 16;
-    if (cfg == 0) cfg = half_tiles(M, N, tiled, false) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
+    if (cfg == 0) cfg = half_tiles(M, N, K, tiled, false) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
     if (tiled == 2 && cfg < 20) cfg = 24;          // gated needs pairs of row tiles
     switch (cfg) {
         case 14: return launch_skinny<1, MT, 4>(x, w, y, M, N, K, y_dtype, tiled, gate, inputs, unit, s);
@@ -508,29 +535,31 @@ static int launch_skinny_fused(const bf16_t* x, const bf16_t* w, bf16_t* y, int 
     gemm_skinny_kernel<1, 1, WAVES, bf16_t, true, false, 2, FUSE_RESIDUAL, XR, true, true><<<(N + 7) / 8, WAVES * 64, 0, s>>>(x, w, y, M, N, K, f)
 #define SKINNY_RSTD_HALF(XR) \
     gemm_skinny_kernel<1, 1, WAVES, bf16_t, true, false, 2, FUSE_RSTD, XR, false, true><<<(N + 7) / 8, WAVES * 64, 0, s>>>(x, w, y, M, N, K, f)
+    const bool lds = f.resid || through_lds(M, K, RT == 2, half, false);
     if constexpr (RT == 1) {
         if (half) {
-            if (f.resid) SKINNY_ROWS(M, SKINNY_RESIDUAL_HALF)
-            else SKINNY_ROWS(M, SKINNY_RSTD_HALF)
+            if (f.resid) SKINNY_ROWS(M, true, SKINNY_RESIDUAL_HALF)
+            else SKINNY_ROWS(M, lds, SKINNY_RSTD_HALF)
             return tli_check_launch("gemm_skinny (norm taken in)");
         }
     }
-    if (f.resid && N % 4 == 0) SKINNY_ROWS(M, SKINNY_RESIDUAL_WHOLE)
-    else if (f.resid) SKINNY_ROWS(M, SKINNY_RESIDUAL)
-    else if (gated) SKINNY_ROWS(M, SKINNY_RSTD_GATED)
-    else SKINNY_ROWS(M, SKINNY_RSTD)
+    if (f.resid && N % 4 == 0) SKINNY_ROWS(M, true, SKINNY_RESIDUAL_WHOLE)
+    else if (f.resid) SKINNY_ROWS(M, true, SKINNY_RESIDUAL)
+    else if (gated) SKINNY_ROWS(M, lds, SKINNY_RSTD_GATED)
+    else if constexpr (RT == 2) SKINNY_ROWS(M, lds, SKINNY_RSTD)
+    else SKINNY_ROWS_16(lds, SKINNY_RSTD)
     return tli_check_launch("gemm_skinny (norm taken in)");
 }
 
 // The launch shape `cfg` of the product with a norm taken in (0: by the sizes), and whether it takes half tiles.
-static int fused_shape(int M, int N, int gated, bool into_residual, int cfg) {
+static int fused_shape(int M, int N, int K, int gated, bool into_residual, int cfg) {
     const long tiles = (N + 15) / 16;
-    if (cfg == 0) cfg = !gated && half_tiles(M, N, 1, into_residual) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
+    if (cfg == 0) cfg = !gated && half_tiles(M, N, K, 1, into_residual) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
     return gated && cfg < 20 ? 24 : cfg;
 }
 
 // How many partial sums of squares a row has after a product into the residual: one for every 8 or 16 columns.
-extern "C" int tli_gemm_skinny_parts(int M, int N, int cfg) { return fused_shape(M, N, 0, true, cfg) == 8 ? (N + 7) / 8 : (N + 15) / 16; }
+extern "C" int tli_gemm_skinny_parts(int M, int N, int cfg) { return fused_shape(M, N, 0, 0, true, cfg) == 8 ? (N + 7) / 8 : (N + 15) / 16; }
 
 // The product with a norm taken in (see the top of this file), for up to 16 rows and W in the
 // decode layout.  Either  resid != null:  resid[M,N] += x . W^T (float32), xw[M,N] =
@@ -557,7 +586,7 @@ extern "C" int tli_gemm_skinny_fused_bf16(const void* x, const void* w, void* y,
     hipStream_t s = (hipStream_t)stream;
     const bf16_t* xp = (const bf16_t*)x;
     const bf16_t* wp = (const bf16_t*)w;
-    cfg = fused_shape(M, N, gated, resid != nullptr, cfg);
+    cfg = fused_shape(M, N, K, gated, resid != nullptr, cfg);
     if (cfg == 8 && resid && N % 4) return tli_fail("gemm_skinny: half tiles into a residual of %d columns (a multiple of 4)", N);
     switch (cfg) {
         case 14: return launch_skinny_fused<1, 4>(xp, wp, (bf16_t*)y, M, N, K, gated, f, s);
