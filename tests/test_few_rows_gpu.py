@@ -165,3 +165,14 @@ def test_a_row_is_the_same_by_either_way_of_its_operands(ops, nk):
     for rows in (slice(0, 1), slice(3, 8), slice(8, 16)):
         for a, b in zip(forms(rows), all_rows):
             assert torch.equal(a, b[rows])
+
+
+def test_short_heads_are_split_later(ops):
+    """A key of a head of 64 is half as many bytes: few rows of them go over several workgroups from a reach of 2,048 keys on,
+    more rows from 4,096; longer heads from 1,024."""
+    if ops.DECODE_WORKGROUPS != 256:
+        pytest.skip("the rule's lines are of 256 compute units")
+    step, *_ = make_step([600], [1], 16, 45, 5, 2, 64, BF, None)
+    for rows, hd, reach, splits in ((1, 64, 1024, 1), (1, 64, 2048, 8), (16, 64, 2048, 8), (17, 64, 2048, 1), (17, 64, 4096, 8), (1, 128, 512, 1),
+                                    (1, 128, 1024, 8), (17, 128, 2048, 8), (1, 192, 1024, 8), (1, 256, 1024, 8)):
+        assert ops._decode_splits(rows, reach, step.cache.group, 4, 2, hd, None)[0] == splits, (rows, hd, reach)

@@ -944,8 +944,8 @@ class HipOps:
         # Against that stand the pass that merges the parts (3 to 5 us; it sums eight of them at once) and
         # the fixed part of a workgroup.  Measured at 32 query and 8 kv heads of 128 (2 and 32 kv heads and
         # heads of 256 agree), from raw projections, us, unsplit / this rule:
-        #   1 row of 520 keys 10.2 / 9.2, of 1,500 19.4 / 12.0; 8 rows of 520 11.4 / 11.9, of 1,000 20.2 /
-        #   16.0; up to a reach of 512 keys no split is better (1 row of 300 keys 8.5 / 9.3).
+        #   1 row of 520 keys 10.2 / 9.2, of 1,500 19.4 / 12.0; 8 rows of 520 12.5 / 12.9 (the reach tells it from
+        #   1,000 no more), of 1,000 17.6 / 15.7; up to a reach of 512 keys no split is better (1 row of 300 keys 8.5 / 9.3).
         #   1 row of 3,000 keys 32.0 / 12.8, of 8,000 97 / 18.1, of 32,000 (32 splits) 34.7, with 16 40.3.
         #   16 rows of 2,000 keys 40.0 / 33.4, of 6,000 103 / 86; of 600 16.9 and in two splits 18.9.
         #   24 rows of 2,100 keys 46.0, in two splits 50.5, of 5,000 98 and 107: from more pairs than half
@@ -961,9 +961,13 @@ class HipOps:
         # one of 4,000: 54.5 unsplit, 35.1 in eight, 48.1 in sixteen), and no split of more rows than a
         # quarter of the units below a reach of 4,096 (one of 900 keys beside 15 of 200: 15.0 and in eight
         # 17.2).  With a window every row walks about as many keys.
+        # Heads below 128 elements hold less a key: they are split from a reach of 2,048 on, and of 4,096 where
+        # the pairs are more than an eighth of the units.  Heads of 64, unsplit and split: 16 rows of 600 keys on
+        # 2 kv heads 9.1 and 10.0, 1 row of 2,000 14.3 and 9.5, 16 14.9 and 11.6; 8 rows on 16 kv heads of 1,030
+        # 12.9 and 14.3, of 2,100 22.4 and 21.4.
         every = groups
         units = self.DECODE_WORKGROUPS
-        least = 4 * self.DECODE_SPLIT_KEYS
+        least = (4 if head_dim >= 128 else 8 if groups <= units // 8 else 16) * self.DECODE_SPLIT_KEYS
         if skew > 1 and not window:
             groups = max(1, groups // skew)
             least = least if every <= units // 4 else 16 * self.DECODE_SPLIT_KEYS
