@@ -342,10 +342,11 @@ class ModelRunner:
         ``feed``: int32 tensor on the device that entries with ``token_from`` take
         their token from (the tokens the previous step sampled).
 
-        The logits that come back belong to the runner: for a recorded decode step they are
-        a view of the recording's output buffer, which the next step of the same shape
+        The logits that come back belong to the runner: for a recorded decode step of a bfloat16
+        run they are a view of the recording's output buffer, which the next step of the same shape
         writes again.  Use them (sample from them, copy them) before the next call of
-        ``step``; ``clone()`` what has to outlive it."""
+        ``step``; ``clone()`` what has to outlive it.  (In a float32 run, whose logits others are checked
+        with, they are a tensor of their own.)"""
         self._check(entries)
         # all or nothing over the whole batch: groups are independent, requests compete
         need = [0] * len(self.cache.groups)
@@ -367,6 +368,8 @@ class ModelRunner:
         if self.use_graphs and wanted == len(entries) and all(len(e.tokens) == 1 for e in entries):
             view = self._pack(entries, feed, pad_to=_decode_bucket(len(entries)))
             logits = self._replay(view, view.num_rows)[:wanted]
+            if self.env.dtype == torch.float32:
+                logits = logits.clone()
         else:
             view = self._pack(entries, feed)
             logits = self.forward(view, wanted)
