@@ -22,9 +22,9 @@ def rnd(shape, seed, std=1.0):
 
 
 # (rows, outputs, k): one row; partial tiles of both; k of less than a step, of a partial last step, of fewer steps than
-# ranges, of many batches; each launch shape (up to 16, 32 and more rows; few, more and many outputs)
-SIZES = [(1, 96, 64), (5, 301, 4), (16, 1000, 100), (7, 16400, 260), (17, 77, 1028), (32, 16448, 64), (33, 130, 4096),
-         (64, 1040, 36), (65, 16385, 132), (200, 8200, 1100), (130, 2050, 516)]
+# ranges, of many batches; each launch shape: up to 16, 32 and more rows; parts of a tile (four or eight columns), one tile, two
+SIZES = [(1, 96, 64), (5, 301, 4), (9, 1500, 68), (16, 2100, 100), (7, 16400, 260), (17, 77, 1028), (20, 1999, 132), (24, 4100, 260),
+         (32, 16448, 64), (33, 130, 4096), (64, 1040, 36), (100, 4100, 132), (65, 16385, 132), (200, 8200, 1100), (130, 2050, 516)]
 
 
 def bound(x, w):
@@ -40,11 +40,12 @@ def test_product(ops, mnk):
     x, w = rnd((M, K), 1), rnd((N, K), 2, 0.05)
     y = ops.linear(x, w)
     assert bool(((y.double() - x.double() @ w.double().T).abs() <= bound(x, w)).all())
-    for lo, hi in ((0, 1), (M // 2, M), (M - 1, M)):
+    for lo, hi in ((0, 1), (M // 2, M), (M - 1, M), (0, min(M, 16)), (0, min(M, 32))):
         assert torch.equal(ops.linear(x[lo:hi].clone(), w), y[lo:hi]), "a row's sums depend on the rows beside it"
 
 
-@pytest.mark.parametrize("mnk", [(1, 32, 64), (5, 48, 100), (16, 24, 36), (33, 1000, 1028), (100, 50, 260), (200, 4100, 516)])
+@pytest.mark.parametrize("mnk", [(1, 32, 64), (5, 48, 100), (16, 24, 36), (17, 40, 100), (32, 1000, 516), (33, 1000, 1028), (100, 50, 260),
+                                 (200, 4100, 516)])
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
 def test_gated_product(ops, mnk, activation):
     from tiny_llm_infer_amd.parts.base import BuildEnv
@@ -59,7 +60,8 @@ def test_gated_product(ops, mnk, activation):
     # are good to a few roundings
     allowed = 0.7 * (1.13 * bound(x, gate) * u.abs() + act.abs() * bound(x, up)) + 16 * 2.0 ** -24 * (0.7 * act * u).abs() + 1e-7
     assert bool(((y.double() - 0.7 * act * u).abs() <= allowed).all())
-    assert torch.equal(ops.linear_swiglu(x[:1].clone(), GatedMatrix(gate, up, env), activation=activation, scale=0.7), y[:1])
+    for lo, hi in ((0, 1), (0, min(M, 16)), (M // 2, M), (0, min(M, 32))):
+        assert torch.equal(ops.linear_swiglu(x[lo:hi].clone(), GatedMatrix(gate, up, env), activation=activation, scale=0.7), y[lo:hi])
 
 
 def test_operands_that_are_not_in_whole_pieces_go_to_the_plain_kernel(ops):

@@ -179,7 +179,12 @@ extern "C" int tli_gemm_f32(const void* x, const void* w, void* y, int M, int N,
     float* yp = (float*)y;
     hipStream_t s = (hipStream_t)stream;
     // Few rows: one tile of W a workgroup while that gives less than two workgroups a compute unit, two beyond (x is then
-    // read half as often).  Many rows: 64 x 64 outputs a workgroup where that fills the chip, else 32 x 64 or 16 x 64.
+    // read half as often).  More than 32 rows: 32 outputs by 64 rows a workgroup where that is a workgroup a compute unit, else 16
+    // by 64.  Cold weights, us, 32 and 16 outputs (the plain kernel): 64 rows, 1,024 columns of k 1,024 14.8 and 11.2 (143), 2,048 of
+    // 6,144 96 and 57 (1,074), 32,768 of 1,024 58.6 and 77.7 (213); 256 rows, 2,048 of 2,048 30.8 and 37.7 (291), 6,144 of 4,096 184
+    // and 214 (666), 1,536 of 1,024 (192 workgroups or 384) 15.2 and 20.3, but 33 rows, 6,144 of 4,096 (the same) 59.4 and 53.7; 512 rows, 4,096 gated of 1,024 108.5 (213); 2,048 rows, 2,048 of 6,144 737 and 842 (1,233) = 70 TFLOP/s.  64
+    // outputs by 64 rows, whose registers leave a SIMD one wave, are nowhere faster: 2,048 rows, 2,048 of 6,144 738, 12,288 gated
+    // of 4,096 at 64 rows 254 and with 32 outputs 170.
     const long tiles = ((long)(gated ? 2 : 1) * N + 15) / 16, units = tli_compute_units();
     // parts of a tile while that gives no more than a workgroup a compute unit (1,024 columns of k 4,096: 64 workgroups of
     // whole tiles, 256 of quarters: 16 decode steps of four layers of width 1,024 4.47 -> 4.19 ms)
@@ -193,7 +198,6 @@ extern "C" int tli_gemm_f32(const void* x, const void* w, void* y, int M, int N,
     if (M <= 32) return tiles < 2 * units && !gated ? launch_f32<1, 2, 4>(xp, wp, yp, M, N, K, gate, s)
                                                     : launch_f32<2, 2, 4>(xp, wp, yp, M, N, K, gate, s);
     const long blocks = tiles * ((M + 63) / 64);
-    if (blocks >= 4 * units) return launch_f32<4, 4, 1>(xp, wp, yp, M, N, K, gate, s);
     if (blocks >= 2 * units || gated) return launch_f32<2, 4, 2>(xp, wp, yp, M, N, K, gate, s);
     return launch_f32<1, 4, 2>(xp, wp, yp, M, N, K, gate, s);
 }
