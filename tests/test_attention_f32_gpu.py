@@ -1,11 +1,12 @@
 """The float32 attention with four lanes a key: beside a float64 reference and the plain kernel at the edges of its blocks
 (16 keys of four waves in turn), pages of 4 and 12 slots, heads of 192 elements, windows; rows that hold no numbers."""
+import dataclasses
 import math
 
 import pytest
 import torch
 
-from test_kernels_gpu import fill_cache, make_step, ref_attention, rnd
+from test_kernels_gpu import close, fill_cache, make_step, ref_attention, rnd
 
 pytestmark = pytest.mark.gpu
 
@@ -44,6 +45,22 @@ def run(ops, case, step, q, plain=False):
         return ops.paged_attention(q.to(DEV), step, step.cache, heads, kv_heads, hd, 1 / math.sqrt(hd), window)
     finally:
         ops.force_plain = False
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}-{c[1]}x{c[2]}-page{c[3]}-window{c[6]}")
+def test_values_and_a_row_alone(ops, case):
+    """As the reference and the plain kernel have it; a row alone is bit for bit the row among others."""
+    step, pos, seq, ks, vs, q = setup(case)
+    heads, kv_heads, hd, window = case[0], case[1], case[2], case[6]
+    assert ops.lib.tli_attention_f32_takes(hd, case[3])
+    want = ref_attention(q, ks, vs, pos, seq, heads, kv_heads, 1 / math.sqrt(hd), window)
+    got = run(ops, case, step, q)
+    close(got, want, F32, "attention")
+    close(run(ops, case, step, q, plain=True), want, F32, "attention of the plain kernel")
+    for row in (0, len(pos) // 2, len(pos) - 1):
+        alone = dataclasses.replace(step, num_rows=1, positions=step.positions[row:row + 1].clone(),
+                                    seq_of_row=step.seq_of_row[row:row + 1].clone())
+        assert torch.equal(run(ops, case, alone, q[row:row + 1])[0], got[row]), row
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}-{c[1]}x{c[2]}-page{c[3]}-window{c[6]}")

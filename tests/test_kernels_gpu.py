@@ -545,17 +545,18 @@ PREFILL_MODES = {"bfloat16-direct": 1, "bfloat16-lds1": 2, "bfloat16-lds2": 3,
                  "bfloat16-two-sets": 10, "bfloat16-one-set": 11}
 
 
-@pytest.mark.parametrize("dtype", DTYPES + ["bfloat16-plain"] + list(PREFILL_MODES))
+@pytest.mark.parametrize("dtype", DTYPES + ["bfloat16-plain", "float32-plain"] + list(PREFILL_MODES))
 @pytest.mark.parametrize("case", ATT_CASES)
 def test_paged_attention(ops, dtype, case):
-    """float32: the plain kernel.  bfloat16: the MFMA kernels (decode when every
-    sequence brings one row, prefill otherwise) in each of the prefill kernel's
+    """float32: four lanes a key where head size and page allow it, and the plain kernel.  bfloat16: the MFMA kernels
+    (decode when every sequence brings one row, prefill otherwise) in each of the prefill kernel's
     forms, and the plain kernel beside them."""
     if case in ATT_CASES[-2:] and dtype in PREFILL_MODES:
         pytest.skip("a case for the launch rule itself; the forced forms have their long cases above")
-    ops.force_plain = dtype == "bfloat16-plain"
+    ops.force_plain = dtype in ("bfloat16-plain", "float32-plain")
     ops.prefill_direct = PREFILL_MODES.get(dtype, 0)
-    dtype = torch.bfloat16 if isinstance(dtype, str) else dtype
+    if isinstance(dtype, str):
+        dtype = torch.float32 if dtype == "float32-plain" else torch.bfloat16
     try:
         _paged_attention_case(ops, dtype, case)
     finally:

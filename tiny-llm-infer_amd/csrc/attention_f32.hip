@@ -6,7 +6,11 @@
 // four are joined at the end.  In a block four lanes share a key (lane 16 c + j: quarter c of key j, 16 bytes a load), then a
 // lane takes every 64th output element and the block's 16 values of it, four to a load.  What bounds a decode step's few short
 // rows is the chain of loads of one block after the other, which is a quarter as long here and has all its loads in flight:
-// 5 rows of up to 52 keys, 16 heads of 64: 15.9 -> 4.8 us, most of it the launch.
+// 5 rows of up to 52 keys, 16 heads of 64: 15.9 -> 4.8 us, most of it the launch.  Longer rows and prompts, the plain kernel and
+// this one (both with the 12 us of a launch from Python), 16 heads of 64 and 32 of 128: 1 row of 200 keys 44.9 -> 13.0 and 46.4 ->
+// 12.9 us, of 4,000 850 -> 97 and 921 -> 148, of 16,000 3,535 -> 408 and 3,668 -> 578; 8 rows of 4,000 887 -> 104 and 929 -> 150; 64
+// of 600 159 -> 35 and 525 -> 135; a prompt of 32 tokens 12.2 -> 12.2 and 14.8 -> 12.6, of 512 441 -> 109 and 1,297 -> 394, of 2,048
+// 5.74 -> 1.46 and 19.6 -> 5.63 ms; heads of 192 and 256 1.04 to 5 times.
 // The order of additions depends on the row's first and last key alone.
 #include "common.h"
 #include <type_traits>
