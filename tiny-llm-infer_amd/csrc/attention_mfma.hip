@@ -979,8 +979,8 @@ attention_decode_solo_kernel(bf16_t* __restrict__ out, bf16_t* __restrict__ k_ca
     }
 }
 
-// grid (heads, rows); one thread per output element
-__global__ void attention_merge_splits_kernel(const float* __restrict__ partial, bf16_t* __restrict__ out,
+// grid (heads, rows); exactly one wave of 64 threads
+__global__ void __launch_bounds__(64) attention_merge_splits_kernel(const float* __restrict__ partial, bf16_t* __restrict__ out,
                                               int heads, int head_dim, int splits) {
     // A lane holds the maximum and sum of one split (64 at a time), so that a head waits for memory twice and not once a
     // split: eight splits of 128 elements 8.7 -> 4.7 us.
