@@ -1531,7 +1531,7 @@ class HipOps:
                             shared_limit=0.0, activation=None, weight_on_input=False, handed_on=False):
         """``apply_experts`` with the shared expert's products taken in, for few rows: ``shared_up`` its gate and up matrices (a
         ``GatedMatrix``, or a ``Matrix`` of gate rows before up rows; without a gate the up matrix), ``shared_down`` (both None:
-        no shared expert); ``handed_on``: ids from E on may occur.  ``ids`` names no expert twice in a row.  The result is a
+        no shared expert); ``handed_on``: ids from E on may occur.  A row may name an expert more than once (slower).  The result is a
         ``DeferredSum``, a part for every place of the choice and one for the shared expert; None where these kernels do not
         apply."""
         T, n = x.shape
