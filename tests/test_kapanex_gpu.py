@@ -157,6 +157,51 @@ def test_delta_rule_kernels_in_portions_and_decoding(ops, dtype, H, G, dk, dv, t
         _close(torch.cat(got[k][1]), want[k][1], 3e-5 if dtype == "float32" else 2e-2, f"{k}: gated norm")
 
 
+@pytest.mark.parametrize("H, G, dk, dv, taps, n", [(4, 2, 16, 24, 4, 8), (2, 2, 8, 8, 1, 64), (3, 1, 40, 20, 2, 2048), (4, 2, 64, 64, 4, 4104),
+                                                   (2, 1, 128, 128, 3, 256), (1, 1, 200, 72, 2, 64), (4, 4, 256, 40, 10, 512), (2, 2, 128, 300, 9, 72)])
+def test_delta_rule_steps_of_one_row_in_one_launch(ops, H, G, dk, dv, taps, n):
+    """Sequences that bring a row a step, some of them new in a slot that was used before: columns in more and less than one round of
+    the workgroup, taps in more than one round, and the same gates, kept rows and state as portions leave."""
+    g = torch.Generator().manual_seed(H * 100 + dk)
+    dt = torch.bfloat16
+    qd, vd = G * dk, H * dv
+    C, ld = 2 * qd + vd, 2 * qd + 2 * vd + 8
+    conv = torch.randn(C, taps, generator=g) * 0.6
+    a_log, dt_bias = torch.rand(H, generator=g) * 3 - 4, torch.randn(H, generator=g) * 0.5
+    norm_w = torch.randn(dv, generator=g) * 0.1 + 1
+    w_gates = (torch.randn(2 * H, n, generator=g) * n ** -0.5).to(dt)
+    lengths = {"a": 14, "b": 6, "c": 13, "d": 5}
+    raw = {k: torch.randn(m, ld, generator=g) for k, m in lengths.items()}
+    x = {k: torch.randn(m, n, generator=g).to(dt) for k, m in lengths.items()}
+    gates = {k: x[k].double() @ w_gates.double().t() for k in lengths}
+    want = {k: _plain_delta_core(raw[k][:, :C + vd], gates[k], conv, a_log, dt_bias, norm_w, 1e-5, H, G, dk, dv, dt)[1] for k in lengths}
+    S = torch.full((3,) + tuple(ops.delta_state_shape(H, dk, dv)), float("nan"), dtype=torch.float32, device="cuda")
+    kept = torch.full((3, max(taps - 1, 1), C), float("nan"), dtype=dt, device="cuda") if taps > 1 else None
+    slot = {"a": 0, "b": 1, "c": 2, "d": 1}
+    conv_d, a_log_d, dt_bias_d, norm_d = conv.t().contiguous().cuda(), a_log.cuda(), dt_bias.cuda(), norm_w.cuda()
+    at, got = {k: 0 for k in lengths}, {k: [] for k in lengths}
+    first = {"a": 3, "c": 2}                                                      # these begin with a portion, on the other kernels
+    while any(at[k] < lengths[k] for k in lengths):
+        keys = [k for k in ("c", "a", "b", "d") if at[k] < lengths[k] and not (k == "d" and at["b"] < lengths["b"])]
+        counts = [first.pop(k, 1) for k in keys]
+        view = _view([at[k] for k in keys], counts, [slot[k] for k in keys])
+        proj = torch.cat([raw[k][at[k]:at[k] + c] for k, c in zip(keys, counts)]).to(dt).cuda()
+        rows = torch.cat([x[k][at[k]:at[k] + c] for k, c in zip(keys, counts)]).cuda()
+        args = (conv_d, a_log_d, dt_bias_d, kept, S, view, H, G, dk, dv, taps)
+        y = ops.delta_step(proj, rows, w_gates.cuda(), *args, norm_d, 1e-5)
+        assert (y is None) == (max(counts) > 1)
+        if y is None:
+            z, turned = ops.small_product(rows, w_gates.cuda())
+            y = ops.gated_rmsnorm(ops.delta_rule(proj, z, *args, gates_transposed=turned), proj, C, norm_d, 1e-5, H, dv, dt)
+        r = 0
+        for k, c in zip(keys, counts):
+            got[k].append(y[r:r + c].cpu())
+            r += c
+            at[k] += c
+    for k in lengths:
+        _close(torch.cat(got[k]), want[k], 2e-2, f"{k}: gated norm")
+
+
 # ------------------------------------------------------------ routed experts ---
 @pytest.mark.parametrize("E, top, groups, keep", [(6, 2, 3, 2), (4, 1, 1, 1), (8, 3, 8, 3), (16, 4, 4, 2), (64, 8, 8, 4), (5, 5, 1, 1)])
 def test_router_choice_and_weights(ops, E, top, groups, keep):

@@ -249,6 +249,170 @@ __global__ void gated_rmsnorm_kernel(const float* __restrict__ o, const T* __res
 }
 
 // ---------------------------------------------------------------------------------------------
+// A decode step: every sequence brings one row, and everything between the layer's products is one launch, a workgroup a
+// (head, row): the two gates' sums, the convolutions of the head's q, k and v, the recurrence and the gated norm (and a launch
+// that moves the kept rows on: the q and k channels of a key head are read by H / G workgroups, so none of them may write them).
+//
+// What bounds such a step is not its bytes (64 KiB of state in and out a workgroup at 128 x 128) but the chain of fetches and
+// launches, so the row's operands are asked for first (loads complete in the order of issue), then the whole state of the
+// head, and the sums over the row are made while it is on its way.  8 rows, 16 heads of 128 x 128, 4 taps, width 2,048, as part of
+// a decode step: five launches (the gates' product 6.7 us, prepare 7.4, kept rows 4.9, recurrence 8 to 11, norm 4.6) and these
+// two: a step of four layers, two of them this one, 431 -> 400 us.
+// ---------------------------------------------------------------------------------------------
+#define DELTA_STEP_THREADS 512
+#define DELTA_STEP_TAPS 8       // taps of a channel that are asked for together
+
+struct DeltaStep {
+    const bf16_t* proj;         // [rows, ld]: q (G dk) | k (G dk) | v (H dv) | gate (H dv)
+    int ld;
+    const bf16_t* x;            // [rows, n]: the layer's input
+    const bf16_t* w_gates;      // [2 H, n]: b, then a
+    int n;
+    const float* conv_w;        // [taps, channels]
+    const bf16_t* kept;         // [slots, taps - 1, channels]
+    const float *a_log, *dt_bias, *weight;
+    const int *positions, *slots;
+    float* state;
+    bf16_t* out;                // [rows, H dv]
+    int H, G, dk, dv, taps;
+    float eps;
+};
+
+template <int RPT>
+__global__ __launch_bounds__(DELTA_STEP_THREADS) void delta_step_kernel(DeltaStep a) {
+    constexpr int WAVES = DELTA_STEP_THREADS / TLI_WAVE;
+    constexpr int TOGETHER = DELTA_STEP_THREADS / DELTA_LANES;           // columns walked side by side: two blocks
+    constexpr int GROUPS = 4;                                            // of them, in flight together
+    constexpr int DKP = DELTA_LANES * RPT;
+    extern __shared__ float ds_lds[];
+    __shared__ float red[2][WAVES];
+    const int head = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid % TLI_WAVE, wave = tid / TLI_WAVE;
+    const int part = tid % DELTA_LANES, local = tid / DELTA_LANES;
+    const int dk = a.dk, dv = a.dv, H = a.H, kvh = head / (H / a.G), qd = a.G * dk, C = 2 * qd + H * dv;
+    float* q_s = ds_lds;                                                 // [DKP], then k [DKP], v and o [dv]
+    float* k_s = q_s + DKP;
+    float* v_s = k_s + DKP;
+    float* o_s = v_s + dv;
+    const int slot = a.slots[row], pos = a.positions[row];
+    const bool fresh = pos == 0;
+    // the two gates' sums: every thread a part of both
+    const bf16_t* xr = a.x + (size_t)row * a.n;
+    const bf16_t* wb = a.w_gates + (size_t)head * a.n;
+    const bf16_t* wa = a.w_gates + (size_t)(H + head) * a.n;
+    float zb = 0.f, za = 0.f;
+    for (int i = tid * 8; i < a.n; i += DELTA_STEP_THREADS * 8) {
+        const uint4 xv = *reinterpret_cast<const uint4*>(xr + i), bv = *reinterpret_cast<const uint4*>(wb + i),
+                    av = *reinterpret_cast<const uint4*>(wa + i);
+        const uint32_t xu[4] = {xv.x, xv.y, xv.z, xv.w}, bu[4] = {bv.x, bv.y, bv.z, bv.w}, au[4] = {av.x, av.y, av.z, av.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float lo = __uint_as_float(xu[e] << 16), hi = __uint_as_float(xu[e] & 0xFFFF0000u);
+            zb = fmaf(lo, __uint_as_float(bu[e] << 16), zb);
+            zb = fmaf(hi, __uint_as_float(bu[e] & 0xFFFF0000u), zb);
+            za = fmaf(lo, __uint_as_float(au[e] << 16), za);
+            za = fmaf(hi, __uint_as_float(au[e] & 0xFFFF0000u), za);
+        }
+    }
+    // the convolutions: a channel of q, k or v a thread and round
+    const bf16_t* mine = a.kept ? a.kept + (size_t)slot * (a.taps - 1) * C : nullptr;
+    for (int e = tid; e < 2 * DKP + dv; e += DELTA_STEP_THREADS) {
+        const int i = e < 2 * DKP ? e % DKP : e - 2 * DKP;
+        float value = 0.f;
+        if (e >= 2 * DKP || i < dk) {
+            const int c = e < DKP ? kvh * dk + i : e < 2 * DKP ? qd + kvh * dk + i : 2 * qd + head * dv + i;
+            float acc = 0.f;
+            for (int j0 = 0; j0 < a.taps; j0 += DELTA_STEP_TAPS) {
+                float x[DELTA_STEP_TAPS], w[DELTA_STEP_TAPS];
+#pragma unroll
+                for (int j = 0; j < DELTA_STEP_TAPS; ++j) {
+                    const int tap = j0 + j, back = a.taps - 1 - tap;     // the tap's row lies this many positions before
+                    x[j] = w[j] = 0.f;
+                    if (tap < a.taps && back <= pos) {
+                        w[j] = a.conv_w[(size_t)tap * C + c];
+                        x[j] = bf16_to_f32(back == 0 ? a.proj[(size_t)row * a.ld + c] : mine[(size_t)tap * C + c]);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < DELTA_STEP_TAPS; ++j)
+                    if (j0 + j < a.taps && a.taps - 1 - j0 - j <= pos) acc = fmaf(w[j], x[j], acc);
+            }
+            value = silu_f(acc);
+        }
+        q_s[e] = value;                                                  // (k and v lie behind q)
+    }
+    const int blocks = (dv + DELTA_COLS - 1) / DELTA_COLS;
+    float* state = a.state + ((size_t)slot * H + head) * blocks * RPT * DELTA_COLS * DELTA_LANES + (local % DELTA_COLS) * DELTA_LANES + part;
+    float S[GROUPS][RPT];
+    auto at = [&](int col) { return state + (size_t)(col / DELTA_COLS) * RPT * DELTA_COLS * DELTA_LANES; };
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) {
+            const int col = c0 + g * TOGETHER + local;
+            const bool there = !fresh && col < blocks * DELTA_COLS;
+#pragma unroll
+            for (int r = 0; r < RPT; ++r) S[g][r] = there ? at(col)[r * DELTA_COLS * DELTA_LANES] : 0.f;
+        }
+    };
+    load(0);
+    zb = wave_sum(zb), za = wave_sum(za);
+    if (lane == 0) red[0][wave] = zb, red[1][wave] = za;
+    __syncthreads();
+    zb = za = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) zb += red[0][w], za += red[1][w];
+    za += a.dt_bias[head];
+    const float beta = 1.0f / (1.0f + expf(-zb));
+    const float decay = expf(-expf(a.a_log[head]) * (fmaxf(za, 0.f) + log1pf(expf(-fabsf(za)))));
+    // unit vectors and their product, every wave for itself (64 elements at a time, in their order, as delta_prepare_kernel adds them)
+    float sq = 0.f, sk = 0.f, dot = 0.f;
+#pragma unroll
+    for (int i = 0; i < DKP; i += TLI_WAVE) {
+        const float qe = i + lane < DKP ? q_s[i + lane] : 0.f, ke = i + lane < DKP ? k_s[i + lane] : 0.f;
+        sq += wave_sum(qe * qe);
+        sk += wave_sum(ke * ke);
+    }
+    const float q_unit = 1.0f / sqrtf(sq + 1e-6f), q_scale = 1.0f / sqrtf((float)dk), k_unit = 1.0f / sqrtf(sk + 1e-6f);
+#pragma unroll
+    for (int i = 0; i < DKP; i += TLI_WAVE) {
+        const float qe = i + lane < DKP ? q_s[i + lane] * q_unit * q_scale : 0.f, ke = i + lane < DKP ? k_s[i + lane] * k_unit : 0.f;
+        dot += wave_sum(qe * ke);
+    }
+    float q[RPT], k[RPT];
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) q[r] = q_s[part + DELTA_LANES * r] * q_unit * q_scale, k[r] = k_s[part + DELTA_LANES * r] * k_unit;
+    for (int c0 = 0; c0 < blocks * DELTA_COLS; c0 += GROUPS * TOGETHER) {
+        if (c0 > 0) load(c0);
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) {
+            const int col = c0 + g * TOGETHER + local;
+            if (col >= blocks * DELTA_COLS) continue;                    // (the 16 lanes of a column alike)
+            const float v = col < dv ? v_s[col] : 0.f;
+            float d1[2] = {0.f, 0.f}, d2[2] = {0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < RPT; ++r) {
+                d1[r & 1] = fmaf(k[r], S[g][r], d1[r & 1]);
+                d2[r & 1] = fmaf(q[r], S[g][r], d2[r & 1]);
+            }
+            const float s1 = row16_sum(d1[0] + d1[1]), s2 = row16_sum(d2[0] + d2[1]);
+            const float u = beta * (v - decay * s1);
+#pragma unroll
+            for (int r = 0; r < RPT; ++r) at(col)[r * DELTA_COLS * DELTA_LANES] = fmaf(k[r], u, decay * S[g][r]);
+            if (part == 0 && col < dv) o_s[col] = fmaf(dot, u, decay * s2);
+        }
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    // the norm over the head's outputs (one wave, in the order of gated_rmsnorm_kernel)
+    const bf16_t* gate = a.proj + (size_t)row * a.ld + C + (size_t)head * dv;
+    float ss = 0.f;
+    for (int i = lane; i < dv; i += TLI_WAVE) ss += o_s[i] * o_s[i];
+    ss = wave_sum(ss);
+    const float scale = 1.0f / sqrtf(ss / (float)dv + a.eps);
+    bf16_t* y = a.out + ((size_t)row * H + head) * dv;
+    for (int i = lane; i < dv; i += TLI_WAVE) from_f32(y + i, o_s[i] * scale * a.weight[i] * silu_f(to_f32(gate[i])));
+}
+
+// ---------------------------------------------------------------------------------------------
 // C ABI
 // ---------------------------------------------------------------------------------------------
 #define DELTA_MAX_DK 256
@@ -338,4 +502,41 @@ extern "C" int tli_gated_rmsnorm(const float* o, const void* gate, int gate_ld, 
     else
         return tli_fail("gated_rmsnorm: unknown dtype %d", dtype);
     return tli_check_launch("gated_rmsnorm");
+}
+
+// A decode step (one row a sequence) in bfloat16, from the projections to the gated norm's output [rows, H dv]: proj as for
+// tli_delta_prepare with the output gate (H dv) behind the channels; x [rows, n], w_gates [2 H, n]; slots and positions per row;
+// the kept rows are moved on.
+extern "C" int tli_delta_step_bf16(const void* proj, int ld, const void* x, const void* w_gates, int n, const float* conv_w, void* kept,
+                                   const float* a_log, const float* dt_bias, const float* weight, const int* positions,
+                                   const int* row_start, const int* seq_start, const int* slots, float* state, void* out, int rows,
+                                   int H, int G, int dk, int dv, int taps, float eps, void* stream) {
+    if (rows <= 0) return 0;
+    if (H <= 0 || G <= 0 || H % G || dk <= 0 || dv <= 0 || taps <= 0 || dk > DELTA_MAX_DK || H > 65535 || rows > 65535)
+        return tli_fail("delta_step: bad sizes (heads %d, key heads %d, dk %d (at most %d), dv %d, taps %d, rows %d)", H, G, dk,
+                        DELTA_MAX_DK, dv, taps, rows);
+    const int C = 2 * G * dk + H * dv;
+    if (ld < C + H * dv) return tli_fail("delta_step: rows of %d hold fewer than the %d channels and the gate", ld, C);
+    if (taps > 1 && !kept) return tli_fail("delta_step: %d taps need the sequences' kept rows", taps);
+    if (n <= 0 || n % 8 || (((uintptr_t)x | (uintptr_t)w_gates) & 15)) return tli_fail("delta_step: the gates' operands must be whole 16-byte pieces");
+    const int rpt = dk <= 16 ? 1 : dk <= 32 ? 2 : dk <= 64 ? 4 : dk <= 128 ? 8 : 16;
+    const size_t lds = (size_t)(2 * DELTA_LANES * rpt + 2 * dv) * sizeof(float);
+    if (lds > 60 * 1024) return tli_fail("delta_step: values of %d do not fit LDS", dv);
+    const DeltaStep a{(const bf16_t*)proj, ld, (const bf16_t*)x, (const bf16_t*)w_gates, n, conv_w, taps > 1 ? (const bf16_t*)kept : nullptr,
+                      a_log, dt_bias, weight, positions, slots, state, (bf16_t*)out, H, G, dk, dv, taps, eps};
+    hipStream_t s = (hipStream_t)stream;
+    const dim3 grid(H, rows);
+#define TLI_DELTA_STEP(RPT) case RPT: delta_step_kernel<RPT><<<grid, DELTA_STEP_THREADS, lds, s>>>(a); break
+    switch (rpt) {
+        TLI_DELTA_STEP(1);
+        TLI_DELTA_STEP(2);
+        TLI_DELTA_STEP(4);
+        TLI_DELTA_STEP(8);
+        default: delta_step_kernel<16><<<grid, DELTA_STEP_THREADS, lds, s>>>(a);
+    }
+#undef TLI_DELTA_STEP
+    if (taps > 1)
+        delta_conv_keep_kernel<bf16_t><<<dim3((C + 255) / 256, rows), 256, 0, s>>>((const bf16_t*)proj, ld, (bf16_t*)kept, row_start, seq_start,
+                                                                                  slots, C, taps);
+    return tli_check_launch("delta_step");
 }

@@ -115,6 +115,7 @@ def load_library():
                               I, I, I, I, I, I, I, I, P],
         "tli_delta_recurrence": [P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, P],
         "tli_delta_state_floats": [I, I],
+        "tli_delta_step_bf16": [P, I, P, P, I, P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, P],
         "tli_gated_rmsnorm": [P, P, I, P, P, I, I, I, F, I, P],
         "tli_moe_route": [P, ctypes.c_longlong, ctypes.c_longlong, P, P, P, I, I, I, I, I, F, I, I, I, I, P, P],
         "tli_moe_router_bf16": [P, P, I, P, P, P, I, I, I, I, I, F, I, I, I, I, P, P],
@@ -1310,21 +1311,14 @@ class HipOps:
             raise KernelError(f"a state of {dk} x {dv} a head is not supported")
         return (heads, n)
 
-    def delta_rule(self, proj, gates, conv, a_log, dt_bias, kept, state, step, heads, kv_heads, dk, dv, taps,
-                   gates_transposed=False):
-        """From the raw projections ``proj`` [T, >= channels] (q, k, v first) and ``gates`` (float32 [T, 2 H]:
-        b, then a; [2 H, T] with ``gates_transposed``) to the heads' outputs of the recurrence, float32 [T, H dv].  ``conv``: float32 [taps,
-        channels], oldest tap first; ``kept`` [slots, taps - 1, channels] and ``state`` (float32 [slots,
-        *delta_state_shape]) are the sequences' state, read (unless a sequence starts at position 0) and replaced."""
+    def _check_delta(self, proj, need, conv, a_log, dt_bias, kept, state, step, heads, kv_heads, dk, dv, taps):
+        """What both forms of the delta rule ask of their operands; ``need``: columns of the projections."""
         T = step.num_rows
         self.check_delta_sizes(heads, kv_heads, dk, dv, taps)
-        qd, vd = kv_heads * dk, heads * dv
-        C = 2 * qd + vd
-        if proj.dim() != 2 or proj.shape[0] != T or proj.shape[1] < C:
-            raise KernelError(f"the projections have shape {tuple(proj.shape)}, expected [{T}, >= {C}]")
+        C = 2 * kv_heads * dk + heads * dv
+        if proj.dim() != 2 or proj.shape[0] != T or proj.shape[1] < need:
+            raise KernelError(f"the projections have shape {tuple(proj.shape)}, expected [{T}, >= {need}]")
         self._want(proj, "projections")
-        self._want(gates, "b and a", torch.float32, (2 * heads, T) if gates_transposed else (T, 2 * heads))
-        ba_row, ba_col = (1, T) if gates_transposed else (2 * heads, 1)
         self._want(conv, "convolution weights", torch.float32, (taps, C))
         self._want(a_log, "A_log", torch.float32, (heads,))
         self._want(dt_bias, "dt_bias", torch.float32, (heads,))
@@ -1336,6 +1330,39 @@ class HipOps:
             self._want(kept, "kept rows of the convolution", proj.dtype, (slots, taps - 1, C))
         if max(step.h_slots, default=0) >= slots:
             raise KernelError("a sequence's slot lies outside the state")
+
+    DELTA_STEP_VALUES = 4096     # a head's values and outputs lie in the workgroup's memory
+
+    def delta_step(self, proj, x, w_gates, conv, a_log, dt_bias, kept, state, step, heads, kv_heads, dk, dv, taps, weight, eps):
+        """A step of one row a sequence in bfloat16, the layer's gates (``x`` [T, n] times ``w_gates`` [2 H, n]: b, then a), ``delta_rule``
+        and ``gated_rmsnorm`` in one: the heads' normed outputs [T, H dv]; the output gate lies behind the channels of ``proj``.  None for
+        other steps, with nothing done."""
+        if (x.dtype != torch.bfloat16 or proj.dtype != torch.bfloat16 or x.shape[1] % 8 or dv > self.DELTA_STEP_VALUES or self.plain_products
+                or not self._single_rows(step)):
+            return None
+        T = step.num_rows
+        self._check_delta(proj, 2 * kv_heads * dk + 2 * heads * dv, conv, a_log, dt_bias, kept, state, step, heads, kv_heads, dk, dv, taps)
+        self._want(x, "layer input", torch.bfloat16, (T, x.shape[1]))
+        self._want(w_gates, "rows of b and a", torch.bfloat16, (2 * heads, x.shape[1]))
+        self._want(weight, "norm weight", torch.float32, (dv,))
+        out = torch.empty((T, heads * dv), dtype=torch.bfloat16, device=self.device)
+        self._call(self.lib.tli_delta_step_bf16, proj.data_ptr(), proj.shape[1], x.data_ptr(), w_gates.data_ptr(), x.shape[1], conv.data_ptr(),
+                   _ptr(kept), a_log.data_ptr(), dt_bias.data_ptr(), weight.data_ptr(), step.positions.data_ptr(), step.row_start.data_ptr(),
+                   step.seq_start.data_ptr(), step.slots.data_ptr(), state.data_ptr(), out.data_ptr(), T, heads, kv_heads, dk, dv, taps,
+                   float(eps), self._stream())
+        return out
+
+    def delta_rule(self, proj, gates, conv, a_log, dt_bias, kept, state, step, heads, kv_heads, dk, dv, taps,
+                   gates_transposed=False):
+        """From the raw projections ``proj`` [T, >= channels] (q, k, v first) and ``gates`` (float32 [T, 2 H]:
+        b, then a; [2 H, T] with ``gates_transposed``) to the heads' outputs of the recurrence, float32 [T, H dv].  ``conv``: float32 [taps,
+        channels], oldest tap first; ``kept`` [slots, taps - 1, channels] and ``state`` (float32 [slots,
+        *delta_state_shape]) are the sequences' state, read (unless a sequence starts at position 0) and replaced."""
+        T = step.num_rows
+        qd, vd = kv_heads * dk, heads * dv
+        self._check_delta(proj, 2 * qd + vd, conv, a_log, dt_bias, kept, state, step, heads, kv_heads, dk, dv, taps)
+        self._want(gates, "b and a", torch.float32, (2 * heads, T) if gates_transposed else (T, 2 * heads))
+        ba_row, ba_col = (1, T) if gates_transposed else (2 * heads, 1)
         f32 = dict(dtype=torch.float32, device=self.device)
         qn, kn = torch.empty((T, qd), **f32), torch.empty((T, qd), **f32)
         vc, out = torch.empty((T, vd), **f32), torch.empty((T, vd), **f32)

@@ -92,8 +92,14 @@ class GatedDeltaRule(Mixer):
     def forward(self, x: torch.Tensor, step: StepView):
         ops = self.env.ops
         main = ops.linear(x, self.w_main)
-        gates, transposed = ops.small_product(x, self.w_gates)
         states = step.state
+        one = getattr(ops, "delta_step", None)
+        if one is not None:                    # (one row a sequence: everything between the products in one launch)
+            y = one(main, x, self.w_gates, self.conv, self.a_log, self.dt_bias, states.get("conv"), states["S"], step,
+                    self.heads, self.kv_heads, self.dk, self.dv, self.taps, self.norm, self.eps)
+            if y is not None:
+                return ops.linear(y, self.w_o, deferred=True)
+        gates, transposed = ops.small_product(x, self.w_gates)
         o = ops.delta_rule(main, gates, self.conv, self.a_log, self.dt_bias, states.get("conv"), states["S"], step,
                            self.heads, self.kv_heads, self.dk, self.dv, self.taps, gates_transposed=transposed)
         y = ops.gated_rmsnorm(o, main, self.channels, self.norm, self.eps, self.heads, self.dv, self.env.dtype)
