@@ -21,13 +21,7 @@
 // what the others do not take.  Steps of few rows in bfloat16 (up to 64, or 32 of many experts) go expert by expert (moe_few.hip),
 // steps of more rows sort the pairs by expert and multiply tile by tile (moe_grouped.hip).
 #include "common.h"
-
-#define MOE_MAX_TOP 32
-
-// What the choice goes by.  A score that is no number (a row with a NaN or an infinity in it) counts as the lowest: a NaN
-// compares as neither larger nor smaller, the lanes of a choice would not agree on the largest, and an expert could be chosen
-// twice.
-__device__ __forceinline__ float choice_score(float v) { return v != v ? -INFINITY : v; }
+#include "moe_route.h"
 
 __global__ void moe_route_kernel(const float* __restrict__ z, long long z_row, long long z_col, int* __restrict__ ids,
                                  float* __restrict__ weights, float* __restrict__ shared_gate, int T, int E,
@@ -97,16 +91,6 @@ __global__ void moe_route_kernel(const float* __restrict__ z, long long z_row, l
     }
 }
 
-// The largest of the lanes' values, ties to the lower index; every lane gets both.  (index < 0: the lane has none)
-__device__ __forceinline__ void wave_best(float& v, int& index) {
-#pragma unroll
-    for (int off = TLI_WAVE / 2; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(v, off, TLI_WAVE);
-        const int oi = __shfl_xor(index, off, TLI_WAVE);
-        if (oi >= 0 && (index < 0 || ov > v || (ov == v && oi < index))) v = ov, index = oi;
-    }
-}
-
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 
 // A workgroup a row: what bounds it is the time of a fetch from memory and the chain of lane exchanges of the choice, so a
@@ -115,25 +99,22 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 #define ROUTER_THREADS 1024
 #define ROUTER_WAVES (ROUTER_THREADS / TLI_WAVE)
 template <int COLS>
-__global__ __launch_bounds__(ROUTER_THREADS) void moe_router_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int D,
-                                                                    int* __restrict__ ids, float* __restrict__ weights,
-                                                                    float* __restrict__ shared_gate, int E, int top, int groups,
-                                                                    int keep, float scale, int has_shared, int softmax_scores,
-                                                                    int group_by_max, int normalize, const float* __restrict__ correction) {
+__global__ __launch_bounds__(ROUTER_THREADS) void moe_router_kernel(const bf16_t* __restrict__ x, int D, RouteArgs a) {
     extern __shared__ float rt_lds[];              // the row's logits [E + 1], then its scores; then the choice scores [E]
+    const int E = a.E;
     float* s = rt_lds;
     float* c = rt_lds + E + 1;
     const size_t t = blockIdx.x;
     const int lane = threadIdx.x % TLI_WAVE, wave = threadIdx.x / TLI_WAVE;
     const bf16_t* xr = x + t * D;
-    const int cols = E + (has_shared ? 1 : 0);
-    for (int e = threadIdx.x; e < E; e += ROUTER_THREADS) c[e] = correction ? correction[e] : 0.f;     // (fetched beside the rows)
+    const int cols = a.cols();
+    for (int e = threadIdx.x; e < E; e += ROUTER_THREADS) c[e] = a.correction ? a.correction[e] : 0.f;     // (fetched beside the rows)
     for (int e0 = wave; e0 < cols; e0 += COLS * ROUTER_WAVES) {
         constexpr int UNROLL = COLS > 2 ? 2 : 4;
         const bf16_t* we[COLS];                    // (past the last row: the last one again, its sum not kept)
-        float a[COLS];
+        float sum[COLS];
 #pragma unroll
-        for (int j = 0; j < COLS; ++j) we[j] = w + (size_t)min(e0 + j * ROUTER_WAVES, cols - 1) * D, a[j] = 0.f;
+        for (int j = 0; j < COLS; ++j) we[j] = a.w + (size_t)min(e0 + j * ROUTER_WAVES, cols - 1) * D, sum[j] = 0.f;
 #pragma unroll UNROLL
         for (int i = lane * 8; i < D; i += TLI_WAVE * 8) {
             const u32x4_t u = *reinterpret_cast<const u32x4_t*>(xr + i);
@@ -144,70 +125,19 @@ __global__ __launch_bounds__(ROUTER_THREADS) void moe_router_kernel(const bf16_t
             for (int j = 0; j < COLS; ++j)
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    a[j] = fmaf(__uint_as_float(u[k] << 16), __uint_as_float(v[j][k] << 16), a[j]);
-                    a[j] = fmaf(__uint_as_float(u[k] & 0xFFFF0000u), __uint_as_float(v[j][k] & 0xFFFF0000u), a[j]);
+                    sum[j] = fmaf(__uint_as_float(u[k] << 16), __uint_as_float(v[j][k] << 16), sum[j]);
+                    sum[j] = fmaf(__uint_as_float(u[k] & 0xFFFF0000u), __uint_as_float(v[j][k] & 0xFFFF0000u), sum[j]);
                 }
         }
 #pragma unroll
         for (int j = 0; j < COLS; ++j) {
-            const float sum = wave_sum(a[j]);
-            if (lane == 0 && e0 + j * ROUTER_WAVES < cols) s[e0 + j * ROUTER_WAVES] = sum;
+            const float z = wave_sum(sum[j]);
+            if (lane == 0 && e0 + j * ROUTER_WAVES < cols) s[e0 + j * ROUTER_WAVES] = z;
         }
     }
     __syncthreads();
     if (wave > 0) return;
-    if (has_shared && lane == 0) shared_gate[t] = 1.0f / (1.0f + expf(-s[E]));
-    if (softmax_scores) {
-        float top_z = -INFINITY, sum = 0.f;
-        for (int e = lane; e < E; e += TLI_WAVE) top_z = fmaxf(top_z, s[e]);
-        top_z = wave_max(top_z);
-        for (int e = lane; e < E; e += TLI_WAVE) {
-            s[e] = expf(s[e] - top_z);
-            sum += s[e];
-        }
-        sum = wave_sum(sum);
-        for (int e = lane; e < E; e += TLI_WAVE) s[e] /= sum;
-    } else {
-        for (int e = lane; e < E; e += TLI_WAVE) s[e] = 1.0f / (1.0f + expf(-s[e]));
-    }
-    for (int e = lane; e < E; e += TLI_WAVE) c[e] = choice_score(correction ? s[e] + c[e] : s[e]);
-    wave_lds_sync();
-    const int per = E / groups;
-    unsigned long long open = ~0ull;               // the `keep` best groups, a bit each (groups <= 64: one a lane)
-    if (keep < groups) {
-        open = 0ull;
-        float a = -INFINITY, b = -INFINITY;        // the two largest of this lane's group
-        if (lane < groups)
-            for (int e = lane * per; e < (lane + 1) * per; ++e) {
-                const float v = c[e];
-                if (v > a) { b = a; a = v; }
-                else if (v > b) b = v;
-            }
-        const float score = (b > -INFINITY && !group_by_max) ? a + b : a;
-        for (int n = 0; n < keep; ++n) {
-            float v = score;
-            int g = lane < groups && !((open >> lane) & 1ull) ? lane : -1;
-            wave_best(v, g);
-            if (g >= 0) open |= 1ull << g;
-        }
-    }
-    uint32_t taken = 0u;                           // of this lane's experts lane, lane + 64, .. (E <= 2048)
-    float total = 0.f, mine = 0.f;                 // the weight of this lane's place in the choice (top <= 32)
-    for (int n = 0; n < top; ++n) {
-        float v = -INFINITY;
-        int best = -1;
-        for (int e = lane, k = 0; e < E; e += TLI_WAVE, ++k)
-            if (!((taken >> k) & 1u) && ((open >> (e / per)) & 1ull) && (best < 0 || c[e] > v)) v = c[e], best = e;
-        wave_best(v, best);
-        if (best < 0) best = 0;                    // (not with sizes that the host lets through)
-        if (best % TLI_WAVE == lane) taken |= 1u << (best / TLI_WAVE);
-        total += s[best];
-        if (lane == n) {
-            mine = s[best];
-            ids[t * top + n] = best;
-        }
-    }
-    if (lane < top) weights[t * top + lane] = mine * (normalize ? scale / (total + 1e-20f) : scale);
+    route_choice(a, s, c, t, lane);
 }
 
 // one workgroup a pair; a wave takes every (waves)th hidden unit, its lanes share out k
@@ -302,16 +232,15 @@ extern "C" int tli_moe_router_bf16(const void* x, const void* w, int D, int* ids
                                    int groups, int keep, float scale, int has_shared, int softmax_scores, int group_by_max,
                                    int normalize, const float* correction, void* stream) {
     if (T <= 0) return 0;
-    if (E <= 0 || E > 2048 || top <= 0 || top > E || top > MOE_MAX_TOP || groups <= 0 || groups > 64 || E % groups || keep <= 0 ||
-        keep > groups || (long long)keep * (E / groups) < top || D <= 0 || D % 8)
+    const RouteArgs a{(const bf16_t*)w, ids, weights, shared_gate, E, top, groups, keep, scale, has_shared, softmax_scores, group_by_max,
+                      normalize, correction};
+    if (route_fault(a) || D <= 0 || D % 8)
         return tli_fail("moe_router: bad sizes (experts %d, top %d (at most %d), groups %d (at most 64), keep %d, width %d)", E, top,
                         MOE_MAX_TOP, groups, keep, D);
     if (((uintptr_t)x | (uintptr_t)w) & 15) return tli_fail("moe_router: operands must be 16-byte aligned");
-    const int rounds = (E + (has_shared ? 1 : 0) + ROUTER_WAVES - 1) / ROUTER_WAVES;
-#define ROUTER_LAUNCH(COLS)                                                                                              \
-    moe_router_kernel<COLS><<<T, ROUTER_THREADS, (size_t)(2 * E + 1) * sizeof(float), (hipStream_t)stream>>>(            \
-        (const bf16_t*)x, (const bf16_t*)w, D, ids, weights, shared_gate, E, top, groups, keep, scale, has_shared,       \
-        softmax_scores, group_by_max, normalize, correction)
+    const int rounds = (a.cols() + ROUTER_WAVES - 1) / ROUTER_WAVES;
+#define ROUTER_LAUNCH(COLS) \
+    moe_router_kernel<COLS><<<T, ROUTER_THREADS, (size_t)(2 * E + 1) * sizeof(float), (hipStream_t)stream>>>((const bf16_t*)x, D, a)
     // As many logits of a wave together as it has, up to four.  Weights from memory, 8 rows, one logit at a time and this rule, us:
     // 16 experts and a shared gate of width 512 5.47 and 5.44, of 1,024 6.34 and 6.05, of 4,096 11.7 and 9.5; 32 of 2,048 10.5 and
     // 8.6; 40 of 2,048 12.3 and 9.9, 64 of 4,096 26.1 and 18.1.  (17 logits whose weights lie in the L2 caches, which they never do

@@ -159,6 +159,8 @@ def load_library():
         "tli_gemm_mid_unit_bf16": [P, P, P, I, I, I, I, P, P, I, I, P],
         "tli_gemm_reduce_unit_bf16": [P, P, I, I, I, I, P, P, I, I, P],
         "tli_token_mixes": [P, P, I, P, P, P, P, P, P, I, I, I, P],
+        "tli_add_layernorm_route_bf16": [P, P, I, P, I, P, P, P, P, I, I, F, P, P, P, P, I, I, I, I, F, I, I, I, I, P, P],
+        "tli_norm_add_norm_route_bf16": [P, P, I, P, F, P, F, P, I, I, P, P, P, P, I, I, I, I, F, I, I, I, I, P, P],
         "tli_norm_rows": [P, I, P, P, I, I, F, I, P],
         "tli_token_gate": [P, P, P, P, I, I, I, I, I, I, I, P],
         "tli_wkv_decays": [P, ctypes.c_longlong, ctypes.c_longlong, P, P, P, I, I, I, I, P],
@@ -1240,11 +1242,7 @@ class HipOps:
         return out
 
     # ---- layer norm ------------------------------------------------------------------------------
-    def add_layernorm(self, resid, deltas, weights, eps, out_dtype, rows=None, num_rows=None):
-        """``resid`` (float32 [T, n]) takes the sum of ``deltas`` (none, one or two tensors [T, n] of
-        ``out_dtype``, or unfinished products: what the parts before still owe it); returns the layer norm (no bias) of its rows
-        once for every weight vector of ``weights`` (one or two: norms of the same rows share their mean
-        and variance).  With ``rows`` only those rows are computed and ``resid`` stays as it is."""
+    def _layernorm_operands(self, resid, deltas, weights, out_dtype):
         total, n = resid.shape
         self._want(resid, "residual", torch.float32)
         deltas, parts = list(deltas), [0, 0]
@@ -1259,6 +1257,33 @@ class HipOps:
             self._want(deltas[i], "residual delta", out_dtype, (total, n))
         for w in weights:
             self._want(w, "norm weight", torch.float32, (n,))
+        return deltas, parts
+
+    def add_layernorm_route(self, resid, deltas, weights, eps, out_dtype, route):
+        """``add_layernorm`` of all rows and the ``router`` of the last output's rows in one launch: (outputs, (ids, weights, gate)); None for
+        what it does not take, with nothing done.  ``route``: the arguments of ``router`` after its input, by name."""
+        if not self._norm_takes_route(resid, out_dtype, route):
+            return None
+        total, n = resid.shape
+        deltas, parts = self._layernorm_operands(resid, deltas, weights, out_dtype)
+        outs = [torch.empty((total, n), dtype=out_dtype, device=self.device) for _ in weights]
+        d1 = deltas[0] if deltas else None
+        d2 = deltas[1] if len(deltas) > 1 else None
+        if not self._aligned(resid, d1, d2, *weights):
+            return None
+        routed, args = self._route_outputs(total, n, route)
+        self._call(self.lib.tli_add_layernorm_route_bf16, resid.data_ptr(), _ptr(d1), parts[0], _ptr(d2), parts[1], weights[0].data_ptr(),
+                   _ptr(weights[1]) if len(weights) > 1 else None, outs[0].data_ptr(), outs[1].data_ptr() if len(weights) > 1 else None,
+                   total, n, float(eps), *args, self._stream())
+        return outs, routed
+
+    def add_layernorm(self, resid, deltas, weights, eps, out_dtype, rows=None, num_rows=None):
+        """``resid`` (float32 [T, n]) takes the sum of ``deltas`` (none, one or two tensors [T, n] of
+        ``out_dtype``, or unfinished products: what the parts before still owe it); returns the layer norm (no bias) of its rows
+        once for every weight vector of ``weights`` (one or two: norms of the same rows share their mean
+        and variance).  With ``rows`` only those rows are computed and ``resid`` stays as it is."""
+        total, n = resid.shape
+        deltas, parts = self._layernorm_operands(resid, deltas, weights, out_dtype)
         out_rows = total
         if rows is not None:
             self._want(rows, "row list", torch.int32)
@@ -1446,6 +1471,33 @@ class HipOps:
                    self.ROUTER_GROUP_SCORES.index(group_score), 1 if normalize else 0, _ptr(correction), self._stream())
         return ids, weights, gate
 
+    NORM_ROUTE_COLS, NORM_ROUTE_WIDTH = 32, 4096          # what a norm with a router in its launch takes (csrc/moe_route.h)
+
+    def _norm_takes_route(self, resid, out_dtype, route) -> bool:
+        T, n = resid.shape
+        return (out_dtype == torch.bfloat16 and n % 8 == 0 and n <= self.NORM_ROUTE_WIDTH and 0 < T <= self.ROUTER_ROWS and not self.separate_norms
+                and not self.plain_products and route["experts"] + (1 if route["has_shared"] else 0) <= self.NORM_ROUTE_COLS
+                and self._aligned(route["w_rows"]))
+
+    @staticmethod
+    def _aligned(*tensors) -> bool:
+        return all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
+
+    def _route_outputs(self, T, n, route):
+        """(ids, weights, gate) of T rows of n elements and the arguments of the C entries for them."""
+        experts, top, has_shared, correction = route["experts"], route["top"], route["has_shared"], route.get("correction")
+        score, group_score = route.get("score", "sigmoid"), route.get("group_score", "top2")
+        self.check_router(score, group_score)
+        self._want(route["w_rows"], "router rows", torch.bfloat16, (experts + (1 if has_shared else 0), n))
+        if correction is not None:
+            self._want(correction, "router correction", torch.float32, (experts,))
+        ids = torch.empty((T, top), dtype=torch.int32, device=self.device)
+        weights = torch.empty((T, top), dtype=torch.float32, device=self.device)
+        gate = torch.empty((T,), dtype=torch.float32, device=self.device) if has_shared else None
+        return (ids, weights, gate), (route["w_rows"].data_ptr(), ids.data_ptr(), weights.data_ptr(), _ptr(gate), experts, top, route["groups"],
+                                      route["keep"], float(route["scale"]), 1 if has_shared else 0, self.ROUTER_SCORES.index(score),
+                                      self.ROUTER_GROUP_SCORES.index(group_score), 1 if route.get("normalize", True) else 0, _ptr(correction))
+
     ROUTER_ROWS = 128            # up to so many rows the router's product and its choice are one launch
 
     def router(self, x, w_rows, experts, top, groups, keep, scale, has_shared, score="sigmoid", group_score="top2", normalize=True,
@@ -1455,18 +1507,12 @@ class HipOps:
         if x.dtype != torch.bfloat16 or n % 8 or not 0 < T <= self.ROUTER_ROWS or self.plain_products:
             z, transposed = self.small_product(x, w_rows)
             return self.route_experts(z, experts, top, groups, keep, scale, has_shared, transposed, score, group_score, normalize, correction)
-        self.check_router(score, group_score)
         self._want(x, "router input")
-        self._want(w_rows, "router rows", torch.bfloat16, (experts + (1 if has_shared else 0), n))
-        if correction is not None:
-            self._want(correction, "router correction", torch.float32, (experts,))
-        ids = torch.empty((T, top), dtype=torch.int32, device=self.device)
-        weights = torch.empty((T, top), dtype=torch.float32, device=self.device)
-        gate = torch.empty((T,), dtype=torch.float32, device=self.device) if has_shared else None
-        self._call(self.lib.tli_moe_router_bf16, x.data_ptr(), w_rows.data_ptr(), n, ids.data_ptr(), weights.data_ptr(), _ptr(gate), T,
-                   experts, top, groups, keep, float(scale), 1 if has_shared else 0, self.ROUTER_SCORES.index(score),
-                   self.ROUTER_GROUP_SCORES.index(group_score), 1 if normalize else 0, _ptr(correction), self._stream())
-        return ids, weights, gate
+        routed, args = self._route_outputs(T, n, dict(w_rows=w_rows, experts=experts, top=top, groups=groups, keep=keep, scale=scale,
+                                                      has_shared=has_shared, score=score, group_score=group_score, normalize=normalize,
+                                                      correction=correction))
+        self._call(self.lib.tli_moe_router_bf16, x.data_ptr(), args[0], n, *args[1:4], T, *args[4:], self._stream())
+        return routed
 
     def apply_experts(self, x, ids, weights, w_gate_up, w_down, packed, shared, shared_gate, limit=0.0, slope=1.0,
                       activation=None, weight_on_input=False):
@@ -1639,6 +1685,21 @@ class HipOps:
         ``rows`` (int32 on the device, the first ``num_rows`` of them) only those rows, and ``resid`` is left as it is."""
         return self._norm_add_norm(resid, y, w_out, eps_out, w_in, eps_in, out_dtype, rows, num_rows, None, None)
 
+    def norm_add_norm_route(self, resid, y, w_out, eps_out, w_in, eps_in, out_dtype, route):
+        """``norm_add_norm`` of all rows and the ``router`` of its output's rows in one launch, (output, (ids, weights, gate)); None for what
+        it does not take, with nothing done.  ``route``: the arguments of ``router`` after its input, by name."""
+        if not self._norm_takes_route(resid, out_dtype, route):
+            return None
+        total, n = resid.shape
+        y, parts = self._norm_add_norm_operands(resid, y, w_out, w_in, out_dtype)
+        if not self._aligned(resid, y, w_out, w_in):
+            return None
+        out = torch.empty((total, n), dtype=out_dtype, device=self.device)
+        routed, args = self._route_outputs(total, n, route)
+        self._call(self.lib.tli_norm_add_norm_route_bf16, resid.data_ptr(), _ptr(y), parts, None if y is None else w_out.data_ptr(),
+                   float(eps_out), w_in.data_ptr(), float(eps_in), out.data_ptr(), total, n, *args, self._stream())
+        return out, routed
+
     def norm_add_norm_mixes(self, resid, y, w_out, eps_out, w_in, eps_in, out_dtype, mixes, step):
         """``norm_add_norm`` and the ``token_mixes`` of its rows in one pass, [mixes, T, n], for a step of one row a sequence;
         None for other steps, with nothing done.  ``mixes`` = (mu [m, n], kept rows)."""
@@ -1646,7 +1707,7 @@ class HipOps:
             return None
         return self._norm_add_norm(resid, y, w_out, eps_out, w_in, eps_in, out_dtype, None, None, mixes, step)
 
-    def _norm_add_norm(self, resid, y, w_out, eps_out, w_in, eps_in, out_dtype, rows, num_rows, mixes, step):
+    def _norm_add_norm_operands(self, resid, y, w_out, w_in, out_dtype):
         total, n = resid.shape
         self._want(resid, "residual", torch.float32)
         if w_in is not None:
@@ -1660,6 +1721,11 @@ class HipOps:
                 y = self.resolve(y)
                 self._want(y, "sublayer output", out_dtype, (total, n))
             self._want(w_out, "norm weight", torch.float32, (n,))
+        return y, parts
+
+    def _norm_add_norm(self, resid, y, w_out, eps_out, w_in, eps_in, out_dtype, rows, num_rows, mixes, step):
+        total, n = resid.shape
+        y, parts = self._norm_add_norm_operands(resid, y, w_out, w_in, out_dtype)
         count = total
         if rows is not None:
             self._want(rows, "rows", torch.int32)

@@ -130,13 +130,20 @@ class RoutedExperts(FeedForward):
     def workspace_elems(self, rows: int) -> int:
         return rows * (self.top * (3 * self.inter + self.hidden) + 3 * (self.shared_inter or 0) + 2 * self.outputs)
 
-    def forward(self, x: torch.Tensor, step: StepView):
-        ops = self.env.ops
-        how = {}
+    def routing(self) -> Dict:
+        """The arguments of the router after its input, by name: for norms whose kernel makes the choice as well."""
+        out = dict(w_rows=self.w_router, experts=self.outputs, top=self.top, groups=self.groups, keep=self.keep, scale=self.scale,
+                   has_shared=self.has_gate)
         if (self.score, self.group_score, self.normalize, self.correction) != ("sigmoid", "top2", True, None):
-            how = dict(score=self.score, group_score=self.group_score, normalize=self.normalize, correction=self.correction)
-        ids, weights, shared_gate = ops.router(x, self.w_router, self.outputs, self.top, self.groups, self.keep, self.scale,
-                                               self.has_gate, **how)
+            out.update(score=self.score, group_score=self.group_score, normalize=self.normalize, correction=self.correction)
+        return out
+
+    def forward(self, x: torch.Tensor, step: StepView, routed=None):
+        """``routed``: (ids, weights, shared gate) of the rows, where their norm's kernel has made them."""
+        ops = self.env.ops
+        if routed is None:
+            routed = ops.router(x, **self.routing())
+        ids, weights, shared_gate = routed
         few = getattr(ops, "experts_of_few_rows", None)
         if few is not None and x.shape[0] <= ops.few_expert_rows(self.experts):
             y = few(x, ids, weights, self.packed, self.shared_gate_up, self.shared_down, shared_gate, limit=self.limit, slope=self.slope,

@@ -53,16 +53,23 @@ class ParallelBlock(Block):
 
     def forward(self, resid: torch.Tensor, pending, step: StepView):
         owed = self._owed(pending)
+        chosen = {}                            # of routed experts, where the norms' kernel chooses them
         if self.pair is not None:
             (w1, w2), eps = self.pair
-            n1, n2 = self.env.ops.add_layernorm(resid, owed, (w1, w2), eps, self.env.dtype)
+            both = None
+            if hasattr(self.ffn, "routing") and hasattr(self.env.ops, "add_layernorm_route"):
+                both = self.env.ops.add_layernorm_route(resid, owed, (w1, w2), eps, self.env.dtype, self.ffn.routing())
+            if both is not None:
+                (n1, n2), chosen["routed"] = both
+            else:
+                n1, n2 = self.env.ops.add_layernorm(resid, owed, (w1, w2), eps, self.env.dtype)
         else:
             n1 = run_norm(self.norm_mixer, resid, self._one(owed))
             n2 = run_norm(self.norm_ffn, resid, None) if self.norm_ffn is not None else None
         a = self.mixer.forward(n1, step)
         if self.ffn is None:
             return (a,)
-        return (a, self.ffn.forward(n2, step))
+        return (a, self.ffn.forward(n2, step, **chosen))
 
     def close(self, resid, pending, final_norm, rows=None, num_rows=None):
         owed = self._owed(pending)

@@ -118,7 +118,8 @@ class SandwichBlock(Block):
         self.side_rms = rms(self.side.norm) if self.side is not None else None
 
     def _read(self, resid, owed, role: str, step: StepView, reader):
-        """The rows that the sublayer ``role`` reads, after what is owed to the residual has been added to it."""
+        """The rows that the sublayer ``role`` reads, after what is owed to the residual has been added to it, and what else
+        the sublayer is given (routed experts: their choice, where the norm's kernel makes it)."""
         ops = self.env.ops
         weight, eps = self.first[role]
         y, w_out, eps_out = (owed.y, owed.weight, owed.eps) if owed is not None else (None, None, 0.0)
@@ -126,8 +127,12 @@ class SandwichBlock(Block):
         if mixes is not None:                     # a reader of mixes of every row with the row before it: made in the same pass
             mixed = ops.norm_add_norm_mixes(resid, y, w_out, eps_out, weight, eps, self.env.dtype, mixes(step), step)
             if mixed is not None:
-                return mixed
-        return ops.norm_add_norm(resid, y, w_out, eps_out, weight, eps, self.env.dtype)
+                return mixed, {}
+        if hasattr(reader, "routing") and hasattr(ops, "norm_add_norm_route"):
+            both = ops.norm_add_norm_route(resid, y, w_out, eps_out, weight, eps, self.env.dtype, reader.routing())
+            if both is not None:
+                return both[0], {"routed": both[1]}
+        return ops.norm_add_norm(resid, y, w_out, eps_out, weight, eps, self.env.dtype), {}
 
     def forward(self, resid: torch.Tensor, pending, step: StepView):
         if pending is not None and not isinstance(pending, NormedDelta):
@@ -137,7 +142,8 @@ class SandwichBlock(Block):
         for role, part in (("mixer", self.mixer), ("ffn", self.ffn)):
             if part is None:
                 continue
-            y = part.forward(self._read(resid, owed, role, step, part), step)
+            rows, more = self._read(resid, owed, role, step, part)
+            y = part.forward(rows, step, **more)
             owed = NormedDelta(y, *self.last[role])
         if self.side is None:
             return owed
