@@ -31,13 +31,22 @@ static inline const char* route_fault(const RouteArgs& a) {
 __device__ __forceinline__ float choice_score(float v) { return v != v ? -INFINITY : v; }
 
 // The largest of the lanes' values, ties to the lower index; every lane gets both.  (index < 0: the lane has none)
+__device__ __forceinline__ void better_of(float& v, int& index, float ov, int oi) {
+    if (oi >= 0 && (index < 0 || ov > v || (ov == v && oi < index))) v = ov, index = oi;
+}
 __device__ __forceinline__ void wave_best(float& v, int& index) {
-#pragma unroll
-    for (int off = TLI_WAVE / 2; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(v, off, TLI_WAVE);
-        const int oi = __shfl_xor(index, off, TLI_WAVE);
-        if (oi >= 0 && (index < 0 || ov > v || (ov == v && oi < index))) v = ov, index = oi;
-    }
+    auto swapped = [&](const auto& a, const auto& b) {
+        v = __uint_as_float(a[0]), index = (int)b[0];
+        better_of(v, index, __uint_as_float(a[1]), (int)b[1]);
+    };
+    swapped(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false),
+            __builtin_amdgcn_permlane32_swap((unsigned)index, (unsigned)index, false, false));
+    swapped(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false),
+            __builtin_amdgcn_permlane16_swap((unsigned)index, (unsigned)index, false, false));
+    better_of(v, index, lane_xor8(v), __float_as_int(lane_xor8(__int_as_float(index))));
+    better_of(v, index, lane_xor4(v), __float_as_int(lane_xor4(__int_as_float(index))));
+    better_of(v, index, lane_xor2(v), __float_as_int(lane_xor2(__int_as_float(index))));
+    better_of(v, index, lane_xor1(v), __float_as_int(lane_xor1(__int_as_float(index))));
 }
 
 // The choice of row t by one wave: s [E (+ 1)] holds the logits, c [E] the correction (or anything); both in LDS
