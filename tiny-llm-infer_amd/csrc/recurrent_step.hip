@@ -6,13 +6,15 @@
 //   wkv:        d = exp(-exp(W2 tanh(z) + w0)) a channel; o = (S + diag(u) k v^T)^T r; S <- diag(d) S + k v^T; RMS times the
 //               weight; silu gate
 // A column of S belongs to 16 lanes of a wave, a lane holding R elements of it (as in lightning.hip: pieces of up to four
-// that lie side by side with the other lanes').  A workgroup takes 16 columns at a time and asks for the first GROUPS x 16
-// columns before anything else, so that the state's bytes, which are nearly all that such a step moves, are on their
-// way while the row's q, k, v and gates are made.
+// that lie side by side with the other lanes').  A workgroup takes 32 columns at a time and asks for the row's own operands, then
+// for the first GROUPS x 32 columns, so that the state's bytes, which are nearly all that such a step moves, are on their way
+// while the row's q, k, v and gates are made, and nothing of the row waits behind them.  With 256 threads, which asked for the state
+// first and for the decays' matrix after the row's tanh, 8 rows of 16 heads of 128 x 128 took (as part of a decode step): retention
+// 9.8 us and now 7.0, mLSTM 11.6 and 8.6, wkv 12.3 and 8.4.
 #include "recurrence.h"
 #include "row_gates.h"
 
-#define RS_THREADS 256
+#define RS_THREADS 512
 
 __device__ __forceinline__ float rs_sum16(float v) {     // over the 16 lanes of a DPP row; every lane gets it
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));
@@ -92,10 +94,11 @@ template <int KIND, int R, typename T, typename TO>
 __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, StepRetention ret, StepMemory mem, StepTimeMix mix) {
     constexpr bool MEMORY = KIND == STEP_MEMORY, WKV = KIND == STEP_WKV;
     constexpr int L = 16, DKP = L * R, NC = RS_THREADS / L;
-    constexpr int GROUPS = R >= 16 ? 4 : R >= 8 ? 8 : 8;               // of NC columns, in flight together
+    constexpr int GROUPS = 4;                                          // of NC columns, in flight together
     constexpr int VW = R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;
     extern __shared__ __align__(16) float rs_lds[];
-    __shared__ float red[16];
+    constexpr int WAVES = RS_THREADS / TLI_WAVE;
+    __shared__ float red[3 * WAVES];
     const int h = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, sub = tid % L, jl = tid / L;
     const int dk = a.dk, dv = a.dv, H = a.H, OV = dv + (MEMORY ? 1 : 0);
     float* q_s = rs_lds;
@@ -154,50 +157,56 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
         for (int g = 0; g < GROUPS; ++g)
             if (j0 + g * NC + jl < dv) load_column(j0 + g * NC + jl, S[g]);
     };
-    if constexpr (MEMORY) {
-        if (jl == 0) load_column(dv, n);
-    }
-    load(0);
+    // The row's operands first, into registers: an element of q or k a thread (2 DKP <= RS_THREADS), one of v, of the gate and of the norm's
+    // weights (more in rounds below), and what the kind needs.  Loads complete in the order of issue, so none of them waits for the
+    // state, and the state is on its way while they are worked on.
+    static_assert(2 * DKP <= RS_THREADS, "an element of q or k a thread");
     const T* src = (const T*)a.proj + (size_t)row * a.ld;
     const T* q_src = src + (size_t)h * dk;
     const T* k_src = src + (size_t)(H + h) * dk;
     const T* v_src = src + (size_t)2 * H * dk + (size_t)h * dv;
+    const T* g_src = src + (size_t)H * (2 * dk + dv) + (size_t)h * dv;
+    const float* weight = MEMORY ? mem.weight + h * dv : WKV ? mix.weight + h * dv : nullptr;
+    const bool is_k = tid >= DKP;
+    const int own = is_k ? tid - DKP : tid;                            // this thread's element
+    const bool owns = tid < 2 * DKP && own < dk;
+    const T* own_src = is_k ? k_src : q_src;
+    T qk_raw{}, other_raw{}, v_raw{}, g_raw{};
+    float weight_raw = 1.f;
+    if (owns) qk_raw = own_src[own];
+    if (tid < dv) {
+        v_raw = v_src[tid];
+        g_raw = g_src[tid];
+        if (MEMORY || WKV) weight_raw = weight[tid];
+    }
     float keep = 0.f, floor_ = 0.f;
+    float turn_cos = 1.f, turn_sin = 0.f;                              // retention: of this thread's element
+    bool turned = false, second = false;
+    constexpr int P = RS_THREADS / DKP;                                // wkv: neighbouring threads that share out a channel's row of W2
+    constexpr int HELD = 4;                                            //      16-byte pieces of it that a thread holds
+    const int channel = tid / P, part = tid % P;
+    const TO* w2 = WKV ? (const TO*)mix.w2 + (size_t)(h * dk + min(channel, dk - 1)) * mix.rank : nullptr;
+    const bool pieces = WKV && sizeof(TO) == 2 && mix.rank % 8 == 0;
+    uint4 w2_raw[WKV ? HELD : 1];
+    float z_raw = 0.f, w0_raw = 0.f, u_raw[WKV ? R : 1];
+    float zi = 0.f, zf = 0.f, ss = 0.f, m0 = 0.f;                      // mLSTM: this thread's parts of the gates' sums
+    float* m_slot = MEMORY ? mem.m_state + (size_t)slot * H + h : nullptr;
     if constexpr (WKV) {
-        for (int i = tid; i < mix.rank; i += RS_THREADS) z_s[i] = tanhf(mix.z[row * mix.z_row + i * mix.z_col]);
-        for (int e = tid; e < DKP; e += RS_THREADS) {
-            q_s[e] = e < dk ? to_f32(q_src[e]) : 0.f;
-            k_s[e] = e < dk ? to_f32(k_src[e]) : 0.f;
-        }
-        for (int j = tid; j < OV; j += RS_THREADS) v_s[j] = to_f32(v_src[j]);
-        __syncthreads();
-        // a channel's decay: P neighbouring threads share out its row of W2
-        constexpr int P = RS_THREADS / DKP;
-        const int c = tid / P, part = tid % P;
-        const TO* w = (const TO*)mix.w2 + (size_t)(h * dk + min(c, dk - 1)) * mix.rank;
-        float acc = 0.f;
-        if (sizeof(TO) == 2 && mix.rank % 8 == 0) {
-            for (int i = part * 8; i < mix.rank; i += 8 * P) {
-                const uint4 raw = *reinterpret_cast<const uint4*>(w + i);
-                const uint32_t b[4] = {raw.x, raw.y, raw.z, raw.w};
+        if (tid < mix.rank) z_raw = mix.z[row * mix.z_row + tid * mix.z_col];
+        w0_raw = mix.w0[h * dk + min(channel, dk - 1)];
+        if (pieces) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    acc = fmaf(z_s[i + 2 * e], __uint_as_float(b[e] << 16), acc);
-                    acc = fmaf(z_s[i + 2 * e + 1], __uint_as_float(b[e] & 0xFFFF0000u), acc);
-                }
+            for (int e = 0; e < HELD; ++e) {
+                const int i = (part + e * P) * 8;
+                w2_raw[e] = i < mix.rank ? *reinterpret_cast<const uint4*>(w2 + i) : make_uint4(0, 0, 0, 0);
             }
-        } else {
-            for (int i = part; i < mix.rank; i += P) acc = fmaf(z_s[i], to_f32(w[i]), acc);
         }
 #pragma unroll
-        for (int off = 1; off < P; off *= 2) acc += __shfl_xor(acc, off, TLI_WAVE);
-        if (part == 0) d_s[c] = c < dk ? expf(-expf(acc + mix.w0[h * dk + c])) : 0.f;
+        for (int r = 0; r < R; ++r) u_raw[r] = at(r) < dk ? mix.u[h * dk + at(r)] : 0.f;
     } else if constexpr (MEMORY) {
-        // the gates' logits: every thread a part of the two dot products
         const T* x = (const T*)mem.x + (size_t)row * mem.n;
         const T* wi = (const T*)mem.w + (size_t)h * mem.n;
         const T* wf = (const T*)mem.w + (size_t)(H + h) * mem.n;
-        float zi = 0.f, zf = 0.f;
         if (mem.n % 8 == 0) {
             for (int i = tid * 8; i < mem.n; i += RS_THREADS * 8) {
                 zi += rs_dot8(x + i, wi + i);
@@ -209,55 +218,78 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
                 zf = fmaf(to_f32(x[i]), to_f32(wf[i]), zf);
             }
         }
-        float ss = 0.f;
         for (int p = tid; p < mem.factor.parts; p += RS_THREADS) ss += mem.factor.ssq[(size_t)p * a.rows + row];
-        float* m_slot = mem.m_state + (size_t)slot * H + h;
-        const float m0 = fresh ? 0.f : *m_slot;
+        if (!fresh) m0 = *m_slot;
+    } else {
+        keep = ret.decay[h];
+        const int pos = ret.positions[row], half = ret.dims / 2;
+        turned = owns && ret.cos_table && pos >= 0 && pos < ret.table_positions && own < ret.dims;
+        if (turned) {
+            second = ret.pairing ? (own & 1) : own >= half;
+            const int pair = ret.pairing ? own / 2 : second ? own - half : own;
+            other_raw = own_src[ret.pairing ? own ^ 1 : second ? own - half : own + half];
+            turn_cos = ret.cos_table[(size_t)pos * half + pair];
+            turn_sin = ret.sin_table[(size_t)pos * half + pair];
+        }
+    }
+    if constexpr (MEMORY) {
+        if (jl == 0) load_column(dv, n);
+    }
+    load(0);
+    float x = to_f32(qk_raw);                                          // (zero past dk)
+    float take = 1.f;
+    if constexpr (WKV) {
+        if (tid < mix.rank) z_s[tid] = tanhf(z_raw);
+        for (int i = tid + RS_THREADS; i < mix.rank; i += RS_THREADS) z_s[i] = tanhf(mix.z[row * mix.z_row + i * mix.z_col]);
+    } else if constexpr (MEMORY) {
         zi = wave_sum(zi), zf = wave_sum(zf), ss = wave_sum(ss);
-        if (tid % TLI_WAVE == 0) red[tid / TLI_WAVE] = zi, red[4 + tid / TLI_WAVE] = zf, red[8 + tid / TLI_WAVE] = ss;
+        if (tid % TLI_WAVE == 0) red[tid / TLI_WAVE] = zi, red[WAVES + tid / TLI_WAVE] = zf, red[2 * WAVES + tid / TLI_WAVE] = ss;
         __syncthreads();                                               // (m0 is read by all as well)
-        zi = red[0] + red[1] + red[2] + red[3];
-        zf = red[4] + red[5] + red[6] + red[7];
+        zi = zf = ss = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) zi += red[w], zf += red[WAVES + w], ss += red[2 * WAVES + w];
         if (mem.factor.parts > 0) {
-            const float f = mem.factor.of_sum(red[8] + red[9] + red[10] + red[11]);
+            const float f = mem.factor.of_sum(ss);
             zi *= f, zf *= f;
         }
         const float gi = gate_capped(zi + mem.bias[h], mem.cap), gf = gate_log_sigmoid(gate_capped(zf + mem.bias[H + h], mem.cap));
         const float m = fmaxf(gf + m0, gi);
         keep = expf(gf + m0 - m);
         floor_ = expf(-m);
-        const float take = expf(gi - m);
+        take = expf(gi - m);
         if (tid == 0) *m_slot = m;
-        for (int e = tid; e < DKP; e += RS_THREADS) {
-            q_s[e] = e < dk ? to_f32(q_src[e]) * mem.q_scale : 0.f;
-            k_s[e] = e < dk ? to_f32(k_src[e]) : 0.f;
-        }
-        for (int j = tid; j < OV; j += RS_THREADS) v_s[j] = j < dv ? to_f32(v_src[j]) * take : take;
+        if (!is_k) x *= mem.q_scale;
     } else {
-        keep = ret.decay[h];
-        const int pos = ret.positions[row], half = ret.dims / 2;
-        const bool turn = ret.cos_table && pos >= 0 && pos < ret.table_positions;
-        const float* cos_row = turn ? ret.cos_table + (size_t)pos * half : nullptr;
-        const float* sin_row = turn ? ret.sin_table + (size_t)pos * half : nullptr;
-        for (int e = tid; e < 2 * DKP; e += RS_THREADS) {
-            const bool is_k = e >= DKP;
-            const int i = is_k ? e - DKP : e;
-            const T* head = is_k ? k_src : q_src;
-            float x = 0.f;
-            if (i < dk) {
-                x = to_f32(head[i]);
-                if (turn && i < ret.dims) {
-                    const bool second = ret.pairing ? (i & 1) : i >= half;
-                    const int pair = ret.pairing ? i / 2 : second ? i - half : i;
-                    const float other = to_f32(head[ret.pairing ? i ^ 1 : second ? i - half : i + half]);
-                    x = second ? rotate_second_half(x, other, cos_row[pair], sin_row[pair])
-                               : rotate_first_half(x, other, cos_row[pair], sin_row[pair]);
+        if (turned)
+            x = second ? rotate_second_half(x, to_f32(other_raw), turn_cos, turn_sin) : rotate_first_half(x, to_f32(other_raw), turn_cos, turn_sin);
+        if (is_k) x *= ret.k_scale;
+    }
+    if (tid < 2 * DKP) q_s[tid] = x;                                   // (k_s lies behind q_s)
+    if (tid < dv) v_s[tid] = to_f32(v_raw) * take;
+    for (int j = tid + RS_THREADS; j < dv; j += RS_THREADS) v_s[j] = to_f32(v_src[j]) * take;
+    if (MEMORY && tid == 0) v_s[dv] = take;
+    if constexpr (WKV) {
+        __syncthreads();
+        float acc = 0.f;
+        if (pieces) {
+            auto piece = [&](const uint4& raw, int i) {
+                const uint32_t b[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    acc = fmaf(z_s[i + 2 * e], __uint_as_float(b[e] << 16), acc);
+                    acc = fmaf(z_s[i + 2 * e + 1], __uint_as_float(b[e] & 0xFFFF0000u), acc);
                 }
-                if (is_k) x *= ret.k_scale;
-            }
-            q_s[e] = x;                                                // (k_s lies behind q_s)
+            };
+#pragma unroll
+            for (int e = 0; e < HELD; ++e)
+                if ((part + e * P) * 8 < mix.rank) piece(w2_raw[e], (part + e * P) * 8);
+            for (int i = (part + HELD * P) * 8; i < mix.rank; i += 8 * P) piece(*reinterpret_cast<const uint4*>(w2 + i), i);
+        } else {
+            for (int i = part; i < mix.rank; i += P) acc = fmaf(z_s[i], to_f32(w2[i]), acc);
         }
-        for (int j = tid; j < OV; j += RS_THREADS) v_s[j] = to_f32(v_src[j]);
+#pragma unroll
+        for (int off = 1; off < P; off *= 2) acc += __shfl_xor(acc, off, TLI_WAVE);
+        if (part == 0) d_s[channel] = channel < dk ? expf(-expf(acc + w0_raw)) : 0.f;
     }
     __syncthreads();
     float q[R], k[R];
@@ -268,7 +300,7 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             d[r] = d_s[at(r)];
-            if (at(r) < dk) bonus = fmaf(q[r] * mix.u[h * dk + at(r)], k[r], bonus);
+            bonus = fmaf(q[r] * u_raw[r], k[r], bonus);
         }
         bonus = rs_sum16(bonus);
     }
@@ -300,19 +332,19 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
     }
     __syncthreads();
     const float by = MEMORY ? 1.f / (fmaxf(fabsf(o_s[dv]), floor_) + 1e-6f) : 1.f;
-    float ss = 0.f;
+    float sum = 0.f;
     for (int j = tid; j < dv; j += RS_THREADS) {
-        const float x = o_s[j] * by;
-        ss = fmaf(x, x, ss);
+        const float o = o_s[j] * by;
+        sum = fmaf(o, o, sum);
     }
-    const float factor = a.scale * by / sqrtf(block_sum(ss, red) / (float)dv + a.eps);
-    const T* g_src = src + (size_t)H * (2 * dk + dv) + (size_t)h * dv;
+    const float factor = a.scale * by / sqrtf(block_sum(sum, red) / (float)dv + a.eps);
     TO* dst = (TO*)a.out + (size_t)row * a.out_ld + (size_t)h * dv;
-    for (int j = tid; j < dv; j += RS_THREADS) {
-        const float z = to_f32(g_src[j]);
-        const float open = (MEMORY ? mem.weight[h * dv + j] : WKV ? z * mix.weight[h * dv + j] : z) / (1.f + expf(-z));
+    auto put = [&](int j, float z, float by_weight) {
+        const float open = (MEMORY ? by_weight : WKV ? z * by_weight : z) / (1.f + expf(-z));
         from_f32(dst + j, o_s[j] * factor * open);
-    }
+    };
+    if (tid < dv) put(tid, to_f32(g_raw), weight_raw);
+    for (int j = tid + RS_THREADS; j < dv; j += RS_THREADS) put(j, to_f32(g_src[j]), MEMORY || WKV ? weight[j] : 1.f);
 }
 
 template <int KIND, typename T, typename TO = T>
