@@ -435,6 +435,37 @@ def test_decoded_rows_whose_keys_are_shared_out(ops, sinks, window, keep, monkey
         _close(y, outs[0].cpu(), 1e-2, "against one workgroup")
 
 
+@pytest.mark.parametrize("sinks", [False, True])
+@pytest.mark.parametrize("heads, kv_heads, key, value, page, window", [(16, 1, 576, 512, 16, None), (1, 1, 16, 16, 16, 1), (5, 1, 96, 64, 32, 33),
+                                                                       (6, 2, 272, 256, 16, 50), (32, 2, 640, 512, 64, 64), (3, 3, 256, 240, 16, 31)])
+def test_decoded_rows_over_a_latent_vector_of_few_heads(ops, heads, kv_heads, key, value, page, window, sinks, monkeypatch):
+    """The four waves share out a key's elements and a value's: sizes with remainders of 32 and of 64, whole and partial rounds of 32
+    keys, empty runs of keys, and pages that are not there."""
+    from tiny_llm_infer_amd.parts.base import GroupView
+    g = torch.Generator().manual_seed(heads + key)
+    lengths = [1, 32, 33, 200, 333]
+    need = [-(-n // page) for n in lengths]
+    ids, width, at = torch.randperm(sum(need), generator=g).to(torch.int32), max(need), 0
+    tables = torch.full((len(lengths), width), -1, dtype=torch.int32)
+    for i, n in enumerate(need):
+        tables[i, :n] = ids[at:at + n]
+        at += n
+    kc = torch.randn(sum(need), kv_heads, page, key, generator=g).to(torch.bfloat16).cuda()
+    q = torch.randn(len(lengths), heads, key, generator=g).to(torch.bfloat16).cuda()
+    group = GroupView(tensors={}, tables=tables.cuda(), table_width=width, page_size=page, window=window)
+    step = _view([n - 1 for n in lengths], [1] * len(lengths), range(len(lengths)))
+    extra = torch.randn(heads, generator=g).cuda() if sinks else None
+    outs = []
+    for splits in (1, 2, 5, 64, None):
+        monkeypatch.setattr(ops, "sized_splits", splits)
+        outs.append(ops.sized_attention(q, step, group, kc, None, heads, kv_heads, 1, key, value, key ** -0.5, window, 0, torch.bfloat16, sinks=extra))
+    monkeypatch.setattr(ops, "force_plain", True)
+    plain = ops.sized_attention(q, step, group, kc, None, heads, kv_heads, 1, key, value, key ** -0.5, window, 0, torch.bfloat16, sinks=extra)
+    for y in outs:
+        _close(y, plain.cpu(), 2e-2, "against the plain kernel")
+        _close(y, outs[0].cpu(), 1e-2, "against one workgroup")
+
+
 # ------------------------------------------------------- one mixer alone, every cut ---
 MIXERS = {
     "latent 4 x 16+8 -> 24": (L, _latent(4, 16, 8, 24, 32, 48, 20)),

@@ -1,10 +1,11 @@
 // Attention over the paged cache for heads whose keys and values have sizes of their own: the matrix-core kernels
 // for bfloat16, key and value sizes in sixteens.  What they compute is what attention_sized_plain.hip computes
 // (maps of a head, values from a cache of their own or the first elements of the keys, a window with kept first
-// keys).  Two kernels:
+// keys).  Three kernels:
 //
 // attention_sized_shared_kernel (further down): portions of prompts, and single rows whose values are their keys'
 //   first elements (all heads read the one latent vector): four waves with 16 columns each share every tile of keys.
+// attention_latent_step_kernel (between them): those single rows where up to 16 heads read the vector.
 // attention_sized_mfma_kernel (first): single decoded rows whose values have a cache of their own.  A workgroup of
 //   four waves takes one row and one (key head, map); its 16 columns are query heads that read that key head.  The keys
 //   the row can see (from the first one it sees to itself, and the kept first ones before them) are walked 16 at a
@@ -381,6 +382,171 @@ __global__ __launch_bounds__(256) void attention_parts_merge_kernel(
         }
         if (d < DV) asm_store4(out + (size_t)row * out_ld + (size_t)head * DV + d, a, inv);
     }
+}
+
+// ---- single rows over a latent vector that up to 16 heads read -----------------------------------------------------
+//
+// A workgroup takes one row, one key head and a run of its keys (gridDim.z runs; their sums go to `parts`); its 16 columns are the
+// key head's query heads.  What bounds such a row is the chain from its position over its block table to its keys and the
+// arithmetic of one tile behind the other, so the four waves share out the arithmetic of every 32 keys: each makes the scores of
+// every fourth 32 elements of a key, the scores' parts meet in LDS, and each multiplies the weights with every fourth 16 value
+// elements.  v_mfma_f32_16x16x32_bf16; the values are read out of the key tile.
+// 8 rows, 16 heads, 512 + 64 elements, 500 keys in 16 runs, as part of a decode step: attention_sized_shared_kernel, where one wave
+// of the four had columns, 15.5 us, this 8.7.
+#define ALS_KEYS 32
+#define ALS_PAD 8
+
+typedef __attribute__((ext_vector_type(8))) __bf16 als_bf16x8;
+union SFrag8 {
+    uint4 u;
+    uint2 h[2];
+    bf16_t e[8];
+    als_bf16x8 v;
+};
+
+static inline int als_row_elems(int key_dim) { return (key_dim + 31) / 32 * 32 + ALS_PAD; }
+static inline size_t als_lds_bytes(int key_dim) {
+    return (size_t)ALS_KEYS * als_row_elems(key_dim) * 2 + (size_t)ASM_WAVES * 2 * 64 * 16;
+}
+
+// NK: 32s of a key a wave takes (a key: up to 128 NK elements); NV: 16s of a value (up to 64 NV).
+template <int NK, int NV>
+__global__ __launch_bounds__(64 * ASM_WAVES) void attention_latent_step_kernel(
+    const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ k_cache, const int* __restrict__ seq_start,
+    const int* __restrict__ tables, int table_width, int page_size, int num_pages, int heads, int kv_heads, int DK, int DV, float scale,
+    int window, const float* __restrict__ sinks, float* __restrict__ parts) {
+    extern __shared__ __align__(16) unsigned char als_lds[];
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int col = lane % 16, grp = lane / 16;
+    const int row = blockIdx.x, kh = blockIdx.y;                        // (a sequence brings one row: row r is sequence r's)
+    const int per_kv = heads / kv_heads, head = kh * per_kv + min(col, per_kv - 1);      // (idle columns repeat the last; never stored)
+    const int hi = seq_start[row], lo = window > 0 ? max(0, hi - window + 1) : 0;
+    const int LD = (DK + 31) / 32 * 32 + ALS_PAD, k32 = (DK + 31) / 32, nv = DV / 16, pieces = DK / 8;
+    bf16_t* kt = reinterpret_cast<bf16_t*>(als_lds);                    // [32][LD]: the keys
+    f32x4* part_s = reinterpret_cast<f32x4*>(kt + (size_t)ALS_KEYS * LD);       // [wave][2][64]: parts of the scores
+    const int rounds = (hi - lo) / ALS_KEYS + 1, each = (rounds + (int)gridDim.z - 1) / (int)gridDim.z;
+    const int first = min((int)blockIdx.z * each, rounds), last = min(first + each, rounds);
+    // a thread brings pieces of 16 bytes of one key: 8 neighbours take 128 bytes in a row
+    constexpr int PASSES = (NK * 128 + 63) / 64;
+    const int kk = tid / 8, p0 = tid % 8;
+    uint4 next[PASSES];
+    const int page_shift = __builtin_ctz(page_size), page_mask = page_size - 1;
+    const size_t k_page = (size_t)kv_heads * page_size * DK;
+    auto fetch = [&](int i) {
+        const int key = lo + i * ALS_KEYS + kk;
+        const int page = key <= hi ? tables[(size_t)row * table_width + (key >> page_shift)] : -1;
+        const bool there = page >= 0 && page < num_pages;
+        const bf16_t* src = k_cache + (size_t)(there ? page : 0) * k_page + ((size_t)kh * page_size + (key & page_mask)) * DK;
+#pragma unroll
+        for (int ps = 0; ps < PASSES; ++ps) {
+            const int p = ps * 8 + p0;
+            next[ps] = make_uint4(0, 0, 0, 0);
+            if (there && p < pieces) next[ps] = *reinterpret_cast<const uint4*>(src + p * 8);
+        }
+    };
+    if (first < last) fetch(first);
+    SFrag8 qf[NK];
+    f32x4 acc[NV];
+    {
+        const bf16_t* q_row = q + ((size_t)row * heads + head) * DK;
+#pragma unroll
+        for (int j = 0; j < NK; ++j) {
+            const int at = (j * ASM_WAVES + wave) * 32 + grp * 8;
+            qf[j].u = make_uint4(0, 0, 0, 0);
+            if (at < DK) qf[j].u = *reinterpret_cast<const uint4*>(q_row + at);          // (DK in eights and more: all 8 or none)
+        }
+#pragma unroll
+        for (int j = 0; j < NV; ++j) acc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    float m = -INFINITY, l = 0.f;
+    for (int it = first; it < last; ++it) {
+        if (it > first) __syncthreads();                                // everyone has read the keys before
+#pragma unroll
+        for (int ps = 0; ps < PASSES; ++ps) {
+            const int p = ps * 8 + p0;
+            if (p < k32 * 4) *reinterpret_cast<uint4*>(kt + (size_t)kk * LD + p * 8) = next[ps];     // (past the key's end zeros)
+        }
+        __syncthreads();
+        if (it + 1 < last) fetch(it + 1);
+        f32x4 s[2] = {(f32x4){0.f, 0.f, 0.f, 0.f}, (f32x4){0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int j = 0; j < NK; ++j) {
+            const int c32 = j * ASM_WAVES + wave;
+            if (c32 < k32) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    SFrag8 a;
+                    a.u = *reinterpret_cast<const uint4*>(kt + (size_t)(t * 16 + col) * LD + c32 * 32 + grp * 8);
+                    s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, qf[j].v, s[t], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) part_s[(wave * 2 + t) * 64 + lane] = s[t];
+        __syncthreads();
+        // this lane: keys k0 + 16 t + 4 grp + i of column col; every wave the same
+        const int k0 = lo + it * ALS_KEYS;
+        float w[8], mx = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            f32x4 sum = part_s[t * 64 + lane];
+#pragma unroll
+            for (int o = 1; o < ASM_WAVES; ++o) {
+                const f32x4 other = part_s[(o * 2 + t) * 64 + lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sum[i] += other[i];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                w[4 * t + i] = k0 + 16 * t + grp * 4 + i <= hi ? sum[i] * scale : -INFINITY;
+                mx = fmaxf(mx, w[4 * t + i]);
+            }
+        }
+        const float m_new = fmaxf(m, quad_rows_max(mx));
+        const float corr = (m_new == -INFINITY) ? 0.f : __expf(m - m_new);
+        SFrag8 p;
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float e = (w[i] == -INFINITY) ? 0.f : __expf(w[i] - m_new);
+            p.e[i] = f32_to_bf16(e);
+            sum += bf16_to_f32(p.e[i]);                                 // the weights as the values meet them
+        }
+        l = l * corr + quad_rows_sum(sum);
+        m = m_new;
+        const bool rescale = __any(corr != 1.0f);                       // (the same for the whole wave)
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int c16 = j * ASM_WAVES + wave;
+            if (c16 < nv) {
+                SFrag8 a;                                               // element 16 c16 + col of the keys 16 t + 4 grp + i
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) a.e[4 * t + i] = kt[(size_t)(t * 16 + grp * 4 + i) * LD + c16 * 16 + col];
+                if (rescale) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[j][i] *= corr;
+                }
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, p.v, acc[j], 0, 0, 0);
+            }
+        }
+    }
+    if (col >= per_kv) return;
+    if (parts) {                                                        // the sums as they are, with m and l behind them
+        float* part = parts + (((size_t)row * heads + head) * gridDim.z + blockIdx.z) * (DV + 4);
+        if (wave == 0 && grp == 0) part[DV] = m, part[DV + 1] = l;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            if (j * ASM_WAVES + wave < nv) asm_store4(part + (j * ASM_WAVES + wave) * 16 + grp * 4, acc[j], 1.0f);
+        return;
+    }
+    float inv = l > 0.f ? 1.0f / l : 0.f;
+    if (sinks) inv = asm_sink_factor(sinks[head], m, l);
+    bf16_t* o_row = out + ((size_t)row * heads + head) * DV;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+        if (j * ASM_WAVES + wave < nv) asm_store4(o_row + (j * ASM_WAVES + wave) * 16 + grp * 4, acc[j], inv);
 }
 
 // ---- steps with portions of prompts: four waves share every tile of keys ----------------------------------------
@@ -826,4 +992,37 @@ extern "C" int tli_attention_pooled_mfma_bf16(
     attention_parts_merge_kernel<<<dim3((pairs + 3) / 4, (value_dim + 255) / 256), 256, 0, (hipStream_t)stream>>>(parts, splits, pairs, heads, value_dim, sinks,
                                                                                    (bf16_t*)out, out_ld, out_scale);
     return tli_check_launch("attention_parts_merge");
+}
+
+// A step of one row a sequence (row r is sequence r's, at seq_start[r]) whose values are the first value_dim elements of the keys, read
+// by up to 16 heads a key head: q [rows, heads, key_dim], out [rows, heads, value_dim], k_cache [pages][kv_heads][slot][key_dim].
+// splits, parts: as for tli_attention_sized_mfma_bf16.
+extern "C" int tli_attention_latent_step_bf16(const void* q, void* out, const void* k_cache, const int* seq_start, int rows, const int* tables,
+                                              int table_width, int page_size, int num_pages, int heads, int kv_heads, int key_dim,
+                                              int value_dim, float scale, int window, const float* sinks, int splits, float* parts,
+                                              void* stream) {
+    if (rows <= 0) return 0;
+    if (!tli_attention_sized_mfma_takes(key_dim, value_dim, page_size, 0))
+        return tli_fail("attention_latent_step: keys of %d and values of %d in pages of %d", key_dim, value_dim, page_size);
+    if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || heads / kv_heads > 16 || kv_heads > 65535)
+        return tli_fail("attention_latent_step: %d heads over %d key heads (at most 16 each)", heads, kv_heads);
+    if (table_width <= 0 || num_pages <= 0 || window < 0) return tli_fail("attention_latent_step: bad cache geometry");
+    if (((uintptr_t)q | (uintptr_t)out | (uintptr_t)k_cache) & 15) return tli_fail("attention_latent_step: operands must be 16-byte aligned");
+    if (splits < 1 || splits > 64 || (splits > 1 && (!parts || ((uintptr_t)parts & 15)))) return tli_fail("attention_latent_step: %d splits", splits);
+    hipStream_t s = (hipStream_t)stream;
+    const dim3 grid(rows, kv_heads, splits);
+#define ALS_RUN(NK, NV)                                                                                                               \
+    attention_latent_step_kernel<NK, NV><<<grid, 64 * ASM_WAVES, als_lds_bytes(key_dim), s>>>(                                        \
+        (const bf16_t*)q, (bf16_t*)out, (const bf16_t*)k_cache, seq_start, tables, table_width, page_size, num_pages, heads, kv_heads, \
+        key_dim, value_dim, scale, window, sinks, splits > 1 ? parts : nullptr)
+    // (at most 49 KiB of LDS)
+    if (key_dim <= 256 && value_dim <= 256) ALS_RUN(2, 4);
+    else ALS_RUN(5, 8);
+#undef ALS_RUN
+    if (splits > 1) {
+        const int pairs = rows * heads;
+        attention_parts_merge_kernel<<<dim3((pairs + 3) / 4, (value_dim + 255) / 256), 256, 0, s>>>(parts, splits, pairs, heads, value_dim, sinks,
+                                                                                                   (bf16_t*)out, heads * value_dim, 1.0f);
+    }
+    return tli_check_launch("attention_latent_step");
 }

@@ -130,6 +130,7 @@ def load_library():
         "tli_head_products_mfma_bf16": [P, ctypes.c_longlong, ctypes.c_longlong, P, P, ctypes.c_longlong, ctypes.c_longlong,
                                         I, I, I, I, P, I, P],
         "tli_attention_sized_mfma_bf16": [P, P, P, P, P, P, I, I, P, I, I, I, I, I, I, I, I, F, I, I, I, I, P, I, P, P],
+        "tli_attention_latent_step_bf16": [P, P, P, P, I, P, I, I, I, I, I, I, I, F, I, P, I, P, P],
         "tli_diff_prepare": [P, I, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P, P, F, I, P],
         "tli_diff_combine": [P, P, I, I, P, I, I, I, F, F, F, I, P],
         "tli_latent_prepare": [P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, I, I, P, F, P, P, I, P],
@@ -1827,6 +1828,11 @@ class HipOps:
                 splits = self._sized_splits(T, step.reach, heads * maps, kv_heads * maps, window, keep)
                 if splits > 1:
                     parts = torch.empty((T * heads * maps * splits * (value_dim + 4),), dtype=torch.float32, device=self.device)
+                if maps == 1 and heads // kv_heads <= 16 and not keep:      # (one wave of the general kernel's four would have heads)
+                    self._call(self.lib.tli_attention_latent_step_bf16, q.data_ptr(), out.data_ptr(), kc.data_ptr(), step.seq_start.data_ptr(),
+                               T, g.tables.data_ptr(), g.table_width, g.page_size, pages, heads, kv_heads, key_dim, value_dim, float(scale),
+                               int(window or 0), _ptr(sinks), splits, _ptr(parts), self._stream())
+                    return out
             self._call(self.lib.tli_attention_sized_mfma_bf16, q.data_ptr(), out.data_ptr(), kc.data_ptr(), _ptr(vc),
                        step.row_start.data_ptr(), step.seq_start.data_ptr(), step.num_seqs, tiles, g.tables.data_ptr(),
                        g.table_width, g.page_size, pages, heads, kv_heads, maps, key_dim, value_dim, float(scale),
