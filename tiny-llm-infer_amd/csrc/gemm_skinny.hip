@@ -597,3 +597,43 @@ extern "C" int tli_gemm_skinny_fused_bf16(const void* x, const void* w, void* y,
         default: return tli_fail("gemm_skinny: unknown configuration %d", cfg);
     }
 }
+
+// The same with float32 outputs (the logits of a step): y = (x . W^T) / sqrt(sum(ssq_in[parts_in][M]) / K + eps).  The launch shape is
+// that of tli_gemm_skinny_bf16 with float32 outputs.  A decode step then has no pass for its last norm (8 rows of 4,096: 4.7 us).
+template <int RT, int WAVES>
+static int launch_skinny_normed_f32(const bf16_t* x, const bf16_t* w, float* y, int M, int N, int K, const SkinnyFuse& f, hipStream_t s,
+                                    bool half = false) {
+    const int blocks = (N + 16 * RT - 1) / (16 * RT);
+    const bool lds = through_lds(M, K, RT == 2, half, true);
+#define SKINNY_NORMED_F32(XR) \
+    gemm_skinny_kernel<RT, 1, WAVES, float, true, false, 2, FUSE_RSTD, XR><<<blocks, WAVES * 64, 0, s>>>(x, w, y, M, N, K, f)
+#define SKINNY_NORMED_F32_HALF(XR) \
+    gemm_skinny_kernel<1, 1, WAVES, float, true, false, 2, FUSE_RSTD, XR, false, true><<<(N + 7) / 8, WAVES * 64, 0, s>>>(x, w, y, M, N, K, f)
+    if constexpr (RT == 1) {
+        if (half) {
+            SKINNY_ROWS(M, lds, SKINNY_NORMED_F32_HALF)
+            return tli_check_launch("gemm_skinny (norm taken in, float32)");
+        }
+    }
+    SKINNY_ROWS_16(lds, SKINNY_NORMED_F32)
+    return tli_check_launch("gemm_skinny (norm taken in, float32)");
+}
+
+extern "C" int tli_gemm_skinny_normed_f32(const void* x, const void* w, void* y, int M, int N, int K, const float* ssq_in, int parts_in,
+                                          float eps, void* stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (M > 16) return tli_fail("gemm_skinny with a norm: %d rows, at most 16", M);
+    if (K <= 0 || K % 8) return tli_fail("gemm_skinny: K = %d must be a positive multiple of 8", K);
+    if (!ssq_in || parts_in <= 0 || !y) return tli_fail("gemm_skinny with sums of squares: missing arguments");
+    if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) return tli_fail("gemm_skinny: operands must be 16-byte aligned");
+    SkinnyFuse f{};
+    f.ssq_in = ssq_in, f.parts_in = parts_in, f.eps = eps;
+    const bf16_t *xp = (const bf16_t*)x, *wp = (const bf16_t*)w;
+    hipStream_t s = (hipStream_t)stream;
+    switch (fused_shape(M, N, K, 0, false, 0)) {
+        case 8: return launch_skinny_normed_f32<1, 8>(xp, wp, (float*)y, M, N, K, f, s, true);
+        case 18: return launch_skinny_normed_f32<1, 8>(xp, wp, (float*)y, M, N, K, f, s);
+        case 28: return launch_skinny_normed_f32<2, 8>(xp, wp, (float*)y, M, N, K, f, s);
+        default: return launch_skinny_normed_f32<2, 4>(xp, wp, (float*)y, M, N, K, f, s);
+    }
+}

@@ -8,7 +8,7 @@ import torch
 
 from ..cache.manager import CacheNeed, StateNeed
 from ..config.base import ConfigError, ModelSpec, PartSpec
-from ..parts.base import BuildEnv, build_part
+from ..parts.base import Block, BuildEnv, build_part, run_norm
 from ..weights.loader import TensorDecl, load_tensors, random_tensors, unique_decls
 
 
@@ -86,11 +86,23 @@ class Model:
         """The residual as the blocks keep it, from the embedding's rows."""
         return self.blocks[self.schedule[0].block].open(x) if self.schedule else x
 
-    def close_residual(self, resid, pending, rows=None, num_rows=None):
+    def embed(self, token_ids, num_rows: int, positions):
+        """The residual as the blocks keep it, from the tokens; and what the first block is given besides: its opening norm's rows,
+        where the embedding makes them in the same pass."""
+        first = self.blocks[self.schedule[0].block] if self.schedule else None
+        norm, normed = getattr(first, "opening_norm", None), getattr(self.embedding, "forward_normed", None)
+        if norm is not None and normed is not None and type(first).open is Block.open:
+            both = normed(token_ids, num_rows, norm)
+            if both is not None:
+                return both[0], {"normed": both[1]}
+        return self.open_residual(self.embedding.forward(token_ids, num_rows, positions)), {}
+
+    def close_residual(self, resid, pending, rows=None, num_rows=None, all_rows=False):
         """The final norm's rows (of ``rows`` only, if given) from the residual and what the last
-        block still owes it."""
+        block still owes it.  ``all_rows``: ``rows`` are all of the residual's, in their order, and the norm's rows go to the head."""
+        if all_rows and (not self.schedule or type(self.blocks[self.schedule[-1].block]).close is Block.close):
+            return run_norm(self.final_norm, resid, pending, consumer=self.head)
         if not self.schedule:
-            from ..parts.base import run_norm
             return run_norm(self.final_norm, resid, pending, rows=rows, num_rows=num_rows)
         return self.blocks[self.schedule[-1].block].close(resid, pending, self.final_norm, rows, num_rows)
 

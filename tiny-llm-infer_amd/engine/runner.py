@@ -277,7 +277,7 @@ class ModelRunner:
             slots=dev[lay["slots"]], sample_rows=dev[lay["sample_rows"]],
             h_row_start=row_start, h_seq_start=starts, h_seq_len=totals,
             h_slots=slots, max_rows_per_seq=max(counts),
-            max_seq_len=max(totals), reach=max(128, 1 << (max(totals) - 1).bit_length()),
+            all_wanted=sample == list(range(rows)), max_seq_len=max(totals), reach=max(128, 1 << (max(totals) - 1).bit_length()),
             skew=min(16, 1 << ((max(totals) * len(totals)) // max(sum(totals), 1)).bit_length() - 1),
             groups=groups)
 
@@ -295,7 +295,7 @@ class ModelRunner:
 
     def _forward(self, step: StepView, num_wanted: int) -> Optional[torch.Tensor]:
         model = self.model
-        resid = model.open_residual(model.embedding.forward(step.token_ids, step.num_rows, step.positions))
+        resid, opening = model.embed(step.token_ids, step.num_rows, step.positions)
         pending = None
         for i, call in enumerate(model.schedule):
             if call.cache >= 0 and call.cache in self.cache.group_of_layer:
@@ -306,12 +306,13 @@ class ModelRunner:
             else:
                 step.cache = None
             step.state = self.states[i]
-            pending = model.blocks[call.block].forward(resid, pending, step)
+            pending = model.blocks[call.block].forward(resid, pending, step, **opening)
+            opening = {}
         step.cache = None
         step.state = None
         if num_wanted == 0:
             return None
-        x = model.close_residual(resid, pending, rows=step.sample_rows, num_rows=num_wanted)
+        x = model.close_residual(resid, pending, rows=step.sample_rows, num_rows=num_wanted, all_rows=step.all_wanted)
         return model.head.forward(x)
 
     def _replay(self, view: StepView, wanted: int) -> torch.Tensor:

@@ -89,6 +89,8 @@ def load_library():
         "tli_gemm_f32": [P, P, P, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_fused_bf16": [P, P, P, I, I, I, I, P, I, F, P, P, P, P, I, I, F, I, P],
+        "tli_gemm_skinny_normed_f32": [P, P, P, I, I, I, P, I, F, P],
+        "tli_embed_rmsnorm": [P, P, P, P, P, I, I, I, F, I, P],
         "tli_gemm_mid_bf16": [P, P, P, P, I, I, I, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_parts": [I, I, I],
         "tli_gemm_mid_splits": [I, I, I],
@@ -368,6 +370,22 @@ class HipOps:
                    num_rows, hidden, vocab, _dtype_code(table.dtype), self._stream())
         return out
 
+    def embed_rmsnorm(self, table, token_ids, num_rows: int, weight, eps):
+        """(``embed`` of the tokens, ``add_rmsnorm`` of those rows with nothing owed) in one pass; None for what it does not take."""
+        vocab, hidden = table.shape
+        if hidden % 4 or hidden > 16384 or self.separate_norms or not self._aligned(table, weight):
+            return None
+        self._want(table, "embedding table")
+        self._want(token_ids, "token ids", torch.int32)
+        self._want(weight, "norm weight", torch.float32, (hidden,))
+        if token_ids.numel() < num_rows:
+            raise KernelError("fewer token ids than rows")
+        resid = torch.empty((num_rows, hidden), dtype=torch.float32, device=self.device)
+        out = torch.empty((num_rows, hidden), dtype=table.dtype, device=self.device)
+        self._call(self.lib.tli_embed_rmsnorm, table.data_ptr(), token_ids.data_ptr(), resid.data_ptr(), weight.data_ptr(), out.data_ptr(),
+                   num_rows, hidden, vocab, float(eps), _dtype_code(table.dtype), self._stream())
+        return resid, out
+
     def resolve(self, y):
         """The tensor of a product that ``linear(..., deferred=True)`` left unfinished."""
         if isinstance(y, PendingProduct):
@@ -538,11 +556,16 @@ class HipOps:
         M, K = x.xw.shape
         if tiled is None:
             raise KernelError("normed rows that still owe their factor need a matrix in the decode layout")
-        if out_dtype not in (None, torch.bfloat16):
-            raise KernelError("normed rows that still owe their factor give bfloat16 products")
         rows_out = _shape_of(m)[0]
         if _shape_of(m)[1] != K:
             raise KernelError(f"linear: input has {K} columns, the matrix {_shape_of(m)[1]}")
+        if out_dtype == torch.float32 and not gated:
+            y = torch.empty((M, rows_out), dtype=torch.float32, device=self.device)
+            self._call(self.lib.tli_gemm_skinny_normed_f32, x.xw.data_ptr(), tiled.data_ptr(), y.data_ptr(), M, rows_out, K, x.ssq.data_ptr(),
+                       x.ssq.shape[0], x.eps, self._stream())
+            return y
+        if out_dtype not in (None, torch.bfloat16):
+            raise KernelError("normed rows that still owe their factor give bfloat16 products, or float32 ones without a gate")
         N = 2 * m.inter if gated else rows_out
         y, y_at, ld = self._rows_into(into, M, m.inter if gated else N, torch.bfloat16)
         self._call(self.lib.tli_gemm_skinny_fused_bf16, x.xw.data_ptr(), tiled.data_ptr(), y_at, M, N, K,

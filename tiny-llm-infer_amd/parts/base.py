@@ -83,6 +83,7 @@ class StepView:
     max_seq_len: int = 1
     reach: int = 1                # max_seq_len rounded up to a power of two: launches are shaped by
                                   # this, so that steps of like shape launch alike (and can be replayed)
+    all_wanted: bool = False      # every row's logits are wanted, in the rows' order (sample_rows counts up)
     skew: int = 1                 # the longest sequence has at least this many times the tokens of the average
                                   # one (a power of two, at most 16): launches may split the long ones' work by it
     groups: List[GroupView] = field(default_factory=list)
@@ -211,6 +212,8 @@ class Block(Part):
     mixer: Mixer
     ffn: FeedForward
     streams = 1          # copies of the residual stream that the arrangement keeps side by side
+    opening_norm = None  # the norm that ``forward`` begins with, of an arrangement whose ``forward`` also takes its rows (``normed``)
+                         # instead of making them, where nothing is owed to the residual (``pending`` None)
 
     def forward(self, resid: torch.Tensor, pending: Optional[torch.Tensor],
                 step: StepView) -> torch.Tensor:

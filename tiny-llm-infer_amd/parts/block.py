@@ -19,7 +19,7 @@ class PreNormBlock(Block):
         super().__init__(spec)
         self.mixer = mixer
         self.ffn = ffn
-        self.norm_mixer = norms["mixer"]
+        self.norm_mixer = self.opening_norm = norms["mixer"]
         self.norm_ffn = norms["ffn"] if ffn is not None else None
         self.replayable = all(p.replayable for p in self._parts())
 
@@ -35,10 +35,10 @@ class PreNormBlock(Block):
             part.load(weights, env)
 
     def forward(self, resid: torch.Tensor, pending: Optional[torch.Tensor],
-                step: StepView) -> torch.Tensor:
+                step: StepView, normed=None) -> torch.Tensor:
         # (a part that gives its input to matrix products only lets the norm before it be
         # taken into those products, if the norm can do that)
-        n = run_norm(self.norm_mixer, resid, pending, consumer=self.mixer)
+        n = normed if normed is not None else run_norm(self.norm_mixer, resid, pending, consumer=self.mixer)
         a = self.mixer.forward(n, step)
         if self.ffn is None:
             return a

@@ -51,8 +51,20 @@ class TokenEmbedding(Part):
                                   positions=positions, pos_table=self.pos_table)
 
 
+    def forward_normed(self, token_ids: torch.Tensor, num_rows: int, norm):
+        """(the residual's rows, their ``norm``) where one pass makes both, else None."""
+        rms, both = norm.as_rms(), getattr(self.env.ops, "embed_rmsnorm", None)
+        if rms is None or both is None or self.pos_table is not None or self.scale != 1.0:
+            return None
+        return both(self.table, token_ids, num_rows, *rms)
+
+
 class LinearHead(Part):
     replayable = True
+
+    @property
+    def takes_normed_rows(self) -> bool:
+        return getattr(getattr(self, "weight", None), "tiled", None) is not None
 
     def __init__(self, spec):
         super().__init__(spec)

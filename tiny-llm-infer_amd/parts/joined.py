@@ -241,6 +241,7 @@ class OneNormParallelBlock(Block):
     def __init__(self, spec, mixer, ffn, norms):
         super().__init__(spec)
         self.mixer, self.ffn, self.norm = mixer, ffn, norms["mixer"]
+        self.opening_norm = self.norm
         self.mult = float(spec.params.get("residual_mult", 1.0))
         for part in self._sublayers():
             if not (hasattr(part, "load_rows") and hasattr(part, "rows")):
@@ -262,8 +263,8 @@ class OneNormParallelBlock(Block):
         self.joined = JoinedRows([p.rows_width for p in parts], [p.output_matrix(weights) for p in parts], env)
         self.takes_normed_rows = all(p.takes_normed_rows for p in parts)
 
-    def forward(self, resid: torch.Tensor, pending: Optional[torch.Tensor], step: StepView):
-        h = run_norm(self.norm, resid, pending, consumer=self)
+    def forward(self, resid: torch.Tensor, pending: Optional[torch.Tensor], step: StepView, normed=None):
+        h = normed if normed is not None else run_norm(self.norm, resid, pending, consumer=self)
         out = self.joined.buffer(step.num_rows)
         for part, at in zip(self._sublayers(), self.joined.at):
             part.rows(h, step, out, at, self.mult)
