@@ -26,6 +26,7 @@
 // (keys up to 128 / 256 / 640 elements, values up to 128 / 256 / 512).
 #include "common.h"
 #include "pooled.h"
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(4))) short bf16x4;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -153,31 +154,44 @@ __global__ __launch_bounds__(64 * ASM_WAVES) void attention_sized_mfma_kernel(
         return is_block(i) ? 16 * (i - n_tokens) : i < n_main ? k_top - 16 * i : 16 * (i - n_main);
     };
 
-    uint4 next[PASSES];
+    // DEPTH tiles' keys and values are on their way together (a wave of a row that is shared out has two or three tiles: they are one
+    // trip to memory, not one each), and a tile's page is looked up once, by a scalar load: a tile of 16 keys lies inside one page.
+    // 8 rows of 1,100 keys and blocks, heads of 128, 8 runs, as part of a decode step: 12.5 us, one tile ahead and its values not, and 10.4 now.
+    constexpr int DEPTH = NKM <= 8 && NVM <= 8 ? 2 : 1;
+    uint4 next[DEPTH][PASSES];
+    constexpr bool VALUES_TOO = !VKEY && DEPTH == 2;                    // (larger heads leave no registers for it)
+    SFrag4 next_v[VALUES_TOO ? DEPTH : 1][VALUES_TOO ? NVM : 1];
     // chunk c = 64 ps + lane is piece c % pieces of key c / pieces: one division a lane, then steps of 64 chunks
     const int key_first = lane / pieces, piece_first = lane - key_first * pieces;
     const int key_step = 64 / pieces, piece_step = 64 - key_step * pieces;
-    auto fetch = [&](int i) {
+    auto fetch_values = [&](int i, auto& v) {                           // from their own cache: dim 16 j + col of the keys k0 + 4 grp + i
+        const int k0 = tile_key(i), key = k0 + grp * 4;
+        const bool block = is_block(i);
+        const int page = (block ? block_table : table)[k0 >> page_shift];
+        const bool there = page >= 0 && page < (block ? pooled.pages : num_pages);
+        const bool some = there && (block ? key < blocks_hi : key <= hi && (key + 3 >= lo || key < kept_hi));
+        const bf16_t* vp = (block ? (const bf16_t*)pooled.v : v_cache) + (size_t)(there ? page : 0) * v_page + ((size_t)g * DV + col) * page_size + (key & page_mask);
+#pragma unroll
+        for (int j = 0; j < NVM; ++j) {
+            v[j].u = make_uint2(0, 0);
+            if (j < nv && some) v[j].u = *reinterpret_cast<const uint2*>(vp + (size_t)j * 16 * page_size);
+        }
+    };
+    auto fetch = [&](int i, auto STAGE) {
+        constexpr int ST = decltype(STAGE)::value;
         const int k0 = tile_key(i);
         const bool block = is_block(i);
-        const int* tab = block ? block_table : table;
-        const bf16_t* keys = block ? (const bf16_t*)pooled.k : k_cache;
-        const int all = block ? pooled.pages : num_pages;
+        const int page = (block ? block_table : table)[k0 >> page_shift];
+        const bool there = page >= 0 && page < (block ? pooled.pages : num_pages);
+        const bf16_t* keys = (block ? (const bf16_t*)pooled.k : k_cache) + (size_t)(there ? page : 0) * k_page + ((size_t)kh * page_size + (k0 & page_mask)) * DK;
         const int t_lo = block ? 0 : lo, t_hi = block ? blocks_hi - 1 : hi, t_kept = block ? 0 : kept_hi;
         int ck = key_first, cp = piece_first;
 #pragma unroll
         for (int ps = 0; ps < PASSES; ++ps) {
             const int c = ps * 64 + lane;
-            next[ps] = make_uint4(0, 0, 0, 0);
-            if (c < chunks) {
-                const int key = k0 + ck;
-                if (key <= t_hi && (key >= t_lo || key < t_kept)) {
-                    const int page = tab[key >> page_shift];
-                    if (page >= 0 && page < all)
-                        next[ps] = *reinterpret_cast<const uint4*>(keys + (size_t)page * k_page +
-                                                                   ((size_t)kh * page_size + (key & page_mask)) * DK + cp * 8);
-                }
-            }
+            next[ST][ps] = make_uint4(0, 0, 0, 0);
+            const int key = k0 + ck;
+            if (c < chunks && there && key <= t_hi && (key >= t_lo || key < t_kept)) next[ST][ps] = *reinterpret_cast<const uint4*>(keys + (size_t)ck * DK + cp * 8);
             ck += key_step;
             cp += piece_step;
             if (cp >= pieces) {
@@ -185,19 +199,20 @@ __global__ __launch_bounds__(64 * ASM_WAVES) void attention_sized_mfma_kernel(
                 ++ck;
             }
         }
+        if constexpr (VALUES_TOO) fetch_values(i, next_v[ST]);
     };
     // with splits (gridDim.z of them) the waves of all the workgroups of one (row, key head) take turns at its tiles
     const int stride = POOLED ? ASM_WAVES * (int)gridDim.z : ASM_WAVES;
     const int first = POOLED ? ASM_WAVES * (int)blockIdx.z + wave : wave;
-    if (first < n_tiles) fetch(first);
-    for (int it = first; it < n_tiles; it += stride) {
+    auto tile_of_keys = [&](int it, auto STAGE) {
+        constexpr int ST = decltype(STAGE)::value;
         const int k0 = tile_key(it);
         {
             int ck = key_first, cp = piece_first;
 #pragma unroll
             for (int ps = 0; ps < PASSES; ++ps) {
                 const int c = ps * 64 + lane;
-                if (c < chunks) *reinterpret_cast<uint4*>(kt + ck * LD + cp * 8) = next[ps];
+                if (c < chunks) *reinterpret_cast<uint4*>(kt + ck * LD + cp * 8) = next[ST][ps];
                 ck += key_step;
                 cp += piece_step;
                 if (cp >= pieces) {
@@ -206,24 +221,14 @@ __global__ __launch_bounds__(64 * ASM_WAVES) void attention_sized_mfma_kernel(
                 }
             }
         }
-        if (it + stride < n_tiles) fetch(it + stride);
-        const bool block = is_block(it);
-        // the values of this tile's keys from their own cache: dim 16 j + col of the keys k0 + 4 grp + i
         SFrag4 vf[VKEY ? 1 : NVM];
-        if (!VKEY) {
-            const int key = k0 + grp * 4;
-            const bf16_t* vp = nullptr;
-            if (block ? key < blocks_hi : key <= hi && (key + 3 >= lo || key < kept_hi)) {
-                const int page = (block ? block_table : table)[key >> page_shift];
-                if (page >= 0 && page < (block ? pooled.pages : num_pages))
-                    vp = (block ? (const bf16_t*)pooled.v : v_cache) + (size_t)page * v_page + ((size_t)g * DV + col) * page_size + (key & page_mask);
-            }
+        if constexpr (VALUES_TOO) {
 #pragma unroll
-            for (int j = 0; j < NVM; ++j) {
-                vf[j].u = make_uint2(0, 0);
-                if (j < nv && vp) vf[j].u = *reinterpret_cast<const uint2*>(vp + (size_t)j * 16 * page_size);
-            }
+            for (int j = 0; j < NVM; ++j) vf[j] = next_v[ST][j];
         }
+        if (it + DEPTH * stride < n_tiles) fetch(it + DEPTH * stride, STAGE);
+        if constexpr (!VKEY && !VALUES_TOO) fetch_values(it, vf);
+        const bool block = is_block(it);
         wave_lds_sync();
         // scores: A = the key k0 + col, this lane group's dims
         // (two sums in turn, so that a matrix instruction does not wait for the one before it)
@@ -285,6 +290,16 @@ __global__ __launch_bounds__(64 * ASM_WAVES) void attention_sized_mfma_kernel(
             }
         }
         wave_lds_sync();                                // the tile is read before the next one is written over it
+    };
+    if (first < n_tiles) fetch(first, std::integral_constant<int, 0>{});
+    if constexpr (DEPTH == 2) {
+        if (first + stride < n_tiles) fetch(first + stride, std::integral_constant<int, 1>{});
+    }
+    for (int it = first; it < n_tiles; it += DEPTH * stride) {
+        tile_of_keys(it, std::integral_constant<int, 0>{});
+        if constexpr (DEPTH == 2) {
+            if (it + stride < n_tiles) tile_of_keys(it + stride, std::integral_constant<int, 1>{});
+        }
     }
     // the four waves' sums into wave 0: each of the others leaves (m, l) a column and its accumulators
     __syncthreads();
