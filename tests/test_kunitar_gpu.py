@@ -466,6 +466,35 @@ def test_decoded_rows_over_a_latent_vector_of_few_heads(ops, heads, kv_heads, ke
         _close(y, outs[0].cpu(), 1e-2, "against one workgroup")
 
 
+@pytest.mark.parametrize("rows", [1, 5, 64])
+@pytest.mark.parametrize("heads, dim, rot, rank", [(16, 128, 64, 512), (3, 64, 32, 96), (2, 256, 16, 16), (5, 48, 16, 112), (1, 272, 32, 64)])
+def test_what_stands_before_the_latent_attention_in_one_launch(ops, rows, heads, dim, rot, rank, monkeypatch):
+    """The queries' products, their turned parts and the cache's entries, with latent vectors of the layer's own and without: the same
+    bits as in two launches (more rows than workgroups that prepare, outputs in one share and in many)."""
+    from tiny_llm_infer_amd.parts.base import GroupView, LayerCache
+    g = torch.Generator().manual_seed(rows + dim)
+    page, key, vdim = 16, rank + rot, 16
+    rnd = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).cuda()
+    query, proj, w_qk, w_v = rnd(rows, heads * (dim + rot) + 8), rnd(rows, key + 4), rnd(heads, rank, dim), rnd(heads, vdim, rank)
+    cos, sin = (torch.randn(4, rot // 2, generator=g).cuda() for _ in range(2))
+    norm = torch.rand(rank, generator=g).cuda()
+    step = _view([i % 3 for i in range(rows)], [1] * rows, range(rows))
+    tables = torch.arange(rows, dtype=torch.int32).cuda()[:, None].contiguous()
+    if rows > 4:
+        tables[4] = -1                                   # a page that is not there
+    got = []
+    for together in (64, 0):
+        monkeypatch.setattr(ops, "LATENT_TOGETHER_ROWS", together)
+        for own in ((proj, 4, norm, 1e-6), None):
+            kc = torch.arange(rows * page * key).view(1, rows, page, key).remainder(97).div(50).to(torch.bfloat16).cuda()
+            group = GroupView(tensors={"latent": kc}, tables=tables, table_width=1, page_size=page, window=None)
+            out = ops.latent_attention(query, 8, own, step, LayerCache(group, 0, own is not None), heads, dim, rot, rank, vdim,
+                                       (cos, sin, rot), key ** -0.5, w_qk, w_v)
+            got.append((out, kc))
+    for a, b in zip(got[:2], got[2:]):
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
 # ------------------------------------------------------- one mixer alone, every cut ---
 MIXERS = {
     "latent 4 x 16+8 -> 24": (L, _latent(4, 16, 8, 24, 32, 48, 20)),

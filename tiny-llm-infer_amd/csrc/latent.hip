@@ -23,42 +23,50 @@ struct HeadGate {
 };
 
 template <typename T>
-__global__ __launch_bounds__(LP_THREADS) void latent_prepare_kernel(
-    const T* __restrict__ q_in, int q_ld, const T* __restrict__ down_in, int down_ld, T* __restrict__ q_out, T* __restrict__ cache, const int* __restrict__ positions,
-    const int* __restrict__ seq_of_row, const int* __restrict__ tables, int table_width, int page_size, int num_pages,
-    int heads, int dim, int rot, int rank, int rot_dims, const float* __restrict__ norm_weight, float eps,
-    const float* __restrict__ cos_t, const float* __restrict__ sin_t) {
-    __shared__ float red[16];
-    const int row = blockIdx.x, tid = threadIdx.x;
-    const T* src = q_in + (size_t)row * q_ld;
-    const int pos = positions[row];
-    const int half = rot_dims / 2;
-    const float* cs = cos_t + (size_t)pos * half;
-    const float* sn = sin_t + (size_t)pos * half;
+struct LatentRows {
+    const T* q_in;
+    int q_ld;
+    const T* down_in;
+    int down_ld;
+    T *q_out, *cache;
+    const int *positions, *seq_of_row, *tables;
+    int table_width, page_size, num_pages, heads, dim, rot, rank, rot_dims;
+    const float* norm_weight;
+    float eps;
+    const float *cos_t, *sin_t;
+};
+
+template <typename T>
+__device__ __forceinline__ void latent_prepare_row(const LatentRows<T>& a, int row, float* red) {
+    const int tid = threadIdx.x, half = a.rot_dims / 2, rot_dims = a.rot_dims, rot = a.rot, rank = a.rank, dim = a.dim;
+    const T* src = a.q_in + (size_t)row * a.q_ld;
+    const int pos = a.positions[row];
+    const float* cs = a.cos_t + (size_t)pos * half;
+    const float* sn = a.sin_t + (size_t)pos * half;
     const int key = rank + rot;
     // the queries' turned parts
-    for (int i = tid; i < heads * rot; i += LP_THREADS) {
+    for (int i = tid; i < a.heads * rot; i += LP_THREADS) {
         const int h = i / rot, d = i % rot;
         const T* part = src + (size_t)h * (dim + rot) + dim;
         float v = to_f32(part[d]);
         if (d < half) v = rotate_first_half(v, to_f32(part[d + half]), cs[d], sn[d]);
         else if (d < rot_dims) v = rotate_second_half(v, to_f32(part[d - half]), cs[d - half], sn[d - half]);
-        from_f32(q_out + ((size_t)row * heads + h) * key + rank + d, v);
+        from_f32(a.q_out + ((size_t)row * a.heads + h) * key + rank + d, v);
     }
-    if (!down_in) return;
-    const int page = tables[(size_t)seq_of_row[row] * table_width + pos / page_size];
-    const T* down = down_in + (size_t)row * down_ld;
+    if (!a.down_in) return;
+    const int page = a.tables[(size_t)a.seq_of_row[row] * a.table_width + pos / a.page_size];
+    const T* down = a.down_in + (size_t)row * a.down_ld;
     float ssq = 0.f;
     for (int d = tid; d < rank; d += LP_THREADS) {
         const float a = to_f32(down[d]);
         ssq = fmaf(a, a, ssq);
     }
-    const float factor = 1.0f / sqrtf(block_sum(ssq, red) / (float)rank + eps);
-    if (page < 0 || page >= num_pages) return;
-    T* dst = cache + ((size_t)page * page_size + pos % page_size) * key;
+    const float factor = 1.0f / sqrtf(block_sum(ssq, red) / (float)rank + a.eps);
+    if (page < 0 || page >= a.num_pages) return;
+    T* dst = a.cache + ((size_t)page * a.page_size + pos % a.page_size) * key;
     for (int d = tid; d < rank; d += LP_THREADS) {
         T r;
-        from_f32(&r, to_f32(down[d]) * factor * norm_weight[d]);
+        from_f32(&r, to_f32(down[d]) * factor * a.norm_weight[d]);
         dst[d] = cache_value(r);
     }
     const T* part = down + rank;
@@ -70,6 +78,12 @@ __global__ __launch_bounds__(LP_THREADS) void latent_prepare_kernel(
         from_f32(&r, v);
         dst[rank + d] = cache_value(r);
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(LP_THREADS) void latent_prepare_kernel(LatentRows<T> a) {
+    __shared__ float red[16];
+    latent_prepare_row(a, blockIdx.x, red);
 }
 
 template <typename T>
@@ -104,14 +118,13 @@ extern "C" int tli_latent_prepare(const void* q_in, int q_ld, const void* down_i
         return tli_fail("latent_prepare: bad sizes");
     if (page_size <= 0 || table_width <= 0 || num_pages <= 0) return tli_fail("latent_prepare: bad cache geometry");
     hipStream_t s = (hipStream_t)stream;
+#define LATENT_ROWS(T)                                                                                                                  \
+    LatentRows<T>{(const T*)q_in, q_ld, (const T*)down_in, down_ld, (T*)q_out, (T*)cache, positions, seq_of_row, tables, table_width,   \
+                  page_size, num_pages, heads, dim, rot, rank, rot_dims, norm_weight, eps, cos_t, sin_t}
     if (dtype == TLI_F32)
-        latent_prepare_kernel<float><<<rows, LP_THREADS, 0, s>>>((const float*)q_in, q_ld, (const float*)down_in, down_ld, (float*)q_out, (float*)cache, positions,
-                                                                 seq_of_row, tables, table_width, page_size, num_pages, heads, dim,
-                                                                 rot, rank, rot_dims, norm_weight, eps, cos_t, sin_t);
+        latent_prepare_kernel<float><<<rows, LP_THREADS, 0, s>>>(LATENT_ROWS(float));
     else if (dtype == TLI_BF16)
-        latent_prepare_kernel<bf16_t><<<rows, LP_THREADS, 0, s>>>((const bf16_t*)q_in, q_ld, (const bf16_t*)down_in, down_ld, (bf16_t*)q_out, (bf16_t*)cache, positions,
-                                                                  seq_of_row, tables, table_width, page_size, num_pages, heads, dim,
-                                                                  rot, rank, rot_dims, norm_weight, eps, cos_t, sin_t);
+        latent_prepare_kernel<bf16_t><<<rows, LP_THREADS, 0, s>>>(LATENT_ROWS(bf16_t));
     else
         return tli_fail("latent_prepare: unknown dtype %d", dtype);
     return tli_check_launch("latent_prepare");
@@ -154,9 +167,9 @@ union HpFrag {
 // (A workgroup's four waves fetch the same blocks of W one after the other: three of them find it in the cache.)
 // EXACT: K is 16 KM (no condition left in the loop over k).
 template <int KM, bool EXACT, int RT>
-__global__ __launch_bounds__(256) void head_products_mfma_kernel(const bf16_t* __restrict__ x, long long x_row, long long x_head,
-                                                                 const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
-                                                                 long long y_row, long long y_head, int T, int N, int K, HeadGate<bf16_t> gate) {
+__device__ __forceinline__ void head_products_mfma(const bf16_t* __restrict__ x, long long x_row, long long x_head,
+                                                   const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
+                                                   long long y_row, long long y_head, int T, int N, int K, HeadGate<bf16_t> gate, int shares) {
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     const int col = lane % 16, grp = lane / 16;
     const int t0 = (blockIdx.x * 4 + wave) * 16 * RT, h = blockIdx.y;
@@ -177,7 +190,7 @@ __global__ __launch_bounds__(256) void head_products_mfma_kernel(const bf16_t* _
 #pragma unroll
     for (int r = 0; r < RT; ++r) by[r] = gate.of(min(t0 + r * 16 + col, T - 1), h);
     // (few rows: the blocks of outputs are shared out over blockIdx.z, an even number each)
-    const int per_z = (((N / 16 + gridDim.z - 1) / gridDim.z) + 1) & ~1;
+    const int per_z = (((N / 16 + shares - 1) / shares) + 1) & ~1;
     const int nblocks = min(N / 16, (int)(blockIdx.z + 1) * per_z);
     for (int nb = blockIdx.z * per_z; nb < nblocks; nb += 2) {
         const bool two = nb + 1 < nblocks;
@@ -216,6 +229,30 @@ __global__ __launch_bounds__(256) void head_products_mfma_kernel(const bf16_t* _
             }
         }
     }
+}
+
+template <int KM, bool EXACT, int RT>
+__global__ __launch_bounds__(256) void head_products_mfma_kernel(const bf16_t* __restrict__ x, long long x_row, long long x_head,
+                                                                 const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
+                                                                 long long y_row, long long y_head, int T, int N, int K, HeadGate<bf16_t> gate) {
+    head_products_mfma<KM, EXACT, RT>(x, x_row, x_head, w, y, y_row, y_head, T, N, K, gate, gridDim.z);
+}
+
+// Steps of few rows: the queries' products into the latent space and prepare, which touch nothing of each other's, as one launch
+// (the last gridDim.z prepares).  8 rows of 16 heads, as part of a decode step: 6.1 and 4.2 us one behind the other, 6.0 together.
+template <int KM, bool EXACT>
+__global__ __launch_bounds__(256) void latent_prepare_products_kernel(LatentRows<bf16_t> a, const bf16_t* __restrict__ w, int T) {
+    __shared__ float red[16];
+    const int shares = gridDim.z - 1, key = a.rank + a.rot;
+    if ((int)blockIdx.z == shares) {
+        for (int row = blockIdx.y * gridDim.x + blockIdx.x; row < T; row += gridDim.x * gridDim.y) {
+            latent_prepare_row(a, row, red);
+            __syncthreads();
+        }
+        return;
+    }
+    head_products_mfma<KM, EXACT, 1>(a.q_in, a.q_ld, a.dim + a.rot, w, a.q_out, (long long)a.heads * key, key, T, a.rank, a.dim,
+                                     HeadGate<bf16_t>{nullptr, 0}, shares);
 }
 
 // Many rows, k of 64, 128, 256 or 512: the head's matrix comes through LDS.  A workgroup takes one head and 64 RT rows
@@ -351,4 +388,36 @@ extern "C" int tli_head_products_mfma_bf16(const void* x, long long x_row, long 
     else HP_ONE(40, false, 1);
 #undef HP_ONE
     return tli_check_launch("head_products_mfma");
+}
+
+// tli_latent_prepare and tli_head_products_mfma_bf16 of the queries with w_qk [heads, rank, dim] into q_out, bfloat16, for up to
+// LPP_ROWS rows.
+#define LPP_ROWS 64
+extern "C" int tli_latent_prepare_products_bf16(const void* q_in, int q_ld, const void* down_in, int down_ld, void* q_out, void* cache,
+                                                const int* positions, const int* seq_of_row, const int* tables, int table_width,
+                                                int page_size, int num_pages, int rows, int heads, int dim, int rot, int rank,
+                                                int rot_dims, const float* norm_weight, float eps, const float* cos_t,
+                                                const float* sin_t, const void* w_qk, void* stream) {
+    if (rows <= 0) return 0;
+    if (heads <= 0 || heads > 65535 || dim <= 0 || rot <= 0 || rank <= 0 || rot_dims <= 0 || rot_dims % 2 || rot_dims > rot || rows > LPP_ROWS ||
+        !q_in || q_ld < heads * (dim + rot) || (down_in && (down_ld < rank + rot || !norm_weight)))
+        return tli_fail("latent_prepare_products: bad sizes");
+    if (page_size <= 0 || table_width <= 0 || num_pages <= 0) return tli_fail("latent_prepare_products: bad cache geometry");
+    const long long key = rank + rot;
+    if (!tli_head_products_mfma_takes(rank, dim, q_ld, dim + rot, heads * key, key) || (((uintptr_t)q_in | (uintptr_t)w_qk | (uintptr_t)q_out) & 7))
+        return tli_fail("latent_prepare_products: the products are not the matrix-core kernel's");
+    const int row_groups = (rows + 63) / 64;
+    int shares = 512 / (row_groups * heads);
+    shares = shares < 1 ? 1 : (shares > rank / 32 ? (rank / 32 < 1 ? 1 : rank / 32) : shares);
+    const dim3 grid(row_groups, heads, shares + 1);
+    hipStream_t s = (hipStream_t)stream;
+    const LatentRows<bf16_t> a = LATENT_ROWS(bf16_t);
+#define LPP_RUN(KM, EXACT) latent_prepare_products_kernel<KM, EXACT><<<grid, 256, 0, s>>>(a, (const bf16_t*)w_qk, rows)
+    if (dim == 64) LPP_RUN(4, true);
+    else if (dim == 128) LPP_RUN(8, true);
+    else if (dim == 256) LPP_RUN(16, true);
+    else if (dim <= 128) LPP_RUN(8, false);
+    else LPP_RUN(40, false);
+#undef LPP_RUN
+    return tli_check_launch("latent_prepare_products");
 }

@@ -136,6 +136,7 @@ def load_library():
         "tli_diff_prepare": [P, I, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P, P, F, I, P],
         "tli_diff_combine": [P, P, I, I, P, I, I, I, F, F, F, I, P],
         "tli_latent_prepare": [P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, I, I, P, F, P, P, I, P],
+        "tli_latent_prepare_products_bf16": [P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, I, I, P, F, P, P, P, P],
         "tli_head_products_plain": [P, ctypes.c_longlong, ctypes.c_longlong, P, P, ctypes.c_longlong, ctypes.c_longlong,
                                     I, I, I, I, P, I, I, P],
         "tli_moe_grouped_tile": [I, I],
@@ -1957,6 +1958,8 @@ class HipOps:
                    T, n, float(eps), _dtype_code(proj.dtype), self._stream())
         return out
 
+    LATENT_TOGETHER_ROWS = 64    # up to so many rows the queries' products and what else stands before the attention are one launch
+
     def latent_attention(self, query, q_at, own, step, cache, heads, dim, rot, rank, vdim, rotary, scale, w_qk, w_v, window=None,
                          sinks=None, gate=None):
         """Attention whose keys and values are made from one latent vector a position, from the raw queries
@@ -1992,14 +1995,17 @@ class HipOps:
         if rd > rot:
             raise KernelError(f"{rd} turned elements do not fit a key part of {rot}")
         q = torch.empty((T, heads, key), dtype=query.dtype, device=self.device)
-        self._call(self.lib.tli_latent_prepare, query.data_ptr() + q_at * es, query.shape[1], down_ptr, down_ld, q.data_ptr(),
-                   kc.data_ptr(), step.positions.data_ptr(),
-                   step.seq_of_row.data_ptr(), g.tables.data_ptr(), g.table_width, g.page_size, pages, T, heads, dim, rot,
-                   rank, rd, norm_ptr, float(norm_eps), cos.data_ptr(), sin.data_ptr(),
-                   _dtype_code(query.dtype), self._stream())
         self._want(w_qk, "matrices into the latent space", query.dtype, (heads, rank, dim))
         self._want(w_v, "matrices out of the latent space", query.dtype, (heads, vdim, rank))
-        self.head_products(query, dim + rot, w_qk, out=q.view(T, heads * key), out_stride=key, x_at=q_at)
+        prepare = (query.data_ptr() + q_at * es, query.shape[1], down_ptr, down_ld, q.data_ptr(), kc.data_ptr(), step.positions.data_ptr(),
+                   step.seq_of_row.data_ptr(), g.tables.data_ptr(), g.table_width, g.page_size, pages, T, heads, dim, rot,
+                   rank, rd, norm_ptr, float(norm_eps), cos.data_ptr(), sin.data_ptr())
+        if (0 < T <= self.LATENT_TOGETHER_ROWS and query.dtype == torch.bfloat16 and not self.plain_products and prepare[0] % 8 == 0
+                and w_qk.data_ptr() % 8 == 0 and self.lib.tli_head_products_mfma_takes(rank, dim, query.shape[1], dim + rot, heads * key, key)):
+            self._call(self.lib.tli_latent_prepare_products_bf16, *prepare, w_qk.data_ptr(), self._stream())
+        else:
+            self._call(self.lib.tli_latent_prepare, *prepare, _dtype_code(query.dtype), self._stream())
+            self.head_products(query, dim + rot, w_qk, out=q.view(T, heads * key), out_stride=key, x_at=q_at)
         o = self.sized_attention(q, step, g, kc.view(pages, 1, g.page_size, key), None, heads, 1, 1, key, rank, scale,
                                  window, 0, query.dtype, sinks=sinks)
         return self.head_products(o.view(T, heads * rank), rank, w_v, gate=gate)
