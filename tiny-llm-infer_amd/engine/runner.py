@@ -277,7 +277,7 @@ class ModelRunner:
             slots=dev[lay["slots"]], sample_rows=dev[lay["sample_rows"]],
             h_row_start=row_start, h_seq_start=starts, h_seq_len=totals,
             h_slots=slots, max_rows_per_seq=max(counts),
-            all_wanted=sample == list(range(rows)), max_seq_len=max(totals), reach=max(128, 1 << (max(totals) - 1).bit_length()),
+            all_wanted=len(sample) == rows and sample == list(range(rows)), max_seq_len=max(totals), reach=max(128, 1 << (max(totals) - 1).bit_length()),
             skew=min(16, 1 << ((max(totals) * len(totals)) // max(sum(totals), 1)).bit_length() - 1),
             groups=groups)
 

@@ -19,7 +19,9 @@ class PreNormBlock(Block):
         super().__init__(spec)
         self.mixer = mixer
         self.ffn = ffn
-        self.norm_mixer = self.opening_norm = norms["mixer"]
+        self.norm_mixer = norms["mixer"]
+        if type(self).forward is PreNormBlock.forward:         # (not of an arrangement derived from this one)
+            self.opening_norm = self.norm_mixer
         self.norm_ffn = norms["ffn"] if ffn is not None else None
         self.replayable = all(p.replayable for p in self._parts())
 

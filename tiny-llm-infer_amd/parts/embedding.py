@@ -54,8 +54,8 @@ class TokenEmbedding(Part):
     def forward_normed(self, token_ids: torch.Tensor, num_rows: int, norm):
         """(the residual's rows, their ``norm``) where one pass makes both, else None."""
         rms, both = norm.as_rms(), getattr(self.env.ops, "embed_rmsnorm", None)
-        if rms is None or both is None or self.pos_table is not None or self.scale != 1.0:
-            return None
+        if rms is None or both is None or self.pos_table is not None or self.scale != 1.0 or type(self).forward is not TokenEmbedding.forward:
+            return None                        # (an embedding derived from this one that makes its rows otherwise)
         return both(self.table, token_ids, num_rows, *rms)
 
 
@@ -64,7 +64,7 @@ class LinearHead(Part):
 
     @property
     def takes_normed_rows(self) -> bool:
-        return getattr(getattr(self, "weight", None), "tiled", None) is not None
+        return type(self).forward is LinearHead.forward and getattr(getattr(self, "weight", None), "tiled", None) is not None
 
     def __init__(self, spec):
         super().__init__(spec)

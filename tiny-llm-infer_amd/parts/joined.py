@@ -241,7 +241,8 @@ class OneNormParallelBlock(Block):
     def __init__(self, spec, mixer, ffn, norms):
         super().__init__(spec)
         self.mixer, self.ffn, self.norm = mixer, ffn, norms["mixer"]
-        self.opening_norm = self.norm
+        if type(self).forward is OneNormParallelBlock.forward:
+            self.opening_norm = self.norm
         self.mult = float(spec.params.get("residual_mult", 1.0))
         for part in self._sublayers():
             if not (hasattr(part, "load_rows") and hasattr(part, "rows")):

@@ -130,6 +130,12 @@ class RoutedExperts(FeedForward):
     def workspace_elems(self, rows: int) -> int:
         return rows * (self.top * (3 * self.inter + self.hidden) + 3 * (self.shared_inter or 0) + 2 * self.outputs)
 
+    @property
+    def takes_choice(self) -> bool:
+        """Whether ``forward`` also takes the choice (``routed``) that a norm's kernel has made: not of a part derived from this one
+        with a ``forward`` of its own."""
+        return type(self).forward is RoutedExperts.forward
+
     def routing(self) -> Dict:
         """The arguments of the router after its input, by name: for norms whose kernel makes the choice as well."""
         out = dict(w_rows=self.w_router, experts=self.outputs, top=self.top, groups=self.groups, keep=self.keep, scale=self.scale,

@@ -57,7 +57,7 @@ class ParallelBlock(Block):
         if self.pair is not None:
             (w1, w2), eps = self.pair
             both = None
-            if hasattr(self.ffn, "routing") and hasattr(self.env.ops, "add_layernorm_route"):
+            if getattr(self.ffn, "takes_choice", False) and hasattr(self.env.ops, "add_layernorm_route"):
                 both = self.env.ops.add_layernorm_route(resid, owed, (w1, w2), eps, self.env.dtype, self.ffn.routing())
             if both is not None:
                 (n1, n2), chosen["routed"] = both

@@ -128,7 +128,7 @@ class SandwichBlock(Block):
             mixed = ops.norm_add_norm_mixes(resid, y, w_out, eps_out, weight, eps, self.env.dtype, mixes(step), step)
             if mixed is not None:
                 return mixed, {}
-        if hasattr(reader, "routing") and hasattr(ops, "norm_add_norm_route"):
+        if getattr(reader, "takes_choice", False) and hasattr(ops, "norm_add_norm_route"):
             both = ops.norm_add_norm_route(resid, y, w_out, eps_out, weight, eps, self.env.dtype, reader.routing())
             if both is not None:
                 return both[0], {"routed": both[1]}
