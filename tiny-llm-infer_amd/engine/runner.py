@@ -138,9 +138,9 @@ class ModelRunner:
         self.inputs = StepInputs(env.device, max(max_batch_tokens, _decode_bucket(max_requests)),
                                  _decode_bucket(max_requests), len(self.cache.groups), max_width)
         self.steps_run = 0
-        # Decode steps (one token for every request, every logit wanted) launch the same
-        # kernels with the same arguments whenever (requests, table width, reach, skew) agree:
-        # their launch sequence is recorded once as a HIP graph and replayed.  (float32 steps too: launched one by
+        # Decode steps (one token for every request, as many places wanted as requests) launch the same
+        # kernels with the same arguments whenever (requests, table width, reach, skew, whether the places are
+        # all rows in their order) agree: their launch sequence is recorded once as a HIP graph and replayed.  (float32 steps too: launched one by
         # one, the 40 kernels of a small model's step take the host longer than the device: 6.1 -> 4.5 ms for 16 steps of
         # four layers of 1,024.)
         parts = [model.embedding, model.final_norm, model.head] + list(model.blocks)
@@ -312,13 +312,14 @@ class ModelRunner:
         step.state = None
         if num_wanted == 0:
             return None
-        x = model.close_residual(resid, pending, rows=step.sample_rows, num_rows=num_wanted, all_rows=step.all_wanted)
+        x = model.close_residual(resid, pending, rows=step.sample_rows, num_rows=num_wanted,
+                                 all_rows=step.all_wanted and num_wanted == step.num_rows)
         return model.head.forward(x)
 
     def _replay(self, view: StepView, wanted: int) -> torch.Tensor:
         """A decode step through its recorded launch sequence.  The step's inputs
         already lie in the device buffer whose layout depends on the key alone."""
-        key = (view.num_seqs, view.groups[0].table_width if view.groups else 0, view.reach, view.skew)
+        key = (view.num_seqs, view.groups[0].table_width if view.groups else 0, view.reach, view.skew, view.all_wanted)
         entry = self.graphs.get(key)
         if entry is None:
             # The first step of a shape runs eagerly (anything lazy happens now) and its result is the
