@@ -9,6 +9,7 @@ import torch
 from ..cache.manager import CacheNeed, StateNeed
 from ..config.base import ConfigError, ModelSpec, PartSpec
 from ..parts.base import Block, BuildEnv, build_part, run_norm
+from ..parts.norm import RMSNorm
 from ..weights.loader import TensorDecl, load_tensors, random_tensors, unique_decls
 
 
@@ -16,6 +17,11 @@ def cache_needs_of(mixer) -> Tuple[CacheNeed, ...]:
     """What a mixer needs of the paged cache: nothing, one need or several."""
     need = mixer.cache_need()
     return () if need is None else (need,) if isinstance(need, CacheNeed) else tuple(need)
+
+
+def _is_stock_rms(norm) -> bool:
+    """Whether the norm's rows are RMSNorm's own: not of a norm derived from it that makes them in a ``forward`` of its own."""
+    return type(norm).forward is RMSNorm.forward
 
 
 class Model:
@@ -91,7 +97,7 @@ class Model:
         where the embedding makes them in the same pass."""
         first = self.blocks[self.schedule[0].block] if self.schedule else None
         norm, normed = getattr(first, "opening_norm", None), getattr(self.embedding, "forward_normed", None)
-        if norm is not None and normed is not None and type(first).open is Block.open:
+        if norm is not None and normed is not None and type(first).open is Block.open and _is_stock_rms(norm):
             both = normed(token_ids, num_rows, norm)
             if both is not None:
                 return both[0], {"normed": both[1]}
@@ -100,7 +106,7 @@ class Model:
     def close_residual(self, resid, pending, rows=None, num_rows=None, all_rows=False):
         """The final norm's rows (of ``rows`` only, if given) from the residual and what the last
         block still owes it.  ``all_rows``: ``rows`` are all of the residual's, in their order, and the norm's rows go to the head."""
-        if all_rows and (not self.schedule or type(self.blocks[self.schedule[-1].block]).close is Block.close):
+        if all_rows and _is_stock_rms(self.final_norm) and (not self.schedule or type(self.blocks[self.schedule[-1].block]).close is Block.close):
             return run_norm(self.final_norm, resid, pending, consumer=self.head)
         if not self.schedule:
             return run_norm(self.final_norm, resid, pending, rows=rows, num_rows=num_rows)
