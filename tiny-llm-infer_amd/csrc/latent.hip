@@ -238,17 +238,18 @@ __global__ __launch_bounds__(256) void head_products_mfma_kernel(const bf16_t* _
     head_products_mfma<KM, EXACT, RT>(x, x_row, x_head, w, y, y_row, y_head, T, N, K, gate, gridDim.z);
 }
 
-// Steps of few rows: the queries' products into the latent space and prepare, which touch nothing of each other's, as one launch
-// (the last gridDim.z prepares).  8 rows of 16 heads, as part of a decode step: 6.1 and 4.2 us one behind the other, 6.0 together.
+// Steps of few rows: the queries' products into the latent space and prepare, which touch nothing of each other's, as one launch: the
+// first `shares` of gridDim.z multiply, the workgroups of the others prepare a row each (a row is a chain of fetches: 64 of them behind one
+// another in a workgroup took 122 us).  8 rows of 16 heads, as part of a decode step: 6.1 and 4.2 us one behind the other, 6.0 together.
+// The whole layer between its projections, 100 keys of 512 + 64, apart and together, us: 16 heads, 1 row 19.6 and 18.0, 8 rows 20.6 and
+// 18.7, 64 rows 36.4 and 34.3; one head, 1 row 17.2 and 14.9, 64 rows 28.6 and 25.6.
 template <int KM, bool EXACT>
-__global__ __launch_bounds__(256) void latent_prepare_products_kernel(LatentRows<bf16_t> a, const bf16_t* __restrict__ w, int T) {
+__global__ __launch_bounds__(256) void latent_prepare_products_kernel(LatentRows<bf16_t> a, const bf16_t* __restrict__ w, int T, int shares) {
     __shared__ float red[16];
-    const int shares = gridDim.z - 1, key = a.rank + a.rot;
-    if ((int)blockIdx.z == shares) {
-        for (int row = blockIdx.y * gridDim.x + blockIdx.x; row < T; row += gridDim.x * gridDim.y) {
-            latent_prepare_row(a, row, red);
-            __syncthreads();
-        }
+    const int key = a.rank + a.rot;
+    if ((int)blockIdx.z >= shares) {
+        const int row = ((blockIdx.z - shares) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+        if (row < T) latent_prepare_row(a, row, red);
         return;
     }
     head_products_mfma<KM, EXACT, 1>(a.q_in, a.q_ld, a.dim + a.rot, w, a.q_out, (long long)a.heads * key, key, T, a.rank, a.dim,
@@ -409,10 +410,11 @@ extern "C" int tli_latent_prepare_products_bf16(const void* q_in, int q_ld, cons
     const int row_groups = (rows + 63) / 64;
     int shares = 512 / (row_groups * heads);
     shares = shares < 1 ? 1 : (shares > rank / 32 ? (rank / 32 < 1 ? 1 : rank / 32) : shares);
-    const dim3 grid(row_groups, heads, shares + 1);
+    const int preparing = (rows + row_groups * heads - 1) / (row_groups * heads);        // (a workgroup a row: each is a chain of fetches)
+    const dim3 grid(row_groups, heads, shares + preparing);
     hipStream_t s = (hipStream_t)stream;
     const LatentRows<bf16_t> a = LATENT_ROWS(bf16_t);
-#define LPP_RUN(KM, EXACT) latent_prepare_products_kernel<KM, EXACT><<<grid, 256, 0, s>>>(a, (const bf16_t*)w_qk, rows)
+#define LPP_RUN(KM, EXACT) latent_prepare_products_kernel<KM, EXACT><<<grid, 256, 0, s>>>(a, (const bf16_t*)w_qk, rows, shares)
     if (dim == 64) LPP_RUN(4, true);
     else if (dim == 128) LPP_RUN(8, true);
     else if (dim == 256) LPP_RUN(16, true);

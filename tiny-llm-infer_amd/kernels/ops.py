@@ -1958,7 +1958,9 @@ class HipOps:
                    T, n, float(eps), _dtype_code(proj.dtype), self._stream())
         return out
 
-    LATENT_TOGETHER_ROWS = 64    # up to so many rows the queries' products and what else stands before the attention are one launch
+    # Up to so many rows the queries' products and what else stands before the attention are one launch (csrc/latent.hip has both
+    # sides' times: 1.3 to 3.8 us less a layer from 1 to 64 rows, 1 to 32 heads; more rows are prompts', whose launches are long).
+    LATENT_TOGETHER_ROWS = 64
 
     def latent_attention(self, query, q_at, own, step, cache, heads, dim, rot, rank, vdim, rotary, scale, w_qk, w_v, window=None,
                          sinks=None, gate=None):
