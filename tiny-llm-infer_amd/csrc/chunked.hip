@@ -295,7 +295,9 @@ __global__ __launch_bounds__(CK_THREADS) void chunk_states_kernel(ChunkRows a, C
     // Two chunks a round.  The next round's keys and values are asked for before this round's products, by every thread and under no
     // condition (a chunk past the last is the last again): a load that may or may not have been issued makes the compiler wait
     // for all that are in flight, which with a chunk's keys asked for by half of the threads was a round trip to memory a chunk.  (Six
-    // prompts, 2,048 rows a step, 16 heads of 128 x 128: retention 55.2 -> 48.1 us, mLSTM 51.5 -> 44.2.)
+    // prompts, 2,048 rows a step, 16 heads of 128 x 128: retention 55.2 -> 48.1 us, mLSTM 51.5 -> 44.2.)  The last round asks for nothing: a
+    // sequence of one or two chunks, such as a decoding request beside a prompt's portion, has no other.  (60 rows alone beside a portion of
+    // 40, retention in all: 109 us with a chunk a round, 117 where the last round asked too, 104 now; 8 portions of 64 33.1, 33.9, 31.2.)
     // (A tile without elements of k, t >= tiles, multiplies what LDS holds and is not stored.)
     bf16_t v0[16], v1[16];
     float end0 = 0.f, end1 = 0.f;                        // the last log A of the chunks whose values are in v0 and v1
@@ -304,14 +306,15 @@ __global__ __launch_bounds__(CK_THREADS) void chunk_states_kernel(ChunkRows a, C
     fetch_values(min(1, chunks - 1), v1, end1);
     store_keys(k_turn);
     __syncthreads();
-    for (int z = 0; z < chunks; z += 2) {
+    int z = 0;
+    for (; z + 2 < chunks; z += 2) {
         bf16_t next0[16], next1[16];
         float next_end0 = 0.f, next_end1 = 0.f;
         fetch_keys(min(z + 2 + k_turn, chunks - 1));
-        fetch_values(min(z + 2, chunks - 1), next0, next_end0);
+        fetch_values(z + 2, next0, next_end0);
         fetch_values(min(z + 3, chunks - 1), next1, next_end1);
         walk(z, v0, end0);
-        if (z + 1 < chunks) walk(z + 1, v1, end1);
+        walk(z + 1, v1, end1);
         __syncthreads();                                 // both chunks' keys are read
         store_keys(z + 2 + k_turn);
         __syncthreads();
@@ -319,6 +322,8 @@ __global__ __launch_bounds__(CK_THREADS) void chunk_states_kernel(ChunkRows a, C
         for (int i = 0; i < 16; ++i) v0[i] = next0[i], v1[i] = next1[i];
         end0 = next_end0, end1 = next_end1;
     }
+    walk(z, v0, end0);                                   // (nothing follows the last round)
+    if (z + 1 < chunks) walk(z + 1, v1, end1);
 #pragma unroll
     for (int t = 0; t < CK_PAIRS; ++t) {
         if (t >= tiles) continue;
