@@ -6,15 +6,13 @@
 //   wkv:        d = exp(-exp(W2 tanh(z) + w0)) a channel; o = (S + diag(u) k v^T)^T r; S <- diag(d) S + k v^T; RMS times the
 //               weight; silu gate
 // A column of S belongs to 16 lanes of a wave, a lane holding R elements of it (as in lightning.hip: pieces of up to four
-// that lie side by side with the other lanes').  A workgroup takes 32 columns at a time and asks for the row's own operands, then
-// for the first GROUPS x 32 columns, so that the state's bytes, which are nearly all that such a step moves, are on their way
-// while the row's q, k, v and gates are made, and nothing of the row waits behind them.  With 256 threads, which asked for the state
-// first and for the decays' matrix after the row's tanh, 8 rows of 16 heads of 128 x 128 took (as part of a decode step): retention
-// 9.8 us and now 7.0, mLSTM 11.6 and 8.6, wkv 12.3 and 8.4.
+// that lie side by side with the other lanes').  A workgroup takes 32 columns at a time (16 with 256 threads: step_wide says which) and
+// asks for the row's own operands, then for the first GROUPS times as many columns, so that the state's bytes, which are nearly all
+// that such a step moves, are on their way while the row's q, k, v and gates are made, and nothing of the row waits behind them.  256 threads
+// that asked for the state first and for the decays' matrix after the row's tanh, and 512 in this order, 8 rows of 16 heads of
+// 128 x 128 as part of a decode step: retention 9.8 us and 7.0, mLSTM 11.6 and 8.6, wkv 12.3 and 8.4.
 #include "recurrence.h"
 #include "row_gates.h"
-
-#define RS_THREADS 512
 
 __device__ __forceinline__ float rs_sum16(float v) {     // over the 16 lanes of a DPP row; every lane gets it
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));
@@ -90,15 +88,15 @@ __device__ __forceinline__ float rs_dot8(const T* a, const T* b) {
 }
 
 // T: of the projections; TO: of the output and the matrices
-template <int KIND, int R, typename T, typename TO>
-__global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, StepRetention ret, StepMemory mem, StepTimeMix mix) {
+template <int KIND, int R, int THREADS, typename T, typename TO>
+__global__ __launch_bounds__(THREADS) void recurrent_step_kernel(StepRows a, StepRetention ret, StepMemory mem, StepTimeMix mix) {
     constexpr bool MEMORY = KIND == STEP_MEMORY, WKV = KIND == STEP_WKV;
-    constexpr int L = 16, DKP = L * R, NC = RS_THREADS / L;
-    constexpr int GROUPS = 4;                                          // of NC columns, in flight together
+    constexpr int L = 16, DKP = L * R, NC = THREADS / L;
+    constexpr int GROUPS = THREADS == 512 ? 4 : 8;                     // of NC columns, in flight together
     constexpr int VW = R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;
     extern __shared__ __align__(16) float rs_lds[];
-    constexpr int WAVES = RS_THREADS / TLI_WAVE;
-    __shared__ float red[3 * WAVES];
+    constexpr int WAVES = THREADS / TLI_WAVE;
+    __shared__ float red[3 * WAVES < 16 ? 16 : 3 * WAVES];              // (block_sum reads 16)
     const int h = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, sub = tid % L, jl = tid / L;
     const int dk = a.dk, dv = a.dv, H = a.H, OV = dv + (MEMORY ? 1 : 0);
     float* q_s = rs_lds;
@@ -157,10 +155,10 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
         for (int g = 0; g < GROUPS; ++g)
             if (j0 + g * NC + jl < dv) load_column(j0 + g * NC + jl, S[g]);
     };
-    // The row's operands first, into registers: an element of q or k a thread (2 DKP <= RS_THREADS), one of v, of the gate and of the norm's
+    // The row's operands first, into registers: an element of q or k a thread (2 DKP <= THREADS), one of v, of the gate and of the norm's
     // weights (more in rounds below), and what the kind needs.  Loads complete in the order of issue, so none of them waits for the
     // state, and the state is on its way while they are worked on.
-    static_assert(2 * DKP <= RS_THREADS, "an element of q or k a thread");
+    static_assert(2 * DKP <= THREADS, "an element of q or k a thread");
     const T* src = (const T*)a.proj + (size_t)row * a.ld;
     const T* q_src = src + (size_t)h * dk;
     const T* k_src = src + (size_t)(H + h) * dk;
@@ -182,8 +180,8 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
     float keep = 0.f, floor_ = 0.f;
     float turn_cos = 1.f, turn_sin = 0.f;                              // retention: of this thread's element
     bool turned = false, second = false;
-    constexpr int P = RS_THREADS / DKP;                                // wkv: neighbouring threads that share out a channel's row of W2
-    constexpr int HELD = 4;                                            //      16-byte pieces of it that a thread holds
+    constexpr int P = THREADS / DKP;                                // wkv: neighbouring threads that share out a channel's row of W2
+    constexpr int HELD = P >= 16 ? 1 : P >= 8 ? 2 : 4;                 //      16-byte pieces of it that a thread holds
     const int channel = tid / P, part = tid % P;
     const TO* w2 = WKV ? (const TO*)mix.w2 + (size_t)(h * dk + min(channel, dk - 1)) * mix.rank : nullptr;
     const bool pieces = WKV && sizeof(TO) == 2 && mix.rank % 8 == 0;
@@ -208,17 +206,17 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
         const T* wi = (const T*)mem.w + (size_t)h * mem.n;
         const T* wf = (const T*)mem.w + (size_t)(H + h) * mem.n;
         if (mem.n % 8 == 0) {
-            for (int i = tid * 8; i < mem.n; i += RS_THREADS * 8) {
+            for (int i = tid * 8; i < mem.n; i += THREADS * 8) {
                 zi += rs_dot8(x + i, wi + i);
                 zf += rs_dot8(x + i, wf + i);
             }
         } else {
-            for (int i = tid; i < mem.n; i += RS_THREADS) {
+            for (int i = tid; i < mem.n; i += THREADS) {
                 zi = fmaf(to_f32(x[i]), to_f32(wi[i]), zi);
                 zf = fmaf(to_f32(x[i]), to_f32(wf[i]), zf);
             }
         }
-        for (int p = tid; p < mem.factor.parts; p += RS_THREADS) ss += mem.factor.ssq[(size_t)p * a.rows + row];
+        for (int p = tid; p < mem.factor.parts; p += THREADS) ss += mem.factor.ssq[(size_t)p * a.rows + row];
         if (!fresh) m0 = *m_slot;
     } else {
         keep = ret.decay[h];
@@ -240,7 +238,7 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
     float take = 1.f;
     if constexpr (WKV) {
         if (tid < mix.rank) z_s[tid] = tanhf(z_raw);
-        for (int i = tid + RS_THREADS; i < mix.rank; i += RS_THREADS) z_s[i] = tanhf(mix.z[row * mix.z_row + i * mix.z_col]);
+        for (int i = tid + THREADS; i < mix.rank; i += THREADS) z_s[i] = tanhf(mix.z[row * mix.z_row + i * mix.z_col]);
     } else if constexpr (MEMORY) {
         zi = wave_sum(zi), zf = wave_sum(zf), ss = wave_sum(ss);
         if (tid % TLI_WAVE == 0) red[tid / TLI_WAVE] = zi, red[WAVES + tid / TLI_WAVE] = zf, red[2 * WAVES + tid / TLI_WAVE] = ss;
@@ -266,7 +264,7 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
     }
     if (tid < 2 * DKP) q_s[tid] = x;                                   // (k_s lies behind q_s)
     if (tid < dv) v_s[tid] = to_f32(v_raw) * take;
-    for (int j = tid + RS_THREADS; j < dv; j += RS_THREADS) v_s[j] = to_f32(v_src[j]) * take;
+    for (int j = tid + THREADS; j < dv; j += THREADS) v_s[j] = to_f32(v_src[j]) * take;
     if (MEMORY && tid == 0) v_s[dv] = take;
     if constexpr (WKV) {
         __syncthreads();
@@ -333,7 +331,7 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
     __syncthreads();
     const float by = MEMORY ? 1.f / (fmaxf(fabsf(o_s[dv]), floor_) + 1e-6f) : 1.f;
     float sum = 0.f;
-    for (int j = tid; j < dv; j += RS_THREADS) {
+    for (int j = tid; j < dv; j += THREADS) {
         const float o = o_s[j] * by;
         sum = fmaf(o, o, sum);
     }
@@ -344,7 +342,17 @@ __global__ __launch_bounds__(RS_THREADS) void recurrent_step_kernel(StepRows a, 
         from_f32(dst + j, o_s[j] * factor * open);
     };
     if (tid < dv) put(tid, to_f32(g_raw), weight_raw);
-    for (int j = tid + RS_THREADS; j < dv; j += RS_THREADS) put(j, to_f32(g_src[j]), MEMORY || WKV ? weight[j] : 1.f);
+    for (int j = tid + THREADS; j < dv; j += THREADS) put(j, to_f32(g_src[j]), MEMORY || WKV ? weight[j] : 1.f);
+}
+
+// Threads of a workgroup: with 512 a head's step is the shorter chain, with 256 more heads' chains fit a compute unit side by side.
+// 512 up to two workgroups of 512 a compute unit where a head has enough columns for them, one where not, none for heads of 16.
+// us with 512 and 256 threads, retention, mLSTM and wkv: 16 heads of 128 x 128, 8 rows 5.8 and 7.5, 8.0 and 9.2, 7.6 and 9.2, 32 rows 10.6
+// and 11.9, 13.1 and 14.0, 13.2 and 14.1, 64 rows 22.7 and 22.4, 25.9 and 22.8, 25.9 and 24.5; of 64 x 64, 32 rows 5.5 and 6.0, 7.9 and
+// 8.0, 7.3 and 7.4, 64 rows 8.0 and 8.3, 11.8 and 10.7, 12.0 and 10.3; of 32 x 32, 16 rows 3.8 and 4.0, 5.8 and 5.8, 4.7 and 4.9, 32 rows
+// 4.4 and 4.2, 6.9 and 6.2, 5.4 and 5.1; of 16 x 16, 8 rows level, 128 rows 7.7 and 5.6, 14.4 and 10.2, 10.1 and 7.6.
+static bool step_wide(const StepRows& a) {
+    return a.dk > 16 && (long long)a.H * a.rows <= ((long long)a.dk * a.dv >= 2048 ? 512 : 256);
 }
 
 template <int KIND, typename T, typename TO = T>
@@ -354,12 +362,16 @@ static int run_step(const StepRows& a, const StepRetention& ret, const StepMemor
     const size_t lds = (size_t)(2 * 16 * R + 2 * (a.dv + 1) + (KIND == STEP_WKV ? 16 * R + mix.rank : 0)) * sizeof(float);
     if (lds > 65536) return tli_fail("recurrent_step: values of %d do not fit LDS", a.dv);
     const dim3 grid(a.H, a.rows);
-#define RS_CASE(R) case R: recurrent_step_kernel<KIND, R, T, TO><<<grid, RS_THREADS, lds, s>>>(a, ret, mem, mix); break;
+    const bool wide = R > 8 || step_wide(a);
+#define RS_RUN(R, THREADS) recurrent_step_kernel<KIND, R, THREADS, T, TO><<<grid, THREADS, lds, s>>>(a, ret, mem, mix)
+#define RS_CASE(R) case R: if (wide) RS_RUN(R, 512); else RS_RUN(R, 256); break;
     switch (R) {
-        RS_CASE(1) RS_CASE(2) RS_CASE(4) RS_CASE(8) RS_CASE(16)
+        RS_CASE(1) RS_CASE(2) RS_CASE(4) RS_CASE(8)
+        case 16: RS_RUN(16, 512); break;
         default: return tli_fail("recurrent_step: keys of %d", a.dk);
     }
 #undef RS_CASE
+#undef RS_RUN
     return tli_check_launch("recurrent_step");
 }
 
