@@ -96,7 +96,7 @@ __global__ __launch_bounds__(THREADS) void recurrent_step_kernel(StepRows a, Ste
     constexpr int VW = R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;
     extern __shared__ __align__(16) float rs_lds[];
     constexpr int WAVES = THREADS / TLI_WAVE;
-    __shared__ float red[3 * WAVES < 16 ? 16 : 3 * WAVES];              // (block_sum reads 16)
+    __shared__ float red[3 * WAVES < 16 ? 16 : 3 * WAVES];              // (block_sum asks for 16)
     const int h = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, sub = tid % L, jl = tid / L;
     const int dk = a.dk, dv = a.dv, H = a.H, OV = dv + (MEMORY ? 1 : 0);
     float* q_s = rs_lds;
