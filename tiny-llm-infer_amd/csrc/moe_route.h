@@ -157,8 +157,8 @@ struct RouteRows {
 // What a norm with a router takes: up to 32 logits (two a wave of 1,024 threads), rows of up to 4,096 elements in 8s: the weights that a
 // wave holds are 64 registers then, of the 128 a lane has with so many threads, and a third logit or a longer row does not fit
 // beside the row.  With the router on its own and in the norm's launch, us, a shared gate beside the experts: rows of 512, 8 experts, 1 row
-// 6.1 and 5.8 (layer norms), 6.4 and 5.7 (norm_add_norm), 128 rows 6.8 and 6.2, 7.0 and 6.1; rows of 4,096, 31 experts, 1 row 13.7 and 12.5, 13.8
-// and 13.0, 128 rows 15.1 and 13.5, 15.1 and 14.0.  (More than 128 rows are prompts' in the main: ROUTER_ROWS of kernels/ops.py.)
+// 6.1 and 5.7 (layer norms), 6.2 and 5.7 (norm_add_norm), 128 rows 6.8 and 6.2, 6.9 and 6.2; rows of 4,096, 31 experts, 1 row 13.3 and 12.5,
+// 13.5 and 12.7, 128 rows 14.7 and 13.5, 14.7 and 13.6.  (More than 128 rows are prompts' in the main: ROUTER_ROWS of kernels/ops.py.)
 #define NORM_ROUTE_THREADS 1024
 #define NORM_ROUTE_COLS 32
 #define NORM_ROUTE_MAX 4096
