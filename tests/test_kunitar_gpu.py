@@ -440,7 +440,7 @@ def test_decoded_rows_whose_keys_are_shared_out(ops, sinks, window, keep, monkey
                                                                        (6, 2, 272, 256, 16, 50), (32, 2, 640, 512, 64, 64), (3, 3, 256, 240, 16, 31)])
 def test_decoded_rows_over_a_latent_vector_of_few_heads(ops, heads, kv_heads, key, value, page, window, sinks, monkeypatch):
     """The four waves share out a key's elements and a value's: sizes with remainders of 32 and of 64, whole and partial rounds of 32
-    keys, empty runs of keys, and pages that are not there."""
+    keys, empty runs of keys, and tables that name no page past a row's last key (every page that a row sees is there)."""
     from tiny_llm_infer_amd.parts.base import GroupView
     g = torch.Generator().manual_seed(heads + key)
     lengths = [1, 32, 33, 200, 333]

@@ -157,6 +157,8 @@ __global__ __launch_bounds__(64 * ASM_WAVES) void attention_sized_mfma_kernel(
     // DEPTH tiles' keys and values are on their way together (a wave of a row that is shared out has two or three tiles: they are one
     // trip to memory, not one each), and a tile's page is looked up once, by a scalar load: a tile of 16 keys lies inside one page.
     // 8 rows of 1,100 keys and blocks, heads of 128, 8 runs, as part of a decode step: 12.5 us, one tile ahead and its values not, and 10.4 now.
+    // Without blocks, two maps of 16 heads of 128 over 4 key heads: 8 rows of 60 keys 6.6 and 6.3 us, of 500 18.0 and 14.0, of 2,000 78 and 43, 64
+    // rows of 60 keys 15.7 and 15.3, of 2,000 138 and 81; maps of 64, 64 rows of 60 keys level.
     constexpr int DEPTH = NKM <= 8 && NVM <= 8 ? 2 : 1;
     uint4 next[DEPTH][PASSES];
     constexpr bool VALUES_TOO = !VKEY && DEPTH == 2;                    // (larger heads leave no registers for it)
@@ -407,7 +409,8 @@ __global__ __launch_bounds__(256) void attention_parts_merge_kernel(
 // every fourth 32 elements of a key, the scores' parts meet in LDS, and each multiplies the weights with every fourth 16 value
 // elements.  v_mfma_f32_16x16x32_bf16; the values are read out of the key tile.
 // 8 rows, 16 heads, 512 + 64 elements, 500 keys in 16 runs, as part of a decode step: attention_sized_shared_kernel, where one wave
-// of the four had columns, 15.5 us, this 8.7.
+// of the four had columns, 15.5 us, this 8.7; 64 rows of 2,000 keys 91 and 60, one row of 100 keys 15.0 and 9.4; one head 86 and 58, 11.2
+// and 8.2.  Every page of the keys that a row sees must be there: keys of one that is not count as zeros, as in that kernel.
 #define ALS_KEYS 32
 #define ALS_PAD 8
 

@@ -1901,13 +1901,17 @@ class HipOps:
                    heads, vdim, float(lam), float(after), float(norm_eps), _dtype_code(proj.dtype), self._stream())
         return out
 
-    SIZED_WORKGROUPS = 256           # decoding rows whose keys are shared out: the workgroups aimed at,
-    SIZED_SPLIT_KEYS = 32            # and the fewest keys of a split (two tiles of 16)
+    # Decoding rows whose keys are shared out: the workgroups aimed at, and the fewest keys of a split: two tiles of 16 of the kernel for more
+    # than 16 heads, one round of 32 of attention_latent_step, for which they were measured again (16 heads of 512 + 64, us, 2, 4, 8, 16 and 32
+    # splits: 1 row of 100 keys 12.2, 9.4, 9.8, 10.4, 11.3; of 500 28.9, 18.4, 12.9, 10.5, 11.5; 16 rows of 500 29.0, 18.8, 14.6, 14.3, 19.2).
+    # There 512 workgroups would be better past 1,000 keys: 16 rows of 2,000 24.1 -> 22.7, 32 rows of 8,000 122 -> 78.
+    SIZED_WORKGROUPS = 256
+    SIZED_SPLIT_KEYS = 32
 
     def _sized_splits(self, T, reach, units, key_heads, window, keep) -> int:
         """Over how many workgroups the keys of one (row, key head) that decodes are shared out, where all heads read one cached
-        vector; ``reach``: a power of two that the longest sequence fits.  A workgroup takes a row's tiles of 16 keys one
-        after the other."""
+        vector; ``reach``: a power of two that the longest sequence fits.  A workgroup takes a run of a row's keys, 16 of
+        them after the other or, up to 16 heads a key head, 32 (csrc/attention_sized_mfma.hip)."""
         keys = min(reach, (window + 15 if window else reach) + keep)
         groups = T * key_heads * ((units // key_heads + 63) // 64)
         return max(1, self.sized_splits or min(self.SIZED_WORKGROUPS // groups, keys // self.SIZED_SPLIT_KEYS, 64))
