@@ -350,7 +350,8 @@ __global__ __launch_bounds__(THREADS) void recurrent_step_kernel(StepRows a, Ste
 // us with 512 and 256 threads, retention, mLSTM and wkv: 16 heads of 128 x 128, 8 rows 5.8 and 7.5, 8.0 and 9.2, 7.6 and 9.2, 32 rows 10.6
 // and 11.9, 13.1 and 14.0, 13.2 and 14.1, 64 rows 22.7 and 22.4, 25.9 and 22.8, 25.9 and 24.5; of 64 x 64, 32 rows 5.5 and 6.0, 7.9 and
 // 8.0, 7.3 and 7.4, 64 rows 8.0 and 8.3, 11.8 and 10.7, 12.0 and 10.3; of 32 x 32, 16 rows 3.8 and 4.0, 5.8 and 5.8, 4.7 and 4.9, 32 rows
-// 4.4 and 4.2, 6.9 and 6.2, 5.4 and 5.1; of 16 x 16, 8 rows level, 128 rows 7.7 and 5.6, 14.4 and 10.2, 10.1 and 7.6.
+// 4.4 and 4.2, 6.9 and 6.2, 5.4 and 5.1; of 16 x 16, 8 rows level, 128 rows 7.7 and 5.6, 14.4 and 10.2, 10.1 and 7.6.  (256 threads that asked for the
+// state first: level or 1 to 15% longer than the better of the two, but heads of 16 x 16 in 2,048 workgroups 9.2 and 6.6 for mLSTM and wkv.)
 static bool step_wide(const StepRows& a) {
     return a.dk > 16 && (long long)a.H * a.rows <= ((long long)a.dk * a.dv >= 2048 ? 512 : 256);
 }
