@@ -39,8 +39,15 @@ __global__ void embed_kernel(const T* __restrict__ table, const int* __restrict_
     for (int i = threadIdx.x; i < hidden; i += blockDim.x) dst[i] = to_f32(src[i]);
 }
 
+template <typename T>
+__device__ __forceinline__ float rounded_to(float v) {
+    T t;
+    from_f32(&t, v);
+    return to_f32(t);
+}
+
 // What a row owes the residual: a row of T, or float32 partial sums [parts][total_rows][n]
-// added in order and rounded to bfloat16.
+// added in order and rounded to T.
 template <typename T>
 struct RowDelta {
     const T* d;
@@ -52,7 +59,7 @@ struct RowDelta {
         if (parts > 0) {
             float a = 0.f;
             for (int s = 0; s < parts; ++s) a += p[s * plane + i];
-            return bf16_to_f32(f32_to_bf16(a));
+            return rounded_to<T>(a);
         }
         return to_f32(d[i]);
     }
@@ -120,6 +127,7 @@ template <typename T, int IT, bool EMBED = false>
 __global__ void add_rmsnorm_vec_kernel(float* __restrict__ resid, const void* __restrict__ delta, int parts,
                                        const float* __restrict__ weight, T* __restrict__ out,
                                        const int* __restrict__ rows, int n, float eps, int total_rows, const T* __restrict__ table) {
+    constexpr int AT_ONCE = sizeof(T) == 4 ? 8 : 4;        // (a float32 product leaves eight planes, a bfloat16 one rarely more than four)
     __shared__ float scratch[16];
     const int out_row = blockIdx.x;
     int r = rows ? rows[out_row] : out_row;
@@ -142,20 +150,20 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ resid, const void* __
             else if (d.any()) {
                 float dv[4];
                 if (d.parts > 0) {
-                    // four planes a round, all asked for before any is added (in plane order; a plane
+                    // AT_ONCE planes a round, all asked for before any is added (in plane order; a plane
                     // past the last is the last again and is not added)
                     float a[4] = {0.f, 0.f, 0.f, 0.f};
-                    for (int s = 0; s < d.parts; s += 4) {
-                        float pv[4][4];
+                    for (int s = 0; s < d.parts; s += AT_ONCE) {
+                        float pv[AT_ONCE][4];
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) load4(d.p + (size_t)min(s + k, d.parts - 1) * d.plane + i, pv[k]);
+                        for (int k = 0; k < AT_ONCE; ++k) load4(d.p + (size_t)min(s + k, d.parts - 1) * d.plane + i, pv[k]);
 #pragma unroll
-                        for (int k = 0; k < 4; ++k)
+                        for (int k = 0; k < AT_ONCE; ++k)
 #pragma unroll
                             for (int e = 0; e < 4; ++e) a[e] = s + k < d.parts ? a[e] + pv[k][e] : a[e];
                     }
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) dv[e] = bf16_to_f32(f32_to_bf16(a[e]));
+                    for (int e = 0; e < 4; ++e) dv[e] = rounded_to<T>(a[e]);
                 } else {
                     load4(d.d + i, dv);
                 }
@@ -268,17 +276,16 @@ extern "C" int tli_embed_rmsnorm(const void* table, const int* ids, float* resid
     return tli_fail("embed_rmsnorm: unknown dtype %d", dtype);
 }
 
-// parts > 0: `delta` holds float32 partial sums [parts][total_rows][n] (bfloat16 rows only).
+// parts > 0: `delta` holds float32 partial sums [parts][total_rows][n].
 extern "C" int tli_add_rmsnorm(float* resid, const void* delta, const float* weight, void* out,
                                const int* rows, int out_rows, int total_rows, int n, float eps,
                                int dtype, int parts, void* stream) {
     if (out_rows <= 0) return 0;
     if (n <= 0) return tli_fail("add_rmsnorm: bad row size %d", n);
-    if (parts < 0 || (parts > 0 && (dtype != TLI_BF16 || !delta)))
-        return tli_fail("add_rmsnorm: partial sums (%d) go with bfloat16 rows only", parts);
+    if (parts < 0 || (parts > 0 && !delta)) return tli_fail("add_rmsnorm: no partial sums (%d)", parts);
     hipStream_t s = (hipStream_t)stream;
     if (dtype == TLI_F32)
-        launch_add_rmsnorm<float>(resid, delta, 0, weight, (float*)out, rows, out_rows, total_rows, n, eps, s);
+        launch_add_rmsnorm<float>(resid, delta, parts, weight, (float*)out, rows, out_rows, total_rows, n, eps, s);
     else if (dtype == TLI_BF16)
         launch_add_rmsnorm<bf16_t>(resid, delta, parts, weight, (bf16_t*)out, rows, out_rows, total_rows, n,
                                    eps, s);

@@ -22,41 +22,11 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 #define GF_RANGES 8
 
-// RT tiles of 16 rows of W and MT tiles of 16 rows of x a workgroup; U steps of 16 k are asked for together, the next U
-// while these are multiplied.  GATED: W holds N gate rows, then N up rows; tiles come in pairs of both and y is
-// act(gate) * up * scale.
-// CT < 16 (one tile of W): a workgroup takes CT of a tile's 16 columns, its lanes of the others repeating them, so that a matrix
-// of few rows is read by more compute units.
-template <int RT, int MT, int U, bool GATED, int CT = 16>
-__global__ void __launch_bounds__(GF_RANGES * 64)
-gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int M, int N, int K,
-                GateOut gate) {
-    constexpr int TOGETHER = GATED ? 2 : 1;                    // row tiles that are finished together
-    __shared__ float red[GF_RANGES][TOGETHER * MT][64][4];
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-    const int r = lane % 16, c = lane / 16;
-    static_assert(CT == 16 || RT == 1, "part of one tile");
-    const int n_base = blockIdx.x * (CT == 16 ? 16 * RT / TOGETHER : CT), m_base = blockIdx.y * (16 * MT);
-
-    f32x4 acc[RT][MT];
-#pragma unroll
-    for (int t = 0; t < RT; ++t)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) acc[t][m] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-    // rows past the end read a valid one and are never stored
-    const float* w_row[RT];
-    const float* x_row[MT];
-#pragma unroll
-    for (int t = 0; t < RT; ++t) {
-        const int n = min(n_base + (t / TOGETHER) * 16 + r % CT, N - 1);
-        w_row[t] = w + (size_t)(n + (GATED && (t & 1) ? N : 0)) * K + c * 4;
-    }
-#pragma unroll
-    for (int m = 0; m < MT; ++m) x_row[m] = x + (size_t)min(m_base + m * 16 + r, M - 1) * K + c * 4;
-
-    const int steps = (K + 15) / 16, each = (steps + GF_RANGES - 1) / GF_RANGES;
-    const int first = min(wave * each, steps), count = min(steps - first, each);
+// acc[t][m] += the products of `count` steps of 16 k from step `first` on; w_row and x_row point at this lane's four k of step 0.
+// U steps are asked for together, the next U while these are multiplied.
+template <int RT, int MT, int U>
+__device__ __forceinline__ void add_range(f32x4 (&acc)[RT][MT], const float* const (&w_row)[RT], const float* const (&x_row)[MT], int first,
+                                          int count, int K, int c) {
     // the last step of k may be partial: it is left to the end, where loads are looked after one by one
     const int whole = min(count, max(0, K / 16 - first));
     const int batches = whole / U;
@@ -116,6 +86,44 @@ gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float*
         for (int t = 0; t < RT; ++t) a[0][0][t] = in ? *reinterpret_cast<const f32x4*>(w_row[t] + k) : zero;
         multiply(0, 0);
     }
+}
+
+// RT tiles of 16 rows of W and MT tiles of 16 rows of x a workgroup; U steps of 16 k are asked for together, the next U
+// while these are multiplied.  GATED: W holds N gate rows, then N up rows; tiles come in pairs of both and y is
+// act(gate) * up * scale.
+// CT < 16 (one tile of W): a workgroup takes CT of a tile's 16 columns, its lanes of the others repeating them, so that a matrix
+// of few rows is read by more compute units.
+template <int RT, int MT, int U, bool GATED, int CT = 16>
+__global__ void __launch_bounds__(GF_RANGES * 64)
+gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int M, int N, int K,
+                GateOut gate) {
+    constexpr int TOGETHER = GATED ? 2 : 1;                    // row tiles that are finished together
+    __shared__ float red[GF_RANGES][TOGETHER * MT][64][4];
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int r = lane % 16, c = lane / 16;
+    static_assert(CT == 16 || RT == 1, "part of one tile");
+    const int n_base = blockIdx.x * (CT == 16 ? 16 * RT / TOGETHER : CT), m_base = blockIdx.y * (16 * MT);
+
+    f32x4 acc[RT][MT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    // rows past the end read a valid one and are never stored
+    const float* w_row[RT];
+    const float* x_row[MT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        const int n = min(n_base + (t / TOGETHER) * 16 + r % CT, N - 1);
+        w_row[t] = w + (size_t)(n + (GATED && (t & 1) ? N : 0)) * K + c * 4;
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) x_row[m] = x + (size_t)min(m_base + m * 16 + r, M - 1) * K + c * 4;
+
+    const int steps = (K + 15) / 16, each = (steps + GF_RANGES - 1) / GF_RANGES;
+    const int first = min(wave * each, steps), count = min(steps - first, each);
+    add_range<RT, MT, U>(acc, w_row, x_row, first, count, K, c);
 
 #pragma unroll
     for (int t0 = 0; t0 < RT; t0 += TOGETHER) {
@@ -144,6 +152,44 @@ gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float*
                 store4(y + (size_t)row * ld + n0, s[0], N - n0, (ld & 3) == 0 && ((uintptr_t)y & 15) == 0);
             }
         }
+    }
+}
+
+// The ranges' sums themselves, [range][M][N], for a reader that adds them in the ranges' order (the same bits as the kernel above): a wave
+// a tile of 16 columns and range, GF_PART_WAVES tiles of a range a workgroup, whose waves share the pieces of x that they read.
+// What it is for: 1,024 columns are 64 tiles, which the kernel above reaches all compute units with only by giving a workgroup a quarter of
+// one, so that three quarters of its matrix instructions and loads repeat.  Here the tiles' eight ranges are 512 waves that repeat nothing,
+// wait for no other wave, and have all their loads in flight (two batches of eight steps).  What bounds it: the launch and one
+// trip to memory; 4,096 k: 3.1 TB/s, a wave's 128 instructions of 32 cycles one after the other.
+// Measured in a recorded chain, cold weights, us, with the norm that adds the sums against the kernel above and the norm: 5 rows, 1,024 columns of
+// k 1,024 7.5 -> 6.0, of 4,096 15.5 -> 8.5; 16 rows 8.6 -> 6.3, 19.4 -> 9.5; 32 rows 10.8 -> 7.2, 26.8 -> 12.4; 1,536 of 1,024 alone 5.4 -> 4.1 (5 rows)
+// and 8.8 -> 6.1 (32).  Non-temporal loads of W are no faster.
+#define GF_PART_WAVES 2
+template <int MT, int U>
+__global__ void __launch_bounds__(GF_PART_WAVES * 64)
+gemm_f32_ranges_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ parts, int M, int N, int K) {
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int r = lane % 16, c = lane / 16;
+    const int n_base = (blockIdx.x * GF_PART_WAVES + wave) * 16, range = blockIdx.y;
+    if (n_base >= N) return;
+    f32x4 acc[1][MT];
+    const float* w_row[1] = {w + (size_t)min(n_base + r, N - 1) * K + c * 4};       // rows past the end read a valid one and are never stored
+    const float* x_row[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        acc[0][m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        x_row[m] = x + (size_t)min(m * 16 + r, M - 1) * K + c * 4;
+    }
+    const int steps = (K + 15) / 16, each = (steps + GF_RANGES - 1) / GF_RANGES;
+    const int first = min(range * each, steps), count = min(steps - first, each);
+    add_range<1, MT, U>(acc, w_row, x_row, first, count, K, c);
+    const int n0 = n_base + c * 4;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int row = m * 16 + r;
+        if (row >= M || n0 >= N) continue;
+        const float s[4] = {acc[0][m][0], acc[0][m][1], acc[0][m][2], acc[0][m][3]};
+        store4(parts + ((size_t)range * M + row) * N + n0, s, N - n0, N % 4 == 0);
     }
 }
 
@@ -200,4 +246,22 @@ extern "C" int tli_gemm_f32(const void* x, const void* w, void* y, int M, int N,
     const long blocks = tiles * ((M + 63) / 64);
     if (blocks >= 2 * units || gated) return launch_f32<2, 4, 2>(xp, wp, yp, M, N, K, gate, s);
     return launch_f32<1, 4, 2>(xp, wp, yp, M, N, K, gate, s);
+}
+
+// How many planes of partial sums tli_gemm_f32_ranges leaves, or 0 where it does not take the product: up to 32 rows (more do not lie in a
+// wave's registers beside W) and no more outputs than the kernel above gives parts of tiles for (with whole tiles the sums cost their
+// reader more than they save: eight planes to read instead of one).
+extern "C" int tli_gemm_f32_ranges_of(int M, int N) {
+    return M > 0 && M <= 32 && N > 0 && ((long)N + 15) / 16 * 2 <= tli_compute_units() ? GF_RANGES : 0;
+}
+
+// parts[GF_RANGES][M][N]: y of tli_gemm_f32 is their sum in order, from zero.
+extern "C" int tli_gemm_f32_ranges(const void* x, const void* w, void* parts, int M, int N, int K, void* stream) {
+    if (!tli_gemm_f32_ranges_of(M, N)) return tli_fail("gemm_f32_ranges: %d rows of %d outputs are not taken", M, N);
+    if (K <= 0 || K % 4) return tli_fail("gemm_f32_ranges: K = %d must be a positive multiple of 4", K);
+    if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)parts) & 15) return tli_fail("gemm_f32_ranges: operands must be 16-byte aligned");
+    const dim3 grid((unsigned)((N + 16 * GF_PART_WAVES - 1) / (16 * GF_PART_WAVES)), GF_RANGES);
+    if (M <= 16) gemm_f32_ranges_kernel<1, 8><<<grid, GF_PART_WAVES * 64, 0, (hipStream_t)stream>>>((const float*)x, (const float*)w, (float*)parts, M, N, K);
+    else gemm_f32_ranges_kernel<2, 8><<<grid, GF_PART_WAVES * 64, 0, (hipStream_t)stream>>>((const float*)x, (const float*)w, (float*)parts, M, N, K);
+    return tli_check_launch("gemm_f32_ranges");
 }

@@ -3,6 +3,21 @@
 #pragma once
 #include "common.h"
 
+// One element of a float32 product: `at` in the product itself (planes 1), or the sum of its partial sums, `plane` elements apart, in their
+// order from zero (eight are asked for together; past the last it is the last again, which is not added).
+__device__ __forceinline__ float sum_planes(const float* __restrict__ at, int planes, size_t plane) {
+    if (planes == 1) return at[0];
+    float a = 0.f;
+    for (int s = 0; s < planes; s += 8) {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = at[(size_t)min(s + k, planes - 1) * plane];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) a = s + k < planes ? a + v[k] : a;
+    }
+    return a;
+}
+
 // Sum of the partial products in split order.  gated: output column j of [M, N/2] takes
 // gate column (j/16)*32 + j%16 and up column 16 further.
 template <typename TO>

@@ -10,14 +10,18 @@
 // q goes to its own [rows, heads*head_dim] buffer.  The cache layout differs from
 // the reference's [page][slot][kv_dim] (kernels/src/paged_attention_cuda.cu:58-67):
 // here the slots of one head in one page are contiguous.
-#include "common.h"
+#include "gemm_reduce.h"
 
 #define QKV_MAX_HEAD_DIM 512
 #define QKV_WAVES 4
 
+// an element of a row, or the sum of its `planes` partial sums (float32 only)
+__device__ __forceinline__ float raw_value(const float* p, int planes, size_t plane) { return sum_planes(p, planes, plane); }
+__device__ __forceinline__ bf16_t raw_value(const bf16_t* p, int, size_t) { return *p; }
+
 template <typename T>
 __global__ void qkv_to_cache_kernel(
-    const T* __restrict__ qkv, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache,
+    const T* __restrict__ qkv, int planes, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache,
     const int* __restrict__ positions, const int* __restrict__ seq_of_row,
     const int* __restrict__ tables, int table_width, int page_size, int num_pages,
     int heads, int kv_heads, int head_dim,
@@ -31,6 +35,7 @@ __global__ void qkv_to_cache_kernel(
     const int stride = q_dim + 2 * kv_dim;
     const int pos = positions[row];
     const T* src_row = qkv + (size_t)row * stride;
+    const size_t plane = (size_t)gridDim.x * stride;
 
     // where this row's keys and values go
     size_t cache_base = 0, v_base = 0;
@@ -60,7 +65,7 @@ __global__ void qkv_to_cache_kernel(
         const int g = h - heads - kv_heads;
         const T* vsrc = src_row + q_dim + kv_dim + (size_t)g * head_dim;
         for (int d = lane; d < head_dim; d += TLI_WAVE)
-            v_cache[v_base + ((size_t)g * head_dim + d) * page_size] = cache_value(vsrc[d]);
+            v_cache[v_base + ((size_t)g * head_dim + d) * page_size] = cache_value(raw_value(vsrc + d, planes, plane));
         return;
     }
     {
@@ -70,7 +75,7 @@ __global__ void qkv_to_cache_kernel(
         const float eps = is_q ? q_eps : k_eps;
         float ss = 0.f;
         for (int i = lane; i < head_dim; i += TLI_WAVE) {
-            const float v = to_f32(src[i]);
+            const float v = to_f32(raw_value(src + i, planes, plane));
             x[i] = v;
             ss += v * v;
         }
@@ -469,9 +474,10 @@ extern "C" int tli_values_to_cache(
     return tli_check_launch("values_to_cache");
 }
 
-// skip_values: the values are written by tli_values_to_cache instead.
+// skip_values: the values are written by tli_values_to_cache instead.  planes > 1 (float32): qkv holds so many partial sums of the
+// projections, [planes][rows][..].
 extern "C" int tli_qkv_to_cache(
-    const void* qkv, void* q_out, void* k_cache, void* v_cache, const int* positions,
+    const void* qkv, int planes, void* q_out, void* k_cache, void* v_cache, const int* positions,
     const int* seq_of_row, const int* tables, int table_width, int page_size, int num_pages,
     int rows, int heads, int kv_heads, int head_dim,
     const float* q_norm_w, float q_eps, const float* k_norm_w, float k_eps,
@@ -485,6 +491,7 @@ extern "C" int tli_qkv_to_cache(
         return tli_fail("qkv_to_cache: rotary_dim %d must be even and at most head_dim %d", rotary_dim, head_dim);
     if (write_cache && (page_size <= 0 || table_width <= 0 || num_pages <= 0))
         return tli_fail("qkv_to_cache: bad cache geometry");
+    if (planes < 1 || (planes > 1 && dtype != TLI_F32)) return tli_fail("qkv_to_cache: %d partial sums (float32 only)", planes);
     hipStream_t s = (hipStream_t)stream;
     const int threads = QKV_WAVES * TLI_WAVE;
     const int units = heads + 2 * kv_heads;
@@ -513,12 +520,12 @@ extern "C" int tli_qkv_to_cache(
     }
     if (dtype == TLI_F32)
         qkv_to_cache_kernel<float><<<grid, threads, 0, s>>>(
-            (const float*)qkv, (float*)q_out, (float*)k_cache, (float*)v_cache, positions, seq_of_row,
+            (const float*)qkv, planes, (float*)q_out, (float*)k_cache, (float*)v_cache, positions, seq_of_row,
             tables, table_width, page_size, num_pages, heads, kv_heads, head_dim, q_norm_w, q_eps,
             k_norm_w, k_eps, cos_table, sin_table, rotary_dim, table_positions, write_cache);
     else if (dtype == TLI_BF16)
         qkv_to_cache_kernel<bf16_t><<<grid, threads, 0, s>>>(
-            (const bf16_t*)qkv, (bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, positions, seq_of_row,
+            (const bf16_t*)qkv, 1, (bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, positions, seq_of_row,
             tables, table_width, page_size, num_pages, heads, kv_heads, head_dim, q_norm_w, q_eps,
             k_norm_w, k_eps, cos_table, sin_table, rotary_dim, table_positions, write_cache);
     else

@@ -26,8 +26,9 @@ class KernelError(RuntimeError):
 
 class PendingProduct:
     """x W^T not run yet: what ``linear(..., deferred=True)`` returns for a decode step's
-    few rows.  ``add_rmsnorm(..., lazy=True)`` runs it with the residual sum and the
-    norm taken into the product; anything else runs it as it is (``resolve``)."""
+    few rows.  ``add_rmsnorm(..., lazy=True)`` runs a bfloat16 one with the residual sum and the
+    norm taken into the product, ``add_rmsnorm`` and ``qkv_attention`` a float32 one as partial sums
+    that they add (``_f32_ranges``); anything else runs it as it is (``resolve``)."""
 
     def __init__(self, x: torch.Tensor, matrix):
         self.x, self.matrix = x, matrix
@@ -79,12 +80,14 @@ def load_library():
         "tli_feed_tokens": [P, P, P, I, I, P],
         "tli_add_rmsnorm": [P, P, P, P, P, I, I, I, F, I, I, P],
         "tli_swiglu": [P, P, I, I, I, F, F, I, F, I, P],
-        "tli_qkv_to_cache": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, F, P, F, P, P, I, I, I, I, I, P],
+        "tli_qkv_to_cache": [P, I, P, P, P, P, P, P, I, I, I, I, I, I, I, P, F, P, F, P, P, I, I, I, I, I, P],
         "tli_values_to_cache": [P, P, P, P, I, I, P, I, I, I, I, I, I, P],
         "tli_keys_values_to_cache": [P, P, P, P, P, I, I, P, I, I, I, I, I, I, P, F, P, P, I, P],
         "tli_attention_plain": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, I, P],
         "tli_attention_f32_takes": [I, I],
         "tli_attention_f32": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, P],
+        "tli_gemm_f32_ranges_of": [I, I],
+        "tli_gemm_f32_ranges": [P, P, P, I, I, I, P],
         "tli_gemm_plain": [P, P, P, I, I, I, I, I, I, P],
         "tli_gemm_f32": [P, P, P, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, I, I, F, I, P],
@@ -223,6 +226,7 @@ class HipOps:
     name = "hip-gfx950"
     MAX_HEAD_DIM = 512
     SKINNY_ROWS = 64
+    F32_RANGES_ROWS = 32         # float32 products of so many rows and few outputs are left as the sums of their ranges of k
     MID_ROWS_FROM = 17           # from this many rows the x-sharing kernel multiplies,
     MID_ROWS_TO = 128            # up to this many
     MID_ROWS_TO_PLAIN = 256      # a product without a gate: up to this many (two blocks of 128 rows side by side)
@@ -251,6 +255,7 @@ class HipOps:
         self.lib = load_library()
         with torch.cuda.device(self.device):
             self.DECODE_WORKGROUPS = int(self.lib.tli_device_compute_units())
+            self.F32_RANGES = int(self.lib.tli_gemm_f32_ranges_of(1, 16))
         self._held_stream = None
         self.force_plain = False     # tests: run the plain attention kernel for bfloat16 too
         self.plain_products = False  # every matrix product through the plain kernel
@@ -408,12 +413,15 @@ class HipOps:
         self._want(resid, "residual", torch.float32)
         self._want(weight, "norm weight", torch.float32, (n,))
         if isinstance(delta, PendingProduct):
-            if lazy and rows is None and not self.separate_norms:
+            if delta.dtype == torch.float32:
+                delta = self._f32_ranges(delta) if out_dtype == torch.float32 else self.resolve(delta)
+            elif lazy and rows is None and not self.separate_norms:
                 return self._product_into_residual(delta, resid, weight, eps)
-            delta = self.resolve(delta)
+            else:
+                delta = self.resolve(delta)
         parts = 0
         if isinstance(delta, DeferredSum):
-            if delta.dtype != out_dtype or out_dtype != torch.bfloat16:
+            if delta.dtype != out_dtype:
                 delta = self.resolve(delta)
             else:
                 parts = delta.parts.shape[0]
@@ -477,6 +485,10 @@ class HipOps:
         if K != K2:
             raise KernelError(f"linear: input has {K} columns, the matrix {K2}")
         self._want(x, "linear input")
+        if ((deferred or sums_only) and x.dtype == torch.float32 and 0 < M <= self.F32_RANGES_ROWS and tiled is None
+                and out_dtype in (None, torch.float32) and not self.separate_norms and (N + 15) // 16 * 2 <= self.DECODE_WORKGROUPS
+                and self._f32_product_takes(x, getattr(w, "w", w))):
+            return PendingProduct(x, w)
         w_dtype = getattr(matrix, "dtype", None) or matrix.w.dtype
         if x.dtype != w_dtype:
             raise KernelError(f"linear: input is {x.dtype}, the matrix {w_dtype}")
@@ -536,6 +548,15 @@ class HipOps:
         """Whether the float32 product on the matrix cores takes these operands: rows of whole 16-byte pieces."""
         return (x.dtype == torch.float32 and w.dtype == torch.float32 and x.shape[1] % 4 == 0
                 and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+    def _f32_ranges(self, p: PendingProduct) -> DeferredSum:
+        """A float32 product of few rows as the sums of its ranges of k, whose sum in order is what ``linear`` gives."""
+        x, w = p.x, getattr(p.matrix, "w", p.matrix)
+        M, N = p.shape
+        self._want(w, "linear matrix", torch.float32, (N, x.shape[1]))
+        parts = torch.empty((self.F32_RANGES, M, N), dtype=torch.float32, device=self.device)
+        self._call(self.lib.tli_gemm_f32_ranges, x.data_ptr(), w.data_ptr(), parts.data_ptr(), M, N, x.shape[1], self._stream())
+        return DeferredSum(parts, torch.float32)
 
     def _product_into_residual(self, p: PendingProduct, resid, weight, eps) -> NormedRows:
         """resid += x W^T, and the rows of the norm that follows, its factor still owed."""
@@ -737,10 +758,15 @@ class HipOps:
     def qkv_to_cache(self, qkv, step, cache, heads, kv_heads, head_dim, q_norm, k_norm, rotary, queries=True):
         """Norms and rotation of q and k, k and v into the cache; returns q.  Without
         ``queries`` only the keys and values are done (bfloat16 heads of 64, 128, 256),
-        the values by a kernel of their own that writes runs of slots."""
+        the values by a kernel of their own that writes runs of slots.  ``qkv`` may be a float32 ``DeferredSum``."""
         T = step.num_rows
         q_dim, kv_dim = heads * head_dim, kv_heads * head_dim
-        self._want(qkv, "qkv", None, (T, q_dim + 2 * kv_dim))
+        planes = 1
+        if isinstance(qkv, DeferredSum):
+            planes, qkv = qkv.parts.shape[0], qkv.parts
+            self._want(qkv, "partial sums of qkv", torch.float32, (planes, T, q_dim + 2 * kv_dim))
+        else:
+            self._want(qkv, "qkv", None, (T, q_dim + 2 * kv_dim))
         q = torch.empty((T, q_dim), dtype=qkv.dtype, device=self.device) if queries else None
         qw, qe = q_norm if q_norm is not None else (None, 0.0)
         kw, ke = k_norm if k_norm is not None else (None, 0.0)
@@ -768,7 +794,7 @@ class HipOps:
                        step.seq_start.data_ptr(), step.num_seqs, T, tab_ptr, width, page, pages, heads, kv_heads,
                        head_dim, _ptr(kw), float(ke), _ptr(cos), _ptr(sin), npos, self._stream())
             return None
-        self._call(self.lib.tli_qkv_to_cache, qkv.data_ptr(), _ptr(q), k_ptr, v_ptr,
+        self._call(self.lib.tli_qkv_to_cache, qkv.data_ptr(), planes, _ptr(q), k_ptr, v_ptr,
                    step.positions.data_ptr(), step.seq_of_row.data_ptr(), tab_ptr, width, page, pages,
                    T, heads, kv_heads, head_dim, _ptr(qw), float(qe), _ptr(kw), float(ke),
                    _ptr(cos), _ptr(sin), rd, npos, write, 0 if queries else 1, _dtype_code(qkv.dtype),
@@ -846,6 +872,11 @@ class HipOps:
         row a sequence) does all of it in the attention kernel where the sizes allow;
         other steps run qkv_to_cache and paged_attention.  ``qkv`` may be a ``DeferredSum``:
         the kernel of a decode step adds the partial sums itself."""
+        if isinstance(qkv, PendingProduct):
+            qkv = self._f32_ranges(qkv) if qkv.dtype == torch.float32 else self.resolve(qkv)
+        if qkv.dtype == torch.float32:
+            q = self.qkv_to_cache(qkv, step, cache, heads, kv_heads, head_dim, q_norm, k_norm, rotary)
+            return self.paged_attention(q, step, cache, heads, kv_heads, head_dim, scale, window)
         sums = None
         if isinstance(qkv, DeferredSum):
             sums = qkv
