@@ -79,13 +79,17 @@ def test_attention_from_projections_left_in_ranges(ops, case):
         step.cache.v.copy_(v0)
         ops.unfused_decode = apart
         try:
-            out = ops.qkv_attention(qkv, step, step.cache, heads, kv_heads, hd, qn, kn, rotary, hd ** -0.5, window)
+            if qkv is None:
+                q = ops.qkv_to_cache(product, step, step.cache, heads, kv_heads, hd, qn, kn, rotary)
+                out = ops.paged_attention(q, step, step.cache, heads, kv_heads, hd, hd ** -0.5, window)
+            else:
+                out = ops.qkv_attention(qkv, step, step.cache, heads, kv_heads, hd, qn, kn, rotary, hd ** -0.5, window)
         finally:
             ops.unfused_decode = False
         return out, step.cache.k.clone(), step.cache.v.clone()
     product = ops.linear(x, w)
     assert not bool(product[0, -hd:].isfinite().any())
-    want = run(product, True)
+    want = run(None, True)
     assert (not torch.equal(want[1], k0)) == writes
     pending = ops.linear(x, w, sums_only=True)
     for qkv in (product, pending, ops._f32_ranges(pending)):

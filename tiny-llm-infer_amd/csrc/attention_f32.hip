@@ -12,16 +12,66 @@
 // of 600 159 -> 35 and 525 -> 135; a prompt of 32 tokens 12.2 -> 12.2 and 14.8 -> 12.6, of 512 441 -> 109 and 1,297 -> 394, of 2,048
 // 5.74 -> 1.46 and 19.6 -> 5.63 ms; heads of 192 and 256 1.04 to 5 times.
 // The order of additions depends on the row's first and last key alone.
-#include "common.h"
+#include "gemm_reduce.h"
 #include <type_traits>
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 #define AF_WAVES 4
 
-template <int DH>            // head_dim / 64
+// The projections of a decode step's rows, [planes][rows][(heads + 2 kv_heads) D] (planes > 1: partial sums), and what is done to them.
+struct RawRows {
+    const float* qkv;
+    int planes;
+    const float *q_norm_w, *k_norm_w;
+    float q_eps, k_eps;
+    const float *cos_table, *sin_table;
+    int rotary_dim, table_positions;
+    int write_cache;
+};
+
+// x[D] in LDS: norm (weight `nw` or null) and rotation of a head that this wavefront takes from `src`, as qkv_to_cache_kernel does them.
+template <int DH>
+__device__ __forceinline__ void head_of_raw_row(float* x, const float* src, size_t plane, const RawRows& raw, const float* nw, float eps,
+                                                const float* cos_row, const float* sin_row, int lane) {
+    constexpr int D = DH * 64;
+    float v[DH], w[DH], ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < DH; ++e) {
+        v[e] = sum_planes(src + e * 64 + lane, raw.planes, plane);
+        w[e] = nw ? nw[e * 64 + lane] : 0.f;
+    }
+#pragma unroll
+    for (int e = 0; e < DH; ++e) ss += v[e] * v[e];
+    if (nw) {
+        const float scale = 1.0f / sqrtf(wave_sum(ss) / (float)D + eps);
+#pragma unroll
+        for (int e = 0; e < DH; ++e) v[e] = w[e] * v[e] * scale;
+    }
+#pragma unroll
+    for (int e = 0; e < DH; ++e) x[e * 64 + lane] = v[e];
+    if (!cos_row) return;
+    wave_lds_sync();
+    const int half = raw.rotary_dim / 2;
+#pragma unroll
+    for (int e = 0; e < DH; ++e) {
+        const int i = e * 64 + lane;
+        if (i < half) v[e] = rotate_first_half(v[e], x[i + half], cos_row[i], sin_row[i]);
+        else if (i < raw.rotary_dim) v[e] = rotate_second_half(v[e], x[i - half], cos_row[i - half], sin_row[i - half]);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int e = 0; e < DH; ++e) x[e * 64 + lane] = v[e];
+}
+
+// RAW: decode steps (one row a sequence) from the projections: every workgroup makes its query and its row's own key and value, the first
+// head of a group writes these into the cache, and every head takes them from LDS, not from the cache, so that nothing waits for a store.
+// The same bits as qkv_to_cache and the kernel without RAW, which is two launches and a trip of q through memory; most of either is launch and
+// latency.  In a recorded chain, 16 heads of 64, projections as eight partial sums, us: 1 row of 30 keys 6.4 -> 4.9, 5 rows of 52 6.9 -> 5.4, 8 of
+// 200 10.8 -> 9.5, 1 of 1,000 29.0 -> 28.6.
+template <int DH, bool RAW>            // head_dim / 64
 __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
-    const float* __restrict__ q, float* __restrict__ out, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
+    const float* __restrict__ q, float* __restrict__ out, float* __restrict__ k_cache, float* __restrict__ v_cache, RawRows raw,
     const int* __restrict__ positions, const int* __restrict__ seq_of_row, const int* __restrict__ tables, int table_width,
     int page_size, int num_pages, int heads, int kv_heads, float scale, int window) {
     constexpr int D = DH * 64;
@@ -40,7 +90,37 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
 
     // this lane's quarter of the query: elements 16 i + 4 c .. + 4
     f32x4 qv[DH * 4];
-    {
+    __shared__ __attribute__((aligned(16))) float own_s[RAW ? 3 : 1][RAW ? D : 4];      // RAW: the query, the row's own key and value
+    const bool own = RAW && raw.write_cache;
+    if constexpr (RAW) {
+        const int width = (heads + 2 * kv_heads) * D;
+        const float* src = raw.qkv + (size_t)row * width;
+        const size_t plane = (size_t)gridDim.x * width;
+        const bool turned = raw.cos_table && pos >= 0 && pos < raw.table_positions;
+        const float* cos_row = turned ? raw.cos_table + (size_t)pos * (raw.rotary_dim / 2) : nullptr;
+        const float* sin_row = turned ? raw.sin_table + (size_t)pos * (raw.rotary_dim / 2) : nullptr;
+        const int page = own && head % (heads / kv_heads) == 0 ? table[pos / page_size] : -1;
+        const bool store = page >= 0 && page < num_pages;
+        if (wave == 0) head_of_raw_row<DH>(own_s[0], src + (size_t)head * D, plane, raw, raw.q_norm_w, raw.q_eps, cos_row, sin_row, lane);
+        if (wave == 1 && own) {
+            head_of_raw_row<DH>(own_s[1], src + (size_t)(heads + g) * D, plane, raw, raw.k_norm_w, raw.k_eps, cos_row, sin_row, lane);
+            if (store)
+#pragma unroll
+                for (int e = 0; e < DH; ++e)                    // (a lane's own elements)
+                    k_cache[(size_t)page * page_stride + ((size_t)g * page_size + pos % page_size) * D + e * 64 + lane] = own_s[1][e * 64 + lane];
+        }
+        if (wave == 2 && own) {
+#pragma unroll
+            for (int e = 0; e < DH; ++e) {
+                const float v = cache_value(sum_planes(src + (size_t)(heads + kv_heads + g) * D + e * 64 + lane, raw.planes, plane));
+                own_s[2][e * 64 + lane] = v;
+                if (store) v_cache[(size_t)page * page_stride + ((size_t)g * D + e * 64 + lane) * page_size + pos % page_size] = v;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < DH * 4; ++i) qv[i] = *reinterpret_cast<const f32x4*>(&own_s[0][i * 16 + c * 4]);
+    } else {
         const float* q_row = q + ((size_t)row * heads + head) * D + c * 4;
 #pragma unroll
         for (int i = 0; i < DH * 4; ++i) qv[i] = *reinterpret_cast<const f32x4*>(q_row + i * 16);
@@ -69,6 +149,20 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
             const float* vp = v_head + (size_t)(held ? v_page[u] : 0) * page_stride + (size_t)lane * page_size + (base + 4 * u) % page_size;
 #pragma unroll
             for (int i = 0; i < DH; ++i) vv[i][u] = *reinterpret_cast<const f32x4*>(vp + (size_t)i * 64 * page_size);
+        }
+        if (own && base + 16 > pos) {
+            // the row's own slot, which another workgroup may be writing just now: what was read of it is not used
+            if (t == pos)
+#pragma unroll
+                for (int i = 0; i < DH * 4; ++i) kv[i] = *reinterpret_cast<const f32x4*>(&own_s[RAW ? 1 : 0][(i * 16 + c * 4) % (RAW ? D : 4)]);
+#pragma unroll
+            for (int i = 0; i < DH; ++i) {
+                const float mine = own_s[RAW ? 2 : 0][RAW ? i * 64 + lane : 0];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) vv[i][u][e] = base + 4 * u + e == pos ? mine : vv[i][u][e];
+            }
         }
         f32x4 dot = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -137,12 +231,28 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
     }
 }
 
+template <bool RAW>
+static void launch_attention_f32(dim3 grid, const float* q, float* out, float* k_cache, float* v_cache, const RawRows& raw, const int* positions,
+                                 const int* seq_of_row, const int* tables, int table_width, int page_size, int num_pages, int heads,
+                                 int kv_heads, int head_dim, float scale, int window, hipStream_t s) {
+#define TLI_AF(DH)                                                                                                                         \
+    attention_f32_kernel<DH, RAW><<<grid, AF_WAVES * 64, 0, s>>>(q, out, k_cache, v_cache, raw, positions, seq_of_row, tables, table_width, \
+                                                                 page_size, num_pages, heads, kv_heads, scale, window)
+    switch (head_dim / 64) {
+        case 1: TLI_AF(1); break;
+        case 2: TLI_AF(2); break;
+        case 3: TLI_AF(3); break;
+        default: TLI_AF(4); break;
+    }
+#undef TLI_AF
+}
+
 extern "C" int tli_attention_f32_takes(int head_dim, int page_size) {
     return head_dim > 0 && head_dim % 64 == 0 && head_dim <= 256 && page_size >= 4 && page_size % 4 == 0;
 }
 
 // As tli_attention_plain, float32.
-extern "C" int tli_attention_f32(const void* q, void* out, const void* k_cache, const void* v_cache, const int* positions,
+extern "C" int tli_attention_f32(const void* q, void* out, void* k_cache, void* v_cache, const int* positions,
                                  const int* seq_of_row, const int* tables, int table_width, int page_size, int num_pages, int rows,
                                  int heads, int kv_heads, int head_dim, float scale, int window, void* stream) {
     if (rows <= 0) return 0;
@@ -153,16 +263,43 @@ extern "C" int tli_attention_f32(const void* q, void* out, const void* k_cache, 
     if (table_width <= 0 || num_pages <= 0) return tli_fail("attention_f32: bad cache geometry");
     if (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) return tli_fail("attention_f32: operands must be 16-byte aligned");
     const dim3 grid(rows, heads);
-#define TLI_AF(DH)                                                                                                                 \
-    attention_f32_kernel<DH><<<grid, AF_WAVES * 64, 0, (hipStream_t)stream>>>((const float*)q, (float*)out, (const float*)k_cache, \
-                                                                               (const float*)v_cache, positions, seq_of_row, tables, \
-                                                                               table_width, page_size, num_pages, heads, kv_heads, scale, window)
-    switch (head_dim / 64) {
-        case 1: TLI_AF(1); break;
-        case 2: TLI_AF(2); break;
-        case 3: TLI_AF(3); break;
-        default: TLI_AF(4); break;
-    }
-#undef TLI_AF
+    launch_attention_f32<false>(grid, (const float*)q, (float*)out, (float*)k_cache, (float*)v_cache, RawRows{}, positions, seq_of_row, tables,
+                                table_width, page_size, num_pages, heads, kv_heads, head_dim, scale, window, (hipStream_t)stream);
     return tli_check_launch("attention_f32");
+}
+
+extern "C" int tli_qkv_to_cache(const void* qkv, int planes, void* q_out, void* k_cache, void* v_cache, const int* positions, const int* seq_of_row,
+                                const int* tables, int table_width, int page_size, int num_pages, int rows, int heads, int kv_heads, int head_dim,
+                                const float* q_norm_w, float q_eps, const float* k_norm_w, float k_eps, const float* cos_table,
+                                const float* sin_table, int rotary_dim, int table_positions, int write_cache, int skip_values, int dtype, void* stream);
+
+// From the rows' projections qkv [planes][rows][(heads + 2 kv_heads) head_dim] (planes > 1: partial sums to be added) to the attention's output.
+// `q` null: a decode step (one row a sequence) in one launch.  Else q [rows][heads * head_dim] takes the queries and it is tli_qkv_to_cache,
+// then tli_attention_f32: a row of a portion also reads the keys of the rows before it.
+extern "C" int tli_qkv_attention_f32(const void* qkv, int planes, void* q, void* out, void* k_cache, void* v_cache, const int* positions,
+                                     const int* seq_of_row, const int* tables, int table_width, int page_size, int num_pages, int rows,
+                                     int heads, int kv_heads, int head_dim, const float* q_norm_w, float q_eps, const float* k_norm_w,
+                                     float k_eps, const float* cos_table, const float* sin_table, int rotary_dim, int table_positions,
+                                     int write_cache, float scale, int window, void* stream) {
+    if (rows <= 0) return 0;
+    if (!tli_attention_f32_takes(head_dim, page_size))
+        return tli_fail("qkv_attention_f32: heads of %d (64, 128, 192, 256) or pages of %d slots are not taken", head_dim, page_size);
+    if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || heads > 65535)
+        return tli_fail("qkv_attention_f32: %d heads cannot be grouped over %d kv heads", heads, kv_heads);
+    if (table_width <= 0 || num_pages <= 0 || planes < 1) return tli_fail("qkv_attention_f32: bad cache geometry or planes");
+    if ((cos_table == nullptr) != (sin_table == nullptr)) return tli_fail("qkv_attention_f32: cos without sin");
+    if (cos_table && (rotary_dim <= 0 || rotary_dim % 2 || rotary_dim > head_dim))
+        return tli_fail("qkv_attention_f32: rotary_dim %d must be even and at most head_dim %d", rotary_dim, head_dim);
+    if (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15) return tli_fail("qkv_attention_f32: the cache must be 16-byte aligned");
+    if (q) {
+        const int fault = tli_qkv_to_cache(qkv, planes, q, k_cache, v_cache, positions, seq_of_row, tables, table_width, page_size, num_pages, rows,
+                                           heads, kv_heads, head_dim, q_norm_w, q_eps, k_norm_w, k_eps, cos_table, sin_table, rotary_dim,
+                                           table_positions, write_cache, 0, TLI_F32, stream);
+        return fault ? fault : tli_attention_f32(q, out, k_cache, v_cache, positions, seq_of_row, tables, table_width, page_size, num_pages, rows,
+                                                 heads, kv_heads, head_dim, scale, window, stream);
+    }
+    const RawRows raw{(const float*)qkv, planes, q_norm_w, k_norm_w, q_eps, k_eps, cos_table, sin_table, rotary_dim, table_positions, write_cache};
+    launch_attention_f32<true>(dim3(rows, heads), nullptr, (float*)out, (float*)k_cache, (float*)v_cache, raw, positions, seq_of_row, tables,
+                               table_width, page_size, num_pages, heads, kv_heads, head_dim, scale, window, (hipStream_t)stream);
+    return tli_check_launch("qkv_attention_f32");
 }

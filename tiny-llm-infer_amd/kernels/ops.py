@@ -86,6 +86,7 @@ def load_library():
         "tli_attention_plain": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, I, P],
         "tli_attention_f32_takes": [I, I],
         "tli_attention_f32": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, P],
+        "tli_qkv_attention_f32": [P, I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, F, P, F, P, P, I, I, I, F, I, P],
         "tli_gemm_f32_ranges_of": [I, I],
         "tli_gemm_f32_ranges": [P, P, P, I, I, I, P],
         "tli_gemm_plain": [P, P, P, I, I, I, I, I, I, P],
@@ -875,8 +876,7 @@ class HipOps:
         if isinstance(qkv, PendingProduct):
             qkv = self._f32_ranges(qkv) if qkv.dtype == torch.float32 else self.resolve(qkv)
         if qkv.dtype == torch.float32:
-            q = self.qkv_to_cache(qkv, step, cache, heads, kv_heads, head_dim, q_norm, k_norm, rotary)
-            return self.paged_attention(q, step, cache, heads, kv_heads, head_dim, scale, window)
+            return self._qkv_attention_f32(qkv, step, cache, heads, kv_heads, head_dim, q_norm, k_norm, rotary, scale, window)
         sums = None
         if isinstance(qkv, DeferredSum):
             sums = qkv
@@ -926,6 +926,32 @@ class HipOps:
                    1 if cache.writes else 0, float(scale), int(window or 0), splits, per_split,
                    None if sums is None else sums.parts.data_ptr(), 0 if sums is None else sums.parts.shape[0],
                    self._stream())
+        return out
+
+    def _qkv_attention_f32(self, qkv, step, cache, heads, kv_heads, head_dim, q_norm, k_norm, rotary, scale, window):
+        """``qkv_attention`` in float32: one call where the sizes allow, which is one launch for a decode step."""
+        T, sums = step.num_rows, isinstance(qkv, DeferredSum)
+        planes, raw = (qkv.parts.shape[0], qkv.parts) if sums else (1, qkv)
+        kc, vc = (cache.record("k"), cache.record("v")) if cache is not None else (None, None)
+        if (cache is None or self.force_plain or not self.lib.tli_attention_f32_takes(head_dim, cache.group.page_size)
+                or (kc.data_ptr() | vc.data_ptr()) % 16):
+            q = self.qkv_to_cache(qkv, step, cache, heads, kv_heads, head_dim, q_norm, k_norm, rotary)
+            return self.paged_attention(q, step, cache, heads, kv_heads, head_dim, scale, window)
+        g, width = cache.group, (heads + 2 * kv_heads) * head_dim
+        self._want(raw, "partial sums of qkv" if sums else "qkv", torch.float32, (planes, T, width) if sums else (T, width))
+        self._check_cache(kc, vc, g, kv_heads, head_dim, torch.float32, step)
+        qw, qe = q_norm if q_norm is not None else (None, 0.0)
+        kw, ke = k_norm if k_norm is not None else (None, 0.0)
+        for w in (qw, kw):
+            if w is not None:
+                self._want(w, "head norm weight", torch.float32, (head_dim,))
+        cos, sin, rd = self._rotary(rotary, step) if rotary is not None else (None, None, 0)
+        out = torch.empty((T, heads * head_dim), dtype=torch.float32, device=self.device)
+        q = torch.empty_like(out) if step.max_rows_per_seq != 1 or self.unfused_decode else None
+        self._call(self.lib.tli_qkv_attention_f32, raw.data_ptr(), planes, _ptr(q), out.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                   step.positions.data_ptr(), step.seq_of_row.data_ptr(), g.tables.data_ptr(), g.table_width, g.page_size, kc.shape[0], T,
+                   heads, kv_heads, head_dim, _ptr(qw), float(qe), _ptr(kw), float(ke), _ptr(cos), _ptr(sin), rd,
+                   0 if cos is None else cos.shape[0], 1 if cache.writes else 0, float(scale), int(window or 0), self._stream())
         return out
 
     def _qkv_attention_prefill(self, qkv, step, cache, heads, kv_heads, head_dim, q_norm, k_norm, rotary,
