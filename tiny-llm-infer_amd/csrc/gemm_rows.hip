@@ -65,6 +65,12 @@ __device__ __forceinline__ void rows_wait_fragments(Pack16r (&a)[RT][4], int j) 
         asm volatile("s_waitcnt vmcnt(%2)" : "+v"(a[0][j].q), "+v"(a[1][j].q) : "n"(N));
 }
 
+// Workgroups that a die gets of `row_blocks` (up to a chunk) of row blocks: the whole column groups that are its own, and its share of the
+// others (see the kernel).
+__host__ __device__ static inline int rows_turns(int row_blocks, int col_groups) {
+    return col_groups / TLI_DIES * row_blocks + (col_groups % TLI_DIES * row_blocks + TLI_DIES - 1) / TLI_DIES;
+}
+
 // RT column tiles a wave, WAVES waves side by side, MT row tiles (ROWS = 16 MT), x fragments
 // taken MH row tiles at a time.  GATED: the column tiles alternate between a gate and an up
 // matrix (tiled = 2 of tli_gemm_skinny_bf16) and y is [M, N/2] = silu(gate) * up.
@@ -100,15 +106,15 @@ gemm_rows_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, bf1
     constexpr int CHUNK = 2048 / ROWS;
     const int row_blocks = (M + ROWS - 1) / ROWS;
     const int col_groups = (n_tiles + RT * WAVES - 1) / (RT * WAVES);
-    const int groups_a_die = (col_groups + TLI_DIES - 1) / TLI_DIES;
     const int die = blockIdx.x % TLI_DIES, turn = blockIdx.x / TLI_DIES;
-    const int chunk = turn / (CHUNK * groups_a_die), in_chunk = turn % (CHUNK * groups_a_die);
-    const int chunk_rows = min(CHUNK, row_blocks - chunk * CHUNK);      // row blocks of this chunk (the last may be short)
     // The column groups that do not make a whole round of the eight dies are dealt out by row
     // blocks instead, so that every die gets as many workgroups as the others (5,120 columns are
     // 20 groups of 256: two for every die, and of the other four each die takes half the row
     // blocks of one).
     const int whole = col_groups / TLI_DIES, left = col_groups % TLI_DIES;
+    const int turns_a_chunk = rows_turns(CHUNK, col_groups);
+    const int chunk = turn / turns_a_chunk, in_chunk = turn % turns_a_chunk;
+    const int chunk_rows = min(CHUNK, row_blocks - chunk * CHUNK);      // row blocks of this chunk (the last may be short)
     int row_block, col_group;
     if (in_chunk < whole * chunk_rows) {
         row_block = chunk * CHUNK + in_chunk % chunk_rows;
@@ -117,7 +123,7 @@ gemm_rows_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, bf1
         const int share = (left * chunk_rows + TLI_DIES - 1) / TLI_DIES; // workgroups of the left-over groups a die takes
         const int j = in_chunk - whole * chunk_rows;
         const int at = die * share + j;                                   // index among the left-over groups' workgroups
-        if (j >= share || at >= left * chunk_rows) return;                // (the grid is rounded up)
+        if (at >= left * chunk_rows) return;                              // (at most seven of a chunk)
         row_block = chunk * CHUNK + at % chunk_rows;
         col_group = whole * TLI_DIES + at / chunk_rows;
     }
@@ -378,8 +384,12 @@ static int launch_rows(const bf16_t* x, const bf16_t* w, bf16_t* y, float* part,
     const int n_tiles = (N + 15) / 16, k_steps = (K + 127) / 128;
     const long col_groups = (n_tiles + RT * WAVES - 1) / (RT * WAVES), row_blocks = (M + MT * 16 - 1) / (MT * 16);
     const long chunk = 2048 / (MT * 16);                     // as the kernel deals the row blocks out
-    const long blocks = (col_groups + TLI_DIES - 1) / TLI_DIES * TLI_DIES * ((row_blocks + chunk - 1) / chunk * chunk);
-    if (blocks > 2147483647L) return tli_fail("gemm_rows: too many workgroups");
+    if (col_groups * (row_blocks + chunk) > 1L << 28) return tli_fail("gemm_rows: too many workgroups");
+    // No workgroup without work between two ranges of k: the compute units are dealt out in turn, so that with the grid rounded up to whole
+    // chunks and whole rounds of dies the second range's workgroups came to the compute units of the first while others had none.
+    // (Product and the norm that adds the ranges, us, before and now: 260 rows, 2,048 columns of k 2,048 in 4 ranges 23.3 and 17.8, 1,024 columns
+    // 20.6 and 15.0, 4,096 of 4,096 32.1 and 30.3; 640 rows, 2,048 of 2,048 26.2 and 21.2; 770 rows, 1,024 of 2,048 24.3 and 18.3.)
+    const long blocks = TLI_DIES * (row_blocks / chunk * rows_turns((int)chunk, (int)col_groups) + rows_turns((int)(row_blocks % chunk), (int)col_groups));
     const int slices_per_split = (k_steps + splits - 1) / splits;
     if (KG == 2 && (slices_per_split % 2 || k_steps % slices_per_split))
         return tli_fail("gemm_rows: two sets of waves need an even number of slices in every range of k (%d of %d)",
