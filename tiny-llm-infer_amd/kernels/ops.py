@@ -1961,9 +1961,13 @@ class HipOps:
     # Decoding rows whose keys are shared out: the workgroups aimed at, and the fewest keys of a split: two tiles of 16 of the kernel for more
     # than 16 heads, one round of 32 of attention_latent_step, for which they were measured again (16 heads of 512 + 64, us, 2, 4, 8, 16 and 32
     # splits: 1 row of 100 keys 12.2, 9.4, 9.8, 10.4, 11.3; of 500 28.9, 18.4, 12.9, 10.5, 11.5; 16 rows of 500 29.0, 18.8, 14.6, 14.3, 19.2).
-    # There 512 workgroups would be better past 1,000 keys: 16 rows of 2,000 24.1 -> 22.7, 32 rows of 8,000 122 -> 78.
+    # There twice as many workgroups where each still has SIZED_WIDE_KEYS of the keys that the rows may have (us, 256 and 512: 16 rows of
+    # 2,100 27.0 and 24.8, of 8,000 61.7 and 45.0; 32 of 1,040 26.4 and 25.0, of 8,000 123 and 80; 64 of 520 26.7 and 25.1, of 1,000
+    # 37.0 and 29.9; 128 of 300 27.9 and 25.7, of 2,000 124 and 81; 8 of 8,000 37.5 and 31.9).  With half the keys it depends on the rows:
+    # 8 of 2,100 20.1 and 22.2, of 4,000 24.9 and 24.3; 32 of 520 19.2 and 20.3, of 1,000 24.0 and 23.1.
     SIZED_WORKGROUPS = 256
     SIZED_SPLIT_KEYS = 32
+    SIZED_WIDE_KEYS = 128
 
     def _sized_splits(self, T, reach, units, key_heads, window, keep) -> int:
         """Over how many workgroups the keys of one (row, key head) that decodes are shared out, where all heads read one cached
@@ -1971,7 +1975,11 @@ class HipOps:
         them after the other or, up to 16 heads a key head, 32 (csrc/attention_sized_mfma.hip)."""
         keys = min(reach, (window + 15 if window else reach) + keep)
         groups = T * key_heads * ((units // key_heads + 63) // 64)
-        return max(1, self.sized_splits or min(self.SIZED_WORKGROUPS // groups, keys // self.SIZED_SPLIT_KEYS, 64))
+        splits = min(self.SIZED_WORKGROUPS // groups, keys // self.SIZED_SPLIT_KEYS, 64)
+        wide = min(2 * self.SIZED_WORKGROUPS // groups, 64)
+        if units // key_heads <= 16 and not keep and keys >= wide * self.SIZED_WIDE_KEYS:
+            splits = max(splits, wide)
+        return max(1, self.sized_splits or splits)
 
     def head_products(self, x, x_stride, w, out=None, out_stride=None, x_at=0, out_at=0, gate=None):
         """y[t, h, :] = w[h] x[t, h, :] for a matrix a head, ``w`` [heads, N, K].  ``x`` is [T, columns]: the input of
