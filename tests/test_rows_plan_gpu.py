@@ -48,3 +48,16 @@ def test_every_output_is_written_once(ops, mn, cfg):
         if splits > 1:
             left = product(ops, x, tiled, N, splits, cfg, deferred=True)
             assert tuple(left.parts.shape) == (splits, M, N) and torch.equal(ops.resolve(left), y)
+
+
+# k of one slice, of fewer than two ranges' worth, of an odd number of slices; few and many columns; rows at the edges of a block of 128
+@pytest.mark.parametrize("mnk", [(257, 16, 128), (385, 1040, 904), (640, 2048, 2048), (641, 2048, 4096), (1000, 3072, 1024), (1537, 512, 1152), (2048, 256, 8192)])
+def test_plan(ops, mnk):
+    """The plan's ranges and launch shape: right, and the ranges within what their sums are laid out for."""
+    M, N, K = mnk
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x = torch.randn((M, K), generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.randn((N, K), generator=g, device=DEV).mul_(0.05).to(torch.bfloat16)
+    splits = ops.lib.tli_gemm_rows_splits(M, N, K)
+    assert 1 <= splits <= 16 and (splits == 1 or splits * 4 <= (K + 127) // 128)
+    assert near(product(ops, x, ops.tile_matrix(w), N, 0, 0), x, w)
