@@ -451,13 +451,29 @@ static bool half_tiles(int M, int N, int K, int tiled, bool into_residual) {
     return into_residual ? N >= 1024 && N % 4 == 0 : K >= N && K >= 256;
 }
 
+// The launch shape (row tiles * 10 + waves) of up to 16 rows.  One tile of 16 columns a workgroup while that gives no more than a workgroup a
+// compute unit, two up to twice as many columns (x is read half as often), two by four waves from four times on.  In between two tiles and
+// eight waves leave a second round of workgroups to a part of the chip, and smaller workgroups share it out better.  Cold weights, us,
+// 28, 14, 18 and 24: 9,216 columns of k 2,048, 1 row 10.9, 9.6, 9.8 and 10.2, of 4,096 18.2, 16.9, 16.1 and 18.4; 11,264 columns, 6 rows 11.8,
+// 10.6, 11.4 and 11.2, of 4,096 20.4, 18.7, 18.3 and 20.9, 16 rows 13.0, 12.5, 12.4 and 12.6; 12,288 12.5, 10.9, 12.3 and 11.6; 14,336
+// columns, 6 rows 13.0, 13.0, 13.2 and 12.2, of 5,120 24 is 1.8% behind 28.  Gated products, whose tiles come in pairs, stay with 28: 24 is 1 to
+// 4% behind.
+static int wide_shape(int N, int K, bool gated) {
+    const long tiles = (N + 15) / 16, units = tli_compute_units();
+    const bool shorter = K < 4096;
+    if (tiles <= units) return 18;
+    if (tiles <= 2 * units || gated || (tiles > 3 * units && !shorter)) return tiles < 4 * units ? 28 : 24;
+    return tiles > 3 * units ? 24 : shorter ? 14 : 18;
+}
+
 template <int MT>
 static int pick_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N, int K, int y_dtype,
                        int tiled, const GateOut& gate, const InputGroups& inputs, const OutUnit& unit, hipStream_t s, int cfg) {
     // cfg 0: by shape.  Narrow outputs get one 16-column tile per workgroup so that
     // even N = 4096 gives 256 workgroups; wide outputs share x over two tiles.
     const long tiles = (N + 15) / 16;
-    if (cfg == 0) cfg = half_tiles(M, N, K, tiled, false) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
+    if (cfg == 0 && MT == 1) cfg = half_tiles(M, N, K, tiled, false) ? 8 : wide_shape(N, K, tiled == 2);
+    if (cfg == 0) cfg = tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
     if (tiled == 2 && cfg < 20) cfg = 24;          // gated needs pairs of row tiles
     switch (cfg) {
         case 14: return launch_skinny<1, MT, 4>(x, w, y, M, N, K, y_dtype, tiled, gate, inputs, unit, s);
@@ -554,7 +570,8 @@ static int launch_skinny_fused(const bf16_t* x, const bf16_t* w, bf16_t* y, int 
 // The launch shape `cfg` of the product with a norm taken in (0: by the sizes), and whether it takes half tiles.
 static int fused_shape(int M, int N, int K, int gated, bool into_residual, int cfg) {
     const long tiles = (N + 15) / 16;
-    if (cfg == 0) cfg = !gated && half_tiles(M, N, K, 1, into_residual) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
+    if (cfg == 0 && !into_residual) cfg = !gated && half_tiles(M, N, K, 1, false) ? 8 : wide_shape(N, K, gated);
+    if (cfg == 0) cfg = half_tiles(M, N, K, 1, true) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
     return gated && cfg < 20 ? 24 : cfg;
 }
 
@@ -634,6 +651,7 @@ extern "C" int tli_gemm_skinny_normed_f32(const void* x, const void* w, void* y,
     hipStream_t s = (hipStream_t)stream;
     switch (fused_shape(M, N, K, 0, false, 0)) {
         case 8: return launch_skinny_normed_f32<1, 8>(xp, wp, (float*)y, M, N, K, f, s, true);
+        case 14: return launch_skinny_normed_f32<1, 4>(xp, wp, (float*)y, M, N, K, f, s);
         case 18: return launch_skinny_normed_f32<1, 8>(xp, wp, (float*)y, M, N, K, f, s);
         case 28: return launch_skinny_normed_f32<2, 8>(xp, wp, (float*)y, M, N, K, f, s);
         default: return launch_skinny_normed_f32<2, 4>(xp, wp, (float*)y, M, N, K, f, s);
