@@ -36,6 +36,9 @@
 //   FUSE_RSTD (the products that read normed rows): x is such a bfloat16(w*h); the rows'
 //       partial sums are added in order, and the outputs are scaled by r (before the
 //       SwiGLU of a gated matrix).
+//   FUSE_SELF (a product that reads normed rows of another's outputs): x are the rows themselves; a wave rounds
+//       w*x for its products, adds up the squares of what it reads, and the outputs are scaled by r.  A launch and a trip of the normed
+//       rows through memory less.
 // Sums, r and the residual are float32 (kernels/src/rmsnorm_kernel_cpu.cpp:27-43); the
 // rounding to bfloat16 happens once, as for a separate norm, only before r is applied
 // instead of after (a scalar factor does not change the relative rounding error).
@@ -70,18 +73,20 @@ __device__ __forceinline__ uint4 load16_or_zero(const bf16_t* p, bool ok) {
 #define FUSE_NONE 0
 #define FUSE_RSTD 1
 #define FUSE_RESIDUAL 2
+#define FUSE_SELF 3
 
 struct SkinnyFuse {
     const float* ssq_in;      // FUSE_RSTD: [parts_in][M] partial sums of squares of the rows of x's source
     int parts_in;
     float eps;
     float* resid;             // FUSE_RESIDUAL: [M][N] float32, updated in place
-    const float* norm_w;      // [N] weights of the norm that follows
+    const float* norm_w;      // [N] weights of the norm that follows; FUSE_SELF: [K] of the rows' own
     bf16_t* xw;               // [M][N] bfloat16(norm_w * resid)
     float* ssq_out;           // [ceil(N/16)][M]
     GateOut gate;             // of a gated matrix
     InputGroups inputs;
     OutUnit unit;             // of a product without a gate and norm
+    int x_ld;                 // FUSE_SELF: elements between two rows of x
 };
 
 template <int RT, int MT, int WAVES, typename TO, bool TILED = false, bool GATED = false, int DEPTH = 2,
@@ -125,7 +130,11 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
     }
     const bf16_t* x_row[MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) x_row[m] = x + (size_t)min(m * 16 + r, M - 1) * K;
+    for (int m = 0; m < MT; ++m) x_row[m] = x + (size_t)min(m * 16 + r, M - 1) * (FUSE == FUSE_SELF ? fuse.x_ld : K);
+    static_assert(FUSE != FUSE_SELF || (MT == 1 && TILED && !GATED && XR == 0), "rows that are normed on their way in");
+    constexpr bool SELF = FUSE == FUSE_SELF;
+    f32x4 own_w[SELF ? DEPTH : 1][SELF ? 8 : 1];               // the norm's weights of a step's 32 elements
+    float own_ssq = 0.f;
 
     // Ring of DEPTH register stages: the loads of the next DEPTH-1 128-wide steps are in
     // flight while the MFMAs of the current one run, so a wave keeps up to
@@ -154,6 +163,10 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
                 for (int j = 0; j < 4; ++j)
                     b[S][m][j].u = *reinterpret_cast<const uint4*>(x_row[m] + k + j * 8);
         }
+        if constexpr (SELF) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) own_w[S][q] = *reinterpret_cast<const f32x4*>(fuse.norm_w + k + q * 4);
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -175,6 +188,18 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
 #pragma unroll
             for (int j = 0; j < 4; ++j) b[0][0][j].w = x_lds[wave][r][(4 * c + j) ^ r];
             wave_lds_sync();
+        }
+        if constexpr (SELF) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t two = b[S][0][j].w[e];
+                    const float lo = __uint_as_float(two << 16), hi = __uint_as_float(two & 0xFFFF0000u);
+                    own_ssq = fmaf(lo, lo, own_ssq);
+                    own_ssq = fmaf(hi, hi, own_ssq);
+                    b[S][0][j].w[e] = pack_bf16x2(lo * own_w[S][2 * j + e / 2][2 * (e % 2)], hi * own_w[S][2 * j + e / 2][2 * (e % 2) + 1]);
+                }
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -289,14 +314,16 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (int i = 0; i < 4; ++i) red[wave][t * MT + m][lane][i] = acc[t][m][i];
-    __shared__ float ssq_red[FUSE == FUSE_RSTD ? WAVES : 1][MT][16];
-    if (FUSE == FUSE_RSTD && c == 0) {
+    constexpr bool SCALED = FUSE == FUSE_RSTD || SELF;
+    if constexpr (SELF) ssq_mine[0] = quad_rows_sum(own_ssq);
+    __shared__ float ssq_red[SCALED ? WAVES : 1][MT][16];
+    if (SCALED && c == 0) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) ssq_red[wave][m][r] = ssq_mine[m];
     }
     __syncthreads();
     float rstd[MT];
-    if (FUSE == FUSE_RSTD) {
+    if (SCALED) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             float a = 0.f;
@@ -361,7 +388,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, T
             if (c == 0 && row < M && (HALF || RT == 1 || n_base + t * 16 < N)) fuse.ssq_out[(size_t)(blockIdx.x * RT + t) * M + row] = ssq;
             continue;
         }
-        if (FUSE == FUSE_RSTD) {
+        if (SCALED) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) s[i] *= rstd[m];
         }
@@ -656,4 +683,35 @@ extern "C" int tli_gemm_skinny_normed_f32(const void* x, const void* w, void* y,
         case 28: return launch_skinny_normed_f32<2, 8>(xp, wp, (float*)y, M, N, K, f, s);
         default: return launch_skinny_normed_f32<2, 4>(xp, wp, (float*)y, M, N, K, f, s);
     }
+}
+
+// y[M,N] = norm(x) . W^T for rows that are part of wider ones: x [M, K], rows x_ld elements apart, the RMS norm over K with weights norm_w [K].
+// Up to 16 rows, W in the decode layout, k in whole steps of 128.  Every workgroup reads all rows anyway and does their arithmetic again, 100 vector
+// instructions a step beside loads that it waits for; the launch of norm_rows is saved.  Norm and product apart and so, in a recorded
+// chain, us: 3,072 columns of k 1,024, 1 row 5.3 and 4.2, 8 rows 5.7 and 4.3, 16 rows 5.8 and 4.3; of 1,536, 8 rows 6.5 and 5.1; 24,576 of 1,536
+// 15.6 and 15.5.
+extern "C" int tli_gemm_skinny_self_bf16(const void* x, int x_ld, const void* w, void* y, int M, int N, int K, const float* norm_w, float eps,
+                                         void* stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (M > 16) return tli_fail("gemm_skinny with a norm: %d rows, at most 16", M);
+    if (K <= 0 || K % 128 || x_ld < K || x_ld % 8) return tli_fail("gemm_skinny with a norm of its own rows: K = %d, rows %d apart", K, x_ld);
+    if (!norm_w || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)norm_w) & 15))
+        return tli_fail("gemm_skinny: operands must be 16-byte aligned");
+    SkinnyFuse f{};
+    f.norm_w = norm_w, f.eps = eps, f.x_ld = x_ld;
+    const bf16_t *xp = (const bf16_t*)x, *wp = (const bf16_t*)w;
+    bf16_t* yp = (bf16_t*)y;
+    hipStream_t s = (hipStream_t)stream;
+#define SKINNY_SELF(RT, WAVES, HALF)                                                                                              \
+    gemm_skinny_kernel<RT, 1, WAVES, bf16_t, true, false, 2, FUSE_SELF, 0, false, HALF>                                             \
+        <<<(N + (HALF ? 8 : 16 * RT) - 1) / (HALF ? 8 : 16 * RT), WAVES * 64, 0, s>>>(xp, wp, yp, M, N, K, f)
+    switch (fused_shape(M, N, K, 0, false, 0)) {
+        case 8: SKINNY_SELF(1, 8, true); break;
+        case 14: SKINNY_SELF(1, 4, false); break;
+        case 18: SKINNY_SELF(1, 8, false); break;
+        case 28: SKINNY_SELF(2, 8, false); break;
+        default: SKINNY_SELF(2, 4, false); break;
+    }
+#undef SKINNY_SELF
+    return tli_check_launch("gemm_skinny (norm of its own rows)");
 }

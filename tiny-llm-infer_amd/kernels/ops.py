@@ -94,6 +94,7 @@ def load_library():
         "tli_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_fused_bf16": [P, P, P, I, I, I, I, P, I, F, P, P, P, P, I, I, F, I, P],
         "tli_gemm_skinny_normed_f32": [P, P, P, I, I, I, P, I, F, P],
+        "tli_gemm_skinny_self_bf16": [P, I, P, P, I, I, I, P, F, P],
         "tli_embed_rmsnorm": [P, P, P, P, P, I, I, I, F, I, P],
         "tli_gemm_mid_bf16": [P, P, P, P, I, I, I, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_parts": [I, I, I],
@@ -2026,6 +2027,22 @@ class HipOps:
         self._call(self.lib.tli_norm_rows, proj.data_ptr() + at * proj.element_size(), proj.shape[1], weight.data_ptr(), out.data_ptr(),
                    T, n, float(eps), _dtype_code(proj.dtype), self._stream())
         return out
+
+    def linear_of_norm(self, proj, at, n, weight, eps, matrix):
+        """``linear(norm_rows(proj, at, n, weight, eps), matrix)``; a decode step's few rows in one launch."""
+        T, tiled = proj.shape[0], getattr(matrix, "tiled", None)
+        if not (0 < T <= 16 and tiled is not None and proj.dtype == torch.bfloat16 and n % 128 == 0 and proj.shape[1] % 8 == 0 and at % 8 == 0
+                and not self.plain_products and not self.separate_norms and self._aligned(proj, weight)):
+            return self.linear(self.norm_rows(proj, at, n, weight, eps), matrix)
+        N, K = _shape_of(matrix)
+        self._want(proj, "projections")
+        self._want(weight, "norm weight", torch.float32, (n,))
+        if at < 0 or at + n > proj.shape[1] or K != n:
+            raise KernelError(f"the elements to norm lie outside their row, or are not the {K} that the matrix reads")
+        y = torch.empty((T, N), dtype=proj.dtype, device=self.device)
+        self._call(self.lib.tli_gemm_skinny_self_bf16, proj.data_ptr() + 2 * at, proj.shape[1], tiled.data_ptr(), y.data_ptr(), T, N, K,
+                   weight.data_ptr(), float(eps), self._stream())
+        return y
 
     # Up to so many rows the queries' products and what else stands before the attention are one launch (csrc/latent.hip has both
     # sides' times: 1.3 to 3.8 us less a layer from 1 to 64 rows, 1 to 32 heads; more rows are prompts', whose launches are long).

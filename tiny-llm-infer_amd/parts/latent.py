@@ -141,8 +141,9 @@ class LatentAttention(Mixer):
         proj = ops.linear(x, self.w_in)
         query, q_at = proj, self.at.get("q")
         if self.q_rank is not None:
-            rows = ops.norm_rows(proj, self.at["down_q"], self.q_rank, self.q_weight, self.q_eps)
-            query, q_at = ops.linear(rows, self.w_uq), 0
+            normed = (proj, self.at["down_q"], self.q_rank, self.q_weight, self.q_eps)
+            together = getattr(ops, "linear_of_norm", None)
+            query, q_at = together(*normed, self.w_uq) if together else ops.linear(ops.norm_rows(*normed), self.w_uq), 0
         own = (proj, self.at["down"], self.norm_weight, self.norm_eps) if self.own else None
         o = ops.latent_attention(query, q_at, own, step, step.cache, self.heads, self.dim, self.rot, self.rank, self.vdim,
                                  self.rotary, self.scale, self.w_qk, self.w_v, window=self.window, sinks=self.sinks,
