@@ -50,7 +50,9 @@ CASES = [(16, 4, 64, 16, True, 64, [1, 16, 17, 52, 65], None, None, True),
          (2, 1, 192, 16, True, 0, [90, 41], None, None, True),
          (2, 2, 256, 16, True, 256, [300, 16], None, 20, True),
          (4, 2, 64, 16, True, 64, [30, 31], None, None, False),
-         (4, 2, 64, 16, True, 64, [30, 45], [3, 1], None, True)]
+         (4, 2, 64, 16, True, 64, [30, 45], [3, 1], None, True),
+         # many heads of more than 64 elements: their squares in one order of roundings
+         (4, 1, 192, 16, True, 192, [9] * 32, None, None, True), (8, 2, 128, 8, True, 128, [20] * 32, None, None, True)]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(v) for v in c[:6]) + f"-{len(c[6])}rows-window{c[8]}-writes{c[9]}")

@@ -42,7 +42,7 @@ __device__ __forceinline__ void head_of_raw_row(float* x, const float* src, size
         w[e] = nw ? nw[e * 64 + lane] : 0.f;
     }
 #pragma unroll
-    for (int e = 0; e < DH; ++e) ss += v[e] * v[e];
+    for (int e = 0; e < DH; ++e) ss = fmaf(v[e], v[e], ss);      // (written out: the sums of qkv_to_cache_kernel, bit for bit)
     if (nw) {
         const float scale = 1.0f / sqrtf(wave_sum(ss) / (float)D + eps);
 #pragma unroll

@@ -77,7 +77,7 @@ __global__ void qkv_to_cache_kernel(
         for (int i = lane; i < head_dim; i += TLI_WAVE) {
             const float v = to_f32(raw_value(src + i, planes, plane));
             x[i] = v;
-            ss += v * v;
+            ss = fmaf(v, v, ss);
         }
         if (nw) {
             ss = wave_sum(ss);
