@@ -13,9 +13,9 @@
 // serves four products, so that a row of W is read in pieces of 64 bytes, the next piece by the next load.
 //
 // Measured with 1 to 5 rows at width 1,024 (the tiled kernel of the vector units in gemm_plain.hip, which walks k with one
-// load in flight, before): q/k/v (6.3 MB) 156 -> 5.8 us, output and down projection (4.2 and 16.8 MB) 378 -> 9.1 us on
-// average, gate/up with its activation (33.6 MB) 160 -> 11.5 us, the head (134 MB) 201 -> 29 us = 4.6 TB/s.  Error against
-// float64 of the logits of four layers 2.9e-6 -> 1.1e-6.
+// load in flight, before): q/k/v (6.3 MB) 156 -> 5.8 us, output and down projection (4.2 and 16.8 MB) 378 -> 9.8 us on
+// average (5.2 where the reader adds the ranges' sums, see gemm_f32_ranges_kernel), gate/up with its activation (33.6 MB) 160 ->
+// 10 us, the head (134 MB) 201 -> 29 us = 4.6 TB/s.  Error against float64 of the logits of four layers 2.9e-6 -> 1.1e-6.
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;

@@ -1972,8 +1972,8 @@ class HipOps:
 
     def _sized_splits(self, T, reach, units, key_heads, window, keep) -> int:
         """Over how many workgroups the keys of one (row, key head) that decodes are shared out, where all heads read one cached
-        vector; ``reach``: a power of two that the longest sequence fits.  A workgroup takes a run of a row's keys, 16 of
-        them after the other or, up to 16 heads a key head, 32 (csrc/attention_sized_mfma.hip)."""
+        vector; ``reach``: a power of two that the longest sequence fits.  A workgroup walks its run of a row's keys in
+        tiles of 16 or, with up to 16 heads a key head, 32 (csrc/attention_sized_mfma.hip)."""
         keys = min(reach, (window + 15 if window else reach) + keep)
         groups = T * key_heads * ((units // key_heads + 63) // 64)
         splits = min(self.SIZED_WORKGROUPS // groups, keys // self.SIZED_SPLIT_KEYS, 64)

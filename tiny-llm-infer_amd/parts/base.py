@@ -94,7 +94,7 @@ class StepView:
 
 class Part:
     # True if forward() looks at nothing on the host but the step's shape (rows,
-    # sequences, table width, reach, skew): then a recorded launch sequence can be replayed
+    # sequences, table width, reach, skew, all_wanted): then a recorded launch sequence can be replayed
     replayable = False
 
     def __init__(self, spec: PartSpec):
