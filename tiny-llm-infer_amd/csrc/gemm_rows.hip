@@ -493,7 +493,8 @@ static double rows_estimate(int M, int N, int K, int splits, int cfg) {
         rounds = wgs <= units ? 1.0 : 1.75 * (double)full + (rem == 0 ? 0.0 : rem <= units ? 1.0 : 1.75);
     }
     const int per = ((K + 127) / 128 + splits - 1) / splits;
-    const double sums = (double)M * N * (splits > 1 ? 8.0 * splits : 4.0) * 1e-6;
+    // (whole blocks of rows: every M of a block has the same plan, hence the same order of sums, which a recorded step filled up with rows relies on)
+    const double sums = (double)row_blocks * 128.0 * N * (splits > 1 ? 8.0 * splits : 4.0) * 1e-6;
     return 6.0 + 0.24 * sums + rounds * (per * f.slice + f.ends);
 }
 static RowsPlan rows_plan(int M, int N, int K) {
@@ -523,6 +524,13 @@ static RowsPlan rows_plan(int M, int N, int K) {
 // How many ranges of k a product of this shape is cut into (the caller sizes `part` by it).
 extern "C" int tli_gemm_rows_splits(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? rows_plan(M, N, K).splits : 1; }
 
+// The launch shape that a product in `splits` ranges of k is given by its sizes (cfg 0 of tli_gemm_rows_bf16).
+extern "C" int tli_gemm_rows_shape(int M, int N, int K, int is_gated, int splits) {
+    if (M <= 0 || N <= 0 || K <= 0 || splits < 1) return 0;
+    const RowsPlan plan = rows_plan(M, N, K);
+    return !is_gated && splits == plan.splits ? plan.cfg : rows_pick(M, N, K, splits, is_gated);
+}
+
 static int gemm_rows(const void* x, const void* w, void* y, float* part, int M, int N, int K, int is_gated, int splits, int cfg, int act,
                      float act_scale, int y_ld, const InputGroups& inputs, void* stream) {
     const GateOut gated = gate_out(is_gated, act, act_scale, y_ld, N / 2);
@@ -539,10 +547,7 @@ static int gemm_rows(const void* x, const void* w, void* y, float* part, int M, 
     if ((size_t)M * K * sizeof(bf16_t) >= (1ull << 32) || (size_t)((N + 15) / 16 * 16) * ((K + 127) / 128 * 128) * sizeof(bf16_t) >= (1ull << 32))
         return tli_fail("gemm_rows: an operand of 4 GiB or more (offsets are 32 bits)");
     if (cfg >= 10) cfg = gated ? cfg / 10 : cfg % 10;       // measurements: one shape for the gated product, one for the others
-    if (cfg == 0) {
-        const RowsPlan plan = rows_plan(M, N, K);
-        cfg = !gated && splits == plan.splits ? plan.cfg : rows_pick(M, N, K, splits, gated);
-    }
+    if (cfg == 0) cfg = tli_gemm_rows_shape(M, N, K, is_gated, splits);
     if (cfg == 1) return launch_rows<2, 8, 16, 1>((const bf16_t*)x, (const bf16_t*)w, (bf16_t*)y, part, M, N, K, gated, inputs, splits, s);
     if (cfg == 2) return launch_rows<4, 4, 8, 1>((const bf16_t*)x, (const bf16_t*)w, (bf16_t*)y, part, M, N, K, gated, inputs, splits, s);
     if (cfg == 3) return launch_rows<4, 8, 8, 1>((const bf16_t*)x, (const bf16_t*)w, (bf16_t*)y, part, M, N, K, gated, inputs, splits, s);

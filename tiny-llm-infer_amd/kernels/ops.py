@@ -103,6 +103,7 @@ def load_library():
         "tli_gemm_mid_reduce": [P, P, I, I, I, I, P],
         "tli_gemm_rows_bf16": [P, P, P, P, I, I, I, I, I, I, I, F, I, P],
         "tli_gemm_rows_splits": [I, I, I],
+        "tli_gemm_rows_shape": [I, I, I, I, I],
         "tli_attention_decode_bf16": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, I, I, P],
         "tli_qkv_attention_decode_bf16": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, F, P, F, P, P, I,
                                           F, I, I, I, P, I, P],
