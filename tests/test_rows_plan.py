@@ -17,3 +17,23 @@ def test_one_plan_for_all_rows_of_a_block(nk):
     for last in list(range(256, 1537, 128)) + [2048, 3072, 3200]:
         want = plan(last)
         assert all(plan(M) == want for M in range(last - 127, last)), last
+
+
+# (rows, columns, k), the ranges that were the faster, gated or columns a matrix; both measured
+@pytest.mark.parametrize("mnk, gated, every, want", [((256, 8192, 4096), 0, 2048, 4), ((129, 8192, 4096), 0, 2048, 4), ((129, 8192, 3072), 0, 2048, 4),
+                                                     ((512, 4096, 4096), 0, 1024, 4), ((640, 8192, 2048), 0, 2048, 1), ((1024, 4096, 1024), 0, 1024, 1),
+                                                     ((640, 8192, 1024), 1, 0, 1), ((512, 4096, 4096), 1, 0, 4), ((129, 8192, 4096), 1, 0, 4),
+                                                     ((256, 4096, 4096), 1, 0, 4)])
+def test_ranges_for_the_shape_that_runs(mnk, gated, every, want):
+    """Gated products and stacked matrices do not run in the shape that a plain product of their sizes would."""
+    assert load_library().tli_gemm_rows_splits_of(*mnk, gated, every) == want
+
+
+def test_ranges_of_every_kind_leave_four_slices_each():
+    lib = load_library()
+    for M in (129, 256, 257, 1000, 3000):
+        for N in (512, 1024, 4096, 12288):
+            for K in (8, 128, 904, 1024, 4096, 17408):
+                for gated, every in ((0, 0), (1, 0), (0, 256), (0, 512)):
+                    splits = lib.tli_gemm_rows_splits_of(M, N, K, gated, every)
+                    assert 1 <= splits <= 16 and (splits == 1 or splits * 4 <= (K + 127) // 128)

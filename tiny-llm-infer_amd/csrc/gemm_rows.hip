@@ -497,22 +497,35 @@ static double rows_estimate(int M, int N, int K, int splits, int cfg) {
     const double sums = (double)row_blocks * 128.0 * N * (splits > 1 ? 8.0 * splits : 4.0) * 1e-6;
     return 6.0 + 0.24 * sums + rounds * (per * f.slice + f.ends);
 }
-static RowsPlan rows_plan(int M, int N, int K) {
+// The launch shape of stacked matrices in `splits` ranges of k (tli_gemm_rows_groups_bf16).
+static int groups_shape(int M, int N, int K, int splits, int every) {
+    const long wgs = (long)((N + 255) / 256) * ((M + 127) / 128) * splits, units = tli_compute_units();
+    const int k_steps = (K + 127) / 128, per = (k_steps + splits - 1) / splits;
+    return every % 512 == 0 && wgs >= 3 * units ? 3 : (wgs <= units || wgs > 2 * units) && per % 2 == 0 && k_steps % per == 0 ? 6 : 2;
+}
+// Gated products and stacked matrices (`every` > 0) have shapes by rules of their own, so that only their ranges are planned, and the pass that
+// adds these is a launch of its own.  us, ranges by the first plan and now: gated 8,192 columns of k 1,024, 640 rows 28.7 (2) and 16.7 (1), 4,096 of 4,096, 256
+// rows 25.9 (8) and 24.1 (4); stacked 4 x 2,048 of 2,048, 640 rows 49.2 (2) and 33.8 (1), 4 x 1,024 of 1,024, 1,024 rows 28.5 (2) and 20.7 (1), 4 x 2,048
+// of 4,096 at 256 rows stays at 4 (39.3; 2 would be 43.6).
+static RowsPlan rows_plan(int M, int N, int K, int is_gated, int every) {
     const long col_groups = ((N + 15) / 16 + 15) / 16, row_blocks = (M + 127) / 128;
     const int k_steps = (K + 127) / 128;
     int splits = 1;
     const long enough = 3L * tli_compute_units() / 4;
     while (col_groups * row_blocks * splits < enough && splits * 2 * 4 <= k_steps && splits < 16) splits *= 2;
-    RowsPlan best{splits, rows_pick(M, N, K, splits, 0)};
+    const bool plain = !is_gated && every == 0;
+    auto shape = [&](int s) { return every > 0 ? groups_shape(M, N, K, s, every) : rows_pick(M, N, K, s, is_gated); };
+    auto estimate = [&](int s, int cfg) { return rows_estimate(M, N, K, s, cfg) + (plain || s == 1 ? 0.0 : 4.0); };
+    RowsPlan best{splits, shape(splits)};
     // (large products are at the costs that rows_pick knows)
     const long large = ((N + 511) / 512 * row_blocks + TLI_DIES - 1) / TLI_DIES;
     if (large >= 3 * tli_units_a_die()) return best;
-    double limit = 0.96 * rows_estimate(M, N, K, best.splits, best.cfg);
+    double limit = 0.96 * estimate(best.splits, best.cfg);
     for (int s = 1; s <= 8 && (s == 1 || s * 4 <= k_steps); s *= 2)
         for (int cfg = 2; cfg <= 6; ++cfg) {
             const int per = (k_steps + s - 1) / s;
-            if (cfg == 6 && (per % 2 || k_steps % per)) continue;
-            const double t = rows_estimate(M, N, K, s, cfg);
+            if (plain ? cfg == 6 && (per % 2 || k_steps % per) : cfg != shape(s)) continue;
+            const double t = estimate(s, cfg);
             if (t < limit) {
                 limit = t;
                 best = RowsPlan{s, cfg};
@@ -521,14 +534,17 @@ static RowsPlan rows_plan(int M, int N, int K) {
     return best;
 }
 
-// How many ranges of k a product of this shape is cut into (the caller sizes `part` by it).
-extern "C" int tli_gemm_rows_splits(int M, int N, int K) { return M > 0 && N > 0 && K > 0 ? rows_plan(M, N, K).splits : 1; }
+// How many ranges of k a product of this shape is cut into (the caller sizes `part` by it); _of: a gated one, or stacked matrices of `every` columns.
+extern "C" int tli_gemm_rows_splits_of(int M, int N, int K, int is_gated, int every) {
+    return M > 0 && N > 0 && K > 0 ? rows_plan(M, N, K, is_gated, every).splits : 1;
+}
+extern "C" int tli_gemm_rows_splits(int M, int N, int K) { return tli_gemm_rows_splits_of(M, N, K, 0, 0); }
 
 // The launch shape that a product in `splits` ranges of k is given by its sizes (cfg 0 of tli_gemm_rows_bf16).
 extern "C" int tli_gemm_rows_shape(int M, int N, int K, int is_gated, int splits) {
     if (M <= 0 || N <= 0 || K <= 0 || splits < 1) return 0;
-    const RowsPlan plan = rows_plan(M, N, K);
-    return !is_gated && splits == plan.splits ? plan.cfg : rows_pick(M, N, K, splits, is_gated);
+    const RowsPlan plan = rows_plan(M, N, K, is_gated, 0);
+    return splits == plan.splits ? plan.cfg : rows_pick(M, N, K, splits, is_gated);
 }
 
 static int gemm_rows(const void* x, const void* w, void* y, float* part, int M, int N, int K, int is_gated, int splits, int cfg, int act,
@@ -568,7 +584,7 @@ static int gemm_rows(const void* x, const void* w, void* y, float* part, int M, 
 
 // y[M,N] = x[M,K] . W^T for any number of rows, bfloat16, W in the decode layout (`gated` as
 // tiled = 2 of tli_gemm_skinny_bf16: N counts gate and up, y is [M, N/2]).  `part`: splits*M*N
-// floats when splits > 1 (splits as returned by tli_gemm_rows_splits, or forced by the
+// floats when splits > 1 (splits as returned by tli_gemm_rows_splits_of, or forced by the
 // caller); with y null the partial sums [splits][M][N] are left for the consumer to add
 // (tli_gemm_mid_reduce, or tli_add_rmsnorm).
 // cfg 0 picks the launch shape; 1: 256 x 256 outputs a workgroup of eight waves, 2: 128 x 256
@@ -589,8 +605,7 @@ extern "C" int tli_gemm_rows_bf16(const void* x, const void* w, void* y, float* 
 extern "C" int tli_gemm_rows_groups_bf16(const void* x, const void* w, void* y, float* part, int M, int N, int K, int splits, int every,
                                          long long step, void* stream) {
     if (every <= 0 || every % 256 || step < (long long)M * K || step % 8) return tli_fail("gemm_rows: bad input groups");
-    const long wgs = (long)((N + 255) / 256) * ((M + 127) / 128) * splits, units = tli_compute_units();
-    const int k_steps = (K + 127) / 128, per = (k_steps + splits - 1) / splits;
-    const int cfg = every % 512 == 0 && wgs >= 3 * units ? 3 : (wgs <= units || wgs > 2 * units) && per % 2 == 0 && k_steps % per == 0 ? 6 : 2;
-    return gemm_rows(x, w, y, part, M, N, K, 0, splits, cfg, 0, 1.0f, 0, InputGroups{every, step}, stream);
+    if (M <= 0 || N <= 0) return 0;
+    if (K <= 0 || splits < 1) return tli_fail("gemm_rows: K = %d, %d splits", K, splits);
+    return gemm_rows(x, w, y, part, M, N, K, 0, splits, groups_shape(M, N, K, splits, every), 0, 1.0f, 0, InputGroups{every, step}, stream);
 }

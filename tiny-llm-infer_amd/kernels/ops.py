@@ -103,6 +103,7 @@ def load_library():
         "tli_gemm_mid_reduce": [P, P, I, I, I, I, P],
         "tli_gemm_rows_bf16": [P, P, P, P, I, I, I, I, I, I, I, F, I, P],
         "tli_gemm_rows_splits": [I, I, I],
+        "tli_gemm_rows_splits_of": [I, I, I, I, I],
         "tli_gemm_rows_shape": [I, I, I, I, I],
         "tli_attention_decode_bf16": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, I, I, P],
         "tli_qkv_attention_decode_bf16": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, F, P, F, P, P, I,
@@ -668,7 +669,7 @@ class HipOps:
         """Any number of rows from the decode layout; k cut into ranges when the output
         alone gives too few workgroups.  ``deferred``: the partial sums of the ranges are
         left for the consumer to add.  ``gate`` as in ``_linear_mid``."""
-        splits = self.rows_splits or self.lib.tli_gemm_rows_splits(M, N, K)
+        splits = self.rows_splits or self.lib.tli_gemm_rows_splits_of(M, N, K, gated, 0)
         part = None
         if splits > 1:
             part = torch.empty((splits, M, N), dtype=torch.float32, device=self.device)
@@ -2451,7 +2452,7 @@ class HipOps:
                                _dtype_code(dtype), every, apart, self._stream())
                 else:
                     mid = M <= self.MID_ROWS_TO
-                    splits = int(self.lib.tli_gemm_mid_splits_rows(M, N, K, 0) if mid else self.lib.tli_gemm_rows_splits(M, N, K))
+                    splits = int(self.lib.tli_gemm_mid_splits_rows(M, N, K, 0) if mid else self.lib.tli_gemm_rows_splits_of(M, N, K, 0, every))
                     part = torch.empty((splits, M, N), dtype=torch.float32, device=self.device) if splits > 1 else None
                     if mid:
                         self._call(self.lib.tli_gemm_mid_groups_bf16, xs.data_ptr(), tiled.data_ptr(), proj.data_ptr(), _ptr(part), M, N, K,
