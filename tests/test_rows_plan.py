@@ -37,3 +37,14 @@ def test_ranges_of_every_kind_leave_four_slices_each():
                 for gated, every in ((0, 0), (1, 0), (0, 256), (0, 512)):
                     splits = lib.tli_gemm_rows_splits_of(M, N, K, gated, every)
                     assert 1 <= splits <= 16 and (splits == 1 or splits * 4 <= (K + 127) // 128)
+
+
+@pytest.mark.parametrize("mnk", [(3200, 12288, 17408), (3200, 12288, 1536), (640, 16384, 1024), (1024, 12288, 17408), (512, 8192, 24576)])
+def test_sizes_that_were_not_measured_keep_the_first_plan(mnk):
+    """Ranges of k only until there are three workgroups of 128 x 256 outputs for every four compute units, four slices of 128 in each."""
+    lib = load_library()
+    M, N, K = mnk
+    groups, splits = -(-N // 256) * -(-M // 128), 1
+    while groups * splits < 3 * lib.tli_device_compute_units() // 4 and splits * 8 <= -(-K // 128) and splits < 16:
+        splits *= 2
+    assert lib.tli_gemm_rows_splits(M, N, K) == splits

@@ -467,13 +467,13 @@ static int rows_pick(int M, int N, int K, int splits, int gated) {
 // compute units, a range keeping at least four slices of 128, and the shape that rows_pick takes for them.  Another plan is taken where
 // its estimate is lower by more than the estimates are good for: that plan is too eager to cut k where k is short (a range of four slices
 // is over before its loads are under way, and all ranges' sums are written and read again by the next norm), and takes 192 columns a workgroup
-// for 256 where two ranges would do.
+// for 256 where two ranges would do.  Only for sizes where both were measured (rows_planned).
 // The estimate, fitted to 1,700 products with the norm behind them (260 to 3,072 rows, 1,024 to 7,168 columns of k 1,024 to 17,408; 7% off on average),
 // in us: 6, 0.24 a MB of sums written and read, and for every round of workgroups on a die its slices and its beginning and end.
-// Product and norm, us, before and now: 2,048 columns of k 2,048, 1,024 rows 30.9 -> 25.0, 2,048 rows 40.7 -> 35.4; of k 4,096, 640 rows 33.6 -> 25.8;
-// of k 8,192 43.9 -> 37.4; 3,072 of 1,024, 1,536 rows 35.6 -> 28.8; 4,096 of 4,096, 640 rows 41.8 -> 38.9; 7,168 of 5,120, 384 rows 51.1 ->
-// 47.0; over the shapes that it was fitted to 3.4% less on average and nowhere more than 1%; over 214 others, the grid without idle
-// workgroups (rows_turns) included, 7% less on average, at most 3.5% more.
+// Product and norm, us, before and now: 2,048 columns of k 2,048, 1,024 rows 30.9 -> 25.0; of k 4,096, 640 rows 33.6 -> 25.8; of k 8,192 43.9 -> 37.4;
+// 3,072 of 1,024, 1,536 rows 35.6 -> 28.8.  Over 954 products with the norm behind them (260 to 3,072 rows, 512 to 8,192 columns, k 512 to
+// 17,408) 2.5% less on average and nowhere more than 2%; the best of all ranges and shapes would be 3.4%.  Over 1,017 without one, which add their ranges
+// in a launch of their own, 4.4% less, nowhere more than 1%.  (With a margin of 4% for the 8% below: 2.7 and 4.9% less, but some 5% more.)
 struct RowsPlan {
     int splits, cfg;
 };
@@ -507,6 +507,12 @@ static int groups_shape(int M, int N, int K, int splits, int every) {
 // adds these is a launch of its own.  us, ranges by the first plan and now: gated 8,192 columns of k 1,024, 640 rows 28.7 (2) and 16.7 (1), 4,096 of 4,096, 256
 // rows 25.9 (8) and 24.1 (4); stacked 4 x 2,048 of 2,048, 640 rows 49.2 (2) and 33.8 (1), 4 x 1,024 of 1,024, 1,024 rows 28.5 (2) and 20.7 (1), 4 x 2,048
 // of 4,096 at 256 rows stays at 4 (39.3; 2 would be 43.6).
+// The sizes between which all ranges and shapes were timed against the first plan; up to 3,072 rows.
+static bool rows_planned(int M, int N, int K, bool plain, int every) {
+    if (M > 3072 || N > 12288) return false;
+    if (plain) return N >= 512 && K >= 512 && K <= 17408 && (long)N * K <= 5120L * 17408;
+    return N >= 1024 && K >= 1024 && K <= (every > 0 ? 4096 : 5120);
+}
 static RowsPlan rows_plan(int M, int N, int K, int is_gated, int every) {
     const long col_groups = ((N + 15) / 16 + 15) / 16, row_blocks = (M + 127) / 128;
     const int k_steps = (K + 127) / 128;
@@ -519,8 +525,8 @@ static RowsPlan rows_plan(int M, int N, int K, int is_gated, int every) {
     RowsPlan best{splits, shape(splits)};
     // (large products are at the costs that rows_pick knows)
     const long large = ((N + 511) / 512 * row_blocks + TLI_DIES - 1) / TLI_DIES;
-    if (large >= 3 * tli_units_a_die()) return best;
-    double limit = 0.96 * estimate(best.splits, best.cfg);
+    if (large >= 3 * tli_units_a_die() || !rows_planned(M, N, K, plain, every)) return best;
+    double limit = 0.92 * estimate(best.splits, best.cfg);
     for (int s = 1; s <= 8 && (s == 1 || s * 4 <= k_steps); s *= 2)
         for (int cfg = 2; cfg <= 6; ++cfg) {
             const int per = (k_steps + s - 1) / s;
