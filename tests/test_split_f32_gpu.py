@@ -98,3 +98,12 @@ def test_attention_from_projections_left_in_ranges(ops, case):
         for apart in (False, True):
             for a, b in zip(run(qkv, apart), want):
                 assert torch.equal(a.nan_to_num(7e30), b.nan_to_num(7e30))
+
+
+def test_the_library_says_which_products_are_left(ops, monkeypatch):
+    """Not a setting of the attention kernels: what ``linear`` leaves is what the kernel for the ranges takes."""
+    monkeypatch.setattr(ops, "DECODE_WORKGROUPS", 4 * ops.DECODE_WORKGROUPS)
+    x, w, weight = rnd((5, 64), 1), rnd((4096, 64), 2), 1 + rnd((4096,), 3, 0.1)
+    left = ops.linear(x, w, deferred=True)
+    assert isinstance(left, torch.Tensor)
+    ops.add_rmsnorm(torch.zeros((5, 4096), device=DEV), left, weight, 1e-6, F32)

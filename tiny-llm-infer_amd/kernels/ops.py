@@ -230,7 +230,6 @@ class HipOps:
     name = "hip-gfx950"
     MAX_HEAD_DIM = 512
     SKINNY_ROWS = 64
-    F32_RANGES_ROWS = 32         # float32 products of so many rows and few outputs are left as the sums of their ranges of k
     MID_ROWS_FROM = 17           # from this many rows the x-sharing kernel multiplies,
     MID_ROWS_TO = 128            # up to this many
     MID_ROWS_TO_PLAIN = 256      # a product without a gate: up to this many (two blocks of 128 rows side by side)
@@ -474,7 +473,8 @@ class HipOps:
         """y = x W^T.  ``w`` is a [N, K] tensor or a ``Matrix`` (row-major tensor plus
         its decode layout).  ``deferred``: the caller hands the result to ``add_rmsnorm``
         (or to ``resolve``) and so also takes a ``PendingProduct`` or a ``DeferredSum``;
-        ``sums_only``: to ``qkv_attention`` (or to ``resolve``), which takes a ``DeferredSum``."""
+        ``sums_only``: to ``qkv_attention`` (or to ``resolve``), which takes a ``DeferredSum`` and, in float32,
+        a ``PendingProduct``."""
         if isinstance(x, NormedRows):
             return self._linear_normed(x, w, getattr(w, "tiled", None), 0, out_dtype)
         if self.plain_products:
@@ -489,9 +489,8 @@ class HipOps:
         if K != K2:
             raise KernelError(f"linear: input has {K} columns, the matrix {K2}")
         self._want(x, "linear input")
-        if ((deferred or sums_only) and x.dtype == torch.float32 and 0 < M <= self.F32_RANGES_ROWS and tiled is None
-                and out_dtype in (None, torch.float32) and not self.separate_norms and (N + 15) // 16 * 2 <= self.DECODE_WORKGROUPS
-                and self._f32_product_takes(x, getattr(w, "w", w))):
+        if ((deferred or sums_only) and x.dtype == torch.float32 and tiled is None and out_dtype in (None, torch.float32)
+                and not self.separate_norms and self.lib.tli_gemm_f32_ranges_of(M, N) and self._f32_product_takes(x, getattr(w, "w", w))):
             return PendingProduct(x, w)
         w_dtype = getattr(matrix, "dtype", None) or matrix.w.dtype
         if x.dtype != w_dtype:
