@@ -107,3 +107,33 @@ def test_the_library_says_which_products_are_left(ops, monkeypatch):
     left = ops.linear(x, w, deferred=True)
     assert isinstance(left, torch.Tensor)
     ops.add_rmsnorm(torch.zeros((5, 4096), device=DEV), left, weight, 1e-6, F32)
+
+
+# outputs that are no multiple of four (rows of the planes without 16-byte alignment, the norm's element-by-element path) and k of every length
+@pytest.mark.parametrize("mnk", SIZES + [(1, 1, 4), (5, 77, 260), (17, 1999, 132), (32, 2047, 1028), (3, 2046, 2304)])
+def test_ranges_whatever_their_reader_would_take(ops, mnk):
+    from tiny_llm_infer_amd.kernels.ops import PendingProduct
+    M, N, K = mnk
+    x, w, resid, weight = rnd((M, K), 1), rnd((N, K), 2, 0.05), rnd((M, N), 3), 1 + rnd((N,), 4, 0.1)
+    parts, product = ops._f32_ranges(PendingProduct(x, w)), ops.linear(x, w)
+    assert torch.equal(ops.resolve(parts), product)
+    for rows in (None, torch.tensor([M - 1, 0], dtype=torch.int32, device=DEV)):
+        one, two = resid.clone(), resid.clone()
+        got = ops.add_rmsnorm(one, parts, weight, 1e-6, F32, rows=rows)
+        want = ops.add_rmsnorm(two, product, weight, 1e-6, F32, rows=rows)
+        assert torch.equal(got, want) and torch.equal(one, two)
+
+
+@pytest.mark.parametrize("nk, pay", [((64, 252), False), ((64, 256), True), ((1024, 256), True), ((1026, 1024), False), ((1028, 1020), False),
+                                     ((1028, 1024), True), ((2047, 2044), False), ((2047, 2048), True)])
+def test_short_products_are_read_whole(ops, nk, pay):
+    from tiny_llm_infer_amd.kernels.ops import DeferredSum, PendingProduct
+    N, K = nk
+    assert isinstance(ops._f32_sums(PendingProduct(rnd((5, K), 1), rnd((N, K), 2))), DeferredSum if pay else torch.Tensor)
+
+
+@pytest.mark.parametrize("hd", [64, 128, 192, 256])
+@pytest.mark.parametrize("window", [None, 17])
+def test_own_key_at_the_edges_of_blocks(ops, hd, window):
+    """The row's own key first, in the middle and last of a block of 16 keys, alone in one, and in every wave's share."""
+    test_attention_from_projections_left_in_ranges(ops, (4, 2, hd, 16, True, hd, [1, 2, 16, 17, 32, 33, 48, 49, 64, 65, 80, 81, 130], None, window, True))

@@ -10,7 +10,7 @@
 // embed_rmsnorm: both, for the first norm of a model: the residual's rows are written and normed from registers
 // swiglu:      out = g / (1 + exp(-g)) * u over a fused [rows, 2*inter] input
 //              (kernels/src/swiglu_kernel_cpu.cpp:20-24)
-#include "common.h"
+#include "gemm_reduce.h"
 
 template <typename T>
 __global__ void embed_kernel(const T* __restrict__ table, const int* __restrict__ ids,
@@ -56,12 +56,7 @@ struct RowDelta {
     size_t plane;
     __device__ __forceinline__ bool any() const { return d != nullptr || parts > 0; }
     __device__ __forceinline__ float at(int i) const {
-        if (parts > 0) {
-            float a = 0.f;
-            for (int s = 0; s < parts; ++s) a += p[s * plane + i];
-            return rounded_to<T>(a);
-        }
-        return to_f32(d[i]);
+        return parts > 0 ? rounded_to<T>(sum_planes(p + i, parts, plane)) : to_f32(d[i]);
     }
 };
 

@@ -159,8 +159,9 @@ gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float*
 // a tile of 16 columns and range, GF_PART_WAVES tiles of a range a workgroup, whose waves share the pieces of x that they read.
 // What it is for: 1,024 columns are 64 tiles, which the kernel above reaches all compute units with only by giving a workgroup a quarter of
 // one, so that three quarters of its matrix instructions and loads repeat.  Here the tiles' eight ranges are 512 waves that repeat nothing,
-// wait for no other wave, and have all their loads in flight (two batches of eight steps).  What bounds it: the launch and one
-// trip to memory; 4,096 k: 3.1 TB/s, a wave's 128 instructions of 32 cycles one after the other.
+// wait for no other wave, and have two batches of eight steps in flight, up to k of 2,048 all of their loads.  What bounds it: the launch and, up to
+// there, one trip to memory; beyond, the loads follow behind the products: 4,096 k (four batches) 3.1 TB/s, a wave's 128 instructions of 32 cycles
+// one after the other.
 // Measured in a recorded chain, cold weights, us, with the norm that adds the sums against the kernel above and the norm: 5 rows, 1,024 columns of
 // k 1,024 7.5 -> 6.0, of 4,096 15.5 -> 8.5; 16 rows 8.6 -> 6.3, 19.4 -> 9.5; 32 rows 10.8 -> 7.2, 26.8 -> 12.4; 1,536 of 1,024 alone 5.4 -> 4.1 (5 rows)
 // and 8.8 -> 6.1 (32).  Non-temporal loads of W are no faster.
@@ -254,6 +255,12 @@ extern "C" int tli_gemm_f32(const void* x, const void* w, void* y, int M, int N,
 extern "C" int tli_gemm_f32_ranges_of(int M, int N) {
     return M > 0 && M <= 32 && N > 0 && ((long)N + 15) / 16 * 2 <= tli_compute_units() ? GF_RANGES : 0;
 }
+
+// Whether leaving the ranges' sums to the norm or the attention behind costs less than the whole product: not where k is short, as the reader has
+// eight planes to read for one.  us, product and norm, whole and left, 1 and 32 rows: 1,024 columns of k 128 4.9, 5.1 and 5.6, 5.8, of 256 5.2, 5.1
+// and 6.5, 6.1, of 1,024 7.5, 6.2 and 11.0, 7.5; 2,048 of 512 6.7, 7.0 and 8.4, 8.9, of 1,024 7.5, 7.2 and 11.3, 9.9; 2,047, whose planes' rows are
+// read element by element, of 1,024 10.8, 12.5 and 15.8, 15.8, of 2,048 14.0, 13.9 and 22.6, 21.3.
+extern "C" int tli_gemm_f32_ranges_pay(int N, int K) { return N <= 1024 ? K >= 256 : K >= (N % 4 ? 2048 : 1024); }
 
 // parts[GF_RANGES][M][N]: y of tli_gemm_f32 is their sum in order, from zero.
 extern "C" int tli_gemm_f32_ranges(const void* x, const void* w, void* parts, int M, int N, int K, void* stream) {

@@ -28,7 +28,7 @@ class PendingProduct:
     """x W^T not run yet: what ``linear(..., deferred=True)`` returns for a decode step's
     few rows.  ``add_rmsnorm(..., lazy=True)`` runs a bfloat16 one with the residual sum and the
     norm taken into the product, ``add_rmsnorm`` and ``qkv_attention`` a float32 one as partial sums
-    that they add (``_f32_ranges``); anything else runs it as it is (``resolve``)."""
+    that they add (``_f32_sums``); anything else runs it as it is (``resolve``)."""
 
     def __init__(self, x: torch.Tensor, matrix):
         self.x, self.matrix = x, matrix
@@ -88,6 +88,7 @@ def load_library():
         "tli_attention_f32": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, P],
         "tli_qkv_attention_f32": [P, I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, F, P, F, P, P, I, I, I, F, I, P],
         "tli_gemm_f32_ranges_of": [I, I],
+        "tli_gemm_f32_ranges_pay": [I, I],
         "tli_gemm_f32_ranges": [P, P, P, I, I, I, P],
         "tli_gemm_plain": [P, P, P, I, I, I, I, I, I, P],
         "tli_gemm_f32": [P, P, P, I, I, I, I, I, F, I, P],
@@ -417,7 +418,7 @@ class HipOps:
         self._want(weight, "norm weight", torch.float32, (n,))
         if isinstance(delta, PendingProduct):
             if delta.dtype == torch.float32:
-                delta = self._f32_ranges(delta) if out_dtype == torch.float32 else self.resolve(delta)
+                delta = self._f32_sums(delta) if out_dtype == torch.float32 else self.resolve(delta)
             elif lazy and rows is None and not self.separate_norms:
                 return self._product_into_residual(delta, resid, weight, eps)
             else:
@@ -551,6 +552,10 @@ class HipOps:
         """Whether the float32 product on the matrix cores takes these operands: rows of whole 16-byte pieces."""
         return (x.dtype == torch.float32 and w.dtype == torch.float32 and x.shape[1] % 4 == 0
                 and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+    def _f32_sums(self, p: PendingProduct):
+        """A float32 product of few rows for a reader that also adds the sums of ranges: those, or the product where they cost more."""
+        return self._f32_ranges(p) if self.lib.tli_gemm_f32_ranges_pay(p.shape[1], p.x.shape[1]) else self.resolve(p)
 
     def _f32_ranges(self, p: PendingProduct) -> DeferredSum:
         """A float32 product of few rows as the sums of its ranges of k, whose sum in order is what ``linear`` gives."""
@@ -876,7 +881,7 @@ class HipOps:
         other steps run qkv_to_cache and paged_attention.  ``qkv`` may be a ``DeferredSum``:
         the kernel of a decode step adds the partial sums itself."""
         if isinstance(qkv, PendingProduct):
-            qkv = self._f32_ranges(qkv) if qkv.dtype == torch.float32 else self.resolve(qkv)
+            qkv = self._f32_sums(qkv) if qkv.dtype == torch.float32 else self.resolve(qkv)
         if qkv.dtype == torch.float32:
             return self._qkv_attention_f32(qkv, step, cache, heads, kv_heads, head_dim, q_norm, k_norm, rotary, scale, window)
         sums = None
