@@ -30,6 +30,29 @@ struct RawRows {
     int write_cache;
 };
 
+// v[e] = sum_planes(at + 64 e, ..), every element's planes asked for before any is added: one trip to memory where one by one they are E.
+template <int E>
+__device__ __forceinline__ void sum_planes_of(float (&v)[E], const float* __restrict__ at, int planes, size_t plane) {
+    if (planes == 1) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = at[e * 64];
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = 0.f;
+    for (int s = 0; s < planes; s += 8) {
+        float p[8][E];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int e = 0; e < E; ++e) p[k][e] = at[(size_t)min(s + k, planes - 1) * plane + e * 64];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int e = 0; e < E; ++e) v[e] = s + k < planes ? v[e] + p[k][e] : v[e];
+    }
+}
+
 // x[D] in LDS: norm (weight `nw` or null) and rotation of a head that this wavefront takes from `src`, as qkv_to_cache_kernel does them.
 template <int DH>
 __device__ __forceinline__ void head_of_raw_row(float* x, const float* src, size_t plane, const RawRows& raw, const float* nw, float eps,
@@ -37,10 +60,8 @@ __device__ __forceinline__ void head_of_raw_row(float* x, const float* src, size
     constexpr int D = DH * 64;
     float v[DH], w[DH], ss = 0.f;
 #pragma unroll
-    for (int e = 0; e < DH; ++e) {
-        v[e] = sum_planes(src + e * 64 + lane, raw.planes, plane);
-        w[e] = nw ? nw[e * 64 + lane] : 0.f;
-    }
+    for (int e = 0; e < DH; ++e) w[e] = nw ? nw[e * 64 + lane] : 0.f;
+    sum_planes_of(v, src + lane, raw.planes, plane);
 #pragma unroll
     for (int e = 0; e < DH; ++e) ss = fmaf(v[e], v[e], ss);      // (written out: the sums of qkv_to_cache_kernel, bit for bit)
     if (nw) {
@@ -68,7 +89,7 @@ __device__ __forceinline__ void head_of_raw_row(float* x, const float* src, size
 // head of a group writes these into the cache, and every head takes them from LDS, not from the cache, so that nothing waits for a store.
 // The same bits as qkv_to_cache and the kernel without RAW, which is two launches and a trip of q through memory; most of either is launch and
 // latency.  In a recorded chain, 16 heads of 64, projections as eight partial sums, us: 1 row of 30 keys 6.4 -> 4.9, 5 rows of 52 6.9 -> 5.4, 8 of
-// 200 10.8 -> 9.5, 1 of 1,000 29.0 -> 28.6.
+// 200 10.8 -> 9.5, 1 of 1,000 29.0 -> 27.4.
 template <int DH, bool RAW>            // head_dim / 64
 __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
     const float* __restrict__ q, float* __restrict__ out, float* __restrict__ k_cache, float* __restrict__ v_cache, RawRows raw,
@@ -110,9 +131,11 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
                     k_cache[(size_t)page * page_stride + ((size_t)g * page_size + pos % page_size) * D + e * 64 + lane] = own_s[1][e * 64 + lane];
         }
         if (wave == 2 && own) {
+            float sums[DH];
+            sum_planes_of(sums, src + (size_t)(heads + kv_heads + g) * D + lane, raw.planes, plane);
 #pragma unroll
             for (int e = 0; e < DH; ++e) {
-                const float v = cache_value(sum_planes(src + (size_t)(heads + kv_heads + g) * D + e * 64 + lane, raw.planes, plane));
+                const float v = cache_value(sums[e]);
                 own_s[2][e * 64 + lane] = v;
                 if (store) v_cache[(size_t)page * page_stride + ((size_t)g * D + e * 64 + lane) * page_size + pos % page_size] = v;
             }
@@ -130,7 +153,8 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
     for (int i = 0; i < DH; ++i) o[i] = 0.f;
     auto page_of = [&](int t) { return t <= pos ? table[t / page_size] : -1; };
 
-    for (int base = (lo / 16 + wave) * 16; base <= pos; base += 16 * AF_WAVES) {
+    // a block of 16 keys; OWN: RAW, and the row's own key may be among them
+    auto block = [&](int base, auto OWN) __attribute__((always_inline)) {
         const int t = base + j;
         const int page = page_of(t);
         const bool seen = t >= lo && page >= 0 && page < num_pages;
@@ -150,7 +174,7 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
 #pragma unroll
             for (int i = 0; i < DH; ++i) vv[i][u] = *reinterpret_cast<const f32x4*>(vp + (size_t)i * 64 * page_size);
         }
-        if (own && base + 16 > pos) {
+        if (decltype(OWN)::value && own && base + 16 > pos) {
             // the row's own slot, which another workgroup may be writing just now: what was read of it is not used
             if (t == pos)
 #pragma unroll
@@ -174,7 +198,7 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
         float top = score;
 #pragma unroll
         for (int off = 8; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 16));
-        if (!__any(score != -INFINITY)) continue;               // (nothing of this block counts: the same for the whole wave)
+        if (!__any(score != -INFINITY)) return;                 // (nothing of this block counts: the same for the whole wave)
         // (a maximum passes NaNs over, the weights and their sum do not: a row with a NaN in it comes out as NaNs)
         const float m_new = fmaxf(m, top);
         const float p = !seen ? -0.f : score == -INFINITY ? 0.f : expf(score - m_new);
@@ -205,7 +229,17 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
         if (__all(seen)) add(std::true_type{});
         else add(std::false_type{});
         wave_lds_sync();
+    };
+    // RAW: the one block with the row's own key apart from the loop, whose registers and order of loads what is done to it would change.  In it and
+    // apart, projections of k 1,024 included, us: 4 heads of 256, 1 row of 2,000 keys 137.5 and 118.5, 16 rows 128.2 and 113.8; 16 heads of 64 60.5 and 57.6,
+    // 63.9 and 60.7.  Not for heads of 128, where it depends on the keys: 8 heads, 8 rows of 700 32.3 and 30.7, 4 rows of 4,000 140 and 149.
+    constexpr bool APART = RAW && DH != 2;
+    int base = (lo / 16 + wave) * 16;
+    for (; APART ? base + 16 <= pos : base <= pos; base += 16 * AF_WAVES) {
+        if (RAW && !APART) block(base, std::true_type{});
+        else block(base, std::false_type{});
     }
+    if (APART && base <= pos) block(base, std::true_type{});
     if (lane == 0) {
         m_s[wave] = m;
         l_s[wave] = l;
