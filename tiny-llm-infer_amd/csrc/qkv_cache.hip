@@ -15,11 +15,9 @@
 #define QKV_MAX_HEAD_DIM 512
 #define QKV_WAVES 4
 
-// an element of a row, or the sum of its `planes` partial sums (float32 only)
-__device__ __forceinline__ float raw_value(const float* p, int planes, size_t plane) { return sum_planes(p, planes, plane); }
-__device__ __forceinline__ bf16_t raw_value(const bf16_t* p, int, size_t) { return *p; }
-
-template <typename T>
+// SUMS (float32): an element of a row is the sum of its `planes` partial sums.  A form of its own, as asking in the other would cost it: 300 rows of 16
+// heads of 64 6.95 us and 6.70 without, 32 rows of 192 4.19 and 4.07.
+template <typename T, bool SUMS>
 __global__ void qkv_to_cache_kernel(
     const T* __restrict__ qkv, int planes, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache,
     const int* __restrict__ positions, const int* __restrict__ seq_of_row,
@@ -36,6 +34,10 @@ __global__ void qkv_to_cache_kernel(
     const int pos = positions[row];
     const T* src_row = qkv + (size_t)row * stride;
     const size_t plane = (size_t)gridDim.x * stride;
+    auto raw = [&](const T* p) {
+        if constexpr (SUMS) return sum_planes(p, planes, plane);
+        else return *p;
+    };
 
     // where this row's keys and values go
     size_t cache_base = 0, v_base = 0;
@@ -65,7 +67,7 @@ __global__ void qkv_to_cache_kernel(
         const int g = h - heads - kv_heads;
         const T* vsrc = src_row + q_dim + kv_dim + (size_t)g * head_dim;
         for (int d = lane; d < head_dim; d += TLI_WAVE)
-            v_cache[v_base + ((size_t)g * head_dim + d) * page_size] = cache_value(raw_value(vsrc + d, planes, plane));
+            v_cache[v_base + ((size_t)g * head_dim + d) * page_size] = cache_value(raw(vsrc + d));
         return;
     }
     {
@@ -75,7 +77,7 @@ __global__ void qkv_to_cache_kernel(
         const float eps = is_q ? q_eps : k_eps;
         float ss = 0.f;
         for (int i = lane; i < head_dim; i += TLI_WAVE) {
-            const float v = to_f32(raw_value(src + i, planes, plane));
+            const float v = to_f32(raw(src + i));
             x[i] = v;
             ss = fmaf(v, v, ss);
         }
@@ -518,17 +520,15 @@ extern "C" int tli_qkv_to_cache(
 #undef WIDE
         return tli_check_launch("qkv_to_cache_wide");
     }
-    if (dtype == TLI_F32)
-        qkv_to_cache_kernel<float><<<grid, threads, 0, s>>>(
-            (const float*)qkv, planes, (float*)q_out, (float*)k_cache, (float*)v_cache, positions, seq_of_row,
-            tables, table_width, page_size, num_pages, heads, kv_heads, head_dim, q_norm_w, q_eps,
-            k_norm_w, k_eps, cos_table, sin_table, rotary_dim, table_positions, write_cache);
-    else if (dtype == TLI_BF16)
-        qkv_to_cache_kernel<bf16_t><<<grid, threads, 0, s>>>(
-            (const bf16_t*)qkv, 1, (bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, positions, seq_of_row,
-            tables, table_width, page_size, num_pages, heads, kv_heads, head_dim, q_norm_w, q_eps,
-            k_norm_w, k_eps, cos_table, sin_table, rotary_dim, table_positions, write_cache);
+#define QKV_TO_CACHE(T, SUMS)                                                                                                           \
+    qkv_to_cache_kernel<T, SUMS><<<grid, threads, 0, s>>>((const T*)qkv, planes, (T*)q_out, (T*)k_cache, (T*)v_cache, positions, seq_of_row, \
+                                                          tables, table_width, page_size, num_pages, heads, kv_heads, head_dim, q_norm_w, \
+                                                          q_eps, k_norm_w, k_eps, cos_table, sin_table, rotary_dim, table_positions, write_cache)
+    if (dtype == TLI_F32 && planes > 1) QKV_TO_CACHE(float, true);
+    else if (dtype == TLI_F32) QKV_TO_CACHE(float, false);
+    else if (dtype == TLI_BF16) QKV_TO_CACHE(bf16_t, false);
     else
         return tli_fail("qkv_to_cache: unknown dtype %d", dtype);
+#undef QKV_TO_CACHE
     return tli_check_launch("qkv_to_cache");
 }
