@@ -52,3 +52,20 @@ def test_rows_that_it_does_not_take_go_through_the_norm(ops):
         proj, w = torch.randn((rows, width), device=DEV).to(BF), as_matrix(torch.randn((64, k), device=DEV).to(BF), env)
         weight = torch.ones(k, device=DEV)
         assert torch.equal(ops.linear_of_norm(proj, at, k, weight, 1e-5, w), ops.linear(ops.norm_rows(proj, at, k, weight, 1e-5), w))
+
+
+# rows, columns, k at both sides of the rule: 16 and 17 rows, k 1,024, 2,048 and a step more, two tiles a compute unit and a tile more
+@pytest.mark.parametrize("size, together", [((16, 64, 2048), True), ((17, 64, 128), False), ((8, 256, 2176), False), ((3, 8192, 1152), True), ((3, 8208, 1152), False),
+                                            ((3, 8208, 1024), True), ((2, 12288, 2048), False)])
+def test_where_the_norm_is_taken_in(ops, size, together):
+    """Longer rows, and many columns of rows that are not short, go through the norm: the same bits as both launches."""
+    from tiny_llm_infer_amd.parts.base import BuildEnv
+    from tiny_llm_infer_amd.parts.linear import as_matrix
+    M, N, K = size
+    env = BuildEnv(dtype=BF, device=torch.device(DEV), ops=ops, max_model_len=64)
+    g = torch.Generator(device=DEV).manual_seed(K)
+    proj, weight = torch.randn((M, K), generator=g, device=DEV).to(BF), 1 + 0.3 * torch.randn((K,), generator=g, device=DEV)
+    matrix = as_matrix(torch.randn((N, K), generator=g, device=DEV).mul_(K ** -0.5).to(BF), env)
+    got, apart = ops.linear_of_norm(proj, 0, K, weight, 1e-5, matrix), ops.linear(ops.norm_rows(proj, 0, K, weight, 1e-5), matrix)
+    assert torch.equal(got, apart) != together
+    assert float((got.double() - apart.double()).norm() / apart.double().norm()) < 2.0 ** -7        # (a rounding to bfloat16 of each side's rows)

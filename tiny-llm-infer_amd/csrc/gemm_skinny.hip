@@ -688,8 +688,13 @@ extern "C" int tli_gemm_skinny_normed_f32(const void* x, const void* w, void* y,
 // y[M,N] = norm(x) . W^T for rows that are part of wider ones: x [M, K], rows x_ld elements apart, the RMS norm over K with weights norm_w [K].
 // Up to 16 rows, W in the decode layout, k in whole steps of 128.  Every workgroup reads all rows anyway and does their arithmetic again, 100 vector
 // instructions a step beside loads that it waits for; the launch of norm_rows is saved.  Norm and product apart and so, in a recorded
-// chain, us: 3,072 columns of k 1,024, 1 row 5.3 and 4.2, 8 rows 5.7 and 4.3, 16 rows 5.8 and 4.3; of 1,536, 8 rows 6.5 and 5.1; 24,576 of 1,536
-// 15.6 and 15.5.
+// chain, us: 3,072 columns of k 1,024, 1 row 5.3 and 4.2, 8 rows 5.7 and 4.3, 16 rows 5.8 and 4.3; of 1,536, 8 rows 6.5 and 5.1; of 2,048, 8 rows 7.2 and
+// 6.4.  The arithmetic is as long as the launch where a wave has more of it than W's loads hide: k beyond 2,048 (8 rows, k 4,096: 256 columns
+// 7.8 and 8.9, 12,288 22.5 and 27.1) and, from more columns on than two tiles a compute unit, beyond 1,024 (12,288 of 2,048 13.4 and 14.5, of 1,024 9.1 and
+// 8.8; 24,576 of 1,536 16.0 and 16.0).
+extern "C" int tli_gemm_skinny_self_takes(int M, int N, int K) {
+    return M > 0 && M <= 16 && N > 0 && K > 0 && K % 128 == 0 && (K <= 1024 || (K <= 2048 && (N + 15) / 16 <= 2 * tli_compute_units()));
+}
 extern "C" int tli_gemm_skinny_self_bf16(const void* x, int x_ld, const void* w, void* y, int M, int N, int K, const float* norm_w, float eps,
                                          void* stream) {
     if (M <= 0 || N <= 0) return 0;

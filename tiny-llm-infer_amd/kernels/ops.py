@@ -95,6 +95,7 @@ def load_library():
         "tli_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, I, I, F, I, P],
         "tli_gemm_skinny_fused_bf16": [P, P, P, I, I, I, I, P, I, F, P, P, P, P, I, I, F, I, P],
         "tli_gemm_skinny_normed_f32": [P, P, P, I, I, I, P, I, F, P],
+        "tli_gemm_skinny_self_takes": [I, I, I],
         "tli_gemm_skinny_self_bf16": [P, I, P, P, I, I, I, P, F, P],
         "tli_embed_rmsnorm": [P, P, P, P, P, I, I, I, F, I, P],
         "tli_gemm_mid_bf16": [P, P, P, P, I, I, I, I, I, I, I, I, F, I, P],
@@ -2037,10 +2038,10 @@ class HipOps:
     def linear_of_norm(self, proj, at, n, weight, eps, matrix):
         """``linear(norm_rows(proj, at, n, weight, eps), matrix)``; a decode step's few rows in one launch."""
         T, tiled = proj.shape[0], getattr(matrix, "tiled", None)
-        if not (0 < T <= 16 and tiled is not None and proj.dtype == torch.bfloat16 and n % 128 == 0 and proj.shape[1] % 8 == 0 and at % 8 == 0
+        N, K = _shape_of(matrix)
+        if not (tiled is not None and proj.dtype == torch.bfloat16 and proj.shape[1] % 8 == 0 and at % 8 == 0 and self.lib.tli_gemm_skinny_self_takes(T, N, n)
                 and not self.plain_products and not self.separate_norms and self._aligned(proj, weight)):
             return self.linear(self.norm_rows(proj, at, n, weight, eps), matrix)
-        N, K = _shape_of(matrix)
         self._want(proj, "projections")
         self._want(weight, "norm weight", torch.float32, (n,))
         if at < 0 or at + n > proj.shape[1] or K != n:
