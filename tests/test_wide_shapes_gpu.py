@@ -36,3 +36,21 @@ def test_launch_shapes(ops, cols, rows, k):
     normed = NormedRows(x, torch.full((1, rows), 4.0 * k, device=DEV), 0.0)
     assert torch.equal(ops.linear(normed, matrix), (0.5 * wide).to(torch.bfloat16))
     assert torch.equal(ops.linear(normed, matrix, out_dtype=torch.float32), 0.5 * wide)
+
+
+# columns at both sides of 9 and of 12 tiles for four compute units; k under which the shapes have different numbers of waves
+@pytest.mark.parametrize("cols, as_before", [(8208, True), (9200, True), (9201, False), (12288, False), (12289, True), (16368, True)])
+@pytest.mark.parametrize("rows", [1, 16])
+def test_row_major_matrices(ops, cols, as_before, rows):
+    """Right, and in the shape of two tiles and eight waves where the others are slower."""
+    g = torch.Generator(device=DEV).manual_seed(cols + rows)
+    x = torch.randn((rows, 2048), generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.randn((cols, 2048), generator=g, device=DEV).mul_(0.05).to(torch.bfloat16)
+    y = ops.linear(x, w, out_dtype=torch.float32)
+    assert near(y, x, w)
+    ops.skinny_cfg = 28
+    try:
+        pairs = ops.linear(x, w, out_dtype=torch.float32)
+    finally:
+        ops.skinny_cfg = 0
+    assert torch.equal(y, pairs) == as_before

@@ -484,12 +484,13 @@ static bool half_tiles(int M, int N, int K, int tiled, bool into_residual) {
 // 28, 14, 18 and 24: 9,216 columns of k 2,048, 1 row 10.9, 9.6, 9.8 and 10.2, of 4,096 18.2, 16.9, 16.1 and 18.4; 11,264 columns, 6 rows 11.8,
 // 10.6, 11.4 and 11.2, of 4,096 20.4, 18.7, 18.3 and 20.9, 16 rows 13.0, 12.5, 12.4 and 12.6; 12,288 12.5, 10.9, 12.3 and 11.6; 14,336
 // columns, 6 rows 13.0, 13.0, 13.2 and 12.2, of 5,120 24 is 1.8% behind 28.  Gated products, whose tiles come in pairs, stay with 28: 24 is 1 to
-// 4% behind.
-static int wide_shape(int N, int K, bool gated) {
+// 4% behind.  Row-major matrices (tiled 0) stay with it outside 9 to 12 tiles for four compute units, 28 and the rule's other shape, us: 8,208 columns of k 5,120, 6
+// and 16 rows 23.8, 23.6 and 28.2, 30.3; 9,216 26.8, 21.7 (1 row) and 33.6, 32.6; 12,288 30.8, 27.8 and 35.4, 35.6; 14,336 of 2,048 15.1, 15.4 and 17.5, 17.4.
+static int wide_shape(int N, int K, int tiled) {
     const long tiles = (N + 15) / 16, units = tli_compute_units();
-    const bool shorter = K < 4096;
+    const bool shorter = K < 4096, pairs = tiled == 2 || (tiled == 0 && (tiles < 2 * units + units / 4 || tiles > 3 * units));
     if (tiles <= units) return 18;
-    if (tiles <= 2 * units || gated || (tiles > 3 * units && !shorter)) return tiles < 4 * units ? 28 : 24;
+    if (tiles <= 2 * units || pairs || (tiles > 3 * units && !shorter)) return tiles < 4 * units ? 28 : 24;
     return tiles > 3 * units ? 24 : shorter ? 14 : 18;
 }
 
@@ -499,7 +500,7 @@ static int pick_skinny(const bf16_t* x, const bf16_t* w, void* y, int M, int N, 
     // cfg 0: by shape.  Narrow outputs get one 16-column tile per workgroup so that
     // even N = 4096 gives 256 workgroups; wide outputs share x over two tiles.
     const long tiles = (N + 15) / 16;
-    if (cfg == 0 && MT == 1) cfg = half_tiles(M, N, K, tiled, false) ? 8 : wide_shape(N, K, tiled == 2);
+    if (cfg == 0 && MT == 1) cfg = half_tiles(M, N, K, tiled, false) ? 8 : wide_shape(N, K, tiled);
     if (cfg == 0) cfg = tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
     if (tiled == 2 && cfg < 20) cfg = 24;          // gated needs pairs of row tiles
     switch (cfg) {
@@ -597,7 +598,7 @@ static int launch_skinny_fused(const bf16_t* x, const bf16_t* w, bf16_t* y, int 
 // The launch shape `cfg` of the product with a norm taken in (0: by the sizes), and whether it takes half tiles.
 static int fused_shape(int M, int N, int K, int gated, bool into_residual, int cfg) {
     const long tiles = (N + 15) / 16;
-    if (cfg == 0 && !into_residual) cfg = !gated && half_tiles(M, N, K, 1, false) ? 8 : wide_shape(N, K, gated);
+    if (cfg == 0 && !into_residual) cfg = !gated && half_tiles(M, N, K, 1, false) ? 8 : wide_shape(N, K, gated ? 2 : 1);
     if (cfg == 0) cfg = half_tiles(M, N, K, 1, true) ? 8 : tiles <= tli_compute_units() ? 18 : (tiles < 4 * tli_compute_units() ? 28 : 24);
     return gated && cfg < 20 ? 24 : cfg;
 }
