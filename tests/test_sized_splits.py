@@ -23,3 +23,11 @@ def test_runs_of_rows(rows, reach, want):
 def test_what_was_not_measured_stays():
     assert splits(32, 8192, units=32) == 8 and splits(32, 8192, keep=4) == 8          # other kernel; kept first keys
     assert splits(32, 8192, window=500) == 8 and splits(16, 8192, units=32, key_heads=2) == 16
+
+
+@pytest.mark.parametrize("rows, reach, want", [(8, 8192, 32), (1, 8192, 64), (16, 8192, 32), (64, 1024, 8)])
+def test_narrow_vectors_go_into_fewer_runs(rows, reach, want):
+    """Short vectors are read faster than many runs' sums of them are merged: 64 runs only where there are no more rows."""
+    stub = types.SimpleNamespace(sized_splits=None, SIZED_WORKGROUPS=HipOps.SIZED_WORKGROUPS, SIZED_SPLIT_KEYS=HipOps.SIZED_SPLIT_KEYS,
+                                 SIZED_WIDE_KEYS=HipOps.SIZED_WIDE_KEYS)
+    assert HipOps._sized_splits(stub, rows, reach, 16, 1, None, 0, 128) == want

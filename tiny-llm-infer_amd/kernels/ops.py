@@ -1914,7 +1914,7 @@ class HipOps:
             tiles = T if grouped else sum((starts[i + 1] - starts[i] + 15) // 16 for i in range(step.num_seqs))
             splits, parts = 1, None
             if grouped and vc is None and out_dtype == torch.bfloat16 and step.num_seqs == T:
-                splits = self._sized_splits(T, step.reach, heads * maps, kv_heads * maps, window, keep)
+                splits = self._sized_splits(T, step.reach, heads * maps, kv_heads * maps, window, keep, key_dim)
                 if splits > 1:
                     parts = torch.empty((T * heads * maps * splits * (value_dim + 4),), dtype=torch.float32, device=self.device)
                 if maps == 1 and heads // kv_heads <= 16 and not keep:      # (one wave of the general kernel's four would have heads)
@@ -1972,19 +1972,22 @@ class HipOps:
     # There twice as many workgroups where each still has SIZED_WIDE_KEYS of the keys that the rows may have (us, 256 and 512: 16 rows of
     # 2,100 27.0 and 24.8, of 8,000 61.7 and 45.0; 32 of 1,040 26.4 and 25.0, of 8,000 123 and 80; 64 of 520 26.7 and 25.1, of 1,000
     # 37.0 and 29.9; 128 of 300 27.9 and 25.7, of 2,000 124 and 81; 8 of 8,000 37.5 and 31.9).  With half the keys it depends on the rows:
-    # 8 of 2,100 20.1 and 22.2, of 4,000 24.9 and 24.3; 32 of 520 19.2 and 20.3, of 1,000 24.0 and 23.1.
+    # 8 of 2,100 20.1 and 22.2, of 4,000 24.9 and 24.3; 32 of 520 19.2 and 20.3, of 1,000 24.0 and 23.1.  All of these 16 heads of 512 + 64; 1, 4 and 8 of
+    # them, and 2 to 16 of 256 + 32, gain as much or more (8 heads, 8 of 4,100 26.0 and 24.0; 64 of 1,000 34.7 and 27.2; of 256 + 32 19.3 and 18.3, 25.7 and
+    # 19.5), also where all rows but one have 100 keys.  Vectors of less than 288 elements only up to 32 runs, of which the second pass reads and adds less
+    # (16 heads of 96 + 32, 32 and 64 runs, 8 of 4,100 13.7 and 14.5, of 8,000 17.5 and 16.0).
     SIZED_WORKGROUPS = 256
     SIZED_SPLIT_KEYS = 32
     SIZED_WIDE_KEYS = 128
 
-    def _sized_splits(self, T, reach, units, key_heads, window, keep) -> int:
+    def _sized_splits(self, T, reach, units, key_heads, window, keep, key_dim=576) -> int:
         """Over how many workgroups the keys of one (row, key head) that decodes are shared out, where all heads read one cached
         vector; ``reach``: a power of two that the longest sequence fits.  A workgroup walks its run of a row's keys in
         tiles of 16 or, with up to 16 heads a key head, 32 (csrc/attention_sized_mfma.hip)."""
         keys = min(reach, (window + 15 if window else reach) + keep)
         groups = T * key_heads * ((units // key_heads + 63) // 64)
         splits = min(self.SIZED_WORKGROUPS // groups, keys // self.SIZED_SPLIT_KEYS, 64)
-        wide = min(2 * self.SIZED_WORKGROUPS // groups, 64)
+        wide = min(2 * self.SIZED_WORKGROUPS // groups, 64 if key_dim >= 288 else 32)
         if units // key_heads <= 16 and not keep and keys >= wide * self.SIZED_WIDE_KEYS:
             splits = max(splits, wide)
         return max(1, self.sized_splits or splits)
