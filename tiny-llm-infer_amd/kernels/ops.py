@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import os
 from ctypes import c_float, c_int, c_void_p
 from typing import Optional, Tuple
@@ -261,6 +262,9 @@ class HipOps:
         with torch.cuda.device(self.device):
             self.DECODE_WORKGROUPS = int(self.lib.tli_device_compute_units())
             self.F32_RANGES = int(self.lib.tli_gemm_f32_ranges_of(1, 16))
+        # by the sizes alone, asked of the library once for each: a step that is not recorded is as long as its host work, and a call takes 0.4 us
+        self._f32_ranges_of = functools.lru_cache(1024)(self.lib.tli_gemm_f32_ranges_of)
+        self._f32_ranges_pay = functools.lru_cache(1024)(self.lib.tli_gemm_f32_ranges_pay)
         self._held_stream = None
         self.force_plain = False     # tests: run the plain attention kernel for bfloat16 too
         self.plain_products = False  # every matrix product through the plain kernel
@@ -492,7 +496,7 @@ class HipOps:
             raise KernelError(f"linear: input has {K} columns, the matrix {K2}")
         self._want(x, "linear input")
         if ((deferred or sums_only) and x.dtype == torch.float32 and tiled is None and out_dtype in (None, torch.float32)
-                and not self.separate_norms and self.lib.tli_gemm_f32_ranges_of(M, N) and self._f32_product_takes(x, getattr(w, "w", w))):
+                and not self.separate_norms and self._f32_ranges_of(M, N) and self._f32_product_takes(x, getattr(w, "w", w))):
             return PendingProduct(x, w)
         w_dtype = getattr(matrix, "dtype", None) or matrix.w.dtype
         if x.dtype != w_dtype:
@@ -556,7 +560,7 @@ class HipOps:
 
     def _f32_sums(self, p: PendingProduct):
         """A float32 product of few rows for a reader that also adds the sums of ranges: those, or the product where they cost more."""
-        return self._f32_ranges(p) if self.lib.tli_gemm_f32_ranges_pay(p.shape[1], p.x.shape[1]) else self.resolve(p)
+        return self._f32_ranges(p) if self._f32_ranges_pay(p.shape[1], p.x.shape[1]) else self.resolve(p)
 
     def _f32_ranges(self, p: PendingProduct) -> DeferredSum:
         """A float32 product of few rows as the sums of its ranges of k, whose sum in order is what ``linear`` gives."""
