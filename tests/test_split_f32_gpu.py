@@ -137,3 +137,10 @@ def test_short_products_are_read_whole(ops, nk, pay):
 def test_own_key_at_the_edges_of_blocks(ops, hd, window):
     """The row's own key first, in the middle and last of a block of 16 keys, alone in one, and in every wave's share."""
     test_attention_from_projections_left_in_ranges(ops, (4, 2, hd, 16, True, hd, [1, 2, 16, 17, 32, 33, 48, 49, 64, 65, 80, 81, 130], None, window, True))
+
+
+@pytest.mark.parametrize("heads, rows", [(16, 16), (16, 17), (24, 13)])
+def test_own_key_of_heads_of_128_on_both_sides_of_a_workgroup_a_compute_unit(ops, heads, rows):
+    """Up to one it is handled in the loop over the keys, from there on apart."""
+    lens = [1, 2, 16, 17, 32, 33, 48, 49, 64, 65, 80, 81, 130, 15, 96, 97, 31][:rows]
+    test_attention_from_projections_left_in_ranges(ops, (heads, 2, 128, 16, True, 128, lens, None, None, True))

@@ -90,7 +90,8 @@ __device__ __forceinline__ void head_of_raw_row(float* x, const float* src, size
 // The same bits as qkv_to_cache and the kernel without RAW, which is two launches and a trip of q through memory; most of either is launch and
 // latency.  In a recorded chain, 16 heads of 64, projections as eight partial sums, us: 1 row of 30 keys 6.4 -> 4.9, 5 rows of 52 6.9 -> 5.4, 8 of
 // 200 10.8 -> 9.5, 1 of 1,000 29.0 -> 27.4.
-template <int DH, bool RAW>            // head_dim / 64
+// APART: the one block with the row's own key apart from the loop, whose registers and order of loads what is done to it would change (RAW only).
+template <int DH, bool RAW, bool APART>            // head_dim / 64
 __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
     const float* __restrict__ q, float* __restrict__ out, float* __restrict__ k_cache, float* __restrict__ v_cache, RawRows raw,
     const int* __restrict__ positions, const int* __restrict__ seq_of_row, const int* __restrict__ tables, int table_width,
@@ -230,10 +231,6 @@ __global__ void __launch_bounds__(AF_WAVES * 64) attention_f32_kernel(
         else add(std::false_type{});
         wave_lds_sync();
     };
-    // RAW: the one block with the row's own key apart from the loop, whose registers and order of loads what is done to it would change.  In it and
-    // apart, projections of k 1,024 included, us: 4 heads of 256, 1 row of 2,000 keys 137.5 and 118.5, 16 rows 128.2 and 113.8; 16 heads of 64 60.5 and 57.6,
-    // 63.9 and 60.7.  Not for heads of 128, where it depends on the keys: 8 heads, 8 rows of 700 32.3 and 30.7, 4 rows of 4,000 140 and 149.
-    constexpr bool APART = RAW && DH != 2;
     int base = (lo / 16 + wave) * 16;
     for (; APART ? base + 16 <= pos : base <= pos; base += 16 * AF_WAVES) {
         if (RAW && !APART) block(base, std::true_type{});
@@ -269,14 +266,21 @@ template <bool RAW>
 static void launch_attention_f32(dim3 grid, const float* q, float* out, float* k_cache, float* v_cache, const RawRows& raw, const int* positions,
                                  const int* seq_of_row, const int* tables, int table_width, int page_size, int num_pages, int heads,
                                  int kv_heads, int head_dim, float scale, int window, hipStream_t s) {
-#define TLI_AF(DH)                                                                                                                         \
-    attention_f32_kernel<DH, RAW><<<grid, AF_WAVES * 64, 0, s>>>(q, out, k_cache, v_cache, raw, positions, seq_of_row, tables, table_width, \
-                                                                 page_size, num_pages, heads, kv_heads, scale, window)
+#define TLI_AF(DH, APART)                                                                                                                  \
+    attention_f32_kernel<DH, RAW, APART><<<grid, AF_WAVES * 64, 0, s>>>(q, out, k_cache, v_cache, raw, positions, seq_of_row, tables,        \
+                                                                        table_width, page_size, num_pages, heads, kv_heads, scale, window)
+    // The row's own key in the loop and apart, projections of k 1,024 included, us: 4 heads of 256, 1 row of 2,000 keys 137.5 and 118.5, 16 rows 128.2
+    // and 113.8; 16 heads of 64 60.5 and 57.6, 63.9 and 60.7.  Heads of 128 are better off in the loop while there is no more than a workgroup a compute
+    // unit, and worse from two on (attention alone; two launches, in the loop, apart): 32 heads, 8 rows of 700 keys 32.4, 28.0 and 30.1, of 4,000 148, 135 and
+    // 147; 16 rows of 2,000 99.4, 102.5 and 96.3; 16 heads, 32 rows of 4,000 255, 263 and 250.
     switch (head_dim / 64) {
-        case 1: TLI_AF(1); break;
-        case 2: TLI_AF(2); break;
-        case 3: TLI_AF(3); break;
-        default: TLI_AF(4); break;
+        case 1: TLI_AF(1, RAW); break;
+        case 2:
+            if (RAW && (long)grid.x * grid.y > tli_compute_units()) TLI_AF(2, RAW);
+            else TLI_AF(2, false);
+            break;
+        case 3: TLI_AF(3, RAW); break;
+        default: TLI_AF(4, RAW); break;
     }
 #undef TLI_AF
 }
