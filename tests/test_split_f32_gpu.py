@@ -139,8 +139,8 @@ def test_own_key_at_the_edges_of_blocks(ops, hd, window):
     test_attention_from_projections_left_in_ranges(ops, (4, 2, hd, 16, True, hd, [1, 2, 16, 17, 32, 33, 48, 49, 64, 65, 80, 81, 130], None, window, True))
 
 
-@pytest.mark.parametrize("heads, rows", [(16, 16), (16, 17), (24, 13)])
+@pytest.mark.parametrize("heads, rows", [(12, 21), (12, 22), (8, 32), (8, 13)])
 def test_own_key_of_heads_of_128_on_both_sides_of_a_workgroup_a_compute_unit(ops, heads, rows):
     """Up to one it is handled in the loop over the keys, from there on apart."""
-    lens = [1, 2, 16, 17, 32, 33, 48, 49, 64, 65, 80, 81, 130, 15, 96, 97, 31][:rows]
+    lens = ([1, 2, 16, 17, 32, 33, 48, 49, 64, 65, 80, 81, 130] * 3)[:rows]
     test_attention_from_projections_left_in_ranges(ops, (heads, 2, 128, 16, True, 128, lens, None, None, True))
