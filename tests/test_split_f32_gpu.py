@@ -144,3 +144,16 @@ def test_own_key_of_heads_of_128_on_both_sides_of_a_workgroup_a_compute_unit(ops
     """Up to one it is handled in the loop over the keys, from there on apart."""
     lens = ([1, 2, 16, 17, 32, 33, 48, 49, 64, 65, 80, 81, 130] * 3)[:rows]
     test_attention_from_projections_left_in_ranges(ops, (heads, 2, 128, 16, True, 128, lens, None, None, True))
+
+
+def test_a_step_with_many_workgroups_is_two_launches(ops, monkeypatch):
+    """By the rule, and the same bits as one launch of it."""
+    rows, heads, hd = 300, 16, 192
+    step, _, pos, _ = make_step([1 + i % 20 for i in range(rows)], [1] * rows, 16, 2 * rows + 3, 7, 4, hd, F32)
+    qkv, outs, given = rnd((rows, (heads + 8) * hd), 5), [], []
+    call = ops._call
+    monkeypatch.setattr(ops, "_call", lambda fn, *args: (given.append(args[2]) if fn == ops.lib.tli_qkv_attention_f32 else None, call(fn, *args))[1])
+    for reach in (step.reach, 256):                      # rows of more keys: one launch
+        step.reach = reach
+        outs.append(ops.qkv_attention(qkv, step, step.cache, heads, 4, hd, None, None, None, hd ** -0.5, None))
+    assert given[0] is not None and given[1] is None and torch.equal(*outs)

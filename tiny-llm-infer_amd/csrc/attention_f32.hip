@@ -311,6 +311,20 @@ extern "C" int tli_qkv_to_cache(const void* qkv, int planes, void* q_out, void* 
                                 const float* q_norm_w, float q_eps, const float* k_norm_w, float k_eps, const float* cos_table,
                                 const float* sin_table, int rotary_dim, int table_positions, int write_cache, int skip_values, int dtype, void* stream);
 
+// Whether a decode step's rows of up to `keys` keys are sooner done in one launch from the projections than in two.  Every workgroup makes its own
+// query and its group's key and value, and has more registers for it, so two launches are as good where the workgroups are many times what the chip
+// holds and each has few keys, with heads of 256 any number of them; and, where no heads share a key, from 2 GB of keys and values on, which come from memory at its
+// rate.  us, two launches and one: 512 rows of 20 keys, 32 heads of 64 43.1, 49.2, of 60 62.2, 62.7; 8 heads of 192 34.0, 35.7 and 55.2, 59.8, of 250 204, 199; 8 heads of 256
+// 47.0, 53.2 and 80.0, 85.7, 16 of them with 500 keys 1,212, 1,234; 16 heads of 128 with a key each, 128 rows of 1,000 366, 380, of 300 128.5, 123.3.
+// At the limits: 4,096 heads of rows of 64, 20 keys 14.6, 14.5, 50 keys 20.7, 18.8; of 128 23.6, 23.4 and 35.6, 33.6; 2,048 of 192 20.5, 19.8 and 28.9, 28.3; 1,536 of 256
+// 20.3, 20.1 and 30.3, 28.3, 2,048 of 300 keys 128, 124.
+extern "C" int tli_qkv_attention_f32_one(int rows, int heads, int kv_heads, int head_dim, int keys) {
+    const long wgs = (long)rows * heads, units = tli_compute_units(), elements = wgs * head_dim;
+    if (heads == kv_heads) return keys <= 128 || elements < 1024 * units || elements * keys < 1024 * 1024 * units;
+    if (keys <= 128) return wgs <= (head_dim <= 128 ? 16 : head_dim <= 192 ? 8 : 6) * units;
+    return head_dim <= 192 || wgs <= 8 * units;
+}
+
 // From the rows' projections qkv [planes][rows][(heads + 2 kv_heads) head_dim] (planes > 1: partial sums to be added) to the attention's output.
 // `q` null: a decode step (one row a sequence) in one launch.  Else q [rows][heads * head_dim] takes the queries and it is tli_qkv_to_cache,
 // then tli_attention_f32: a row of a portion also reads the keys of the rows before it.

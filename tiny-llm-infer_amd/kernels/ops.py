@@ -87,6 +87,7 @@ def load_library():
         "tli_attention_plain": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, I, P],
         "tli_attention_f32_takes": [I, I],
         "tli_attention_f32": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, P],
+        "tli_qkv_attention_f32_one": [I, I, I, I, I],
         "tli_qkv_attention_f32": [P, I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, F, P, F, P, P, I, I, I, F, I, P],
         "tli_gemm_f32_ranges_of": [I, I],
         "tli_gemm_f32_ranges_pay": [I, I],
@@ -941,7 +942,7 @@ class HipOps:
         return out
 
     def _qkv_attention_f32(self, qkv, step, cache, heads, kv_heads, head_dim, q_norm, k_norm, rotary, scale, window):
-        """``qkv_attention`` in float32: one call where the sizes allow, which is one launch for a decode step."""
+        """``qkv_attention`` in float32: one call where the sizes allow, which is one launch for a decode step where that is the sooner done."""
         T, sums = step.num_rows, isinstance(qkv, DeferredSum)
         planes, raw = (qkv.parts.shape[0], qkv.parts) if sums else (1, qkv)
         kc, vc = (cache.record("k"), cache.record("v")) if cache is not None else (None, None)
@@ -959,7 +960,10 @@ class HipOps:
                 self._want(w, "head norm weight", torch.float32, (head_dim,))
         cos, sin, rd = self._rotary(rotary, step) if rotary is not None else (None, None, 0)
         out = torch.empty((T, heads * head_dim), dtype=torch.float32, device=self.device)
-        q = torch.empty_like(out) if step.max_rows_per_seq != 1 or self.unfused_decode else None
+        keys = min(step.reach, window) if window else step.reach
+        one = (step.max_rows_per_seq == 1 and not self.unfused_decode
+               and self.lib.tli_qkv_attention_f32_one(T, heads, kv_heads, head_dim, keys))
+        q = None if one else torch.empty_like(out)
         self._call(self.lib.tli_qkv_attention_f32, raw.data_ptr(), planes, _ptr(q), out.data_ptr(), kc.data_ptr(), vc.data_ptr(),
                    step.positions.data_ptr(), step.seq_of_row.data_ptr(), g.tables.data_ptr(), g.table_width, g.page_size, kc.shape[0], T,
                    heads, kv_heads, head_dim, _ptr(qw), float(qe), _ptr(kw), float(ke), _ptr(cos), _ptr(sin), rd,
