@@ -55,8 +55,16 @@ struct RowDelta {
     int parts;
     size_t plane;
     __device__ __forceinline__ bool any() const { return d != nullptr || parts > 0; }
+    // EIGHT: asked for eight at once, which a float32 product leaves; a bfloat16 one leaves two or four
+    template <bool EIGHT>
     __device__ __forceinline__ float at(int i) const {
-        return parts > 0 ? rounded_to<T>(sum_planes(p + i, parts, plane)) : to_f32(d[i]);
+        if (EIGHT) return rounded_to<T>(sum_planes(p + i, parts, plane));
+        if (parts > 0) {
+            float a = 0.f;
+            for (int s = 0; s < parts; ++s) a += p[s * plane + i];
+            return rounded_to<T>(a);
+        }
+        return to_f32(d[i]);
     }
 };
 
@@ -68,7 +76,10 @@ __device__ __forceinline__ RowDelta<T> row_delta(const void* delta, int parts, i
     return rd;
 }
 
-template <typename T>
+// EIGHT (here and below): rows of a float32 product left as eight planes of sums.  Forms of their own, as the registers of eight planes cost the others (us,
+// with them and without: float32 rows without sums, 512 of 4,096 elements 6.5 and 5.8, 4,096 rows 43.6 and 39.6; bfloat16, 4,065 elements, 1,015 rows in four planes
+// and the product before 78.1 and 69.4).
+template <typename T, bool EIGHT>
 __global__ void add_rmsnorm_kernel(float* __restrict__ resid, const void* __restrict__ delta, int parts,
                                    const float* __restrict__ weight, T* __restrict__ out,
                                    const int* __restrict__ rows, int n, float eps, int total_rows) {
@@ -82,7 +93,7 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ resid, const void* __rest
     float ss = 0.f;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         float v = x[i];
-        if (d.any()) v += d.at(i);
+        if (d.any()) v += d.template at<EIGHT>(i);
         if (update) x[i] = v;
         ss += v * v;
     }
@@ -91,7 +102,7 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ resid, const void* __rest
     T* o = out + (size_t)out_row * n;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         float v = x[i];
-        if (d.any() && !update) v += d.at(i);
+        if (d.any() && !update) v += d.template at<EIGHT>(i);
         from_f32(o + i, weight[i] * v * scale);
     }
 }
@@ -118,11 +129,11 @@ __device__ __forceinline__ void store4(bf16_t* p, const float v[4]) {
 }
 
 // EMBED: the rows are those of a table [vocab, n] that `rows` names, and become the residual's.
-template <typename T, int IT, bool EMBED = false>
+template <typename T, int IT, bool EMBED = false, bool EIGHT = false>
 __global__ void add_rmsnorm_vec_kernel(float* __restrict__ resid, const void* __restrict__ delta, int parts,
                                        const float* __restrict__ weight, T* __restrict__ out,
                                        const int* __restrict__ rows, int n, float eps, int total_rows, const T* __restrict__ table) {
-    constexpr int AT_ONCE = sizeof(T) == 4 ? 8 : 4;        // (a float32 product leaves eight planes, a bfloat16 one rarely more than four)
+    constexpr int AT_ONCE = EIGHT ? 8 : 4;        // (a bfloat16 product rarely leaves more than four)
     __shared__ float scratch[16];
     const int out_row = blockIdx.x;
     int r = rows ? rows[out_row] : out_row;
@@ -185,21 +196,20 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ resid, const void* __
     }
 }
 
-template <typename T>
+template <typename T, bool EIGHT>
 static void launch_add_rmsnorm(float* resid, const void* delta, int parts, const float* weight, T* out,
                                const int* rows, int out_rows, int total_rows, int n, float eps, hipStream_t s) {
     const int groups = n / 4;
     if (n % 4 == 0 && groups <= 4096) {
         int threads = groups <= 1024 ? (groups + 63) / 64 * 64 : 1024;
-        if (groups <= 1024)
-            add_rmsnorm_vec_kernel<T, 1><<<out_rows, threads, 0, s>>>(resid, delta, parts, weight, out, rows, n, eps, total_rows, nullptr);
-        else if (groups <= 2048)
-            add_rmsnorm_vec_kernel<T, 2><<<out_rows, threads, 0, s>>>(resid, delta, parts, weight, out, rows, n, eps, total_rows, nullptr);
-        else
-            add_rmsnorm_vec_kernel<T, 4><<<out_rows, threads, 0, s>>>(resid, delta, parts, weight, out, rows, n, eps, total_rows, nullptr);
+#define ADD_NORM(IT) add_rmsnorm_vec_kernel<T, IT, false, EIGHT><<<out_rows, threads, 0, s>>>(resid, delta, parts, weight, out, rows, n, eps, total_rows, nullptr)
+        if (groups <= 1024) ADD_NORM(1);
+        else if (groups <= 2048) ADD_NORM(2);
+        else ADD_NORM(4);
+#undef ADD_NORM
         return;
     }
-    add_rmsnorm_kernel<T><<<out_rows, n >= 2048 ? 512 : 256, 0, s>>>(resid, delta, parts, weight, out, rows, n, eps, total_rows);
+    add_rmsnorm_kernel<T, EIGHT><<<out_rows, n >= 2048 ? 512 : 256, 0, s>>>(resid, delta, parts, weight, out, rows, n, eps, total_rows);
 }
 
 template <typename T>
@@ -280,9 +290,10 @@ extern "C" int tli_add_rmsnorm(float* resid, const void* delta, const float* wei
     if (parts < 0 || (parts > 0 && !delta)) return tli_fail("add_rmsnorm: no partial sums (%d)", parts);
     hipStream_t s = (hipStream_t)stream;
     if (dtype == TLI_F32)
-        launch_add_rmsnorm<float>(resid, delta, parts, weight, (float*)out, rows, out_rows, total_rows, n, eps, s);
+        (parts > 0 ? launch_add_rmsnorm<float, true> : launch_add_rmsnorm<float, false>)(resid, delta, parts, weight, (float*)out, rows, out_rows, total_rows,
+                                                                                         n, eps, s);
     else if (dtype == TLI_BF16)
-        launch_add_rmsnorm<bf16_t>(resid, delta, parts, weight, (bf16_t*)out, rows, out_rows, total_rows, n,
+        launch_add_rmsnorm<bf16_t, false>(resid, delta, parts, weight, (bf16_t*)out, rows, out_rows, total_rows, n,
                                    eps, s);
     else
         return tli_fail("add_rmsnorm: unknown dtype %d", dtype);
