@@ -157,3 +157,9 @@ def test_a_step_with_many_workgroups_is_two_launches(ops, monkeypatch):
         step.reach = reach
         outs.append(ops.qkv_attention(qkv, step, step.cache, heads, 4, hd, None, None, None, hd ** -0.5, None))
     assert given[0] is not None and given[1] is None and torch.equal(*outs)
+
+
+@pytest.mark.parametrize("nk, pay", [((848, 392), False), ((848, 384), True), ((800, 640), True), ((512, 392), True), ((250, 256), True), ((322, 256), False),
+                                     ((322, 512), True), ((893, 1020), False), ((893, 1024), True)])
+def test_uneven_ranges_and_rows_read_element_by_element_are_left_later(ops, nk, pay):
+    test_short_products_are_read_whole(ops, nk, pay)

@@ -257,10 +257,15 @@ extern "C" int tli_gemm_f32_ranges_of(int M, int N) {
 }
 
 // Whether leaving the ranges' sums to the norm or the attention behind costs less than the whole product: not where k is short, as the reader has
-// eight planes to read for one.  us, product and norm, whole and left, 1 and 32 rows: 1,024 columns of k 128 4.9, 5.1 and 5.6, 5.8, of 256 5.2, 5.1
-// and 6.5, 6.1, of 1,024 7.5, 6.2 and 11.0, 7.5; 2,048 of 512 6.7, 7.0 and 8.4, 8.9, of 1,024 7.5, 7.2 and 11.3, 9.9; 2,047, whose planes' rows are
-// read element by element, of 1,024 10.8, 12.5 and 15.8, 15.8, of 2,048 14.0, 13.9 and 22.6, 21.3.
-extern "C" int tli_gemm_f32_ranges_pay(int N, int K) { return N <= 1024 ? K >= 256 : K >= (N % 4 ? 2048 : 1024); }
+// eight planes to read for one, nor where the eight ranges of a short k are not alike.  us, product and norm, whole and left, 1 and 32 rows: 1,024 columns of k 128 4.9, 5.1
+// and 5.6, 5.8, of 256 5.2, 5.1 and 6.5, 6.1, of 1,024 7.5, 6.2 and 11.0, 7.5; 848 of k 392 5.7, 6.3 and 6.8, 7.5, 800 of 640 5% less; 2,048 of 512 6.7, 7.0 and 8.4, 8.9, of
+// 1,024 7.5, 7.2 and 11.3, 9.9.  Rows that are no multiple of four are read element by element, which costs more of them: 250 of 256 6% less (1 row), 322 of 256
+// 6% more, of 512 level, 893 of 512 7.7, 8.4 (1 row), of 1,024 5% less; 2,046 of 1,024 12% more, of 2,048 level.
+extern "C" int tli_gemm_f32_ranges_pay(int N, int K) {
+    if (N % 4) return K >= (N <= 256 ? 256 : N <= 512 ? 512 : N <= 1024 ? 1024 : 2048);
+    if (N > 1024) return K >= 1024;
+    return K >= (N > 512 && K % (16 * GF_RANGES) ? 640 : 256);
+}
 
 // parts[GF_RANGES][M][N]: y of tli_gemm_f32 is their sum in order, from zero.
 extern "C" int tli_gemm_f32_ranges(const void* x, const void* w, void* parts, int M, int N, int K, void* stream) {
