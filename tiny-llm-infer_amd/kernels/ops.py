@@ -31,8 +31,9 @@ class PendingProduct:
     norm taken into the product, ``add_rmsnorm`` and ``qkv_attention`` a float32 one as partial sums
     that they add (``_f32_sums``); anything else runs it as it is (``resolve``)."""
 
-    def __init__(self, x: torch.Tensor, matrix):
+    def __init__(self, x: torch.Tensor, matrix, pays: Optional[bool] = None):
         self.x, self.matrix = x, matrix
+        self.pays = pays         # float32: whether partial sums cost less (None: not asked yet)
         self.shape = (x.shape[0], _shape_of(matrix)[0])
         self.dtype = x.dtype
 
@@ -263,9 +264,10 @@ class HipOps:
         with torch.cuda.device(self.device):
             self.DECODE_WORKGROUPS = int(self.lib.tli_device_compute_units())
             self.F32_RANGES = int(self.lib.tli_gemm_f32_ranges_of(1, 16))
-        # by the sizes alone, asked of the library once for each: a step that is not recorded is as long as its host work, and a call takes 0.4 us
-        self._f32_ranges_of = functools.lru_cache(1024)(self.lib.tli_gemm_f32_ranges_of)
-        self._f32_ranges_pay = functools.lru_cache(1024)(self.lib.tli_gemm_f32_ranges_pay)
+        # (rows, outputs, k) -> whether the sums of a float32 product's ranges cost a reader that adds them less than the product; None: they are not
+        # left.  Asked of the library once for each: a step that is not recorded is as long as its host work, and a call takes 0.4 us.
+        lib = self.lib
+        self._f32_left = functools.lru_cache(1024)(lambda M, N, K: bool(lib.tli_gemm_f32_ranges_pay(N, K)) if lib.tli_gemm_f32_ranges_of(M, N) else None)
         self._held_stream = None
         self.force_plain = False     # tests: run the plain attention kernel for bfloat16 too
         self.plain_products = False  # every matrix product through the plain kernel
@@ -497,8 +499,8 @@ class HipOps:
             raise KernelError(f"linear: input has {K} columns, the matrix {K2}")
         self._want(x, "linear input")
         if ((deferred or sums_only) and x.dtype == torch.float32 and tiled is None and out_dtype in (None, torch.float32)
-                and not self.separate_norms and self._f32_ranges_of(M, N) and self._f32_product_takes(x, getattr(w, "w", w))):
-            return PendingProduct(x, w)
+                and not self.separate_norms and self._f32_left(M, N, K) is not None and self._f32_product_takes(x, getattr(w, "w", w))):
+            return PendingProduct(x, w, self._f32_left(M, N, K))
         w_dtype = getattr(matrix, "dtype", None) or matrix.w.dtype
         if x.dtype != w_dtype:
             raise KernelError(f"linear: input is {x.dtype}, the matrix {w_dtype}")
@@ -561,7 +563,8 @@ class HipOps:
 
     def _f32_sums(self, p: PendingProduct):
         """A float32 product of few rows for a reader that also adds the sums of ranges: those, or the product where they cost more."""
-        return self._f32_ranges(p) if self._f32_ranges_pay(p.shape[1], p.x.shape[1]) else self.resolve(p)
+        pays = self._f32_left(*p.shape, p.x.shape[1]) if p.pays is None else p.pays
+        return self._f32_ranges(p) if pays else self.resolve(p)
 
     def _f32_ranges(self, p: PendingProduct) -> DeferredSum:
         """A float32 product of few rows as the sums of its ranges of k, whose sum in order is what ``linear`` gives."""
