@@ -17,11 +17,13 @@
 // load of this kernel, and a fragment's wait carries the fragment's registers through so
 // that its products come after it.
 // (The compiler takes the outputs of these loads as there at once: a launch shape has to fit the vector registers, or it moves
-// fragments to other registers while they are on their way.  tests/test_compiled_loads.py looks at the compiled code for that, and at
-// the counts; a new shape passes it before it runs.)
-// What bounds it: a compute unit takes a load of 1 KiB in 16 clocks, and a wave that waits for its turn issues no products.  44
-// workgroups of 128 x 192 outputs, one a compute unit, a slice of 128: products 0.78 us, loads 0.53 us, together 1.28 to 1.30; read further
-// ahead (x by two slices, W by one, fragments in LDS by three) 1.30 to 1.33.
+// fragments to other registers while they are on their way.  tests/test_compiled_loads.py walks the compiled kernels for that, and for
+// the counts of the waits; a new shape passes it before it runs, and one whose sums then differ from the other shapes' is not run again.)
+// What bounds it is not settled.  256 rows, 4,096 columns of k 12,288 as 44 workgroups of 128 x 192 outputs, one a compute unit: 122 us, 1.28 a
+// slice of 128.  Parts were left out of a trial form only (three slots of x, LDS fragments read three ahead, one workgroup a compute unit), us:
+// there 125 whole, 94 without the loads of W, 88 without the copies of x, 75 without both, 125 without the LDS reads; on the whole chip (2,048 rows, 24,576
+// columns of k 4,096, 128 x 512 outputs) 332, 265, 308, 252 and 287.  So loads and copies hide behind each other in part.  (Without its LDS reads
+// the form multiplies no random numbers any more, which alone is faster on the whole chip: its power sets the clock.)
 // (The same kernel on v_mfma_f32_32x32x16_bf16, its W operands put together from pairs of
 // these fragments by v_permlane16_swap and v_permlane32_swap, was measured 7% slower.)
 //
